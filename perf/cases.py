@@ -11,7 +11,7 @@ options of the same ranges.
 
 Model states are the framework's own new starts (model.build_box) of the two decks in
 geoflac_amd/configs on meshes of other sizes.  The host state of a mesh is built once
-per process; a seed then gives each model its own cohesion factors, geotherm noise,
+per process; a seed then gives each model its own cohesion factors, thermal anomaly,
 friction, and pulling velocity.
 """
 import functools
@@ -122,7 +122,10 @@ def _new_model(deck, nelx, nelz, option, precision, rng):
     gp, st = type(gp0).from_buffer_copy(gp0), st0.copy()
     ez, ex = nelz, nelx
     st.coh_scale = np.asfortranarray((1.0 + 0.01 * rng.uniform(-1.0, 1.0, size=(ez, ex))).astype(np.float32))
-    st.temp[1:-1, :] += rng.uniform(-0.5, 0.5, size=(nelz - 1, nelx + 1))
+    # a smooth thermal anomaly of some kelvin between the fixed surface and base
+    x, z = np.linspace(0.0, math.pi, nelx + 1)[None, :], np.linspace(0.0, math.pi, nelz + 1)[:, None]
+    for k in (1, 2, 3, 5):
+        st.temp[1:-1, :] += (rng.uniform(-10.0, 10.0) / k * np.cos(k * x + rng.uniform(0.0, 3.0)) * np.sin(k * z))[1:-1]
     st.temp0[...] = st.temp
     f = 1.0 + 0.1 * float(rng.uniform(-1.0, 1.0))
     st.bc *= f

@@ -53,10 +53,11 @@ def alg_bytes(kernel, E, N, nact, p, area_frac=0.0, mixfrac=1.0):
         per_n = 16 + 16                                                # vel, cord
         # with the move's areas pending: no dvol read, area and dvol written
         return E * (per_e + 32 * area_frac) + N * per_n
-    if kernel in ("k_therm_tile", "k_therm_pipe"):
-        return N * (8 + 8 + 8 + 16) + E * (16 + 4 + 8)                # temp, temp0 out, x out, cord | area(1:2) iphase source
-    if kernel in ("k_therm_tile_extra", "k_therm_pipe_extra"):
-        return N * (8 + 8 + 8 + 16) + E * (16 + 4 + 8)                # temp0, x in, x out, cord | area(1:2) iphase source
+    if kernel == "k_therm_strip":
+        # temp, temp0 (the extrapolated start), result, cord | iphase source (areas from the coordinates)
+        return N * (8 + 8 + 8 + 16) + E * (4 + 8)
+    if kernel == "k_therm_strip_extra":
+        return N * (8 + 8 + 8 + 16) + E * (4 + 8)                      # temp, x in, x out, cord | iphase source
     if kernel == "k_node":
         return E * (96 + 32) + N * (16 + 16 + 16 + 8 + 16 + 16 + 16)  # stress0(1:3) area | cord rmass+amass vel ncod bc, vel+force out
     if kernel == "k_node_t":  # the step's fl_node also writes the moved coordinates
@@ -82,19 +83,8 @@ def alg_bytes(kernel, E, N, nact, p, area_frac=0.0, mixfrac=1.0):
         return E * (8 + 4) + N * 32                                    # visn iphase | cord vel
     if kernel == "k_move_cord":
         return N * 48
-    if kernel == "k_therm_bc":  # the boundary conditions, copied to temp
-        return N * 16
-    if kernel == "k_therm_tail":
-        # the boundary conditions in place on the boundary nodes of the result, which
-        # becomes temp (a fallback pass inside k_therm_tail is added where it ran)
-        return (2 * p.nx + 2 * p.nz) * 16
     if kernel == "k_area_check":
         return N * 16                                                  # cord (the move's negative-area test)
-    if kernel == "k_therm_check":
-        # the border check: 78 border values of each 64x16-node tile (54x12 outputs)
-        # against the assembled iterate; fallback passes are added where they ran
-        ntiles = -(-p.nz // 54) * -(-p.nx // 12)
-        return ntiles * 78 * 16
     return 0
 
 
@@ -457,9 +447,9 @@ def main():
     n0 = m.state.clock.nloop
     m.step(args.profile_steps)
     afrac = area_pending_fraction(gp, n0, args.profile_steps)
-    kernels = ["k_rheol1<false>", "k_rheol1<true>", "k_rheol", "k_visc<double>", "k_therm_pipe",
-               "k_therm_pipe_extra", "k_therm_check", "k_node<0>", "k_node_t<0>", "k_move_elem<0>",
-               "k_move_area", "k_move_rot<0>", "k_move_cord<double>", "k_therm_bc", "k_therm_tail", "k_dens<double>", "k_rmass", "k_dt_reduce<double>", "k_amass", "k_masses",
+    kernels = ["k_rheol1<false>", "k_rheol1<true>", "k_rheol", "k_visc<double>", "k_therm_strip",
+               "k_therm_strip_extra", "k_therm_check", "k_node<0>", "k_node_t<0>", "k_move_elem<0>",
+               "k_move_area", "k_move_rot<0>", "k_move_cord<double>", "k_therm_rest", "k_dens<double>", "k_rmass", "k_dt_reduce<double>", "k_amass", "k_masses",
                "k_area_check", "k_clock"]
     times = {k: m.kernel_time(k) for k in kernels}
     m.set_timing(False)
@@ -469,12 +459,11 @@ def main():
     nact = int((host_state.phase_ratio >= 0.01).any(axis=(1, 2)).sum())
     mixfrac = float((host_state.phase_ratio.max(axis=0) < 1.0).mean())  # elements of more than one phase
     ab = alg_bytes(dom, E, N, nact, gp, afrac, mixfrac)
-    # a fallback pass and its check count only where the pass ran (the launches after a
-    # proven pass exit at once)
+    # a further thermal pass counts only where it ran (k_therm_rest exits at once after a
+    # proven pass)
     step_bytes = sum(alg_bytes(k, E, N, nact, gp, afrac, mixfrac) * v[1] for k, v in times.items()
-                     if k not in ("k_therm_pipe_extra", "k_therm_check"))
-    step_bytes += alg_bytes("k_therm_pipe_extra", E, N, nact, gp) * th[1]
-    step_bytes += alg_bytes("k_therm_check", E, N, nact, gp) * (args.profile_steps + th[1])
+                     if k != "k_therm_strip_extra")
+    step_bytes += alg_bytes("k_therm_strip_extra", E, N, nact, gp) * th[1]
     step_bytes //= args.profile_steps
     step_ms = sum(v[0] for v in times.values()) / args.profile_steps
     avg_s = ms_tot / 1e3 / max(nl, 1)

@@ -47,6 +47,7 @@ struct GfDevParams {
     double t_top, t_bot, bot_bc, g, demf, ten_off, tau_heal, v_min, v_max;
     double frac, fracm, strain_inert, dt_scale, xReyn, vbc, rxbo, rzbo, pisos, drosub;
     double vbc_over_rxbo;
+    double diff_max;     // largest thermal diffusivity of the phases
     double topo_kappa;   // surface diffusion (src/fl_move.f90:40), 0: none
     GfPhase ph[GF_MAXPH];
 };

@@ -18,7 +18,8 @@ struct GfDevArrays {
     int *iphase;
     double *pr;           // phase ratio planes of the active phases: pr[a*ne + e]
     double *xa, *xb;      // thermal fixed-point iterates (pass p writes xa if p is even)
-    double *tbord;        // thermal tiles' border values
+    double *tbord;        // thermal strips' (tiles') border values
+    double *tpre;         // GF_NPRE slots: boundary rows and columns before the boundary conditions
     double *dens;         // per-element density scratch (rmasses)
     // Mixed precision: velocity and force in FP32, and the stress as an FP32 deviation
     // from a per-element isotropic reference -pref*I kept in FP64 (the element's mean
@@ -98,10 +99,11 @@ template <> GF_DEV float *sv_ptr<float>(double *d, float *f) { return f; }
 // Kernels indexed this way are launched with GF_BLOCK threads per workgroup (a
 // compile-time constant: reading blockDim.x costs a memory round trip per wave).
 #define GF_BLOCK 256
-GF_DEV long xcd_lin()
+// skip: workgroups at the start of the launch that do something else (a multiple of 8)
+GF_DEV long xcd_lin(unsigned skip = 0)
 {
-    const unsigned q = gridDim.x / 8;
-    return (long)((blockIdx.x % 8) * q + blockIdx.x / 8) * GF_BLOCK + threadIdx.x;
+    const unsigned q = (gridDim.x - skip) / 8, b = blockIdx.x - skip;
+    return (long)((b % 8) * q + b / 8) * GF_BLOCK + threadIdx.x;
 }
 __global__ void k_copy(double *__restrict__ dst, const double *__restrict__ src, long n)
 {
@@ -582,20 +584,6 @@ GF_DEV void therm_tile_one(const GfDevParams *__restrict__ P, GfDevClock *ck, co
 #undef LIDX
 }
 
-// pass 0 runs one workgroup per tile; later passes, which are rarely needed, run a
-// smaller grid that loops (so that a pass that is not needed costs little)
-__global__ void __launch_bounds__(1024) k_therm_tile(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                     int pass)
-{
-    if (pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) return;  // already proven
-    const int ntiles = therm_ntj(P) * therm_nti(P);
-    const int nwg = 8 * ((ntiles + 7) / 8);
-    for (int wg = blockIdx.x; wg < nwg; wg += gridDim.x) {
-        const int tile = xcd_tile(wg, ntiles);
-        if (tile >= 0) therm_tile_one(P, ck, A, pass, tile);
-    }
-}
-
 // ---------------------------------------------------------------- pipelined thermal tiles
 // The single-model step runs the tiles above with one workgroup per CU walking a
 // list of tiles.  A tile's inputs are needed only while its coefficients are built;
@@ -970,8 +958,9 @@ GF_DEV void therm_tile_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, c
 template <int XIN, bool DIS>
 // arp: the element areas of the last move are pending (formed from the coordinates)
 __global__ void __launch_bounds__(1024) k_therm_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                     int pass, double stol, int arp, int wt0)
+                                                     int pass, double stol, int arp, int wt0, int ops)
 {
+    if (ops && blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
     if (pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) return;  // already proven
     __shared__ ThermRaw raw;
     __shared__ double sU[TH_NF * TH_NE];
@@ -1035,15 +1024,6 @@ GF_DEV void therm_check_body(const GfDevParams *__restrict__ P, GfDevClock *ck, 
     atomicAdd(&ck->therm_mismatch, 1ull);  // (statistics)
     atomicMax(&ck->therm_mismatch_ulp, (unsigned long long)(a > b ? a - b : b - a));
     if (bad) atomicOr(&ck->therm_pass_changed[pass], 1u);
-}
-
-// (grid-stride: a launch for a fallback pass may use fewer workgroups than entries)
-__global__ void __launch_bounds__(256) k_therm_check(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                     int pass, int arp, long total)
-{
-    if (pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) return;  // that pass did not run
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (long)gridDim.x * blockDim.x)
-        therm_check_body(P, ck, A, pass, t, arp);
 }
 
 // Boundary conditions src/fl_therm.f90:575-598 applied to the proven iterate.
@@ -1139,12 +1119,6 @@ GF_DEV void therm_bc_body(const GfDevParams *__restrict__ P, GfDevClock *ck, con
     therm_bc_apply(P, ck, A, t, passes, proof, proven);
 }
 
-__global__ void __launch_bounds__(256) k_therm_bc(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                  int passes, int proof)
-{
-    therm_bc_body(P, ck, A, xcd_lin(), passes, proof);
-}
-
 // Grid-wide barrier of a launch whose workgroups are all resident.  Every wave
 // waits for its own memory operations; thread 0 then publishes the workgroup's writes
 // (agent-scope release), counts in, waits for the last workgroup to bump the
@@ -1184,56 +1158,14 @@ GF_DEV bool grid_sync(GfDevClock *ck)
     return s_ok != 0;
 }
 
-// The rest of fl_therm after pass 0 and its border check, in one launch (one
-// workgroup per CU, at most the CUs).  When pass 0 is proven (nearly every step) this is the
-// boundary conditions alone.  Otherwise the fallback passes run here, each over all
-// tiles with the launch's workgroups and followed by its border check, with grid
-// barriers between the phases, until one is proven or TH passes ran; then the
-// boundary conditions.  The same arithmetic as the launch-per-phase sequence
-// (k_therm_pipe, k_therm_check, k_therm_bc).  The flags that decide another pass are
-// read with coherent loads after a barrier, so every workgroup takes the same
-// decision; flag 0 was written by earlier launches.  rot: the result becomes the new
-// temperature in xa (therm_bc_rot) instead of being copied to temp.
-template <bool DIS>
-__global__ void __launch_bounds__(1024) k_therm_tail(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                     double stol, int arp, int npass, int proof, long nchk, int rot)
+// the boundary conditions of FP32-arithmetic mode's single pass, in place
+__global__ void __launch_bounds__(256) k_therm_bc(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A)
 {
-    const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x, nthr = (long)gridDim.x * blockDim.x;
-    int proven = -1;
-    if (!proof || ck->therm_pass_changed[0] == 0u) {
-        proven = 0;
-    } else {
-        __shared__ ThermRaw raw;
-        __shared__ double sU[TH_NF * TH_NE];
-        __shared__ int sFlag[3];
-        const int ntiles = therm_ntj(P) * therm_nti(P);
-        const int q = (ntiles + 7) / 8, x = blockIdx.x % 8, r = blockIdx.x / 8, RW = gridDim.x / 8;
-        const int first = x * q + r, end = min((x + 1) * q, ntiles);
-        for (int pass = 1; pass < npass; pass++) {
-            if (first < end) {
-                therm_store_raw<1, DIS>(therm_prefetch<1, DIS>(P, ck, A, pass, first, arp, 0), raw);
-                for (int t = first; t < end; t += RW) {
-                    lds_barrier();
-                    therm_tile_pipe<1, DIS>(P, ck, A, pass, t, P, ck, A, t + RW < end ? t + RW : -1, raw, sU, sFlag,
-                                            stol, arp, 0);
-                }
-            }
-            if (!grid_sync(ck)) return;  // every tile's iterate is written
-            for (long t = tid; t < nchk; t += nthr) therm_check_body(P, ck, A, pass, t, arp, 0);
-            if (!grid_sync(ck)) return;  // every border is checked
-            if (__hip_atomic_load(&ck->therm_pass_changed[pass], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
-                proven = pass;
-                break;
-            }
-        }
-    }
-    if (rot) {  // the result becomes temp in place (therm_bc_rot)
-        therm_bc_rot(P, ck, A, tid, nthr, npass, proof, proven);
-        return;
-    }
-    const long nn = (long)P->nz * P->nx;
-    for (long t = tid; t < nn; t += nthr) therm_bc_apply(P, ck, A, t, npass, proof, proven);
+    const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    therm_bc_rot(P, ck, A, tid, (long)gridDim.x * blockDim.x, 1, 0, 0);
 }
+
+#include "gf_therm.h"
 
 // ------------------------------------------------------------------ material properties
 // src/matprops.f90:136-215
@@ -2058,27 +1990,39 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
 
 template <bool SHEARH>
 __global__ void __launch_bounds__(256) k_rheol1(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                int avgsr, int rot)
+                                                int avgsr, int rot, ThermChk chk)
 {
-    long e = xcd_lin();
+    if (blockIdx.x < (unsigned)chk.grid) {
+        therm_chk_block(P, ck, A, chk);
+        return;
+    }
+    long e = xcd_lin((unsigned)chk.grid);
     if (e >= NE) return;
     rheol_single<SHEARH, double, double>(P, P->ph, ck, A, e, avgsr, rot);
 }
 // mixed precision: FP32 strain rate and stress
 template <bool SHEARH>
 __global__ void __launch_bounds__(256) k_rheol1m(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                 int avgsr, int rot)
+                                                 int avgsr, int rot, ThermChk chk)
 {
-    long e = xcd_lin();
+    if (blockIdx.x < (unsigned)chk.grid) {
+        therm_chk_block(P, ck, A, chk);
+        return;
+    }
+    long e = xcd_lin((unsigned)chk.grid);
     if (e >= NE) return;
     rheol_single<SHEARH, float, float>(P, P->ph, ck, A, e, avgsr, rot);
 }
 // FP32 storage, FP64 arithmetic
 template <bool SHEARH>
 __global__ void __launch_bounds__(256) k_rheol1s(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                 int avgsr, int rot)
+                                                 int avgsr, int rot, ThermChk chk)
 {
-    long e = xcd_lin();
+    if (blockIdx.x < (unsigned)chk.grid) {
+        therm_chk_block(P, ck, A, chk);
+        return;
+    }
+    long e = xcd_lin((unsigned)chk.grid);
     if (e >= NE) return;
     rheol_single<SHEARH, float, double>(P, P->ph, ck, A, e, avgsr, rot);
 }
@@ -2670,14 +2614,17 @@ GF_DEV void node_tile_update(const GfDevParams *__restrict__ P, GfDevClock *ck, 
 // while computing the current one ran slower: two workgroups per CU instead of three.)
 template <int M, bool MOVE>
 __global__ void __launch_bounds__(256) k_node_t(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                double *cord_out)
+                                                double *cord_out, int ops)
 {
     __shared__ NodeLds<M> L;
     const int ntiles = node_ntj(P) * node_nti(P);
     const int q = (ntiles + 7) / 8, tile = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
     if (tile >= ntiles) return;  // the whole workgroup
     const NodeClk kc = node_clk(ck);
-    if (MOVE && blockIdx.x == 0 && threadIdx.x == 0) ck->dt_move = kc.dt;  // the move's dt (no other reader here)
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (MOVE) ck->dt_move = kc.dt;  // the move's dt (no other reader here)
+        if (ops) clock_op(ck, ops);     // (fields nothing here reads)
+    }
     const NodePf<M> pf = node_prefetch<M>(P, A, tile);
     node_stage<M>(pf, L);
     __syncthreads();

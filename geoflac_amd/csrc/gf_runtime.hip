@@ -96,14 +96,16 @@ struct gf_ctx {
     // passes when needed); 1: FP32-arithmetic mode takes the single tile pass as it is
     int therm_passes = TH_MAXPASS;
     bool therm_proof = true;  // false: FP32-arithmetic mode, the single pass is not proven
-    // Fallback thermal passes launch with few workgroups (they exit at once when the
-    // pass before was proven) unless the last call needed one: then with the full grid
-    bool therm_fb_full = true;
-    // the thermal step's fallback passes and boundary conditions as one launch
-    // (k_therm_tail) instead of a launch per phase (GF_THERM=multi, or a device on which
-    // a workgroup of it does not fit on every CU)
-    bool therm_tail = false;
-    unsigned long long therm_extra_seen = 0;
+    // the thermal step's further passes as one launch (k_therm_rest) instead of a launch
+    // per pass and check (GF_THERM=multi, or a device on which a workgroup of it does not
+    // fit on every CU)
+    bool therm_rest = false;
+    int therm_w = 0;     // output columns of a thermal strip
+    int therm_call = 0;  // thermal calls, modulo 3: the slot of a.tpre this call writes
+    ThermChk chk{};      // the border check of the thermal call under way
+    int node_ops = 0;    // clock updates left to the step's fl_node
+    bool therm_clean = true;  // the flags of the thermal passes are 0 on the device
+    int therm_hist = 0;  // calls before it (at most 2) whose slots hold their boundary values
     // per-kernel event timing
     bool timing = false;
     std::vector<hipEvent_t> ev_pool;
@@ -129,6 +131,37 @@ static int set_err(gf_ctx *c, int code, const char *fmt, ...)
         if (e_ != hipSuccess)                                                                 \
             return set_err(ctx, GF_ERR_HIP, "%s failed: %s", #call, hipGetErrorString(e_));   \
     } while (0)
+
+static ThermGeo therm_geo_host(const gf_params &p, int w)
+{
+    ThermGeo g;
+    g.nz = p.nz;
+    g.nx = p.nx;
+    g.w = w;
+    g.nr = g.nz <= 64 ? 1 : (g.nz - 2 * TS_HB + TS_OJ - 1) / TS_OJ;
+    g.ns = (g.nx + w - 1) / w;
+    return g;
+}
+// Output columns of a thermal strip.  A strip of w columns takes some w + 6 column times
+// (halo, ring, start); a column takes a wave alone on its SIMD 1.3 us (latency), n waves
+// 0.6 us more each, 0.9 us each where issue bounds.  The width of least time over the
+// 1024 SIMDs.  Measured, us a step (whole step) at widths 2, 4, 8, 16, 24: 401x101 nodes
+// 38, 41, 47, 59, 70; 902x302 101, 97, 102, 110, 121; 2001x1001 541, 508, 492, 493, 497.
+static int therm_strip_width(const gf_params &p)
+{
+    int best = 2;
+    double least = 1e300;
+    for (int w = 2; w <= 32; w++) {
+        const ThermGeo g = therm_geo_host(p, w);
+        const double n = (double)g.nr * g.ns / 1024.0;
+        const double col = n <= 1.0 ? 1.3 : std::max(1.3 + 0.6 * (n - 1.0), 0.9 * n);
+        if ((w + 6) * col < least) {
+            least = (w + 6) * col;
+            best = w;
+        }
+    }
+    return best;
+}
 
 // workgroups of 256 for n threads, rounded up to a multiple of the 8 XCDs (kernels
 // renumber workgroups per XCD and return for indices past n)
@@ -163,6 +196,7 @@ static int build_dev_params(gf_ctx *ctx)
     d.xReyn = p.xReyn; d.vbc = p.vbc; d.rxbo = p.rxbo; d.rzbo = p.rzbo; d.pisos = p.pisos; d.drosub = p.drosub;
     d.vbc_over_rxbo = p.vbc / p.rxbo;
     d.topo_kappa = p.topo_kappa;
+    d.diff_max = 0.0;
     for (int k = 0; k < GF_MAXPH; k++) {
         GfPhase &ph = d.ph[k];
         ph.irheol = p.irheol[k];
@@ -185,6 +219,7 @@ static int build_dev_params(gf_ctx *ctx)
             ph.pln_r = p.pln[k] * 8.31448;                      // src/matprops.f90:160,195
         }
         if (p.den[k] != 0.0 && p.cp[k] != 0.0) ph.diff = p.conduct[k] / p.den[k] / p.cp[k];
+        if (k < p.nphase && ph.diff > d.diff_max) d.diff_max = ph.diff;
         // pre_plast (src/rh_plastic.f90:249-284) of a one-phase element at aps = 0
         {
             const double aps0 = 0.0;
@@ -293,9 +328,9 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
         ctx->therm_grid = (unsigned)std::max(8, ncu / 8 * 8);
         int nb = 0;
         const char *tm = getenv("GF_THERM");
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_therm_tail<true>, TH_J * TH_I, 0) != hipSuccess)
-            nb = 0;
-        ctx->therm_tail = nb >= 1 && ncu >= 8 && !(tm && strcmp(tm, "multi") == 0);
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_therm_rest<true>, 256, 0) != hipSuccess) nb = 0;
+        ctx->therm_rest = nb >= 1 && ncu >= 8 && !(tm && strcmp(tm, "multi") == 0);
+        ctx->therm_w = therm_strip_width(*p);
         (void)hipGetLastError();
     }
     ALLOC(ctx->dp, sizeof(GfDevParams));
@@ -333,8 +368,14 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
     ALLOC(ctx->a.pr, 8 * ne * GF_MAXACT);
     ALLOC(ctx->a.xa, 8 * nn);
     ALLOC(ctx->a.xb, 8 * nn);
-    ALLOC(ctx->therm_border, 8 * (size_t)TH_NB * ((p->nz + TH_OJ - 1) / TH_OJ) * ((p->nx + TH_OI - 1) / TH_OI));
+    {
+        const ThermGeo g = therm_geo_host(*p, ctx->therm_w);
+        const size_t nb = (size_t)g.nr * g.ns * TS_NB(g.w),
+                     nt = (size_t)TH_NB * ((p->nz + TH_OJ - 1) / TH_OJ) * ((p->nx + TH_OI - 1) / TH_OI);
+        ALLOC(ctx->therm_border, 8 * std::max(nb, nt));
+    }
     ctx->a.tbord = ctx->therm_border;
+    ALLOC(ctx->a.tpre, 8 * (size_t)GF_NPRE * 2 * (p->nx + p->nz));
     ALLOC(ctx->a.dens, 8 * ne);
     ALLOC(ctx->a.iphx, 4 * ne);
     if (hipMemset(ctx->a.iphx, 0, 4 * ne) != hipSuccess) {
@@ -381,7 +422,7 @@ extern "C" void gf_destroy(gf_ctx *ctx)
                     ctx->a.force, ctx->a.amass, ctx->a.rmass, ctx->a.bc, ctx->a.ncod, ctx->a.stress0,
                     ctx->a.area, ctx->a.dvol, ctx->a.strain, ctx->a.se2sr, ctx->a.aps, ctx->a.visn,
                     ctx->a.e2sr, ctx->a.sshrheat, ctx->a.shrheat, ctx->a.source, ctx->a.iphase, ctx->a.pr,
-                    ctx->a.xa, ctx->a.xb, ctx->a.dens, ctx->therm_border, ctx->a.stress0f, ctx->a.velf,
+                    ctx->a.xa, ctx->a.xb, ctx->a.dens, ctx->therm_border, ctx->a.tpre, ctx->a.stress0f, ctx->a.velf,
                     ctx->a.forcef, ctx->a.pref, ctx->sur_samples, ctx->sur_w, ctx->sur_m, ctx->sur_v,
                     ctx->sur_grad, ctx->sur_partial, ctx->sur_cfg, ctx->sur_stats, ctx->sur_list,
                     ctx->sur_cnt, ctx->sur_lval, ctx->sur_wgs, ctx->cord_alt, ctx->out_buf, ctx->a.mark_age,
@@ -744,6 +785,12 @@ static int upload_iphase_present(gf_ctx *ctx)
 }
 
 static int flush_rot(gf_ctx *ctx);
+// the next thermal call starts from the old temperature alone
+static void therm_forget(gf_ctx *ctx)
+{
+    ctx->temp0_prev = false;
+    ctx->therm_hist = 0;
+}
 
 extern "C" int gf_upload(gf_ctx *ctx, uint32_t mask)
 {
@@ -751,7 +798,7 @@ extern "C" int gf_upload(gf_ctx *ctx, uint32_t mask)
     if (!ctx->bound) return set_err(ctx, GF_ERR_STATE, "gf_upload before gf_bind_host");
     int frc = flush_rot(ctx);  // the upload overwrites the moved state
     if (frc) return frc;
-    ctx->temp0_prev = false;  // temp and temp0 may no longer be consecutive steps
+    therm_forget(ctx);  // temp and temp0 may no longer be consecutive steps
     HIPCHK(hipStreamSynchronize(ctx->stream));
     for (const FieldDesc &f : kFields) {
         if (!(mask & f.bit)) continue;
@@ -1008,10 +1055,6 @@ static int fetch_clock(gf_ctx *ctx, gf_clock *c)
     GfDevClock ck;
     HIPCHK(hipStreamSynchronize(ctx->stream));
     HIPCHK(hipMemcpy(&ck, ctx->dck, sizeof(ck), hipMemcpyDeviceToHost));
-    // the last call's fallback passes decide the grid of the next call's fallback launches
-    if (ck.therm_extra_passes < ctx->therm_extra_seen) ctx->therm_extra_seen = 0;  // (statistics were reset)
-    ctx->therm_fb_full = ck.therm_extra_passes > ctx->therm_extra_seen;
-    ctx->therm_extra_seen = ck.therm_extra_passes;
     if (ctx->markers_uploaded && ctx->p.topo_kappa > 0.0) ctx->a.nmarkers = ck.nmarkers;  // (resurface appends)
     if (ck.bar_timeout != 0) {  // (not expected: every workgroup of the launch is resident)
         GfDevClock z = ck;
@@ -1035,6 +1078,7 @@ static int fetch_clock(gf_ctx *ctx, gf_clock *c)
         z.error_code = 0;
         z.error_index = (long long)1 << 62;
         HIPCHK(hipMemcpy(ctx->dck, &z, sizeof(z), hipMemcpyHostToDevice));
+        if (ck.error_code == GF_ERR_THERM_SWEEPS) therm_forget(ctx);  // (its result is not known to be the serial one)
         return set_err(ctx, ck.error_code, "reference STOP %d at element (j,i)=(%d,%d)", ck.error_code,
                        ctx->err_j, ctx->err_i);
     }
@@ -1083,7 +1127,8 @@ static int collect_timing(gf_ctx *ctx)
 }
 
 #define LAUNCH(kern, n, ...) LAUNCH_NAMED(#kern, kern, n, __VA_ARGS__)
-#define LAUNCH_NAMED(name, kern, n, ...)                                                   \
+#define LAUNCH_NAMED(name, kern, n, ...) LAUNCH_DIM(name, kern, nblk(n), 256, __VA_ARGS__)
+#define LAUNCH_DIM(name, kern, grid, block, ...)                                           \
     do {                                                                                   \
         hipEvent_t e0_ = nullptr, e1_ = nullptr;                                           \
         if (ctx->timing) {                                                                 \
@@ -1091,7 +1136,7 @@ static int collect_timing(gf_ctx *ctx)
             e1_ = next_event(ctx);                                                         \
             if (e0_) (void)hipEventRecord(e0_, ctx->stream);                               \
         }                                                                                  \
-        hipLaunchKernelGGL(kern, dim3(nblk(n)), dim3(256), 0, ctx->stream, __VA_ARGS__);   \
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, ctx->stream, __VA_ARGS__);    \
         int rc_ = launch_check(ctx, name);                                                 \
         if (rc_) return rc_;                                                               \
         if (ctx->timing && e0_ && e1_) {                                                   \
@@ -1152,84 +1197,85 @@ static int flush_rot(gf_ctx *ctx)
 // stop sweeping once no node changes by more than this many kelvin (the GS iteration
 // contracts geometrically, so the remaining error is of this order)
 #define GF_THERM_STOL 1.0e-9
-static int enq_therm(gf_ctx *ctx, bool clock_done = false)
+// ops: clock updates for the first kernel of the call to make (or a launch of their own);
+// defer: the border check of pass 0 goes into the launch of fl_rheol (ctx->chk), after
+// which enq_therm_rest ends the call
+static int enq_therm_rest(gf_ctx *ctx);
+static int enq_therm(gf_ctx *ctx, int ops = 0, bool defer = false)
 {
     int rc;
-    if (!clock_done && (rc = enq_clock(ctx, CK_THERM_BEGIN))) return rc;
-    const int ntiles = ((ctx->p.nz + TH_OJ - 1) / TH_OJ) * ((ctx->p.nx + TH_OI - 1) / TH_OI);
-    const int npass = ctx->therm_passes;
-    // The single-model call turns three buffers over instead of copying: the old
-    // temperature (temp) is read, temp0 holds the previous call's starting temperature
-    // (the extrapolated start), and the result is formed in xa; then xa becomes temp,
-    // temp becomes temp0 (src/fl_therm.f90:52) and temp0 the next call's xa.  Not while
-    // a batch holds the context's array pointers (in_batch), and not in the
-    // launch-per-phase sequence.
-    const bool rot = ctx->therm_tail && ctx->in_batch == 0 && ctx->p.nz >= 3 && ctx->p.nx >= 3;
-    for (int pass = 0; pass < (ctx->therm_tail ? 1 : npass); pass++) {
-        const dim3 grid(pass == 0 || ctx->therm_fb_full ? ctx->therm_grid : 32u);
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        if (ctx->timing) {
-            e0 = next_event(ctx);
-            e1 = next_event(ctx);
-            if (e0) (void)hipEventRecord(e0, ctx->stream);
-        }
-        const bool dis = ctx->p.ishearh == 1 && ctx->p.itherm != 2;
-        // pass 0 starts from the extrapolation 2 temp - temp0 once temp0 holds the
-        // previous step's starting temperature.  A tile reads temp0 of its halo, which
-        // the neighbouring tiles overwrite with this step's value as they go: the
-        // start then depends on the order the tiles run in, which only the proven
-        // passes are free of (their fixed point is exact), so the unproven single pass
-        // of FP32-arithmetic mode starts from the old temperature.
-        const bool ex = ctx->temp0_prev && !ctx->therm_noguess && ctx->therm_proof;
-        auto kern = pass > 0 ? (dis ? k_therm_pipe<1, true> : k_therm_pipe<1, false>)
-                    : ex     ? (dis ? k_therm_pipe<2, true> : k_therm_pipe<2, false>)
-                             : (dis ? k_therm_pipe<0, true> : k_therm_pipe<0, false>);
-        hipLaunchKernelGGL(kern, grid, dim3(TH_J * TH_I), 0, ctx->stream, ctx->dp, ctx->dck, ctx->a, pass,
-                           ctx->therm_proof ? 0.0 : GF_THERM_STOL, ctx->area_pending ? 1 : 0, rot ? 0 : 1);
-        if ((rc = launch_check(ctx, "k_therm_pipe"))) return rc;
-        if (ctx->timing && e0 && e1) {
-            (void)hipEventRecord(e1, ctx->stream);
-            ctx->pending.push_back({pass == 0 ? "k_therm_pipe" : "k_therm_pipe_extra", {e0, e1}});
-        }
-        if (ctx->therm_proof) {
-            const long nchk = (long)ntiles * TH_NB;
-            LAUNCH(k_therm_check, pass == 0 || ctx->therm_fb_full ? nchk : 64L * 256, ctx->dp, ctx->dck, ctx->a, pass,
-                   ctx->area_pending ? 1 : 0, nchk);
-        }
+    // the flags of the passes start at 0: the last step's fl_node cleared them, or this
+    if (!ctx->therm_clean && (rc = enq_clock(ctx, CK_THERM_BEGIN))) return rc;
+    ctx->therm_clean = false;
+    const bool dis = ctx->p.ishearh == 1 && ctx->p.itherm != 2;
+    const int arp = ctx->area_pending ? 1 : 0;
+    if (!ctx->therm_proof) {
+        // FP32-arithmetic mode: one tile pass, whose result (which depends on the sweeps
+        // it made) is taken as it is, then the boundary conditions
+        auto kern = dis ? k_therm_pipe<0, true> : k_therm_pipe<0, false>;
+        LAUNCH_DIM("k_therm_pipe", kern, ctx->therm_grid, TH_J * TH_I, ctx->dp, ctx->dck, ctx->a, 0, GF_THERM_STOL,
+                   arp, 0, ops);
+        LAUNCH(k_therm_bc, 2L * (ctx->p.nx + ctx->p.nz), ctx->dp, ctx->dck, ctx->a);
+        return enq_therm_rest(ctx);
     }
-    if (ctx->therm_tail) {
+    const ThermGeo g = therm_geo_host(ctx->p, ctx->therm_w);
+    const unsigned grid = 8u * (unsigned)((g.nr * g.ns + 7) / 8);
+    const long nb = (long)g.nr * g.ns * TS_NB(g.w);
+    ctx->chk = ThermChk{(int)nblk(nb), g.w, arp, therm_slots(ctx->therm_call, ctx->therm_hist), ctx->a.temp, ctx->a.xa};
+    // pass 0 starts from the extrapolation 2 temp - temp0 once temp0 holds the
+    // previous step's starting temperature
+    const bool ex = ctx->temp0_prev && !ctx->therm_noguess;
+    auto kern = ex ? (dis ? k_therm_strip<true, 2> : k_therm_strip<false, 2>)
+                   : (dis ? k_therm_strip<true, 0> : k_therm_strip<false, 0>);
+    LAUNCH_DIM("k_therm_strip", kern, grid, 64, ctx->dp, ctx->dck, ctx->a, g.w, 0, arp, ctx->chk.sl, ops);
+    if (defer) return GF_OK;
+    LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, g.w, 0, arp, ctx->chk.sl, nb);
+    return enq_therm_rest(ctx);
+}
+
+// the further passes, if pass 0 was not proven, and the end of the call
+static int enq_therm_rest(gf_ctx *ctx)
+{
+    if (ctx->therm_proof) {
         const bool dis = ctx->p.ishearh == 1 && ctx->p.itherm != 2;
-        double stol = ctx->therm_proof ? 0.0 : GF_THERM_STOL;
-        int arp = ctx->area_pending ? 1 : 0, np = npass, proof = ctx->therm_proof ? 1 : 0, irot = rot ? 1 : 0;
-        long nchk = (long)ntiles * TH_NB;
-        void *args[] = {(void *)&ctx->dp, (void *)&ctx->dck, (void *)&ctx->a, &stol, &arp, &np, &proof, &nchk, &irot};
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        if (ctx->timing) {
-            e0 = next_event(ctx);
-            e1 = next_event(ctx);
-            if (e0) (void)hipEventRecord(e0, ctx->stream);
+        const int npass = ctx->therm_passes, w = ctx->chk.w, arp = ctx->chk.arp;
+        const ThermSlots sl = ctx->chk.sl;
+        if (ctx->therm_rest) {
+            // A plain launch: its grid (one workgroup per CU, at most the CUs) is resident
+            // once the kernels before it on this stream are done, unless other streams hold
+            // CUs, whose kernels then finish first.  The grid barriers of the further passes
+            // wait boundedly, so a launch that is not resident reports an error instead of
+            // waiting for ever.  (A cooperative launch guarantees residency but costs
+            // ~16 us more per launch on MI355X, more than the launches it replaces.)
+            auto rest = dis ? k_therm_rest<true> : k_therm_rest<false>;
+            LAUNCH_DIM("k_therm_rest", rest, ctx->therm_grid, 256, ctx->dp, ctx->dck, ctx->a, w, arp, sl, npass);
+        } else {
+            const ThermGeo g = therm_geo_host(ctx->p, w);
+            const unsigned grid = 8u * (unsigned)((g.nr * g.ns + 7) / 8);
+            const long nb = (long)g.nr * g.ns * TS_NB(w);
+            auto extra = dis ? k_therm_strip<true, 1> : k_therm_strip<false, 1>;
+            for (int pass = 1; pass < npass; pass++) {
+                LAUNCH_DIM("k_therm_strip_extra", extra, grid, 64, ctx->dp, ctx->dck, ctx->a, w, pass, arp, sl, 0);
+                LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, w, pass, arp, sl, nb);
+            }
+            LAUNCH_DIM("k_therm_last", k_therm_last, ctx->therm_grid, 256, ctx->dp, ctx->dck, ctx->a, sl, npass);
         }
-        // A plain launch: its grid (one workgroup per CU, at most the CUs) is resident
-        // once the kernels before it on this stream are done, unless other streams hold
-        // CUs, whose kernels then finish first.  The grid barriers of the fallback passes
-        // wait boundedly, so a launch that is not resident reports an error instead of
-        // waiting for ever.  (A cooperative launch guarantees residency but costs
-        // ~16 us more per launch on MI355X, more than the launches it replaces.)
-        const void *kern = dis ? (const void *)k_therm_tail<true> : (const void *)k_therm_tail<false>;
-        hipError_t e = hipLaunchKernel(kern, dim3(ctx->therm_grid), dim3(TH_J * TH_I), args, 0, ctx->stream);
-        if (e != hipSuccess) return set_err(ctx, GF_ERR_HIP, "launch of k_therm_tail failed: %s", hipGetErrorString(e));
-        if (ctx->timing && e0 && e1) {
-            (void)hipEventRecord(e1, ctx->stream);
-            ctx->pending.push_back({"k_therm_tail", {e0, e1}});
-        }
-    } else {
-        LAUNCH(k_therm_bc, ctx->nn, ctx->dp, ctx->dck, ctx->a, npass, ctx->therm_proof ? 1 : 0);
+        ctx->therm_call = (ctx->therm_call + 1) % 3;
+        ctx->therm_hist = std::min(ctx->therm_hist + 1, 2);
+        ctx->chk.grid = 0;
     }
-    if (rot) {
+    // Three buffers turn over instead of the result being copied: the old temperature
+    // (temp) is read, temp0 holds the previous call's starting temperature (the
+    // extrapolated start), and the result is formed in xa; then xa becomes temp, temp
+    // becomes temp0 (src/fl_therm.f90:52) and temp0 the next call's xa.  Not while a
+    // batch holds the context's array pointers.
+    if (ctx->in_batch == 0) {
         double *t = ctx->a.temp;
         ctx->a.temp = ctx->a.xa;
         ctx->a.xa = ctx->a.temp0;
         ctx->a.temp0 = t;
+    } else {
+        LAUNCH(k_therm_copy, ctx->nn, ctx->dp, ctx->a);
     }
     ctx->temp0_prev = true;  // temp0 holds this call's starting temperature at every node
     return GF_OK;
@@ -1281,22 +1327,32 @@ static int enq_rheol(gf_ctx *ctx, bool clock_done = false, bool last = true)
         else if (mstore) LAUNCH_NAMED("k_visc<float>", k_visc<2>, ctx->ne, ctx->dp, ctx->dck, ctx->a, vr);
         else LAUNCH_NAMED("k_visc<double>", k_visc<0>, ctx->ne, ctx->dp, ctx->dck, ctx->a, vr);
     }
+    // (a thermal border check that was left to this launch runs in its first workgroups)
+    const ThermChk chk = ctx->chk;
+    const unsigned grid = nblk(ctx->ne) + (unsigned)chk.grid;
+#define RHEOL_LAUNCH(K) \
+    LAUNCH_DIM(#K, K, grid, 256, ctx->dp, ctx->dck, ctx->a, avgsr, rot, chk)
     if (ctx->rheol_quad && !mixed && !mstore)
         LAUNCH(k_rheol, 4 * ctx->ne, ctx->dp, ctx->dck, ctx->a, avgsr);
     else if (mstore && ctx->p.ishearh == 1)
-        LAUNCH(k_rheol1s<true>, ctx->ne, ctx->dp, ctx->dck, ctx->a, avgsr, rot);
+        RHEOL_LAUNCH(k_rheol1s<true>);
     else if (mstore)
-        LAUNCH(k_rheol1s<false>, ctx->ne, ctx->dp, ctx->dck, ctx->a, avgsr, rot);
+        RHEOL_LAUNCH(k_rheol1s<false>);
     else if (mixed && ctx->p.ishearh == 1)
-        LAUNCH(k_rheol1m<true>, ctx->ne, ctx->dp, ctx->dck, ctx->a, avgsr, rot);
+        RHEOL_LAUNCH(k_rheol1m<true>);
     else if (mixed)
-        LAUNCH(k_rheol1m<false>, ctx->ne, ctx->dp, ctx->dck, ctx->a, avgsr, rot);
+        RHEOL_LAUNCH(k_rheol1m<false>);
     else if (ctx->p.ishearh == 1)
-        LAUNCH(k_rheol1<true>, ctx->ne, ctx->dp, ctx->dck, ctx->a, avgsr, rot);
+        RHEOL_LAUNCH(k_rheol1<true>);
     else
-        LAUNCH(k_rheol1<false>, ctx->ne, ctx->dp, ctx->dck, ctx->a, avgsr, rot);
+        RHEOL_LAUNCH(k_rheol1<false>);
+#undef RHEOL_LAUNCH
     if (avgsr == 1) {
-        if ((rc = enq_clock(ctx, CK_DTAVG_RESET))) return rc;
+        // (the step's fl_node resets it)
+        if (clock_done && !ctx->node_direct)
+            ctx->node_ops |= CK_DTAVG_RESET;
+        else if ((rc = enq_clock(ctx, CK_DTAVG_RESET)))
+            return rc;
         ctx->nsrate = 0;
     }
     ctx->nsrate = ctx->nsrate + 1;
@@ -1318,13 +1374,19 @@ static int enq_node(gf_ctx *ctx, bool move)
     const bool fuse = move && ctx->p.movegrid != 0 && ctx->in_batch == 0;
     const int M = ctx->precision == GF_PREC_MIXED ? 1 : ctx->precision == GF_PREC_MIXED_STORAGE ? 2 : 0;
     double *out = fuse ? ctx->cord_alt : nullptr;
+    // in the step also the clock updates that no kernel up to here could make
+    const int ops = move ? ctx->node_ops | CK_THERM_BEGIN : 0;
+    if (move) {
+        ctx->node_ops = 0;
+        ctx->therm_clean = true;
+    }
     // (timed under one name per precision, with or without the move)
-    if (M == 1 && fuse) LAUNCH_NAMED("k_node_t<1>", (k_node_t<1, true>), n, ctx->dp, ctx->dck, ctx->a, out);
-    else if (M == 1) LAUNCH_NAMED("k_node_t<1>", (k_node_t<1, false>), n, ctx->dp, ctx->dck, ctx->a, out);
-    else if (M == 2 && fuse) LAUNCH_NAMED("k_node_t<2>", (k_node_t<2, true>), n, ctx->dp, ctx->dck, ctx->a, out);
-    else if (M == 2) LAUNCH_NAMED("k_node_t<2>", (k_node_t<2, false>), n, ctx->dp, ctx->dck, ctx->a, out);
-    else if (fuse) LAUNCH_NAMED("k_node_t<0>", (k_node_t<0, true>), n, ctx->dp, ctx->dck, ctx->a, out);
-    else LAUNCH_NAMED("k_node_t<0>", (k_node_t<0, false>), n, ctx->dp, ctx->dck, ctx->a, out);
+    if (M == 1 && fuse) LAUNCH_NAMED("k_node_t<1>", (k_node_t<1, true>), n, ctx->dp, ctx->dck, ctx->a, out, ops);
+    else if (M == 1) LAUNCH_NAMED("k_node_t<1>", (k_node_t<1, false>), n, ctx->dp, ctx->dck, ctx->a, out, ops);
+    else if (M == 2 && fuse) LAUNCH_NAMED("k_node_t<2>", (k_node_t<2, true>), n, ctx->dp, ctx->dck, ctx->a, out, ops);
+    else if (M == 2) LAUNCH_NAMED("k_node_t<2>", (k_node_t<2, false>), n, ctx->dp, ctx->dck, ctx->a, out, ops);
+    else if (fuse) LAUNCH_NAMED("k_node_t<0>", (k_node_t<0, true>), n, ctx->dp, ctx->dck, ctx->a, out, ops);
+    else LAUNCH_NAMED("k_node_t<0>", (k_node_t<0, false>), n, ctx->dp, ctx->dck, ctx->a, out, ops);
     if (fuse) {
         std::swap(ctx->a.cord, ctx->cord_alt);
         ctx->cord_moved = true;
@@ -1509,12 +1571,18 @@ static int enq_flac(gf_ctx *ctx, int pending = 0, bool last = true)
 {
     int rc;
     const bool mech = ctx->p.itherm != 2;
-    // fl_therm's and fl_rheol's clock updates in one launch (neither touches dt)
-    if ((rc = enq_clock(ctx, pending | CK_THERM_BEGIN | (mech ? CK_DTAVG_ADD : 0)))) return rc;
-    if ((rc = enq_therm(ctx, true))) return rc;
+    const bool phases = ctx->nloop % ctx->p.ifreq_rmasses == 0;
+    // fl_rheol's launch also checks the thermal step's borders where nothing up to it
+    // reads the temperature (change_phase, Eff_visc, thermal stresses) or writes what the
+    // check reads (the shear heating)
+    const bool defer = mech && ctx->therm_proof && !phases && ctx->nloop % ctx->p.ifreq_visc != 0 &&
+                       ctx->p.istress_therm == 0 && ctx->p.ishearh != 1 && !ctx->rheol_quad;
+    // the thermal kernel makes its own and fl_rheol's clock updates (it reads only dt)
+    if ((rc = enq_therm(ctx, pending | (mech ? CK_DTAVG_ADD : 0), defer))) return rc;
     if (mech) {
-        if (ctx->nloop % ctx->p.ifreq_rmasses == 0 && (rc = enq_change_phase(ctx))) return rc;
+        if (phases && (rc = enq_change_phase(ctx))) return rc;
         if ((rc = enq_rheol(ctx, true, last))) return rc;
+        if (defer && (rc = enq_therm_rest(ctx))) return rc;
         if (ctx->p.nystressbc == 1 && (rc = enq_bc_update(ctx))) return rc;
         if ((rc = enq_node(ctx, true))) return rc;
         if ((rc = enq_move(ctx))) return rc;
@@ -2710,6 +2778,8 @@ extern "C" int gf_batch_step(gf_batch *b, int32_t nsteps)
         c->rot_pending = b->rot_pending;  // completed by the model's own k_move_rot where needed
         c->area_pending = b->area_pending;
         c->temp0_prev = b->temp0_prev;
+        c->therm_hist = 0;  // (the batch keeps no boundary values)
+        c->therm_clean = false;
         int r = fetch_clock(c, nullptr);
         if (r && first == GF_OK) first = r;
     }

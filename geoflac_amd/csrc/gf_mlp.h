@@ -8,8 +8,8 @@
 //  * Samples come from the solver itself: k_visc_sample evaluates the features and
 //    the exact formula for every element of the current state.
 //  * Training runs on the device in FP32 (k_mlp_grad: forward and hand-written
-//    backward of a mean-squared loss over a minibatch, per-workgroup partial
-//    gradients; k_mlp_reduce: their sum in a fixed order; k_mlp_adam: the update).
+//    backward of a mean-squared loss over a minibatch on the matrix cores, per-workgroup
+//    partial gradients; k_mlp_reduce: their sum in a fixed order; k_mlp_adam: the update).
 //  * Inference (k_mlp_infer for tests, k_visc_mlp in the step) runs the two hidden
 //    layers on the matrix cores: BF16 operands, FP32 accumulation
 //    (v_mfma_f32_32x32x8bf16_1k), 32 elements per matrix tile.
@@ -77,15 +77,8 @@ GF_DEV bool mlp_in_distribution(const MlpCfg *cfg, const MlpStats *st, const flo
     return ((cfg->occ[r] & ~st->bad[r]) >> c) & 1u;
 }
 
-GF_DEV float mlp_sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
-GF_DEV float mlp_silu(float z) { return z * mlp_sigmoid(z); }
 // inference: the hardware reciprocal (1 ulp) in place of the rounded division
 GF_DEV float mlp_silu_fast(float z) { return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
-GF_DEV float mlp_dsilu(float z)
-{
-    const float s = mlp_sigmoid(z);
-    return s * (1.0f + z * (1.0f - s));
-}
 GF_DEV unsigned short f2bf(float f)  // round to nearest, ties to even
 {
     unsigned int u = __float_as_uint(f);
@@ -151,140 +144,347 @@ __global__ void __launch_bounds__(256) k_visc_sample(const GfDevParams *__restri
 }
 
 // ------------------------------------------------------------------ training
-// Workgroup of 256 threads over tiles of 64 samples.  Thread t works on unit
-// n = t % 64 and on the 16 samples (or 16 inputs) of group g = t / 64.
-#define MLP_TS 64
-#define MLP_LD (MLP_NH + 1)  // padded LDS row
-__global__ void __launch_bounds__(256) k_mlp_grad(const float *__restrict__ w, const float *__restrict__ samples,
-                                                  long nsamples, long first, long batch, long perm_a, long perm_c,
-                                                  const MlpCfg *__restrict__ cfg, int per_block,
-                                                  float *__restrict__ partial)
+// The gradient's three 64 x 64 products (layer 2, its weights' gradient, the gradient
+// passed back to layer 1) run on the matrix cores in FP32 (v_mfma_f32_32x32x2f32,
+// v_mfma_f32_16x16x4f32: FP32 operands and sums), a wave to a tile of 32 samples.
+// Products are formed transposed, units x samples: lane l holds sample l % 32, and result
+// register r of row block T holds unit 32 T + (r & 3) + 8 (r >> 2) + 4 (l / 32).  That is
+// a valid order of the next product's K as it stands, so the activations go from one
+// product to the next in registers; W2 waits in LDS in the order of that K (w2a by rows,
+// w2t by columns, four K steps a 16-byte read).  Only the products over samples (the
+// weights' gradients) need their operands turned, through this wave's LDS rows.
+// What bounds it: a tile takes a wave 13.8k cycles of FP32 matrix work and 9k of
+// activations and LDS turns, which two waves of a SIMD do not overlap (25 us a 65536
+// samples with one or two), and some 12 us for the launch, the weights' turn into LDS and
+// the waves' sum.  With the reduction, us: 175 (products on the vector ALU from LDS) ->
+// 43 at 65536 samples, 965 -> 174 at 400000, 47 -> 24 at 1000.
+#define MG_W 8    // waves of a workgroup
+#define MG_TS 32  // samples of a tile
+#define MG_LD 36  // padded LDS row of samples (16-byte aligned; rows 4 banks apart)
+typedef float mg_f16 __attribute__((ext_vector_type(16)));
+typedef float mg_f4 __attribute__((ext_vector_type(4)));
+typedef float mg_f4u __attribute__((ext_vector_type(4), aligned(4)));  // (a caller's samples: any float address)
+
+struct MgTiles {
+    float w2a[MLP_NH * MLP_NH], w2t[MLP_NH * MLP_NH];
+    float u[MG_W][MLP_NH][MG_LD];     // units x samples of a wave: dy H2, dZ2, dZ1 in turn
+    float h[MG_W][MLP_NH / 2][MG_LD]; // half of H1
+    float x[MG_W][8][MG_LD];          // features x samples, then a row of ones
+};
+union MgShared {
+    MgTiles t;
+    float part[MG_W][MLP_NP + 1];  // at the end: each wave's gradient
+};
+static_assert(sizeof(MgShared) <= 160 * 1024 - 1024, "one workgroup per CU");
+
+// the sigmoid by the hardware reciprocal and one Newton step (the bound keeps an
+// overflowed exponential from giving 0 inf)
+GF_DEV float mg_sigmoid(float z)
 {
-    __shared__ float sw[MLP_NP];               // W2 is read from sW2 (rows padded: no bank conflicts)
-    __shared__ float sW2[MLP_NH][MLP_LD];
-    __shared__ float sX[MLP_TS][8], sT[MLP_TS], sDY[MLP_TS];
-    __shared__ float sZ1[MLP_TS][MLP_LD], sH1[MLP_TS][MLP_LD], sZ2[MLP_TS][MLP_LD], sH2[MLP_TS][MLP_LD];
-    __shared__ float sRed[4][MLP_NH];
-    const int t = threadIdx.x, n = t % MLP_NH, g = t / MLP_NH;
-    for (int q = t; q < MLP_NP; q += blockDim.x) sw[q] = w[q];
-    for (int q = t; q < MLP_NH * MLP_NH; q += blockDim.x) sW2[q / MLP_NH][q % MLP_NH] = w[MLP_OW2 + q];
-    float aW2[16], aW1[2], aB1 = 0.0f, aB2 = 0.0f, aW3 = 0.0f, aB3 = 0.0f, aLoss = 0.0f;
-    for (int q = 0; q < 16; q++) aW2[q] = 0.0f;
-    aW1[0] = aW1[1] = 0.0f;
-    const float inv_b = 1.0f / (float)batch;
-    const long b0 = (long)blockIdx.x * per_block;
-    for (int tile = 0; tile < per_block; tile += MLP_TS) {
-        __syncthreads();
-        if (t < MLP_TS) {  // gather one sample per thread
-            const long bpos = b0 + tile + t;
-            float xs[MLP_SW];
-            bool ok = bpos < batch;
-            if (ok) {
-                const long idx = (perm_a * ((first + bpos) % nsamples) + perm_c) % nsamples;
-                for (int f = 0; f < MLP_SW; f++) xs[f] = samples[idx * MLP_SW + f];
-                ok = xs[MLP_NIN] == xs[MLP_NIN];  // NaN marks an element outside the domain
-            }
-            for (int f = 0; f < MLP_NIN; f++) sX[t][f] = ok ? (xs[f] - cfg->xmean[f]) / cfg->xstd[f] : 0.0f;
-            sX[t][MLP_NIN] = ok ? 1.0f : 0.0f;  // weight of the sample in the loss
-            sT[t] = ok ? (xs[MLP_NIN] - cfg->ymean) / cfg->ystd : 0.0f;
+    const float d = fminf(1.0f + __expf(-z), 1.0e38f), y = __builtin_amdgcn_rcpf(d);
+    return __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
+}
+// LDS written by some lanes of a wave and read by others: keeps the compiler from
+// reordering (the hardware runs a wave's LDS operations in order)
+GF_DEV void mg_lds_turn()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// keeps the compiler from holding values formed from z across this point
+GF_DEV void mg_opaque(mg_f16 z[2]) { asm volatile("" : "+v"(z[0]), "+v"(z[1])); }
+
+// cfg null: the samples are taken as they are.  Workgroup b takes tiles b, b + grid, ...,
+// its waves in turn.
+__global__ void __launch_bounds__(64 * MG_W) k_mlp_grad(const float *__restrict__ w, const float *__restrict__ samples,
+                                                        long nsamples, long first, long batch, long perm_a, long perm_c,
+                                                        const MlpCfg *__restrict__ cfg, float *__restrict__ partial)
+{
+    __shared__ __align__(16) MgShared S;
+    __shared__ __align__(16) float sB2[MLP_NH], sW3[MLP_NH];
+    const int t = threadIdx.x, wv = t / 64, l = t % 64, s = l & 31, h = l >> 5;
+    {
+        constexpr int NQ = MLP_NH * MLP_NH / (64 * MG_W);
+        float va[NQ], vt[NQ];  // (all loads in flight)
+#pragma unroll
+        for (int u = 0; u < NQ; u++) {
+            const int q = t + u * 64 * MG_W;
+            va[u] = w[MLP_OW2 + q % MLP_NH * MLP_NH + q / MLP_NH];
+            vt[u] = w[MLP_OW2 + q];
         }
-        __syncthreads();
-#pragma unroll 2
-        for (int q = 0; q < 16; q++) {  // layer 1
-            const int s = g * 16 + q;
-            float z = sw[MLP_OB1 + n];
-            for (int k = 0; k < MLP_NIN; k++) z += sw[MLP_OW1 + n * MLP_NIN + k] * sX[s][k];
-            sZ1[s][n] = z;
-            sH1[s][n] = mlp_silu(z);
-        }
-        __syncthreads();
-#pragma unroll 2
-        for (int q = 0; q < 16; q++) {  // layer 2
-            const int s = g * 16 + q;
-            float z = sw[MLP_OB2 + n];
-            for (int k = 0; k < MLP_NH; k++) z += sW2[n][k] * sH1[s][k];
-            sZ2[s][n] = z;
-            sH2[s][n] = mlp_silu(z);
-        }
-        __syncthreads();
-        if (t < MLP_TS) {  // output and loss
-            float y = sw[MLP_OB3];
-            for (int k = 0; k < MLP_NH; k++) y += sw[MLP_OW3 + k] * sH2[t][k];
-            const float r = (y - sT[t]) * sX[t][MLP_NIN];
-            aLoss += r * r;
-            sDY[t] = 2.0f * r * inv_b;
-        }
-        __syncthreads();
-#pragma unroll 2
-        for (int q = 0; q < 16; q++) {  // dZ2 in place; dW3, dB3
-            const int s = g * 16 + q;
-            aW3 += sDY[s] * sH2[s][n];
-            sZ2[s][n] = sDY[s] * sw[MLP_OW3 + n] * mlp_dsilu(sZ2[s][n]);
-        }
-        if (t == 0)
-            for (int s = 0; s < MLP_TS; s++) aB3 += sDY[s];
-        __syncthreads();
-#pragma unroll 2
-        for (int s = 0; s < MLP_TS; s++) {  // dW2[n][16g .. 16g+15], dB2
-            const float d = sZ2[s][n];
-            for (int q = 0; q < 16; q++) aW2[q] += d * sH1[s][g * 16 + q];
-            if (g == 0) aB2 += d;
-        }
-#pragma unroll 2
-        for (int q = 0; q < 16; q++) {  // dZ1 = (W2^T dZ2) * silu'(Z1), thread = input unit n
-            const int s = g * 16 + q;
-            float dh = 0.0f;
-            for (int m = 0; m < MLP_NH; m++) dh += sZ2[s][m] * sW2[m][n];
-            sH2[s][n] = dh * mlp_dsilu(sZ1[s][n]);  // H2 is free now
-        }
-        __syncthreads();
-        for (int s = 0; s < MLP_TS; s++) {  // dW1[n][2g, 2g+1], dB1
-            const float d = sH2[s][n];
-            for (int q = 0; q < 2; q++) {
-                const int k = 2 * g + q;
-                if (k < MLP_NIN) aW1[q] += d * sX[s][k];
-            }
-            if (g == 3) aB1 += d;
+#pragma unroll
+        for (int u = 0; u < NQ; u++) {
+            const int q = t + u * 64 * MG_W, lo = q % MLP_NH, hi = q / MLP_NH;
+            // W2[m = lo][k = hi], lanes along m; W2[m = hi][n = lo], lanes along n
+            const int kk = ((hi >> 5) * 4 + ((hi >> 3) & 3)) * 2 + (lo >> 5);
+            const int at = (kk * 64 + (lo & 31) + 32 * ((hi >> 2) & 1)) * 4 + (hi & 3);
+            S.t.w2a[at] = va[u];
+            S.t.w2t[at] = vt[u];
         }
     }
-    // partial gradient of this workgroup (plus its loss sum in the last slot)
+    if (t < MLP_NH) {
+        sB2[t] = w[MLP_OB2 + t];
+        sW3[t] = w[MLP_OW3 + t];
+    }
+    float w1[2][4];  // W1 with b1 as its column 7: rows 32 M + s, columns 2 j + h
+#pragma unroll
+    for (int M = 0; M < 2; M++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int m = 32 * M + s, k = 2 * j + h;
+            w1[M][j] = k < MLP_NIN ? w[MLP_OW1 + m * MLP_NIN + k] : w[MLP_OB1 + m];
+        }
+    const float b3 = w[MLP_OB3], inv_b = 1.0f / (float)batch;
+    float(*U)[MG_LD] = S.t.u[wv], (*H)[MG_LD] = S.t.h[wv], (*X)[MG_LD] = S.t.x[wv];
+    __syncthreads();
+    mg_f16 aW2[2][2] = {};
+    mg_f4 aW1[4] = {};
+    float aB2 = 0.0f, aW3 = 0.0f, aB3 = 0.0f, aLoss = 0.0f;
+    const long ntiles = (batch + MG_TS - 1) / MG_TS;
+    for (long tile = blockIdx.x + (long)gridDim.x * wv; tile < ntiles; tile += (long)gridDim.x * MG_W) {
+        // ---- one sample per lane (both halves the same)
+        const long bpos = tile * MG_TS + s;
+        float xs[8];
+        bool ok = bpos < batch;
+        float tg = 0.0f;
+        {
+            long idx = 0;
+            if (ok) {  // (the whole set in order needs no 64-bit remainders)
+                if (perm_a == 1 && perm_c == 0 && first == 0 && batch <= nsamples)
+                    idx = bpos;
+                else
+                    idx = (perm_a * ((first + bpos) % nsamples) + perm_c) % nsamples;
+            }
+            const mg_f4u v0 = *(const mg_f4u *)(samples + idx * MLP_SW), v1 = *(const mg_f4u *)(samples + idx * MLP_SW + 4);
+            for (int k = 0; k < 4; k++) {
+                xs[k] = v0[k];
+                xs[4 + k] = v1[k];
+            }
+            tg = xs[MLP_NIN];
+            ok = ok && tg == tg;  // NaN marks an element outside the domain
+            if (cfg) {
+                for (int k = 0; k < MLP_NIN; k++) xs[k] = (xs[k] - cfg->xmean[k]) / cfg->xstd[k];
+                tg = (tg - cfg->ymean) / cfg->ystd;
+            }
+            for (int k = 0; k < MLP_NIN; k++) xs[k] = ok ? xs[k] : 0.0f;
+            tg = ok ? tg : 0.0f;
+            xs[7] = 1.0f;
+        }
+        for (int k = 0; k < 4; k++) X[4 * h + k][s] = h ? xs[4 + k] : xs[k];
+        // ---- layer 1
+        // (only Z1 is kept: H1 and silu' are formed again where they are read, which costs
+        // less than the registers that would hold them)
+        mg_f16 z1[2];
+#pragma unroll
+        for (int M = 0; M < 2; M++) {
+            z1[M] = mg_f16{};
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                z1[M] = __builtin_amdgcn_mfma_f32_32x32x2f32(w1[M][j], h ? xs[2 * j + 1] : xs[2 * j], z1[M], 0, 0, 0);
+        }
+        // ---- layer 2
+        mg_f16 z2[2];
+#pragma unroll
+        for (int M = 0; M < 2; M++)
+#pragma unroll
+            for (int rq = 0; rq < 4; rq++) {
+                const mg_f4 b = *(const mg_f4 *)&sB2[32 * M + 8 * rq + 4 * h];
+#pragma unroll
+                for (int i = 0; i < 4; i++) z2[M][4 * rq + i] = b[i];
+            }
+#pragma unroll
+        for (int T = 0; T < 2; T++)
+#pragma unroll
+            for (int rq = 0; rq < 4; rq++) {
+                const mg_f4 a0 = *(const mg_f4 *)&S.t.w2a[(((T * 4 + rq) * 2 + 0) * 64 + l) * 4];
+                const mg_f4 a1 = *(const mg_f4 *)&S.t.w2a[(((T * 4 + rq) * 2 + 1) * 64 + l) * 4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float z = z1[T][4 * rq + i], h1 = z * mg_sigmoid(z);
+                    z2[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[i], h1, z2[0], 0, 0, 0);
+                    z2[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[i], h1, z2[1], 0, 0, 0);
+                }
+            }
+        mg_opaque(z1);
+        // ---- output, loss, dZ2
+        float y = 0.0f;
+#pragma unroll
+        for (int M = 0; M < 2; M++)
+#pragma unroll
+            for (int rq = 0; rq < 4; rq++) {
+                const mg_f4 w3 = *(const mg_f4 *)&sW3[32 * M + 8 * rq + 4 * h];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int r = 4 * rq + i;
+                    const float z = z2[M][r], sg = mg_sigmoid(z), h2 = z * sg;
+                    y += w3[i] * h2;
+                    U[32 * M + 8 * rq + 4 * h + i][s] = h2;
+                    z2[M][r] = w3[i] * (sg * (1.0f + z * (1.0f - sg)));  // times dy: dZ2
+                }
+            }
+        y += __shfl_xor(y, 32);
+        const float res = ok ? (y + b3) - tg : 0.0f;
+        const float dy = 2.0f * res * inv_b;
+        if (h == 0) {
+            aLoss += res * res;
+            aB3 += dy;
+            H[0][s] = dy;
+        }
+        mg_lds_turn();
+        {  // dW3: dy H2 over the samples, unit l
+            float v = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const mg_f4 p = *(const mg_f4 *)&U[l][4 * q], d = *(const mg_f4 *)&H[0][4 * q];
+                v += (p[0] * d[0] + p[1] * d[1]) + (p[2] * d[2] + p[3] * d[3]);
+            }
+            aW3 += v;
+        }
+        mg_lds_turn();
+#pragma unroll
+        for (int M = 0; M < 2; M++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                z2[M][r] = dy * z2[M][r];
+                U[32 * M + (r & 3) + 8 * (r >> 2) + 4 * h][s] = z2[M][r];
+            }
+        mg_lds_turn();
+        {  // dB2
+            float v = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const mg_f4 p = *(const mg_f4 *)&U[l][4 * q];
+                v += (p[0] + p[1]) + (p[2] + p[3]);
+            }
+            aB2 += v;
+        }
+        // ---- dW2 = dZ2 H1^T over the samples (half h takes samples 16 h + k)
+#pragma unroll
+        for (int T = 0; T < 2; T++) {
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                H[(r & 3) + 8 * (r >> 2) + 4 * h][s] = z1[T][r] * mg_sigmoid(z1[T][r]);
+            mg_lds_turn();
+#pragma unroll
+            for (int kq = 0; kq < 4; kq++) {
+                const mg_f4 a0 = *(const mg_f4 *)&U[s][16 * h + 4 * kq], a1 = *(const mg_f4 *)&U[32 + s][16 * h + 4 * kq];
+                const mg_f4 b = *(const mg_f4 *)&H[s][16 * h + 4 * kq];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    aW2[0][T] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[i], b[i], aW2[0][T], 0, 0, 0);
+                    aW2[1][T] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[i], b[i], aW2[1][T], 0, 0, 0);
+                }
+            }
+            mg_lds_turn();
+        }
+        mg_opaque(z1);
+        // ---- dH1 = W2^T dZ2, dZ1
+        mg_f16 dh[2] = {};
+#pragma unroll
+        for (int T = 0; T < 2; T++)
+#pragma unroll
+            for (int rq = 0; rq < 4; rq++) {
+                const mg_f4 a0 = *(const mg_f4 *)&S.t.w2t[(((T * 4 + rq) * 2 + 0) * 64 + l) * 4];
+                const mg_f4 a1 = *(const mg_f4 *)&S.t.w2t[(((T * 4 + rq) * 2 + 1) * 64 + l) * 4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    dh[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[i], z2[T][4 * rq + i], dh[0], 0, 0, 0);
+                    dh[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[i], z2[T][4 * rq + i], dh[1], 0, 0, 0);
+                }
+            }
+#pragma unroll
+        for (int N = 0; N < 2; N++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float z = z1[N][r], sg = mg_sigmoid(z);
+                U[32 * N + (r & 3) + 8 * (r >> 2) + 4 * h][s] = dh[N][r] * (sg * (1.0f + z * (1.0f - sg)));
+            }
+        mg_lds_turn();
+        // ---- dW1 and dB1 (column 7) = dZ1 X^T (quarter l / 16 takes samples 8 (l / 16) + k)
+        {
+            const int c = l & 15, qd = l >> 4;
+            mg_f4 b0{}, b1{};
+            if (c < 8) {
+                b0 = *(const mg_f4 *)&X[c][8 * qd];
+                b1 = *(const mg_f4 *)&X[c][8 * qd + 4];
+            }
+#pragma unroll
+            for (int N = 0; N < 4; N++) {
+                const mg_f4 a0 = *(const mg_f4 *)&U[16 * N + c][8 * qd], a1 = *(const mg_f4 *)&U[16 * N + c][8 * qd + 4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) aW1[N] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[i], b0[i], aW1[N], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) aW1[N] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[i], b1[i], aW1[N], 0, 0, 0);
+            }
+        }
+        mg_lds_turn();
+    }
+    // ---- the waves' gradients, then their sum in wave order (and the loss sum, last)
+    double dLoss = aLoss, dB3 = aB3;
+    for (int o = 16; o; o >>= 1) {
+        dLoss += __shfl_xor(dLoss, o);
+        dB3 += __shfl_xor(dB3, o);
+    }
+    __syncthreads();
+    float *pw = S.part[wv];
+#pragma unroll
+    for (int M = 0; M < 2; M++)
+#pragma unroll
+        for (int T = 0; T < 2; T++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                pw[MLP_OW2 + (32 * M + (r & 3) + 8 * (r >> 2) + 4 * h) * MLP_NH + 32 * T + s] = aW2[M][T][r];
+#pragma unroll
+    for (int N = 0; N < 4; N++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int n = 16 * N + 4 * (l >> 4) + r, k = l & 15;
+            if (k < MLP_NIN) pw[MLP_OW1 + n * MLP_NIN + k] = aW1[N][r];
+            if (k == MLP_NIN) pw[MLP_OB1 + n] = aW1[N][r];
+        }
+    pw[MLP_OB2 + l] = aB2;
+    pw[MLP_OW3 + l] = aW3;
+    if (l == 0) {
+        pw[MLP_OB3] = (float)dB3;
+        pw[MLP_NP] = (float)dLoss;
+    }
+    __syncthreads();
     float *pg = partial + (long)blockIdx.x * (MLP_NP + 1);
-    for (int q = 0; q < 16; q++) pg[MLP_OW2 + n * MLP_NH + g * 16 + q] = aW2[q];
-    for (int q = 0; q < 2; q++) {
-        const int k = 2 * g + q;
-        if (k < MLP_NIN) pg[MLP_OW1 + n * MLP_NIN + k] = aW1[q];
-    }
-    if (g == 0) pg[MLP_OB2 + n] = aB2;
-    if (g == 3) pg[MLP_OB1 + n] = aB1;
-    sRed[g][n] = aW3;
-    __syncthreads();
-    if (g == 0) pg[MLP_OW3 + n] = ((sRed[0][n] + sRed[1][n]) + sRed[2][n]) + sRed[3][n];
-    if (t < MLP_TS) sDY[t] = aLoss;
-    __syncthreads();
-    if (t == 0) {
-        float l = 0.0f;
-        for (int s = 0; s < MLP_TS; s++) l += sDY[s];
-        pg[MLP_OB3] = aB3;
-        pg[MLP_NP] = l;
+    for (int q = t; q <= MLP_NP; q += 64 * MG_W) {
+        double v = S.part[0][q];
+        for (int k = 1; k < MG_W; k++) v += S.part[k][q];
+        pg[q] = (float)v;
     }
 }
 
 // gradient (and loss) = sum of the workgroups' partials, MLP_RED_PARAMS parameters per
-// workgroup: wave q adds the partials of workgroups q, q+4, q+8, ... and the four sums
-// are added in wave order (a fixed order: the result does not depend on timing)
-#define MLP_RED_PARAMS 64
+// workgroup: group q adds the partials of workgroups q, q+8, q+16, ..., eight loads at a
+// time, and the eight sums are added in order (a fixed order: the result does not depend
+// on timing), in FP64, so that the sum adds one rounding
+#define MLP_RED_PARAMS 32
 __global__ void __launch_bounds__(256) k_mlp_reduce(const float *__restrict__ partial, int nblocks,
                                                     float *__restrict__ grad)
 {
-    __shared__ float part[4][MLP_RED_PARAMS];
+    __shared__ double part[8][MLP_RED_PARAMS];
     const int l = threadIdx.x % MLP_RED_PARAMS, q = threadIdx.x / MLP_RED_PARAMS;
     const int p = blockIdx.x * MLP_RED_PARAMS + l;
-    float s = 0.0f;
-    if (p <= MLP_NP)
-        for (int b = q; b < nblocks; b += 4) s += partial[(long)b * (MLP_NP + 1) + p];
+    double s = 0.0;
+    if (p <= MLP_NP) {
+        int b = q;
+        for (; b + 56 < nblocks; b += 64) {
+            float v[8];
+            for (int k = 0; k < 8; k++) v[k] = partial[(long)(b + 8 * k) * (MLP_NP + 1) + p];
+            for (int k = 0; k < 8; k++) s += v[k];
+        }
+        for (; b < nblocks; b += 8) s += partial[(long)b * (MLP_NP + 1) + p];
+    }
     part[q][l] = s;
     __syncthreads();
-    if (q == 0 && p <= MLP_NP) grad[p] = ((part[0][l] + part[1][l]) + part[2][l]) + part[3][l];
+    if (q == 0 && p <= MLP_NP) {
+        for (int k = 1; k < 8; k++) s += part[k][l];
+        grad[p] = (float)s;
+    }
 }
 
 // every stride-th sample, packed (the training set-up's statistics read them on the

@@ -2058,22 +2058,16 @@ static int sur_alloc(gf_ctx *ctx)
     return GF_OK;
 }
 
-// one Adam step on a minibatch of `batch` samples starting at permuted position `first`
-// workgroups and samples per workgroup of a gradient launch over `batch` samples
-static void grad_grid(long batch, int &nblocks, int &per_block)
-{
-    const long tiles = (batch + MLP_TS - 1) / MLP_TS;
-    nblocks = (int)std::min<long>(tiles, MLP_GRAD_BLOCKS);
-    per_block = (int)((tiles + nblocks - 1) / nblocks) * MLP_TS;
-}
+// workgroups of a gradient over `batch` samples: a tile each as long as they last
+static int grad_grid(long batch) { return (int)std::min<long>((batch + MG_TS - 1) / MG_TS, MLP_GRAD_BLOCKS); }
 
+// one Adam step on a minibatch of `batch` samples starting at permuted position `first`
 static int sur_train_step(gf_ctx *ctx, long nsamples, long first, long batch, long pa, long pc, float lr, int step,
                           hipStream_t s)
 {
-    int nb, per_block;
-    grad_grid(batch, nb, per_block);
-    hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(256), 0, s, ctx->sur_w, ctx->sur_samples, nsamples, first, batch,
-                       pa, pc, ctx->sur_cfg, per_block, ctx->sur_partial);
+    const int nb = grad_grid(batch);
+    hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(64 * MG_W), 0, s, ctx->sur_w, ctx->sur_samples, nsamples, first,
+                       batch, pa, pc, ctx->sur_cfg, ctx->sur_partial);
     hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NP + MLP_RED_PARAMS) / MLP_RED_PARAMS), dim3(256), 0, s, ctx->sur_partial, nb,
                        ctx->sur_grad);
     hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NP + 255) / 256), dim3(256), 0, s, ctx->sur_w, ctx->sur_m, ctx->sur_v,
@@ -2285,31 +2279,24 @@ extern "C" int gf_mlp_grad(const float *x, const float *t, int64_t n, const floa
 {
     if (!x || !t || !w || !grad || n < 1) return GF_ERR_ARG;
     float *ds = nullptr, *dw = nullptr, *dp = nullptr, *dg = nullptr;
-    MlpCfg *dc = nullptr;
     int rc = GF_OK;
     std::vector<float> smp((size_t)n * MLP_SW);
     for (int64_t q = 0; q < n; q++) {
         for (int f = 0; f < MLP_NIN; f++) smp[q * MLP_SW + f] = x[q * MLP_NIN + f];
         smp[q * MLP_SW + MLP_NIN] = t[q];
     }
-    MlpCfg c{};
-    for (int f = 0; f < 8; f++) { c.xmean[f] = 0; c.xstd[f] = 1; }
-    c.ymean = 0; c.ystd = 1;
-    int nb, per_block;
-    grad_grid((long)n, nb, per_block);
+    const int nb = grad_grid((long)n);
     std::vector<float> out(MLP_NP + 1);
     if (hipMalloc((void **)&ds, sizeof(float) * smp.size()) != hipSuccess ||
         hipMalloc((void **)&dw, sizeof(float) * MLP_NP) != hipSuccess ||
         hipMalloc((void **)&dp, sizeof(float) * (MLP_NP + 1) * MLP_GRAD_BLOCKS) != hipSuccess ||
         hipMalloc((void **)&dg, sizeof(float) * (MLP_NP + 1)) != hipSuccess ||
-        hipMalloc((void **)&dc, sizeof(MlpCfg)) != hipSuccess ||
         hipMemcpy(ds, smp.data(), sizeof(float) * smp.size(), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(dw, w, sizeof(float) * MLP_NP, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(dc, &c, sizeof(c), hipMemcpyHostToDevice) != hipSuccess) {
+        hipMemcpy(dw, w, sizeof(float) * MLP_NP, hipMemcpyHostToDevice) != hipSuccess) {
         rc = GF_ERR_HIP;
     } else {
-        hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(256), 0, 0, dw, ds, (long)n, 0L, (long)n, 1L, 0L, dc, per_block,
-                           dp);
+        hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(64 * MG_W), 0, 0, dw, ds, (long)n, 0L, (long)n, 1L, 0L,
+                           (const MlpCfg *)nullptr, dp);
         hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NP + MLP_RED_PARAMS) / MLP_RED_PARAMS), dim3(256), 0, 0, dp, nb, dg);
         if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess ||
             hipMemcpy(out.data(), dg, sizeof(float) * (MLP_NP + 1), hipMemcpyDeviceToHost) != hipSuccess)
@@ -2319,19 +2306,16 @@ extern "C" int gf_mlp_grad(const float *x, const float *t, int64_t n, const floa
         memcpy(grad, out.data(), sizeof(float) * MLP_NP);
         if (loss) *loss = out[MLP_NP] / (float)n;
     }
-    for (void *b : {(void *)ds, (void *)dw, (void *)dp, (void *)dg, (void *)dc})
+    for (void *b : {(void *)ds, (void *)dw, (void *)dp, (void *)dg})
         if (b) (void)hipFree(b);
     return rc;
 }
 
 // ---- gf_mlp_grad_noalloc: the gradient kernels on device-resident data with their
-// scratch memory in a fixed device array (no allocation per call).  Layout of scratch:
-// the identity normalisation (MlpCfg) in the first 512 bytes, then the partial
-// gradients of at most MLP_GRAD_BLOCKS workgroups (MLP_NP + 1 floats each).  Every call
-// rewrites both before they are read; calls that overlap on one GPU race on them.
-#define GF_NOALLOC_CFG_BYTES 512
-#define GF_NOALLOC_SCRATCH_BYTES (GF_NOALLOC_CFG_BYTES + sizeof(float) * (MLP_NP + 1) * MLP_GRAD_BLOCKS)
-static_assert(sizeof(MlpCfg) <= GF_NOALLOC_CFG_BYTES, "the normalisation block fits its slot");
+// scratch memory in a fixed device array (no allocation per call): the partial gradients
+// of at most MLP_GRAD_BLOCKS workgroups (MLP_NP + 1 floats each).  Every call rewrites
+// those it reads; calls that overlap on one GPU race on them.
+#define GF_NOALLOC_SCRATCH_BYTES (sizeof(float) * (MLP_NP + 1) * MLP_GRAD_BLOCKS)
 static __device__ __align__(256) unsigned char scratch[GF_NOALLOC_SCRATCH_BYTES];
 
 #define GF_NOALLOC_MAXDEV 64
@@ -2354,37 +2338,18 @@ static int noalloc_scratch(void **out)
     return GF_OK;
 }
 
-__global__ void k_mlp_cfg_identity(MlpCfg *c)
-{
-    const int f = threadIdx.x;
-    if (f < 8) {
-        c->xmean[f] = 0.0f;
-        c->xstd[f] = 1.0f;
-        c->xlo[f] = 0.0f;
-        c->xhi[f] = 0.0f;
-    }
-    if (f == 0) {
-        c->ymean = 0.0f;
-        c->ystd = 1.0f;
-    }
-}
-
 extern "C" int gf_mlp_grad_noalloc(const float *samples, int64_t n, const float *w, float *grad, void *stream)
 {
     if (!samples || !w || !grad || n < 1) return GF_ERR_ARG;
-    if (n > GF_MLP_NOALLOC_MAXN) return GF_ERR_ARG;  // (per-workgroup sample counts are 32-bit)
+    if (n > GF_MLP_NOALLOC_MAXN) return GF_ERR_ARG;
     void *base = nullptr;
     int rc = noalloc_scratch(&base);
     if (rc) return rc;
-    MlpCfg *cfg = (MlpCfg *)base;
-    float *partial = (float *)((unsigned char *)base + GF_NOALLOC_CFG_BYTES);
-    int nb, per_block;
-    grad_grid((long)n, nb, per_block);
-    if (nb > MLP_GRAD_BLOCKS) return GF_ERR_ARG;
+    float *partial = (float *)base;
+    const int nb = grad_grid((long)n);
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_mlp_cfg_identity, dim3(1), dim3(64), 0, s, cfg);
-    hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(256), 0, s, w, samples, (long)n, 0L, (long)n, 1L, 0L, cfg,
-                       per_block, partial);
+    hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(64 * MG_W), 0, s, w, samples, (long)n, 0L, (long)n, 1L, 0L,
+                       (const MlpCfg *)nullptr, partial);
     hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NP + MLP_RED_PARAMS) / MLP_RED_PARAMS), dim3(256), 0, s, partial, nb,
                        grad);
     return hipGetLastError() == hipSuccess ? GF_OK : GF_ERR_HIP;

@@ -207,7 +207,8 @@ __global__ void __launch_bounds__(256) kb_dt_reduce(const BatchEntry *__restrict
 __global__ void kb_dt_scalars(const BatchEntry *__restrict__ tab, BatchMap map)
 {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m < map.nm) dt_scalars_body(tab[m].P, tab[m].ck);
+    if (m < map.nm)
+        dt_scalars_body(tab[m].P, tab[m].ck, dlmin_of(__longlong_as_double((long long)tab[m].ck->dly_bits)));
 }
 
 // change_phase of every model with markers (gf_phase.h)
@@ -221,15 +222,11 @@ __global__ void kb_phase_plan(const BatchEntry *__restrict__ tab, BatchMap map)
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m < map.nm && tab[m].A.phstamp) phase_plan_body(const_cast<GfDevParams *>(tab[m].P), tab[m].ck);
 }
-__global__ void __launch_bounds__(256) kb_phase_replane(const BatchEntry *__restrict__ tab, BatchMap map)
+__global__ void __launch_bounds__(256) kb_phase_update(const BatchEntry *__restrict__ tab, BatchMap map)
 {
     batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) {
-        if (b.A.phstamp && b.ck->ph_replan) phase_replane_body(b.P, b.ck, b.A, e);
-    });
-}
-__global__ void __launch_bounds__(256) kb_phase_recount(const BatchEntry *__restrict__ tab, BatchMap map)
-{
-    batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) {
-        if (b.A.phstamp) phase_recount_body(b.P, b.ck, b.A, e);
+        if (!b.A.phstamp) return;
+        if (b.ck->ph_replan) phase_replane_body(b.P, b.ck, b.A, e);
+        phase_recount_body(b.P, b.ck, b.A, e);
     });
 }

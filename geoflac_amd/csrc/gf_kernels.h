@@ -21,6 +21,7 @@ struct GfDevArrays {
     double *tbord;        // thermal strips' (tiles') border values
     double *tpre;         // GF_NPRE slots: boundary rows and columns before the boundary conditions
     double *dens;         // per-element density scratch (rmasses)
+    unsigned long long *dtred;  // dt_mass's maxima of a step that runs both masses (DTR_SLOTS lines)
     // Mixed precision: velocity and force in FP32, and the stress as an FP32 deviation
     // from a per-element isotropic reference -pref*I kept in FP64 (the element's mean
     // normal stress when it was uploaded), so that the FP32 planes carry the tectonic
@@ -99,6 +100,10 @@ template <> GF_DEV float *sv_ptr<float>(double *d, float *f) { return f; }
 // Kernels indexed this way are launched with GF_BLOCK threads per workgroup (a
 // compile-time constant: reading blockDim.x costs a memory round trip per wave).
 #define GF_BLOCK 256
+// dt_mass's maxima of a step that runs both masses (k_dens): DTR_SLOTS cells of two
+// values, a 128-byte line each
+#define DTR_SLOTS 64
+#define DTR_PAD 16
 // skip: workgroups at the start of the launch that do something else (a multiple of 8)
 GF_DEV long xcd_lin(unsigned skip = 0)
 {
@@ -2625,6 +2630,9 @@ __global__ void __launch_bounds__(256) k_node_t(const GfDevParams *__restrict__ 
         if (MOVE) ck->dt_move = kc.dt;  // the move's dt (no other reader here)
         if (ops) clock_op(ck, ops);     // (fields nothing here reads)
     }
+    // dt_mass's maxima of this step start at 0 (k_dens)
+    if ((ops & CK_DT_BEGIN) && blockIdx.x == 0 && threadIdx.x < 2 * DTR_SLOTS)
+        A.dtred[(threadIdx.x >> 1) * DTR_PAD + (threadIdx.x & 1)] = 0ull;
     const NodePf<M> pf = node_prefetch<M>(P, A, tile);
     node_stage<M>(pf, L);
     __syncthreads();
@@ -2921,16 +2929,48 @@ GF_DEV void dens_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const G
 {
     A.dens[e] = eff_dens_value<M>(P, ck, A, e, rot);
 }
-// dtb: also starts dt_mass's minima for a k_dt_reduce that follows (CK_DT_BEGIN; no
-// kernel of this launch reads them)
-template <int M>
+// DTR: also dt_mass's maxima over the element (elem_dly's product and its corners'
+// velocities: every node is a corner), for the k_masses that follows.  They go to
+// DTR_SLOTS cells on lines of their own, one atomic per workgroup and cell at most: on
+// one address the atomics of a launch serialise (a reduction launch of 1024 workgroups
+// took 12-15 us on the smallest mesh).  The step's fl_node cleared the cells.
+template <bool ARP> GF_DEV double elem_dly(const GfDevParams *P, const GfDevArrays &A, long t);
+template <int M, bool DTR>
 __global__ void __launch_bounds__(256) k_dens(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, int rot,
-                                              int dtb)
+                                              int arp)
 {
-    long e = xcd_lin();
-    if (e >= NE) return;
-    if (dtb && e == 0) clock_op(ck, CK_DT_BEGIN);
-    dens_body<M>(P, ck, A, e, rot);
+    typedef typename Prec<M>::SV SV;
+    const long e = xcd_lin();
+    if (!DTR && e >= NE) return;
+    double dly = 0.0, vmax = 0.0;
+    if (e < NE) {
+        dens_body<M>(P, ck, A, e, rot);
+        if (DTR) {
+            const int j = (int)((unsigned)e % (unsigned)(NZ - 1)) + 1, i = (int)((unsigned)e / (unsigned)(NZ - 1)) + 1;
+            dly = fmax(dly, arp ? elem_dly<true>(P, A, e) : elem_dly<false>(P, A, e));
+            const SV *vel = sv_ptr<SV>(A.vel, A.velf);
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                vmax = fmax(vmax, fabs((double)vel[IN(j + (q & 1), i + ((q >> 1) & 1)) + NN * (q >> 2)]));
+        }
+    }
+    if (!DTR) return;
+    __shared__ double s_max[2][4];
+    for (int off = 32; off > 0; off >>= 1) {
+        dly = fmax(dly, __shfl_xor(dly, off));
+        vmax = fmax(vmax, __shfl_xor(vmax, off));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s_max[0][threadIdx.x >> 6] = dly;
+        s_max[1][threadIdx.x >> 6] = vmax;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const double *q = s_max[threadIdx.x];
+        const unsigned long long v = (unsigned long long)__double_as_longlong(fmax(fmax(q[0], q[1]), fmax(q[2], q[3])));
+        unsigned long long *cell = A.dtred + (blockIdx.x % DTR_SLOTS) * DTR_PAD + threadIdx.x;
+        if (v > __hip_atomic_load(cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(cell, v);
+    }
 }
 
 // The reference scatters each element's 4 triangles to their nodes in 2x2 colour
@@ -3131,7 +3171,7 @@ GF_DEV double side_len(const GfDevParams *P, const GfDevArrays &A, int ja, int i
 // negative-area STOP ends the run.)
 // ARP: the last move's areas are pending: formed from the moved coordinates
 // (move_area_body's arithmetic) instead of being read
-template <bool ARP = false>
+template <bool ARP>
 GF_DEV double elem_dly(const GfDevParams *P, const GfDevArrays &A, long t)
 {
     const int j = (int)((unsigned)t % (unsigned)(NZ - 1)) + 1, i = (int)((unsigned)t / (unsigned)(NZ - 1)) + 1;
@@ -3225,22 +3265,21 @@ __global__ void __launch_bounds__(256) k_dt_reduce(const GfDevParams *__restrict
 
 // Scalars of src/dt_mass.f90:31-51,122-158.  dtmax_therm and dt_maxwell depend on
 // the element only through its phase, so their minima run over the phases present.
-GF_DEV void dt_scalars_body(const GfDevParams *__restrict__ P, GfDevClock *ck)
+// dlmin from the reduction's largest product (elem_dly): min(1e28, 1/max)
+GF_DEV double dlmin_of(double dly) { return dly > 0.0 ? fmin(1.0e28, 1.0 / dly) : 1.0e28; }
+GF_DEV double dt_elastic_of(const GfDevParams *__restrict__ P, const GfDevClock *ck, double dlmin)
 {
     const double sec_year = 3.1558e+7;
-    {  // dlmin from the reduction's largest product (elem_dly): min(1e28, 1/max)
-        const double dly = __longlong_as_double((long long)ck->dly_bits);
-        if (dly > 0.0) ck->dlmin_bits = (unsigned long long)__double_as_longlong(fmin(1.0e28, 1.0 / dly));
-    }
-    double dlmin = __longlong_as_double((long long)ck->dlmin_bits);
-    if (P->idt_scale == 1) {
-        ck->dt_elastic = P->dt_scale;
-    } else if (P->idt_scale == 2) {
-        if (P->vbc == 0)
-            ck->dt_elastic = dlmin * P->frac * P->strain_inert / (1.0 / sec_year / 100);
-        else
-            ck->dt_elastic = dlmin * P->frac * P->strain_inert / P->vbc;
-    }
+    if (P->idt_scale == 1) return P->dt_scale;
+    if (P->idt_scale == 2)
+        return P->vbc == 0 ? dlmin * P->frac * P->strain_inert / (1.0 / sec_year / 100)
+                           : dlmin * P->frac * P->strain_inert / P->vbc;
+    return ck->dt_elastic;
+}
+GF_DEV void dt_scalars_body(const GfDevParams *__restrict__ P, GfDevClock *ck, double dlmin)
+{
+    ck->dlmin_bits = (unsigned long long)__double_as_longlong(dlmin);
+    ck->dt_elastic = dt_elastic_of(P, ck, dlmin);
     double dtmax_therm = 1.0e28, dt_maxwell = 1.0e28;
     for (int k = 1; k <= GF_MAXPH; k++) {
         if (ck->ph_count[k - 1] <= 0) continue;  // no element has this iphase
@@ -3259,11 +3298,20 @@ GF_DEV void dt_scalars_body(const GfDevParams *__restrict__ P, GfDevClock *ck)
 
 __global__ void k_dt_scalars(const GfDevParams *__restrict__ P, GfDevClock *ck)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) dt_scalars_body(P, ck);
+    if (threadIdx.x == 0 && blockIdx.x == 0)
+        dt_scalars_body(P, ck, dlmin_of(__longlong_as_double((long long)ck->dly_bits)));
 }
 
 // inertial masses, src/dt_mass.f90:64-120 (gather form of the coloured scatter)
-GF_DEV double amass_sum(const GfDevParams *__restrict__ P, GfDevClock *ck, const CornerSlots &cs,
+struct DtScal {
+    double dlmin, vel_max, dt_elastic;
+};
+GF_DEV DtScal dt_scal(const GfDevClock *ck)
+{
+    return DtScal{__longlong_as_double((long long)ck->dlmin_bits), __longlong_as_double((long long)ck->velmax_bits),
+                  ck->dt_elastic};
+}
+GF_DEV double amass_sum(const GfDevParams *__restrict__ P, const DtScal &ds, const CornerSlots &cs,
                         const double (&ar)[4][3], const int (&ip)[4]);
 GF_DEV void amass_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long t, int arp = 0)
 {
@@ -3280,16 +3328,14 @@ GF_DEV void amass_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const 
 #pragma unroll
     for (int sl = 0; sl < 4; sl++) ip[sl] = bldi(bI, cs.e[sl] * 4u, 0);
     corner_areas(P, A, j, i, cs, arp, ar);
-    A.amass[t] = amass_sum(P, ck, cs, ar, ip);
+    A.amass[t] = amass_sum(P, dt_scal(ck), cs, ar, ip);
 }
 // the inertial mass of a node from its slots' areas and phases (src/dt_mass.f90:74-154)
-GF_DEV double amass_sum(const GfDevParams *__restrict__ P, GfDevClock *ck, const CornerSlots &cs,
+GF_DEV double amass_sum(const GfDevParams *__restrict__ P, const DtScal &ds, const CornerSlots &cs,
                         const double (&ar)[4][3], const int (&ip)[4])
 {
     const double c1d12 = 1.0 / 12.0;
-    const double dlmin = __longlong_as_double((long long)ck->dlmin_bits);
-    const double vel_max = __longlong_as_double((long long)ck->velmax_bits);
-    const double dt_elastic = ck->dt_elastic;
+    const double dlmin = ds.dlmin, vel_max = ds.vel_max, dt_elastic = ds.dt_elastic;
     double pw[4];
 #pragma unroll
     for (int sl = 0; sl < 4; sl++) pw[sl] = cs.ok[sl] ? PHASE(ip[sl]).pwave : 0.0;
@@ -3316,9 +3362,9 @@ __global__ void __launch_bounds__(256) k_amass(const GfDevParams *__restrict__ P
     amass_body(P, ck, A, t, arp);
 }
 // rmasses and dt_mass's inertial masses in one pass, in a step that runs both (after
-// k_dens, k_dt_reduce and k_dt_scalars, none of which reads rmass): the node's areas
-// are loaded or formed once for both sums, each summed in its own kernel's order
-GF_DEV void masses_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long t, int arp)
+// k_dens, which does not read rmass): the node's areas are loaded or formed once for
+// both sums, each summed in its own kernel's order
+GF_DEV void masses_body(const GfDevParams *__restrict__ P, const DtScal &ds, const GfDevArrays &A, long t, int arp)
 {
     const int j = (int)((unsigned)t % (unsigned)NZ) + 1, i = (int)((unsigned)t / (unsigned)NZ) + 1;
     const double c1d12 = 1.0 / 12.0;
@@ -3340,12 +3386,30 @@ GF_DEV void masses_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const
 #pragma unroll
             for (int q = 0; q < 3; q++) sum = sum + c1d12 / ar[sl][q] * dn[sl];
     A.rmass[t] = sum;
-    A.amass[t] = P->idt_scale == 0 ? sum : amass_sum(P, ck, cs, ar, ip);  // (dt_mass.f90:66: amass = rmass)
+    A.amass[t] = P->idt_scale == 0 ? sum : amass_sum(P, ds, cs, ar, ip);  // (dt_mass.f90:66: amass = rmass)
 }
+// Every wave takes the maxima that k_dens left in A.dtred and forms dlmin and dt_elastic
+// from them; the first thread of the launch also stores them and dt (nothing else in the
+// launch reads those)
 __global__ void __launch_bounds__(256) k_masses(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
                                                 int arp)
 {
-    long t = xcd_lin();
+    static_assert(DTR_SLOTS == 64, "a cell a lane");
+    const int lane = threadIdx.x & 63;
+    double dly = __longlong_as_double((long long)A.dtred[lane * DTR_PAD]);
+    double vmax = __longlong_as_double((long long)A.dtred[lane * DTR_PAD + 1]);
+    for (int off = 32; off > 0; off >>= 1) {
+        dly = fmax(dly, __shfl_xor(dly, off));
+        vmax = fmax(vmax, __shfl_xor(vmax, off));
+    }
+    const double dlmin = dlmin_of(dly);
+    const DtScal ds{dlmin, vmax, dt_elastic_of(P, ck, dlmin)};
+    const long t = xcd_lin();
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ck->dly_bits = (unsigned long long)__double_as_longlong(dly);
+        ck->velmax_bits = (unsigned long long)__double_as_longlong(vmax);
+        dt_scalars_body(P, ck, dlmin);
+    }
     if (t >= NN) return;
-    masses_body(P, ck, A, t, arp);
+    masses_body(P, ds, A, t, arp);
 }

@@ -4,7 +4,7 @@
 // The reference loops over every marker, applies the pressure-temperature rules of
 // the marker's phase, flags the elements whose markers changed (itmp), then
 // recounts the phase ratios, the dominant phase and the plastic strain of the
-// flagged elements.  Here that is four launches every ifreq_rmasses steps:
+// flagged elements.  Here that is three launches every ifreq_rmasses steps:
 //
 //   k_phase_rules    one thread per element: unless bounds from the element's corners
 //                    show that no rule of a phase its markers may hold can fire, the
@@ -17,10 +17,9 @@
 //                    reference's loops over phases, so every phase mix adds in the
 //                    reference's order).  Phases that just appeared get a plane,
 //                    phases left in no element lose theirs; at most GF_MAXACT;
-//   k_phase_replane  one thread per element, when the plan changed: moves the
-//                    element's ratios to their new planes;
-//   k_phase_recount  one thread per element stamped by this call: counts its
-//                    markers per phase, writes the ratios, iphase and aps.
+//   k_phase_update   one thread per element: when the plan changed, moves the
+//                    element's ratios to their new planes; when this call stamped it,
+//                    counts its markers per phase, writes the ratios, iphase and aps.
 //
 // The rules read only the markers, cord, temp and the phase ratios of elements
 // below, none of which the rule pass writes, so the result is independent of the
@@ -96,38 +95,14 @@ GF_DEV bool phase_rule_may_fire(const GfDevParams *__restrict__ P, int iph, doub
     return phase_has_rule(iph);
 }
 
-// src/change_phase.f90:58-230 for marker kk
-GF_DEV void phase_rules_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long kk)
+// the new phase (0: none) of a marker of phase iph in element (j, i) at the given depth
+// and temperature, src/change_phase.f90:100-230
+GF_DEV int phase_rule(const GfDevParams *__restrict__ P, const GfDevArrays &A, int iph, int j, int i, double depth,
+                      double tmpr)
 {
-    if (A.mark_dead[kk] == 0) return;
-    const int iph = A.mark_phase[kk];
-    if (!phase_has_rule(iph)) return;
     const double max_basalt_depth = 150.e3, min_eclogite_temp = 400.0, min_eclogite_depth = 20e3,
                  mantle_density = 3000.0, max_melting_depth = 200.e3, serpentine_temp = 550.0;
-    const int n = A.mark_ntriag[kk];
-    const int k = (n - 1) % 2 + 1;
-    const int j = ((n - k) / 2) % (NZ - 1) + 1;
-    const int i = (n - k) / 2 / (NZ - 1) + 1;
-    // the marker's triangle: corners (c1, c2, c3) as the interpolation below weighs them
-    const int j1 = k == 1 ? j : j, i1 = k == 1 ? i : i + 1;
-    const int j3 = k == 1 ? j : j + 1, i3 = i + 1;
-    const double y1 = CORD(j1, i1, 2), y2 = CORD(j + 1, i, 2), y3 = CORD(j3, i3, 2);
-    const double t1 = TEMP(j1, i1), t2 = TEMP(j + 1, i), t3 = TEMP(j3, i3);
-    const double ysurf = 0.5 * (CORD(1, i, 2) + CORD(1, i + 1, 2));
-    // Markers whose rules cannot fire anywhere in their triangle are skipped before
-    // their barycentric coordinates are read.
-    {
-        const double tmax = fmax(fmax(t1, t2), t3);
-        const double ylo = fmin(fmin(y1, y2), y3), yhi = fmax(fmax(y1, y2), y3);
-        const double dm = 1e-6 * (fabs(ysurf) + fabs(ylo) + fabs(yhi) + 1.0), tm = 1e-9 * (fabs(tmax) + 1.0);
-        const double dlo = ysurf - yhi - dm, dhi = ysurf - ylo + dm;  // depth range
-        if (!phase_rule_may_fire(P, iph, dlo, dhi, tmax, tm)) return;
-    }
-    const double a1 = A.mark_a1[kk], a2 = A.mark_a2[kk];
-    const double yy = y1 * a1 + y2 * a2 + y3 * (1 - a1 - a2);
-    const double tmpr = t1 * a1 + t2 * a2 + t3 * (1 - a1 - a2);
-    const double depth = ysurf - yy;
-    if (depth > max_melting_depth) return;
+    if (depth > max_melting_depth) return 0;
     int newph = 0;
     double trpres, trpres2, press;
     switch (iph) {
@@ -199,11 +174,46 @@ GF_DEV void phase_rules_body(const GfDevParams *__restrict__ P, GfDevClock *ck, 
     default:
         break;
     }
-    if (newph) {
-        A.mark_phase[kk] = (signed char)newph;
-        A.phstamp[IE(j, i)] = ck->ph_call + 1;  // every changing marker of the element writes the same
-        atomicOr(&ck->ph_newmask, 1u << (newph - 1));
+    return newph;
+}
+GF_DEV void phase_set(GfDevClock *ck, const GfDevArrays &A, long kk, long e, int newph)
+{
+    A.mark_phase[kk] = (signed char)newph;
+    A.phstamp[e] = ck->ph_call + 1;  // every changing marker of the element writes the same
+    atomicOr(&ck->ph_newmask, 1u << (newph - 1));
+}
+
+// src/change_phase.f90:58-230 for marker kk
+GF_DEV void phase_rules_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long kk)
+{
+    if (A.mark_dead[kk] == 0) return;
+    const int iph = A.mark_phase[kk];
+    if (!phase_has_rule(iph)) return;
+    const int n = A.mark_ntriag[kk];
+    const int k = (n - 1) % 2 + 1;
+    const int j = ((n - k) / 2) % (NZ - 1) + 1;
+    const int i = (n - k) / 2 / (NZ - 1) + 1;
+    // the marker's triangle: corners (c1, c2, c3) as the interpolation below weighs them
+    const int j1 = k == 1 ? j : j, i1 = k == 1 ? i : i + 1;
+    const int j3 = k == 1 ? j : j + 1, i3 = i + 1;
+    const double y1 = CORD(j1, i1, 2), y2 = CORD(j + 1, i, 2), y3 = CORD(j3, i3, 2);
+    const double t1 = TEMP(j1, i1), t2 = TEMP(j + 1, i), t3 = TEMP(j3, i3);
+    const double ysurf = 0.5 * (CORD(1, i, 2) + CORD(1, i + 1, 2));
+    // Markers whose rules cannot fire anywhere in their triangle are skipped before
+    // their barycentric coordinates are read.
+    {
+        const double tmax = fmax(fmax(t1, t2), t3);
+        const double ylo = fmin(fmin(y1, y2), y3), yhi = fmax(fmax(y1, y2), y3);
+        const double dm = 1e-6 * (fabs(ysurf) + fabs(ylo) + fabs(yhi) + 1.0), tm = 1e-9 * (fabs(tmax) + 1.0);
+        const double dlo = ysurf - yhi - dm, dhi = ysurf - ylo + dm;  // depth range
+        if (!phase_rule_may_fire(P, iph, dlo, dhi, tmax, tm)) return;
     }
+    const double a1 = A.mark_a1[kk], a2 = A.mark_a2[kk];
+    const double yy = y1 * a1 + y2 * a2 + y3 * (1 - a1 - a2);
+    const double tmpr = t1 * a1 + t2 * a2 + t3 * (1 - a1 - a2);
+    const double depth = ysurf - yy;
+    const int newph = phase_rule(P, A, iph, j, i, depth, tmpr);
+    if (newph) phase_set(ck, A, kk, IE(j, i), newph);
 }
 
 __global__ void __launch_bounds__(256) k_phase_rules_mk(const GfDevParams *__restrict__ P, GfDevClock *ck,
@@ -229,14 +239,54 @@ GF_DEV void phase_rules_elem_body(const GfDevParams *__restrict__ P, GfDevClock 
     const double ylo = fmin(fmin(y1, y2), fmin(y3, y4)), yhi = fmax(fmax(y1, y2), fmax(y3, y4));
     const double dm = 1e-6 * (fabs(ysurf) + fabs(ylo) + fabs(yhi) + 1.0), tm = 1e-9 * (fabs(tmax) + 1.0);
     const double dlo = ysurf - yhi - dm, dhi = ysurf - ylo + dm;
-    // the phases markers may hold, lowest id first (the plane lookup once per element)
+    // the phases markers may hold whose rules may fire (the plane lookup once per element)
     const int sed_ocean = phase_sed_ocean(P) ? 1 : 0;
-    bool may = false;
-    for (unsigned m = present; m != 0u && !may; m &= m - 1u)
-        may = phase_rule_may_fire(P, __ffs(m), dlo, dhi, tmax, tm, sed_ocean);
-    if (!may) return;
+    unsigned fire = 0u;
+    for (unsigned m = present; m != 0u; m &= m - 1u)
+        if (phase_rule_may_fire(P, __ffs(m), dlo, dhi, tmax, tm, sed_ocean)) fire |= m & (0u - m);
+    if (!fire) return;
     const int nm = A.nmark_elem[e];
-    for (int q = 0; q < nm; q++) phase_rules_body(P, ck, A, (long)A.mark_id_elem[q + (long)GF_MAX_MARKERS_PER_ELEM * e] - 1);
+    // Markers three at a time, each level of their loads together (list, marker, its
+    // coordinates): the chain of loads bounds an element whose rules may fire.  The
+    // corners of a marker's triangle are the element's.
+    constexpr int MK = 3;
+    for (int q0 = 0; q0 < nm; q0 += MK) {
+        long kk[MK];
+        int iph[MK], n[MK];
+        bool go[MK];
+#pragma unroll
+        for (int u = 0; u < MK; u++) kk[u] = q0 + u < nm ? (long)A.mark_id_elem[q0 + u + (long)GF_MAX_MARKERS_PER_ELEM * e] - 1 : -1;
+#pragma unroll
+        for (int u = 0; u < MK; u++) {
+            go[u] = kk[u] >= 0;
+            iph[u] = n[u] = 0;
+            if (go[u]) {
+                go[u] = A.mark_dead[kk[u]] != 0;
+                iph[u] = A.mark_phase[kk[u]];
+                n[u] = A.mark_ntriag[kk[u]];
+            }
+        }
+        double a1[MK], a2[MK];
+#pragma unroll
+        for (int u = 0; u < MK; u++) {
+            go[u] = go[u] && iph[u] >= 1 && iph[u] <= GF_MAXPH && ((fire >> (iph[u] - 1)) & 1u);
+            a1[u] = a2[u] = 0.0;
+            if (go[u]) {
+                a1[u] = A.mark_a1[kk[u]];
+                a2[u] = A.mark_a2[kk[u]];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < MK; u++) {
+            if (!go[u]) continue;
+            const bool k1 = (n[u] - 1) % 2 == 0;  // triangle 1 or 2 of the element
+            const double c1y = k1 ? y1 : y3, c3y = k1 ? y3 : y4, c1t = k1 ? t1 : t3, c3t = k1 ? t3 : t4;
+            const double yy = c1y * a1[u] + y2 * a2[u] + c3y * (1 - a1[u] - a2[u]);
+            const double tmpr = c1t * a1[u] + t2 * a2[u] + c3t * (1 - a1[u] - a2[u]);
+            const int newph = phase_rule(P, A, iph[u], j, i, ysurf - yy, tmpr);
+            if (newph) phase_set(ck, A, kk[u], e, newph);
+        }
+    }
 }
 
 __global__ void __launch_bounds__(256) k_phase_rules(const GfDevParams *__restrict__ P, GfDevClock *ck,
@@ -311,15 +361,6 @@ GF_DEV void phase_replane_body(const GfDevParams *__restrict__ P, const GfDevClo
     for (int b = 0; b < nnew; b++) A.pr[b * ne + e] = w[b];
 }
 
-__global__ void __launch_bounds__(256) k_phase_replane(const GfDevParams *__restrict__ P, const GfDevClock *ck,
-                                                       GfDevArrays A)
-{
-    if (!ck->ph_replan) return;
-    const long e = xcd_lin();
-    if (e >= NE) return;
-    phase_replane_body(P, ck, A, e);
-}
-
 // src/change_phase.f90:247-260 with count_phase_ratio (src/marker_data.f90:140-174);
 // aps_share 0: count_phase_ratio alone (resurface, src/fl_move.f90:413-416)
 GF_DEV void phase_recount_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long e,
@@ -392,10 +433,12 @@ __global__ void __launch_bounds__(256) k_iphx(const GfDevParams *__restrict__ P,
     iphx_body(P, A, e);
 }
 
-__global__ void __launch_bounds__(256) k_phase_recount(const GfDevParams *__restrict__ P, GfDevClock *ck,
-                                                       GfDevArrays A, int aps_share)
+// an element's ratios to their new planes (when the plan changed), then its recount
+__global__ void __launch_bounds__(256) k_phase_update(const GfDevParams *__restrict__ P, GfDevClock *ck,
+                                                      GfDevArrays A, int aps_share)
 {
     const long e = xcd_lin();
     if (e >= NE) return;
+    if (ck->ph_replan) phase_replane_body(P, ck, A, e);
     phase_recount_body(P, ck, A, e, aps_share);
 }

@@ -377,6 +377,7 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
     ctx->a.tbord = ctx->therm_border;
     ALLOC(ctx->a.tpre, 8 * (size_t)GF_NPRE * 2 * (p->nx + p->nz));
     ALLOC(ctx->a.dens, 8 * ne);
+    ALLOC(ctx->a.dtred, 8 * DTR_SLOTS * DTR_PAD);
     ALLOC(ctx->a.iphx, 4 * ne);
     if (hipMemset(ctx->a.iphx, 0, 4 * ne) != hipSuccess) {
         rc = set_err(ctx, GF_ERR_HIP, "hipMemset failed");
@@ -422,7 +423,7 @@ extern "C" void gf_destroy(gf_ctx *ctx)
                     ctx->a.force, ctx->a.amass, ctx->a.rmass, ctx->a.bc, ctx->a.ncod, ctx->a.stress0,
                     ctx->a.area, ctx->a.dvol, ctx->a.strain, ctx->a.se2sr, ctx->a.aps, ctx->a.visn,
                     ctx->a.e2sr, ctx->a.sshrheat, ctx->a.shrheat, ctx->a.source, ctx->a.iphase, ctx->a.pr,
-                    ctx->a.xa, ctx->a.xb, ctx->a.dens, ctx->therm_border, ctx->a.tpre, ctx->a.stress0f, ctx->a.velf,
+                    ctx->a.xa, ctx->a.xb, ctx->a.dens, ctx->a.dtred, ctx->therm_border, ctx->a.tpre, ctx->a.stress0f, ctx->a.velf,
                     ctx->a.forcef, ctx->a.pref, ctx->sur_samples, ctx->sur_w, ctx->sur_m, ctx->sur_v,
                     ctx->sur_grad, ctx->sur_partial, ctx->sur_cfg, ctx->sur_stats, ctx->sur_list,
                     ctx->sur_cnt, ctx->sur_lval, ctx->sur_wgs, ctx->cord_alt, ctx->out_buf, ctx->a.mark_age,
@@ -1420,49 +1421,49 @@ static int enq_move(gf_ctx *ctx)
     return GF_OK;
 }
 
-// dtb: k_dens also starts the dt minima of a dt_mass that follows (enq_masses)
-static int enq_rmasses(gf_ctx *ctx, int dtb = 0)
+// dtr: k_dens also takes dt_mass's maxima for the k_masses that follows (enq_masses)
+static int enq_rmasses(gf_ctx *ctx, bool dtr = false)
 {
     // the masses form pending areas from the moved coordinates (corner_areas)
     const int arp = ctx->area_pending ? 1 : 0;
     // Eff_dens rotates the stress it reads by a pending move itself (the move stays
     // pending for the next fl_rheol)
     const int rot = ctx->rot_pending ? 1 : 0;
-    if (ctx->precision == GF_PREC_MIXED)
-        LAUNCH_NAMED("k_dens<float>", k_dens<1>, ctx->ne, ctx->dp, ctx->dck, ctx->a, rot, dtb);
-    else if (ctx->precision == GF_PREC_MIXED_STORAGE)
-        LAUNCH_NAMED("k_dens<float>", k_dens<2>, ctx->ne, ctx->dp, ctx->dck, ctx->a, rot, dtb);
-    else
-        LAUNCH_NAMED("k_dens<double>", k_dens<0>, ctx->ne, ctx->dp, ctx->dck, ctx->a, rot, dtb);
-    if (!dtb) LAUNCH(k_rmass, ctx->nn, ctx->dp, ctx->dck, ctx->a, arp);
+    const int M = ctx->precision == GF_PREC_MIXED ? 1 : ctx->precision == GF_PREC_MIXED_STORAGE ? 2 : 0;
+    auto kern = dtr ? (M == 1 ? k_dens<1, true> : M == 2 ? k_dens<2, true> : k_dens<0, true>)
+                    : (M == 1 ? k_dens<1, false> : M == 2 ? k_dens<2, false> : k_dens<0, false>);
+    LAUNCH_NAMED(M == 0 ? "k_dens<double>" : "k_dens<float>", kern, ctx->ne, ctx->dp, ctx->dck, ctx->a, rot, arp);
+    if (!dtr) LAUNCH(k_rmass, ctx->nn, ctx->dp, ctx->dck, ctx->a, arp);
     return GF_OK;
 }
 
+// workgroups of a reduction over the elements (four elements a thread, at most DT_RED_BLOCKS)
+static long dt_red_threads(const gf_ctx *ctx)
+{
+    return std::min<long>(DT_RED_BLOCKS, (ctx->ne + 1023) / 1024) * 256;
+}
 static int enq_dt_mass(gf_ctx *ctx)
 {
     int rc;
     // the dt minima and inertial masses form pending areas from the moved coordinates
     const int arp = ctx->area_pending ? 1 : 0;
     if ((rc = enq_clock(ctx, CK_DT_BEGIN))) return rc;
-    LAUNCH_SV(k_dt_reduce, (long)DT_RED_BLOCKS * 256, ctx->dp, ctx->dck, ctx->a, arp);
+    LAUNCH_SV(k_dt_reduce, dt_red_threads(ctx), ctx->dp, ctx->dck, ctx->a, arp);
     hipLaunchKernelGGL(k_dt_scalars, dim3(1), dim3(64), 0, ctx->stream, ctx->dp, ctx->dck);
     if ((rc = launch_check(ctx, "k_dt_scalars"))) return rc;
     LAUNCH(k_amass, ctx->nn, ctx->dp, ctx->dck, ctx->a, arp);
     return GF_OK;
 }
 
-// rmasses and dt_mass of one step (src/flac.f90:68-72) with one pass over the nodes
-// for both masses: k_dens (which also starts the dt minima), k_dt_reduce,
-// k_dt_scalars, then k_masses (rmass and amass; dt_mass does not read rmass except as
-// amass = rmass, src/dt_mass.f90:66)
+// rmasses and dt_mass of one step (src/flac.f90:68-72) in two launches: k_dens with
+// dt_mass's maxima, then k_masses, which forms the dt scalars from them and both masses in
+// one pass over the nodes (dt_mass reads rmass only as amass = rmass,
+// src/dt_mass.f90:66)
 static int enq_masses(gf_ctx *ctx)
 {
     int rc;
     const int arp = ctx->area_pending ? 1 : 0;
-    if ((rc = enq_rmasses(ctx, 1))) return rc;
-    LAUNCH_SV(k_dt_reduce, (long)DT_RED_BLOCKS * 256, ctx->dp, ctx->dck, ctx->a, arp);
-    hipLaunchKernelGGL(k_dt_scalars, dim3(1), dim3(64), 0, ctx->stream, ctx->dp, ctx->dck);
-    if ((rc = launch_check(ctx, "k_dt_scalars"))) return rc;
+    if ((rc = enq_rmasses(ctx, true))) return rc;
     LAUNCH(k_masses, ctx->nn, ctx->dp, ctx->dck, ctx->a, arp);
     return GF_OK;
 }
@@ -1534,8 +1535,7 @@ static int enq_change_phase(gf_ctx *ctx)
     hipLaunchKernelGGL(k_phase_plan, dim3(1), dim3(64), 0, ctx->stream, ctx->dp, ctx->dck);
     int rc = launch_check(ctx, "k_phase_plan");
     if (rc) return rc;
-    LAUNCH(k_phase_replane, ctx->ne, ctx->dp, ctx->dck, ctx->a);
-    LAUNCH(k_phase_recount, ctx->ne, ctx->dp, ctx->dck, ctx->a, 1);
+    LAUNCH(k_phase_update, ctx->ne, ctx->dp, ctx->dck, ctx->a, 1);
     return GF_OK;
 }
 
@@ -1551,8 +1551,7 @@ static int enq_diff_topo(gf_ctx *ctx)
     if ((rc = launch_check(ctx, "k_resurface"))) return rc;
     hipLaunchKernelGGL(k_phase_plan, dim3(1), dim3(64), 0, ctx->stream, ctx->dp, ctx->dck);
     if ((rc = launch_check(ctx, "k_phase_plan"))) return rc;
-    LAUNCH(k_phase_replane, ctx->ne, ctx->dp, ctx->dck, ctx->a);
-    LAUNCH(k_phase_recount, ctx->ne, ctx->dp, ctx->dck, ctx->a, 0);
+    LAUNCH(k_phase_update, ctx->ne, ctx->dp, ctx->dck, ctx->a, 0);
     return GF_OK;
 }
 
@@ -1584,10 +1583,12 @@ static int enq_flac(gf_ctx *ctx, int pending = 0, bool last = true)
         if ((rc = enq_rheol(ctx, true, last))) return rc;
         if (defer && (rc = enq_therm_rest(ctx))) return rc;
         if (ctx->p.nystressbc == 1 && (rc = enq_bc_update(ctx))) return rc;
+        const bool rm = phases, im = ctx->nloop % ctx->p.ifreq_imasses == 0;
+        const bool both = rm && im && !ctx->node_direct;
+        if (both) ctx->node_ops |= CK_DT_BEGIN;  // (fl_node starts dt_mass's maxima)
         if ((rc = enq_node(ctx, true))) return rc;
         if ((rc = enq_move(ctx))) return rc;
-        const bool rm = ctx->nloop % ctx->p.ifreq_rmasses == 0, im = ctx->nloop % ctx->p.ifreq_imasses == 0;
-        if (rm && im) {
+        if (both) {
             if ((rc = enq_masses(ctx))) return rc;
         } else {
             if (rm && (rc = enq_rmasses(ctx))) return rc;
@@ -2600,8 +2601,7 @@ static int enq_batch_flac(gf_batch *b)
         if (b->markers && b->nloop % p.ifreq_rmasses == 0) {  // change_phase
             if (b->tot_m > 0) BLAUNCH(kb_phase_rules, bgrid(b->tot_m, 256), 256, b->dtab, map);
             BLAUNCH(kb_phase_plan, gm, 64, b->dtab, map);
-            BLAUNCH(kb_phase_replane, bgrid(b->tot_e, 256), 256, b->dtab, map);
-            BLAUNCH(kb_phase_recount, bgrid(b->tot_e, 256), 256, b->dtab, map);
+            BLAUNCH(kb_phase_update, bgrid(b->tot_e, 256), 256, b->dtab, map);
         }
         const int rot = (b->rot_pending ? RH_ROT : 0) | (b->area_pending ? RH_AREA : 0);
         if (do_visc) BLAUNCH(kb_visc<M>, bgrid(b->tot_e, 256), 256, b->dtab, map, (rot & RH_ROT) ? 1 : 0);

@@ -12,10 +12,18 @@
 #include "gf_kernels.h"
 #include "gf_phase.h"
 
+// The temperature turns over three buffers and the coordinates two, as in a model alone,
+// but in the table: kb_begin turns them at the start of each step, so that a captured step
+// can be replayed.  Within a step A.temp is the step's result (formed by the thermal
+// launches) and A.temp0 its old temperature; A.cord are the coordinates before the move and
+// cord_next those after it (the current ones between steps; where the grid does not move,
+// A.cord throughout).
 struct BatchEntry {
     const GfDevParams *P;
     GfDevClock *ck;
     GfDevArrays A;
+    double *tprev;      // the starting temperature of the call before (the next call's result)
+    double *cord_next;
     long pe, pn, pt, pb, pm;  // first global index: elements, nodes, thermal tiles, border entries, markers
     long ce, cn, ct, cb, cm;  // counts of the same
 };
@@ -78,23 +86,133 @@ __global__ void kb_clock(const BatchEntry *__restrict__ tab, BatchMap map, int o
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m < map.nm) clock_op(tab[m].ck, op);
 }
-
-__global__ void __launch_bounds__(1024) kb_therm_tile(const BatchEntry *__restrict__ tab, BatchMap map, long total,
-                                                      int pass)
+// the boundary values that earlier thermal calls left are not this batch's
+__global__ void kb_fresh(const BatchEntry *__restrict__ tab, BatchMap map)
 {
-    for (long g = blockIdx.x; g < total; g += gridDim.x) {
-        const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_TILE][g]));
-        if (pass > 0 && b.ck->therm_pass_changed[pass - 1] == 0u) continue;  // this model is proven
-        therm_tile_one(b.P, b.ck, b.A, pass, (int)(g - b.pt));
+    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (m < map.nm) tab[m].ck->th_hist = 0;
+}
+// the start of a step: clock updates, the buffers turned over (cord: the coordinates
+// too), the thermal calls counted
+__global__ void kb_begin(BatchEntry *tab, BatchMap map, int op, int cord)
+{
+    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= map.nm) return;
+    BatchEntry &b = tab[m];
+    clock_op(b.ck, op);
+    b.ck->th_call = (b.ck->th_call + 1) % 3;
+    b.ck->th_hist = min(b.ck->th_hist + 1, 3);
+    double *t = b.tprev;
+    b.tprev = b.A.temp0;
+    b.A.temp0 = b.A.temp;
+    b.A.temp = t;
+    if (cord) {
+        double *c = b.A.cord;
+        b.A.cord = b.cord_next;
+        b.cord_next = c;
     }
 }
 
-// the thermal pipeline over the tiles of all models (k_therm_pipe, one workgroup per
-// CU walking a list of tiles); a tile of a model that is already proven only passes
-// the prefetch on
-template <int XIN, bool DIS>
+// the arrays as the thermal kernels name them (temp the old temperature, xa the result,
+// temp0 the call before's old temperature), and as the kernels after the move do
+GF_DEV GfDevArrays bthermal(const BatchEntry &b)
+{
+    GfDevArrays A = b.A;
+    A.temp = b.A.temp0;
+    A.xa = b.A.temp;
+    A.temp0 = b.tprev;
+    return A;
+}
+GF_DEV GfDevArrays bmoved(const BatchEntry &b)
+{
+    GfDevArrays A = b.A;
+    A.cord = b.cord_next;
+    return A;
+}
+GF_DEV ThermSlots bslots(const BatchEntry &b) { return therm_slots(b.ck->th_call, b.ck->th_hist - 1); }
+
+// The proven thermal step of every model (k_therm_strip, k_therm_check, k_therm_rest):
+// one wave a strip over the strips of all models
+template <bool DIS, int MODE>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+kb_therm_strip(const BatchEntry *__restrict__ tab, BatchMap map, int total, int w, int arp)
+{
+    __shared__ double sPh[4][GF_MAXPH];
+    const int q = (total + 7) / 8, g = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= q || g >= total) return;
+    const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_TILE][g]));
+    const GfDevArrays A = bthermal(b);
+    therm_phase_table(b.P, sPh);
+    const ThermIter it{A.xb, A.xa, arp, 0};
+    const int t = g - (int)b.pt;
+    therm_strip<DIS, MODE>(b.P, b.ck, A, therm_geo(b.P, w), t, it, bslots(b), A.tbord + (long)t * TS_NB(w), b.ck->dt,
+                           sPh);
+}
+__global__ void __launch_bounds__(256) kb_therm_check(const BatchEntry *__restrict__ tab, BatchMap map, int w, int arp)
+{
+    batch_apply<BK_BORD>(tab, map, [&](const BatchEntry &b, long t) {
+        therm_check_one(b.P, b.ck, bthermal(b), therm_geo(b.P, w), t, 0, arp, bslots(b));
+    });
+}
+// Returns at once when every model's pass 0 is proven.  Otherwise the further passes of
+// the models that are not, with grid barriers on the first model's counters (one workgroup
+// per CU at most, as k_therm_rest).
+template <bool DIS>
+__global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restrict__ tab, BatchMap map, int total, int w,
+                                                     long border, int arp, int npass)
+{
+    auto flag = [&](int m, int pass) {  // written by other workgroups of this launch too
+        return __hip_atomic_load(&tab[m].ck->therm_pass_changed[pass], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // whether a model's pass is not proven (nor any before it: later flags stay 0 then)
+    auto open_after = [&](int pass) {
+        int any = 0;
+        for (int m = threadIdx.x; m < map.nm; m += 256) any |= flag(m, pass) != 0u;
+        return __syncthreads_or(any) != 0;
+    };
+    if (!open_after(0)) return;
+    __shared__ double sPhw[4][4][GF_MAXPH];
+    double(*sPh)[GF_MAXPH] = sPhw[threadIdx.x / 64];
+    GfDevClock *bar = tab[0].ck;
+    const long tid = (long)blockIdx.x * 256 + threadIdx.x, nthr = (long)gridDim.x * 256;
+    for (int pass = 1; pass < npass; pass++) {
+        for (int g = (int)(tid / 64); g < total; g += (int)(nthr / 64)) {
+            const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_TILE][g]));
+            if (__hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
+                continue;
+            const GfDevArrays A = bthermal(b);
+            therm_phase_table(b.P, sPh);
+            const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, arp, pass};
+            const int t = g - (int)b.pt;
+            therm_strip<DIS, 1>(b.P, b.ck, A, therm_geo(b.P, w), t, it, bslots(b), A.tbord + (long)t * TS_NB(w),
+                                b.ck->dt, sPh);
+        }
+        if (!grid_sync(bar)) return;  // every strip's iterate is written
+        for (long g = (long)blockIdx.x * 256; g < border; g += nthr) {
+            const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_BORD][g / BATCH_ALIGN]));
+            const long t = g + threadIdx.x - b.pb;
+            if (t < b.cb &&
+                __hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)
+                therm_check_one(b.P, b.ck, bthermal(b), therm_geo(b.P, w), t, pass, arp, bslots(b));
+        }
+        if (!grid_sync(bar)) return;  // every border is checked
+        if (!open_after(pass)) break;
+    }
+    for (int m = 0; m < map.nm; m++) {
+        if (flag(m, 0) == 0u) continue;
+        int proven = -1;
+        for (int k = npass - 1; k >= 0; k--)
+            if (flag(m, k) == 0u) proven = k;
+        if (tid == 0) therm_outcome(tab[m].ck, proven);
+        therm_settle(tab[m].P, bthermal(tab[m]), bslots(tab[m]), proven < 0 ? npass - 1 : proven, tid, nthr);
+    }
+}
+
+// FP32-arithmetic mode: the thermal pipeline over the tiles of all models (k_therm_pipe,
+// one workgroup per CU walking a list of tiles)
+template <bool DIS>
 __global__ void __launch_bounds__(1024) kb_therm_pipe(const BatchEntry *__restrict__ tab, BatchMap map, long total,
-                                                      int pass, double stol, int arp)
+                                                      double stol, int arp, int fold)
 {
     __shared__ ThermRaw raw;
     __shared__ double sU[TH_NF * TH_NE];
@@ -105,28 +223,21 @@ __global__ void __launch_bounds__(1024) kb_therm_pipe(const BatchEntry *__restri
     auto entry = [&](long t) -> const BatchEntry & { return bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_TILE][t])); };
     {
         const BatchEntry &b = entry(first);
-        therm_store_raw<XIN, DIS>(therm_prefetch<XIN, DIS>(b.P, b.ck, b.A, pass, (int)(first - b.pt), arp), raw);
+        therm_store_raw<DIS>(therm_prefetch<DIS>(b.P, b.ck, bthermal(b), (int)(first - b.pt), arp), raw);
     }
     for (long t = first; t < end; t += RW) {
         lds_barrier();  // this tile's inputs are in; the previous tile is done with sU
         const BatchEntry &b = entry(t);
         const long tn = t + RW;
         const BatchEntry &bn = entry(tn < end ? tn : t);
-        therm_tile_pipe<XIN, DIS>(b.P, b.ck, b.A, pass, (int)(t - b.pt), bn.P, bn.ck, bn.A,
-                                  tn < end ? (int)(tn - bn.pt) : -1, raw, sU, sFlag, stol, arp);
+        therm_tile_pipe<DIS>(b.P, b.ck, bthermal(b), (int)(t - b.pt), bn.P, bn.ck, bthermal(bn),
+                             tn < end ? (int)(tn - bn.pt) : -1, raw, sU, sFlag, stol, arp, fold);
     }
 }
-
-__global__ void __launch_bounds__(256) kb_therm_check(const BatchEntry *__restrict__ tab, BatchMap map, int pass)
+// its boundary conditions where the tiles do not apply them
+__global__ void __launch_bounds__(256) kb_therm_bc(const BatchEntry *__restrict__ tab, BatchMap map)
 {
-    batch_apply<BK_BORD>(tab, map, [&](const BatchEntry &b, long t) { therm_check_body(b.P, b.ck, b.A, pass, t); });
-}
-
-__global__ void __launch_bounds__(256) kb_therm_bc(const BatchEntry *__restrict__ tab, BatchMap map, int passes,
-                                                   int proof)
-{
-    batch_apply<BK_NODE>(tab, map,
-                         [&](const BatchEntry &b, long t) { therm_bc_body(b.P, b.ck, b.A, t, passes, proof); });
+    batch_apply<BK_NODE>(tab, map, [&](const BatchEntry &b, long t) { therm_bc_node(b.P, bthermal(b), t); });
 }
 
 template <int M>
@@ -145,63 +256,58 @@ __global__ void __launch_bounds__(256) kb_rheol(const BatchEntry *__restrict__ t
     });
 }
 
+// move: the coordinates move into cord_next as the node has its velocity (and the move's
+// dt is recorded, for the rotation and the areas left pending)
 template <int M>
-__global__ void __launch_bounds__(256) kb_node(const BatchEntry *__restrict__ tab, BatchMap map)
-{
-    batch_apply<BK_NODE>(tab, map, [&](const BatchEntry &b, long t) { node_body<M>(b.P, b.ck, b.A, t); });
-}
-
-// also records each model's move dt (for a rotation and areas left pending)
-template <typename SV>
-__global__ void __launch_bounds__(256) kb_move_cord(const BatchEntry *__restrict__ tab, BatchMap map)
+__global__ void __launch_bounds__(256) kb_node(const BatchEntry *__restrict__ tab, BatchMap map, int move)
 {
     batch_apply<BK_NODE>(tab, map, [&](const BatchEntry &b, long t) {
-        move_cord_body<SV>(b.P, b.ck, b.A, t);
-        if (t == 0) b.ck->dt_move = b.ck->dt;
+        node_body<M>(b.P, b.ck, b.A, t, move ? b.cord_next : nullptr);
+        if (move && t == 0) b.ck->dt_move = b.ck->dt;
     });
-}
-
-template <int M>
-__global__ void __launch_bounds__(256) kb_move_elem(const BatchEntry *__restrict__ tab, BatchMap map)
-{
-    batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) { move_elem_body<M>(b.P, b.ck, b.A, e); });
-}
-// the areas, dvol and negative-area STOP of the move (the rotation is left to kb_rheol)
-__global__ void __launch_bounds__(256) kb_move_area(const BatchEntry *__restrict__ tab, BatchMap map)
-{
-    batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) { move_area_body(b.P, b.ck, b.A, e, 0); });
 }
 // the negative-area STOP of moves whose areas are still pending (coordinates only)
 __global__ void __launch_bounds__(256) kb_area_check(const BatchEntry *__restrict__ tab, BatchMap map)
 {
-    batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) { area_check_body(b.P, b.ck, b.A, e); });
+    batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) { area_check_body(b.P, b.ck, bmoved(b), e); });
 }
 
+// the masses and dt minima after the step's move (arp: its areas are pending)
 template <int M>
 __global__ void __launch_bounds__(256) kb_dens(const BatchEntry *__restrict__ tab, BatchMap map, int rot)
 {
-    batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) { dens_body<M>(b.P, b.ck, b.A, e, rot); });
+    batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) { dens_body<M>(b.P, b.ck, bmoved(b), e, rot); });
 }
 
-__global__ void __launch_bounds__(256) kb_rmass(const BatchEntry *__restrict__ tab, BatchMap map)
+__global__ void __launch_bounds__(256) kb_rmass(const BatchEntry *__restrict__ tab, BatchMap map, int arp)
 {
-    batch_apply<BK_NODE>(tab, map, [&](const BatchEntry &b, long t) { rmass_body(b.P, b.ck, b.A, t); });
+    batch_apply<BK_NODE>(tab, map, [&](const BatchEntry &b, long t) { rmass_body(b.P, b.ck, bmoved(b), t, arp); });
 }
 
-__global__ void __launch_bounds__(256) kb_amass(const BatchEntry *__restrict__ tab, BatchMap map)
+__global__ void __launch_bounds__(256) kb_amass(const BatchEntry *__restrict__ tab, BatchMap map, int arp)
 {
-    batch_apply<BK_NODE>(tab, map, [&](const BatchEntry &b, long t) { amass_body(b.P, b.ck, b.A, t); });
+    batch_apply<BK_NODE>(tab, map, [&](const BatchEntry &b, long t) { amass_body(b.P, b.ck, bmoved(b), t, arp); });
+}
+// both masses, with the dt scalars from the maxima of kb_dt_reduce (k_masses)
+__global__ void __launch_bounds__(256) kb_masses(const BatchEntry *__restrict__ tab, BatchMap map, int arp)
+{
+    batch_apply<BK_NODE>(tab, map, [&](const BatchEntry &b, long t) {
+        const double dlmin = dlmin_of(__longlong_as_double((long long)b.ck->dly_bits));
+        const DtScal ds{dlmin, __longlong_as_double((long long)b.ck->velmax_bits), dt_elastic_of(b.P, b.ck, dlmin)};
+        if (t == 0) dt_scalars_body(b.P, b.ck, dlmin);  // (nothing else here reads what it stores)
+        masses_body(b.P, ds, bmoved(b), t, arp);
+    });
 }
 
 // dt minima: `per` workgroups of 256 threads per model
 #define BATCH_DT_BLOCKS 16
 template <typename SV>
-__global__ void __launch_bounds__(256) kb_dt_reduce(const BatchEntry *__restrict__ tab, BatchMap map)
+__global__ void __launch_bounds__(256) kb_dt_reduce(const BatchEntry *__restrict__ tab, BatchMap map, int arp)
 {
     const int m = blockIdx.x / BATCH_DT_BLOCKS;
     if (m >= map.nm) return;
     const BatchEntry &b = bentry(tab, m);
-    dt_reduce_body<SV>(b.P, b.ck, b.A, blockIdx.x % BATCH_DT_BLOCKS, BATCH_DT_BLOCKS);
+    dt_reduce_body<SV>(b.P, b.ck, bmoved(b), blockIdx.x % BATCH_DT_BLOCKS, BATCH_DT_BLOCKS, arp);
 }
 
 __global__ void kb_dt_scalars(const BatchEntry *__restrict__ tab, BatchMap map)

@@ -80,6 +80,9 @@ struct GfDevClock {
     // dt_mass's minimum side measure as the largest product area x side length over
     // the elements (bits of a non-negative double); dlmin is its reciprocal
     unsigned long long dly_bits;
+    // a batch's thermal calls: their number modulo 3, and how many before this one left
+    // their boundary values (0..2, counted one ahead)
+    int th_call, th_hist;
     // itest_mesh's smallest triangle angle, as an order-preserving key (rem_angle_key)
     unsigned long long rem_key;
 };

@@ -161,26 +161,15 @@ __global__ void k_math_check(const double *x, const double *y, double *out, long
 // A sweep evaluates that same formula at every node, taking the new values from
 // the previous iterate X (X_0 = old temp).  The map is lower-triangular in the
 // serial order, so its only fixed point is the serial result, and a sweep that
-// changes no bit proves it has been reached.  Sweeps run inside a workgroup on a
-// tile of 64 x 16 nodes held in LDS, with halos of TH_HJ rows above and below and
-// TH_HI columns to the left (the coupling to the previous column is ~(dz/dx)^2
-// weaker); the per-node coefficients of the six triangles are formed once, in the
-// reference's order, and kept in registers.  A tile iterates until it is still.
-// Proof without a second full pass: when a tile is still, every node of its output
-// region is a fixed point of the map evaluated with the tile's own values of its
-// neighbours.  The output nodes' neighbours outside the output region (the row above,
-// the column to the left and the row below it, 2*TH_OI + TH_OJ nodes) are halo nodes
-// whose tile values are saved to a border buffer; k_therm_check compares them with
-// the values their owning tiles wrote.  If all are bit-equal, the assembled global
-// iterate is a fixed point of the global map at every node, hence the serial result.
-// Otherwise another pass starts from the assembled iterate (halos now near exact).
-// Tiles are numbered so that each XCD runs a contiguous range of column-major tiles,
-// which keeps the halo re-reads of neighbouring tiles in the same L2.
-// Halo sizes: each halo row damps the influence of the halo's unsettled edge by the
-// vertical coupling (about 1e-3 per row on the 4000x1000 box), each column by the
-// weaker horizontal one.  Measured there: 5 rows and 4 columns need a fallback pass
-// about once in 40 steps (6 rows: never; 4 rows or 3 columns: most steps), and the
-// 54 output rows per tile instead of 52 save 8% of the tiles.
+// changes no bit proves it has been reached.  The proven step (gf_therm.h) marches
+// over columns; FP32-arithmetic mode keeps the tiles below, whose single pass stops at a
+// tolerance and is not proven: its result depends on the sweeps a tile makes.  Sweeps run
+// inside a workgroup on a tile of 64 x 16 nodes held in LDS, with halos of TH_HJ rows
+// above and below and TH_HI columns to the left (the coupling to the previous column is
+// ~(dz/dx)^2 weaker); the per-node coefficients of the six triangles are formed once, in
+// the reference's order, and kept in registers.  Tiles are numbered so that each XCD runs
+// a contiguous range of column-major tiles, which keeps the halo re-reads of neighbouring
+// tiles in the same L2.
 #define TH_J 64
 #define TH_I 16
 #define TH_HJ 5
@@ -192,33 +181,9 @@ __global__ void k_math_check(const double *x, const double *y, double *out, long
 #define TH_MAXPASS 4
 #define TH_MAXSWEEP 48
 #define TH_SWEEP0 3   // sweeps run before the first stillness test
-#define TH_NB (2 * TH_OI + TH_OJ)  // border entries per tile
 
-// logical tile of workgroup `wg` when consecutive workgroups go to the 8 XCDs in turn:
-// XCD x runs tiles [x*q, (x+1)*q); -1 for the padding workgroups of the last range
-GF_DEV int xcd_tile(int wg, int ntiles)
-{
-    const int q = (ntiles + 7) / 8;
-    const int t = (wg % 8) * q + wg / 8;
-    return t < ntiles ? t : -1;
-}
 GF_DEV int therm_ntj(const GfDevParams *P) { return (P->nz + TH_OJ - 1) / TH_OJ; }
 GF_DEV int therm_nti(const GfDevParams *P) { return (P->nx + TH_OI - 1) / TH_OI; }
-// tile-local (lj, li) of border entry k: the row above the output region (TH_OI),
-// the row below it up to the last column but one (TH_OI - 1, left-down neighbours of
-// the last output row), the column to its left from the first output row to the row
-// below the region (TH_OJ + 1)
-GF_DEV void therm_border_pos(int k, int &lj, int &li)
-{
-    if (k < TH_OI) {
-        lj = TH_HJ - 1; li = TH_HI + k;
-    } else if (k < 2 * TH_OI - 1) {
-        lj = TH_J - TH_HJ; li = TH_HI + (k - TH_OI);
-    } else {
-        lj = TH_HJ + (k - (2 * TH_OI - 1)); li = TH_HI - 1;
-    }
-}
-
 struct ThermCoef {
     // rhs = rhs + P_t - Q_t * S_t for the triangles t present, in the reference order:
     // t1 B of (j-1,i-1), t2 A of (j-1,i), t3 B of (j-1,i), t4 A of (j,i-1), t5 B of (j,i-1), t6 A of (j,i)
@@ -362,233 +327,6 @@ GF_DEV double therm_eval_full(const ThermCoef &c, double xu, double xl, double x
     return c.told + div_fma(rhs * dt, c.area_n, c.rarea);
 }
 
-// The old temperature comes from A.temp in every pass (nothing writes temp before the
-// boundary conditions at the end of the call); pass 0 also copies it to temp0
-// (src/fl_therm.f90:52); passes > 0 start from the previous pass's iterate xin.
-// A tile's global reads (its node footprint: temperature and coordinates; its 65 x 17
-// elements: areas, phase, source) are issued together into LDS, so that each tile pays
-// the memory latency once; everything after that reads LDS.
-GF_DEV void therm_tile_one(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, int pass,
-                           int tile)
-{
-    const double *__restrict__ xin = (pass % 2 == 1) ? A.xa : A.xb;
-    double *__restrict__ xout = (pass % 2 == 0) ? A.xa : A.xb;
-    double *__restrict__ bord = A.tbord;
-    const int ntj = therm_ntj(P);
-    constexpr int NL = TH_LI * TH_LJ;
-    __shared__ double sT[NL], sCx[NL], sCy[NL];     // old temperature, coordinates
-    __shared__ double sAr[2][TH_NE];                // area of triangles A and B
-    __shared__ double sDm[TH_NE], sDf[TH_NE];       // dummye and diffusivity per element
-    __shared__ double sU[TH_NF * TH_NE];            // element table by rounds, then the two iterates
-    __shared__ double sPh[3][GF_MAXPH];             // den, cp, diff per phase
-    double(*sX)[NL] = reinterpret_cast<double(*)[NL]>(sU);
-    for (int q = threadIdx.x; q < GF_MAXPH; q += blockDim.x) {
-        sPh[0][q] = P->ph[q].den;
-        sPh[1][q] = P->ph[q].cp;
-        sPh[2][q] = P->ph[q].diff;
-    }
-    const bool with_dissip = P->ishearh == 1 && P->itherm != 2;
-    __syncthreads();  // the previous tile's LDS reads are done (and the phase table is in)
-    const int tj = threadIdx.x % TH_J, ti = threadIdx.x / TH_J;
-    const int j0 = (tile % ntj) * TH_OJ + 1 - TH_HJ;  // 1-based row of tile row 0
-    const int i0 = (tile / ntj) * TH_OI + 1 - TH_HI;  // 1-based column of tile column 0
-    const double *told_g = A.temp;
-#define LIDX(lj, li) (((li) + 1) * TH_LJ + ((lj) + 1))
-    // Each thread has two node slots (q and q + 1024 of the 66 x 18 footprint) and two
-    // element slots (e and e + 1024 of the 65 x 17 table).  All loads are issued before
-    // the first LDS store so that the tile waits for memory once.
-    constexpr int NT = TH_J * TH_I;
-    const int e0 = threadIdx.x, e1 = threadIdx.x + NT;
-    auto node_at = [&](int q, long &ix) {
-        const int jj = j0 + q % TH_LJ - 1, ii = i0 + q / TH_LJ - 1;
-        ix = IN(jj, ii);
-        return q < NL && jj >= 1 && jj <= NZ && ii >= 1 && ii <= NX;
-    };
-    auto elem_ok = [&](int e, int &je, int &ie) {
-        je = j0 + e % TH_EJ - 1;
-        ie = i0 + e / TH_EJ - 1;
-        return e < TH_NE && je >= 1 && je <= NZ - 1 && ie >= 1 && ie <= NX - 1;
-    };
-    long nix0, nix1;
-    const bool nin0 = node_at(e0, nix0), nin1 = node_at(e1, nix1);
-    int je0, ie0, je1, ie1;
-    const bool ein0 = elem_ok(e0, je0, ie0), ein1 = elem_ok(e1, je1, ie1);
-    const long eix0 = ein0 ? IE(je0, ie0) : 0, eix1 = ein1 ? IE(je1, ie1) : 0;
-    double tv0 = 0.0, cx0 = 0.0, cy0 = 0.0, tv1 = 0.0, cx1 = 0.0, cy1 = 0.0;
-    if (nin0) { tv0 = told_g[nix0]; cx0 = A.cord[nix0]; cy0 = A.cord[nix0 + NN]; }
-    if (nin1) { tv1 = told_g[nix1]; cx1 = A.cord[nix1]; cy1 = A.cord[nix1 + NN]; }
-    double a10 = 0.0, a20 = 0.0, sr0 = 0.0, sh0 = 0.0, a11 = 0.0, a21 = 0.0, sr1 = 0.0, sh1 = 0.0;
-    int ph0 = 1, ph1 = 1;
-    if (ein0) {
-        a10 = A.area[eix0]; a20 = A.area[eix0 + NE]; ph0 = A.iphase[eix0]; sr0 = A.source[eix0];
-        if (with_dissip) sh0 = A.shrheat[eix0];
-    }
-    if (ein1) {
-        a11 = A.area[eix1]; a21 = A.area[eix1 + NE]; ph1 = A.iphase[eix1]; sr1 = A.source[eix1];
-        if (with_dissip) sh1 = A.shrheat[eix1];
-    }
-    sT[e0] = tv0; sCx[e0] = cx0; sCy[e0] = cy0;
-    if (e1 < NL) { sT[e1] = tv1; sCx[e1] = cx1; sCy[e1] = cy1; }
-    // dummye = (source + dissip/den)/cp (src/fl_therm.f90:405-414; dissip 0 unless shear heating)
-    if (ein0) {
-        sAr[0][e0] = a10; sAr[1][e0] = a20;
-        sDm[e0] = (sr0 + sh0 / sPh[0][ph0 - 1]) / sPh[1][ph0 - 1];
-        sDf[e0] = sPh[2][ph0 - 1];
-    }
-    if (ein1) {
-        sAr[0][e1] = a11; sAr[1][e1] = a21;
-        sDm[e1] = (sr1 + sh1 / sPh[0][ph1 - 1]) / sPh[1][ph1 - 1];
-        sDf[e1] = sPh[2][ph1 - 1];
-    }
-    __syncthreads();
-    const int j = j0 + tj, i = i0 + ti;
-    const bool valid = j >= 1 && j <= NZ && i >= 1 && i <= NX;
-    const bool is_out = valid && tj >= TH_HJ && tj < TH_J - TH_HJ && ti >= TH_HI;
-    // Node coefficients, as therm_coef forms them, from per-element data built once per
-    // element in three rounds through the table sU: round 0 ra13, P = dummye*ra13 and
-    // Q = 0.5*diff*inv_area of triangles A and B; round 1 the symmetric products
-    // K(a,b) of A; round 2 those of B (a product commutes exactly, so K(a,b) and K(b,a)
-    // are the same bits).
-    auto elem_store = [&](int e, int round) {
-        int je, ie;
-        if (!elem_ok(e, je, ie)) return;
-        if (round == 0) {
-            for (int tri = 0; tri < 2; tri++) {
-                const double inv_area = 1.0 / sAr[tri][e];
-                const double ra13 = div_fma(inv_area, 6.0, GF_RSIX);
-                sU[(3 * tri + 0) * TH_NE + e] = ra13;
-                sU[(3 * tri + 1) * TH_NE + e] = sDm[e] * ra13;
-                sU[(3 * tri + 2) * TH_NE + e] = 0.5 * sDf[e] * inv_area;
-            }
-            return;
-        }
-        const double ar = sAr[round - 1][e];
-        const int ej = e % TH_EJ - 1, ei = e / TH_EJ - 1;
-        double d[6];
-        if (round == 1) {  // A: (ej,ei), (ej+1,ei), (ej,ei+1)
-            const int n1 = LIDX(ej, ei), n2 = LIDX(ej + 1, ei), n3 = LIDX(ej, ei + 1);
-            const double y1 = sCy[n1], y2 = sCy[n2], y3 = sCy[n3], x1 = sCx[n1], x2 = sCx[n2], x3 = sCx[n3];
-            d[0] = (y2 - y3) * ar; d[1] = (y3 - y1) * ar; d[2] = (y1 - y2) * ar;
-            d[3] = (x3 - x2) * ar; d[4] = (x1 - x3) * ar; d[5] = (x2 - x1) * ar;
-        } else {           // B: (ej+1,ei), (ej,ei+1), (ej+1,ei+1)
-            const int n2 = LIDX(ej + 1, ei), n3 = LIDX(ej, ei + 1), n4 = LIDX(ej + 1, ei + 1);
-            const double y2 = sCy[n2], y3 = sCy[n3], y4 = sCy[n4], x2 = sCx[n2], x3 = sCx[n3], x4 = sCx[n4];
-            d[0] = (y2 - y4) * ar; d[1] = (y4 - y3) * ar; d[2] = (y3 - y2) * ar;
-            d[3] = (x4 - x2) * ar; d[4] = (x3 - x4) * ar; d[5] = (x2 - x3) * ar;
-        }
-        sU[0 * TH_NE + e] = KAB(d, 1, 1);
-        sU[1 * TH_NE + e] = KAB(d, 1, 2);
-        sU[2 * TH_NE + e] = KAB(d, 1, 3);
-        sU[3 * TH_NE + e] = KAB(d, 2, 2);
-        sU[4 * TH_NE + e] = KAB(d, 2, 3);
-        sU[5 * TH_NE + e] = KAB(d, 3, 3);
-    };
-    ThermCoef c;
-    c.mask = 0;
-    if (valid) {
-        if (j != 1 && i != 1) c.mask |= 1;
-        if (j != 1 && i != NX) c.mask |= 2 | 4;
-        if (j != NZ && i != 1) c.mask |= 8 | 16;
-        if (j != NZ && i != NX) c.mask |= 32;
-    }
-    c.area_n = 0.0;
-    // the element and triangle (0 A, 1 B) of each of the node's six triangles, in order
-    const int te[6] = {EIDX(tj - 1, ti - 1), EIDX(tj - 1, ti), EIDX(tj - 1, ti), EIDX(tj, ti - 1), EIDX(tj, ti - 1),
-                       EIDX(tj, ti)};
-    for (int round = 0; round < 3; round++) {
-        elem_store(e0, round);
-        elem_store(e1, round);
-        __syncthreads();
-        if (valid) {
-            auto T = [&](int jj, int ii) { return sT[LIDX(jj - j0, ii - i0)]; };
-            auto F = [&](int t, int f) { return sU[f * TH_NE + te[t]]; };
-            const double tme = T(j, i);
-            if (round == 0) {
-#pragma unroll
-                for (int t = 0; t < 6; t++) {
-                    if (!(c.mask & (1 << t))) continue;
-                    const int tri = (t == 0 || t == 2 || t == 4) ? 1 : 0;
-                    c.area_n = c.area_n + F(t, 3 * tri);
-                    c.P[t] = F(t, 3 * tri + 1);
-                    c.Q[t] = F(t, 3 * tri + 2);
-                }
-                c.rarea = 1.0 / c.area_n;
-            } else if (round == 1) {  // triangles A: K11 K12 K13 K22 K23 K33 at 0..5
-                if (c.mask & 2) {  // element (j-1,i), node is vertex 2
-                    c.k21 = F(1, 1); c.c22 = tme * F(1, 3); c.c23 = T(j - 1, i + 1) * F(1, 4);
-                }
-                if (c.mask & 8) {  // element (j,i-1), node is vertex 3
-                    c.k41 = F(3, 2); c.k42 = F(3, 4); c.c43 = tme * F(3, 5);
-                }
-                if (c.mask & 32)  // element (j,i), node is vertex 1
-                    c.qs6 = c.Q[5] * (tme * F(5, 0) + T(j + 1, i) * F(5, 1) + T(j, i + 1) * F(5, 2));
-            } else {  // triangles B
-                if (c.mask & 1) {  // element (j-1,i-1), node is vertex 3
-                    c.k11 = F(0, 2); c.k12 = F(0, 4); c.c13 = tme * F(0, 5);
-                }
-                if (c.mask & 4)  // element (j-1,i), node is vertex 2
-                    c.qs3 = c.Q[2] * (T(j - 1, i + 1) * F(2, 1) + tme * F(2, 3) + T(j, i + 1) * F(2, 4));
-                if (c.mask & 16) {  // element (j,i-1), node is vertex 1
-                    c.c51 = tme * F(4, 0); c.k52 = F(4, 1); c.c53 = T(j + 1, i) * F(4, 2);
-                }
-            }
-        }
-        __syncthreads();
-    }
-    c.told = valid ? sT[LIDX(tj, ti)] : 0.0;
-    // starting iterate (the element table is no longer needed): the old temperature in
-    // pass 0, the previous pass's result later
-    for (int q = threadIdx.x; q < NL; q += blockDim.x) {
-        double xv = sT[q];
-        if (pass > 0) {
-            const int jj = j0 + q % TH_LJ - 1, ii = i0 + q / TH_LJ - 1;
-            xv = (jj >= 1 && jj <= NZ && ii >= 1 && ii <= NX) ? xin[IN(jj, ii)] : 0.0;
-        }
-        sX[0][q] = xv;
-        sX[1][q] = xv;
-    }
-    __syncthreads();
-
-    const double dt = ck->dt;
-    const int me = LIDX(tj, ti), up = LIDX(tj - 1, ti), lf = LIDX(tj, ti - 1), dl = LIDX(tj + 1, ti - 1);
-    int cur = 0, nsweep = 0;
-    bool still = false;
-    // the first TH_SWEEP0 sweeps are never the last one: no stillness test for them
-    // (a sweep at the fixed point changes nothing, so more sweeps cannot change the result)
-    for (; nsweep < TH_SWEEP0; nsweep++) {
-        if (valid) sX[cur ^ 1][me] = therm_eval(c, sX[cur][up], sX[cur][lf], sX[cur][dl], dt);
-        __syncthreads();
-        cur ^= 1;
-    }
-    while (nsweep < TH_MAXSWEEP) {
-        bool changed = false;
-        double tn = 0.0;
-        if (valid) {
-            tn = therm_eval(c, sX[cur][up], sX[cur][lf], sX[cur][dl], dt);
-            changed = __double_as_longlong(tn) != __double_as_longlong(sX[cur][me]);
-            sX[cur ^ 1][me] = tn;
-        }
-        int any = __syncthreads_or(changed);
-        cur ^= 1;
-        nsweep++;
-        if (!any) {
-            still = true;
-            break;
-        }
-    }
-    if (is_out) {
-        xout[IN(j, i)] = sX[cur][me];
-        if (pass == 0) A.temp0[IN(j, i)] = c.told;
-    }
-    if (threadIdx.x < TH_NB) {  // save the tile's values of the output region's outer neighbours
-        int lj, li;
-        therm_border_pos(threadIdx.x, lj, li);
-        bord[(long)tile * TH_NB + threadIdx.x] = sX[cur][LIDX(lj, li)];
-    }
-    if (threadIdx.x == 0 && !still) atomicOr(&ck->therm_pass_changed[pass], 2u);
-#undef LIDX
-}
-
 // ---------------------------------------------------------------- pipelined thermal tiles
 // The single-model step runs the tiles above with one workgroup per CU walking a
 // list of tiles.  A tile's inputs are needed only while its coefficients are built;
@@ -606,22 +344,19 @@ static_assert(2 * TH_LJ * TH_LI <= TH_NF * TH_NE, "the iterates fit in the eleme
 
 struct ThermRaw {
     double t[TR_NLP], cx[TR_NLP], cy[TR_NLP];     // old temperature, coordinates
-    double x[TR_NLP];                             // starting iterate (passes > 0)
     double a0[TR_NEP], a1[TR_NEP], src[TR_NEP];   // areas of triangles A and B, heat source
     double sh[TR_NEP];                            // shear heating (when it heats)
     int iph[TR_NEP];                              // phase
     double ph[3][GF_MAXPH];                       // den, cp, diff per phase of the tile's model
     double dt;                                    // the model's dt
-    int active, pad;                              // 0: the model is already proven (passes > 0)
 };
 // one thread's share of a tile's inputs: node slots q and q + 1024, element slots
 // e and e + 1024 (0 outside the mesh); thread q < 3 GF_MAXPH: phase table entry q;
-// thread 0: dt and the activity flag
+// thread 0: dt
 struct ThermPf {
-    double t[2], cx[2], cy[2], x[2], a0[2], a1[2], src[2], sh[2];
+    double t[2], cx[2], cy[2], a0[2], a1[2], src[2], sh[2];
     int iph[2];
     double phv, dtv;
-    int act;
 };
 // a load through a global-memory pointer (never the flat path, whose counter the LDS
 // barriers would also wait for)
@@ -644,22 +379,15 @@ GF_DEV void therm_tile_origin(const GfDevParams *P, int tile, int &j0, int &i0)
 
 // node q = (q % 66, q / 66) - 1 of the footprint, element e = (e % 65, e / 65) - 1 of
 // the table
-// XIN: the starting iterate -- 0: the old temperature (pass 0), 1: loaded from the
-// previous pass's iterate (passes > 0), 2: extrapolated in time from the old
-// temperature and temp0, the temperature at the start of the previous step (pass 0;
-// where pass 0 copies the old temperature to temp0, temp0 of this tile's neighbours
-// may already hold this step's value, and then the extrapolation is the old
-// temperature: only the number of sweeps changes, the fixed point is the same).
 // DIS: the shear heating is loaded
-template <int XIN, bool DIS>
-GF_DEV ThermPf therm_prefetch(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, int pass,
-                              int tile, int arp = 0, int gate = 1)
+template <bool DIS>
+GF_DEV ThermPf therm_prefetch(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, int tile,
+                              int arp)
 {
     int j0, i0;
     therm_tile_origin(P, tile, j0, i0);
     const long nz = P->nz, nx = P->nx, nn = nz * nx, ne = (nz - 1) * (nx - 1);
     const double *told_g = A.temp;
-    const double *xin = (pass % 2 == 1) ? A.xa : A.xb;
     ThermPf f;
     // the model's scalars first, used at once: waiting for them later would also wait
     // for the tile loads below
@@ -670,24 +398,18 @@ GF_DEV ThermPf therm_prefetch(const GfDevParams *__restrict__ P, GfDevClock *ck,
         f.phv = w == 0 ? ph.den : w == 1 ? ph.cp : ph.diff;
     }
     f.dtv = 0.0;
-    f.act = 1;
-    if (threadIdx.x == 0) {
-        f.dtv = ck->dt;
-        f.act = (gate && pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) ? 0 : 1;
-    }
-    asm volatile("" ::"v"(f.phv), "v"(f.dtv), "v"(f.act));
+    if (threadIdx.x == 0) f.dtv = ck->dt;
+    asm volatile("" ::"v"(f.phv), "v"(f.dtv));
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         const int q = threadIdx.x + k * TH_J * TH_I;
         const int jj = j0 + q % TH_LJ - 1, ii = i0 + q / TH_LJ - 1;
-        f.t[k] = f.cx[k] = f.cy[k] = f.x[k] = 0.0;
+        f.t[k] = f.cx[k] = f.cy[k] = 0.0;
         if (q < TH_LJ * TH_LI && jj >= 1 && jj <= nz && ii >= 1 && ii <= nx) {
             const long ix = (jj - 1) + nz * (ii - 1);
             f.t[k] = gld(told_g, ix);
             f.cx[k] = gld(A.cord, ix);
             f.cy[k] = gld(A.cord, ix + nn);
-            if (XIN == 1) f.x[k] = gld(xin, ix);
-            if (XIN == 2) f.x[k] = gld(A.temp0, ix);
         }
         const int je = j0 + q % TH_EJ - 1, ie = i0 + q / TH_EJ - 1;
         f.a0[k] = f.a1[k] = f.src[k] = f.sh[k] = 0.0;
@@ -705,7 +427,7 @@ GF_DEV ThermPf therm_prefetch(const GfDevParams *__restrict__ P, GfDevClock *ck,
     }
     return f;
 }
-template <int XIN, bool DIS>
+template <bool DIS>
 GF_DEV void therm_store_raw(const ThermPf &f, ThermRaw &R)
 {
 #pragma unroll
@@ -715,7 +437,6 @@ GF_DEV void therm_store_raw(const ThermPf &f, ThermRaw &R)
             R.t[q] = f.t[k];
             R.cx[q] = f.cx[k];
             R.cy[q] = f.cy[k];
-            if (XIN != 0) R.x[q] = f.x[k];
         }
         if (q < TH_NE) {
             R.a0[q] = f.a0[k];
@@ -726,28 +447,21 @@ GF_DEV void therm_store_raw(const ThermPf &f, ThermRaw &R)
         }
     }
     if (threadIdx.x < 3 * GF_MAXPH) R.ph[threadIdx.x / GF_MAXPH][threadIdx.x % GF_MAXPH] = f.phv;
-    if (threadIdx.x == 0) {
-        R.dt = f.dtv;
-        R.active = f.act;
-    }
+    if (threadIdx.x == 0) R.dt = f.dtv;
 }
 
-// One tile (P, ck, A, tile) from its inputs in R (the arithmetic of therm_tile_one,
-// bit for bit); loads tile `next` of (Pn, ckn, An) (if next >= 0) during the sweeps
-// and leaves it in R.  sU: element table by rounds, then the two iterates.  Nothing
-// after the prefetch is issued reads global memory (a wait for it would also wait
-// for the prefetch): the mesh size is held in registers, the phase table, dt and the
-// activity flag came with the tile's inputs.  wt0: pass 0 copies the old temperature
-// to temp0 (0 where the caller turns temp0 over by itself: the rotating buffers of
-// the single-model step).
-template <int XIN, bool DIS>
-GF_DEV void therm_tile_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, int pass,
-                            int tile, const GfDevParams *__restrict__ Pn, GfDevClock *ckn, const GfDevArrays &An,
-                            int next, ThermRaw &R, double *sU, int *sFlag, double stol, int arp = 0, int gate = 1,
-                            int wt0 = 1)
+// One tile (P, ck, A, tile) from its inputs in R; loads tile `next` of (Pn, ckn, An) (if
+// next >= 0) during the sweeps and leaves it in R.  sU: element table by rounds, then the
+// two iterates.  Nothing after the prefetch is issued reads vector memory (a wait for it
+// would also wait for the prefetch): the mesh size is held in registers, the phase table
+// and dt came with the tile's inputs.  fold: the boundary conditions (:575-598) are applied
+// to what is stored (not with a bottom heat flux, which reads a row another tile may own).
+template <bool DIS>
+GF_DEV void therm_tile_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, int tile,
+                            const GfDevParams *__restrict__ Pn, GfDevClock *ckn, const GfDevArrays &An, int next,
+                            ThermRaw &R, double *sU, int *sFlag, double stol, int arp, int fold)
 {
-    double *__restrict__ xout = (pass % 2 == 0) ? A.xa : A.xb;
-    double *__restrict__ bord = A.tbord;
+    double *__restrict__ xout = A.xa;
     constexpr int NL = TH_LI * TH_LJ, NT = TH_J * TH_I;
     double(*sX)[NL] = reinterpret_cast<double(*)[NL]>(sU);
     const int nz = P->nz, nx = P->nx;
@@ -756,11 +470,6 @@ GF_DEV void therm_tile_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, c
         const int ntj = (nz + TH_OJ - 1) / TH_OJ;
         j0 = (tile % ntj) * TH_OJ + 1 - TH_HJ;
         i0 = (tile / ntj) * TH_OI + 1 - TH_HI;
-    }
-    if (!R.active) {  // a proven model (passes > 0): nothing to do but the prefetch
-        lds_barrier();
-        if (next >= 0) therm_store_raw<XIN, DIS>(therm_prefetch<XIN, DIS>(Pn, ckn, An, pass, next, arp, gate), R);
-        return;
     }
     const double(*sPh)[GF_MAXPH] = R.ph;
     const int tj = threadIdx.x % TH_J, ti = threadIdx.x / TH_J;
@@ -784,7 +493,7 @@ GF_DEV void therm_tile_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, c
         if (ein1) moved_area(e1);
     }
     // round 0: ra13, P = dummye*ra13, Q = 0.5*diff*inv_area of triangles A and B;
-    // rounds 1 and 2: the K(a,b) products of A, of B (as in therm_tile_one)
+    // rounds 1 and 2: the K(a,b) products of A, of B
     auto elem_store = [&](int e, int round) {
         if (round == 0) {
             const int ph = R.iph[e];
@@ -879,23 +588,17 @@ GF_DEV void therm_tile_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, c
         lds_barrier();
     }
     c.told = valid ? R.t[nb] : 0.0;
-    // starting iterate: the old temperature in pass 0, the previous pass's result later
+    // starting iterate: the old temperature
     {
-        const double v0 = XIN == 1 ? R.x[e0] : XIN == 2 ? 2.0 * R.t[e0] - R.x[e0] : R.t[e0];
-        sX[0][e0] = v0;
-        sX[1][e0] = v0;
-        if (e1 < NL) {
-            const double v1 = XIN == 1 ? R.x[e1] : XIN == 2 ? 2.0 * R.t[e1] - R.x[e1] : R.t[e1];
-            sX[0][e1] = v1;
-            sX[1][e1] = v1;
-        }
+        sX[0][e0] = sX[1][e0] = R.t[e0];
+        if (e1 < NL) sX[0][e1] = sX[1][e1] = R.t[e1];
         if (threadIdx.x < 3) sFlag[threadIdx.x] = 0;
     }
     lds_barrier();
     const double dt = R.dt;
     asm volatile("" ::"v"(dt));
     ThermPf pf;
-    if (next >= 0) pf = therm_prefetch<XIN, DIS>(Pn, ckn, An, pass, next, arp, gate);  // R is free now
+    if (next >= 0) pf = therm_prefetch<DIS>(Pn, ckn, An, next, arp);  // R is free now
 
     const int me = nb, up = nb - 1, lf = nb - TH_LJ, dl = nb - TH_LJ + 1;
     int cur = 0, nsweep = 0;
@@ -943,30 +646,39 @@ GF_DEV void therm_tile_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, c
         sweeps(std::false_type{});
     // the next tile's inputs go to R before this tile's outputs are stored, so that
     // waiting for the loads does not wait for the stores
-    if (next >= 0) therm_store_raw<XIN, DIS>(pf, R);
+    if (next >= 0) therm_store_raw<DIS>(pf, R);
     if (is_out) {
-        xout[oix] = sX[cur][me];
-        if (pass == 0 && wt0) A.temp0[oix] = c.told;
+        double v = sX[cur][me];
+        if (!fold) {
+            xout[oix] = v;
+        } else {
+            if (j == 1)
+                v = P->t_top;
+            else if (j == nz && P->itemp_bc == 1)
+                v = P->bot_bc;
+            // (the side columns take their neighbours' values)
+            if (i != 1 && i != nx) {
+                xout[oix] = v;
+                if (i == 2) xout[oix - nz] = v;
+                if (i == nx - 1) xout[oix + nz] = v;
+            }
+        }
     }
-    if (threadIdx.x < TH_NB) {
-        int lj, li;
-        therm_border_pos(threadIdx.x, lj, li);
-        bord[(long)tile * TH_NB + threadIdx.x] = sX[cur][LIDX(lj, li)];
-    }
-    if (threadIdx.x == 0 && !still) atomicOr(&ck->therm_pass_changed[pass], 2u);
+    // a tile that did not settle within TH_MAXSWEEP: the call counts as unconverged, once
+    if (threadIdx.x == 0 && !still && atomicOr(&ck->therm_pass_changed[0], 2u) == 0u)
+        atomicAdd(&ck->therm_unconverged, 1ull);
 #undef LIDX
 }
 
 // Workgroup w (of a grid that is a multiple of 8, one per CU) runs on XCD w % 8, which
 // owns the contiguous tile range [x q, (x+1) q); its r-th workgroup there takes tiles
 // x q + r, + R, + 2R, ... with R = grid / 8.
-template <int XIN, bool DIS>
 // arp: the element areas of the last move are pending (formed from the coordinates)
+template <bool DIS>
 __global__ void __launch_bounds__(1024) k_therm_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                     int pass, double stol, int arp, int wt0, int ops)
+                                                     double stol, int arp, int fold, int ops)
 {
     if (ops && blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
-    if (pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) return;  // already proven
     __shared__ ThermRaw raw;
     __shared__ double sU[TH_NF * TH_NE];
     __shared__ int sFlag[3];
@@ -974,69 +686,15 @@ __global__ void __launch_bounds__(1024) k_therm_pipe(const GfDevParams *__restri
     const int q = (ntiles + 7) / 8, x = blockIdx.x % 8, r = blockIdx.x / 8, RW = gridDim.x / 8;
     const int first = x * q + r, end = min((x + 1) * q, ntiles);
     if (first >= end) return;
-    therm_store_raw<XIN, DIS>(therm_prefetch<XIN, DIS>(P, ck, A, pass, first, arp), raw);
+    therm_store_raw<DIS>(therm_prefetch<DIS>(P, ck, A, first, arp), raw);
     for (int t = first; t < end; t += RW) {
         lds_barrier();  // this tile's inputs are in; the previous tile is done with sU
-        therm_tile_pipe<XIN, DIS>(P, ck, A, pass, t, P, ck, A, t + RW < end ? t + RW : -1, raw, sU, sFlag, stol, arp,
-                                  1, wt0);
+        therm_tile_pipe<DIS>(P, ck, A, t, P, ck, A, t + RW < end ? t + RW : -1, raw, sU, sFlag, stol, arp, fold);
     }
 }
 
-// Compares each tile's border values with the global iterate written by the owning
-// tiles.  A border node whose tile value differs is harmless when every output node
-// that reads it still satisfies x = F(x) with the global values: those (at most three)
-// nodes are re-evaluated here.  This matters on the top row, whose pre-boundary-
-// condition temperature is close to zero, so that differences far below the other
-// rows' rounding still show up as a few ulp there.  Any remaining difference (or a
-// tile that did not settle) sends the next pass.
-GF_DEV void therm_check_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, int pass,
-                             long t, int arp = 0, int gate = 1)
-{
-    if (gate && pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) return;
-    const double *__restrict__ x = (pass % 2 == 0) ? A.xa : A.xb;
-    const double *__restrict__ bord = A.tbord;
-    const int ntj = therm_ntj(P);
-    if (t >= (long)ntj * therm_nti(P) * TH_NB) return;
-    const int tile = (int)(t / TH_NB), k = (int)(t % TH_NB);
-    int lj, li;
-    therm_border_pos(k, lj, li);
-    const int j0 = (tile % ntj) * TH_OJ + 1 - TH_HJ, i0 = (tile / ntj) * TH_OI + 1 - TH_HI;
-    const int j = j0 + lj, i = i0 + li;
-    if (j < 1 || j > NZ || i < 1 || i > NX) return;
-    const long long a = __double_as_longlong(bord[t]), b = __double_as_longlong(x[IN(j, i)]);
-    if (a == b) return;
-    // output nodes of this tile that read (j,i): as up (j+1,i), left (j,i+1), left-down (j-1,i+1)
-    const int dj[3] = {1, 0, -1}, di[3] = {0, 1, 1};
-    const double dt = ck->dt;
-    auto T = [&](int jj, int ii) { return A.temp[IN(jj, ii)]; };  // the old temperature
-    // the (up to three) evaluations first, the flag after them, so that no atomic
-    // orders the loads of one evaluation after another's
-    bool bad = false;
-#pragma unroll
-    for (int q = 0; q < 3; q++) {
-        const int mj = j + dj[q], mi = i + di[q];
-        const int mlj = mj - j0, mli = mi - i0;
-        if (mlj < TH_HJ || mlj >= TH_J - TH_HJ || mli < TH_HI || mli >= TH_I) continue;
-        if (mj < 1 || mj > NZ || mi < 1 || mi > NX) continue;
-        ThermCoef c;
-        therm_coef(P, A, mj, mi, T, c, arp);
-        const double xu = mj > 1 ? x[IN(mj - 1, mi)] : 0.0;
-        const double xl = mi > 1 ? x[IN(mj, mi - 1)] : 0.0;
-        const double xd = (mi > 1 && mj < NZ) ? x[IN(mj + 1, mi - 1)] : 0.0;
-        const double f = therm_eval(c, xu, xl, xd, dt);
-        bad |= __double_as_longlong(f) != __double_as_longlong(x[IN(mj, mi)]);
-    }
-    atomicAdd(&ck->therm_mismatch, 1ull);  // (statistics)
-    atomicMax(&ck->therm_mismatch_ulp, (unsigned long long)(a > b ? a - b : b - a));
-    if (bad) atomicOr(&ck->therm_pass_changed[pass], 1u);
-}
-
-// Boundary conditions src/fl_therm.f90:575-598 applied to the proven iterate.
-// passes: the fixed-point passes that ran; proof: their results carry the border
-// proof (FP64), and a call that no pass proved raises GF_ERR_THERM_SWEEPS (its last
-// pass is used, but the result is not known to be the serial one); without proof the
-// single tile pass is taken as it is (FP32-arithmetic mode)
-// proven: the first pass whose border check found no difference (-1: none)
+// Boundary conditions src/fl_therm.f90:575-598 of FP32-arithmetic mode where its tiles do
+// not apply them (a bottom heat flux)
 // the value of node (j, i) after the conditions (:575-598), from the iterate x: the
 // top and bottom conditions (:575-588), then the side columns copy their neighbours
 // (only boundary nodes change: an interior node keeps x)
@@ -1058,70 +716,29 @@ GF_DEV double therm_bc_value(const GfDevParams *__restrict__ P, const GfDevArray
     if (i == NX) return tb(j, NX - 1);
     return tb(j, i);
 }
-// the counters of the call's outcome; the iterate that is the result (pass p wrote xa
-// when p is even, xb when odd)
-GF_DEV const double *therm_bc_outcome(GfDevClock *ck, const GfDevArrays &A, bool first, int passes, int proof,
-                                      int &proven)
+// in place: only the boundary nodes (rows 1 and nz, columns 1 and nx) change, each
+// computed from interior nodes, or from boundary nodes that keep their value.  Entry t of
+// them.  (nz, nx >= 3.)
+GF_DEV void therm_bc_node(const GfDevParams *__restrict__ P, const GfDevArrays &A, long t)
 {
-    if (!proof) proven = 0;
-    if (first && (proven < 0 || (!proof && ck->therm_pass_changed[0] != 0u)))
-        atomicAdd(&ck->therm_unconverged, 1ull);
-    if (first && proof && proven < 0) raise_error(ck, GF_ERR_THERM_SWEEPS, 0);
-    if (first && proven > 0) atomicAdd(&ck->therm_extra_passes, (unsigned long long)proven);
-    return (proven < 0 ? (passes - 1) : proven) % 2 == 0 ? A.xa : A.xb;
-}
-GF_DEV void therm_bc_apply(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long t,
-                           int passes, int proof, int proven)
-{
-    const double *__restrict__ x = therm_bc_outcome(ck, A, t == 0, passes, proof, proven);
-    if (t >= NN) return;
-    const int j = (int)((unsigned)t % (unsigned)NZ) + 1, i = (int)((unsigned)t / (unsigned)NZ) + 1;
-    A.temp[t] = therm_bc_value(P, A, x, j, i);
-}
-// The same conditions where the result becomes the new temperature in place (xa, which
-// the caller then takes as temp): after an even pass the result is in xa already and
-// only its boundary nodes (rows 1 and nz, columns 1 and nx) change, each computed from
-// interior nodes, or from boundary nodes that keep their value; after an odd pass every
-// node is formed from xb into xa.  Thread tid of nthr.  (nz, nx >= 3.)
-GF_DEV void therm_bc_rot(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long tid,
-                         long nthr, int passes, int proof, int proven)
-{
-    const double *x = therm_bc_outcome(ck, A, tid == 0, passes, proof, proven);
-    double *out = A.xa;
     const int nz = NZ, nx = NX;
-    if (x == out) {
-        const long nb = 2L * nx + 2L * (nz - 2);
-        for (long t = tid; t < nb; t += nthr) {
-            int j, i;
-            if (t < nx) {
-                j = 1; i = (int)t + 1;
-            } else if (t < 2L * nx) {
-                j = nz; i = (int)(t - nx) + 1;
-            } else if (t < 2L * nx + nz - 2) {
-                j = (int)(t - 2L * nx) + 2; i = 1;
-            } else {
-                j = (int)(t - 2L * nx - (nz - 2)) + 2; i = nx;
-            }
-            out[IN(j, i)] = therm_bc_value(P, A, x, j, i);
-        }
+    int j, i;
+    if (t < nx) {
+        j = 1; i = (int)t + 1;
+    } else if (t < 2L * nx) {
+        j = nz; i = (int)(t - nx) + 1;
+    } else if (t < 2L * nx + nz - 2) {
+        j = (int)(t - 2L * nx) + 2; i = 1;
+    } else if (t < 2L * nx + 2L * (nz - 2)) {
+        j = (int)(t - 2L * nx - (nz - 2)) + 2; i = nx;
     } else {
-        for (long t = tid; t < NN; t += nthr) {
-            const int j = (int)((unsigned)t % (unsigned)nz) + 1, i = (int)((unsigned)t / (unsigned)nz) + 1;
-            out[t] = therm_bc_value(P, A, x, j, i);
-        }
+        return;
     }
+    A.xa[IN(j, i)] = therm_bc_value(P, A, A.xa, j, i);
 }
-
-GF_DEV void therm_bc_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long t,
-                          int passes, int proof)
+__global__ void __launch_bounds__(256) k_therm_bc(const GfDevParams *__restrict__ P, GfDevArrays A)
 {
-    int proven = -1;
-    for (int k = 0; k < passes; k++)
-        if (ck->therm_pass_changed[k] == 0u) {
-            proven = k;
-            break;
-        }
-    therm_bc_apply(P, ck, A, t, passes, proof, proven);
+    therm_bc_node(P, A, (long)blockIdx.x * 256 + threadIdx.x);
 }
 
 // Grid-wide barrier of a launch whose workgroups are all resident.  Every wave
@@ -1161,13 +778,6 @@ GF_DEV bool grid_sync(GfDevClock *ck)
     }
     __syncthreads();
     return s_ok != 0;
-}
-
-// the boundary conditions of FP32-arithmetic mode's single pass, in place
-__global__ void __launch_bounds__(256) k_therm_bc(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A)
-{
-    const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    therm_bc_rot(P, ck, A, tid, (long)gridDim.x * blockDim.x, 1, 0, 0);
 }
 
 #include "gf_therm.h"
@@ -2373,8 +1983,10 @@ GF_DEV NodeVel<typename Prec<M>::SV> node_update(const GfDevParams *__restrict__
 // damping and the velocity update.
 // The force and velocity arithmetic runs in SV (double: the reference's, bit for bit;
 // float: mixed precision); geometry is formed in double from the FP64 coordinates.
+// cord_out: the moved coordinates (null: no move)
 template <int M>
-GF_DEV void node_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long t)
+GF_DEV void node_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, long t,
+                      double *cord_out = nullptr)
 {
     typedef typename Prec<M>::SV SV;
     const int j = (int)((unsigned)t % (unsigned)NZ) + 1, i = (int)((unsigned)t / (unsigned)NZ) + 1;
@@ -2422,7 +2034,12 @@ GF_DEV void node_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const G
         }
         p = pr[el];
     };
-    node_update<M>(P, ck, A, t, j, i, src, [&]() { return node_own<SV>(P, A, t); }, node_clk(ck));
+    const NodeClk kc = node_clk(ck);
+    const NodeVel<SV> nv = node_update<M>(P, ck, A, t, j, i, src, [&]() { return node_own<SV>(P, A, t); }, kc);
+    if (cord_out) {  // (move_cord_body)
+        cord_out[t] = cx[1][1] + (double)nv.v1 * kc.dt;
+        cord_out[t + NN] = cy[1][1] + (double)nv.v2 * kc.dt;
+    }
 }
 
 template <int M>

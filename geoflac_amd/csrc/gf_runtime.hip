@@ -105,6 +105,7 @@ struct gf_ctx {
     ThermChk chk{};      // the border check of the thermal call under way
     int node_ops = 0;    // clock updates left to the step's fl_node
     bool therm_clean = true;  // the flags of the thermal passes are 0 on the device
+    void *therm_batch = nullptr;  // the batch whose steps were the model's last thermal calls
     int therm_hist = 0;  // calls before it (at most 2) whose slots hold their boundary values
     // per-kernel event timing
     bool timing = false;
@@ -142,18 +143,22 @@ static ThermGeo therm_geo_host(const gf_params &p, int w)
     g.ns = (g.nx + w - 1) / w;
     return g;
 }
-// Output columns of a thermal strip.  A strip of w columns takes some w + 6 column times
+// Output columns of the thermal strips of one or more meshes in a launch.  A strip of w columns takes some w + 6 column times
 // (halo, ring, start); a column takes a wave alone on its SIMD 1.3 us (latency), n waves
 // 0.6 us more each, 0.9 us each where issue bounds.  The width of least time over the
 // 1024 SIMDs.  Measured, us a step (whole step) at widths 2, 4, 8, 16, 24: 401x101 nodes
 // 38, 41, 47, 59, 70; 902x302 101, 97, 102, 110, 121; 2001x1001 541, 508, 492, 493, 497.
-static int therm_strip_width(const gf_params &p)
+static int therm_strip_width(const std::vector<const gf_params *> &ps)
 {
     int best = 2;
     double least = 1e300;
     for (int w = 2; w <= 32; w++) {
-        const ThermGeo g = therm_geo_host(p, w);
-        const double n = (double)g.nr * g.ns / 1024.0;
+        long strips = 0;
+        for (const gf_params *p : ps) {
+            const ThermGeo g = therm_geo_host(*p, w);
+            strips += (long)g.nr * g.ns;
+        }
+        const double n = (double)strips / 1024.0;
         const double col = n <= 1.0 ? 1.3 : std::max(1.3 + 0.6 * (n - 1.0), 0.9 * n);
         if ((w + 6) * col < least) {
             least = (w + 6) * col;
@@ -330,7 +335,7 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
         const char *tm = getenv("GF_THERM");
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_therm_rest<true>, 256, 0) != hipSuccess) nb = 0;
         ctx->therm_rest = nb >= 1 && ncu >= 8 && !(tm && strcmp(tm, "multi") == 0);
-        ctx->therm_w = therm_strip_width(*p);
+        ctx->therm_w = therm_strip_width({p});
         (void)hipGetLastError();
     }
     ALLOC(ctx->dp, sizeof(GfDevParams));
@@ -370,9 +375,7 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
     ALLOC(ctx->a.xb, 8 * nn);
     {
         const ThermGeo g = therm_geo_host(*p, ctx->therm_w);
-        const size_t nb = (size_t)g.nr * g.ns * TS_NB(g.w),
-                     nt = (size_t)TH_NB * ((p->nz + TH_OJ - 1) / TH_OJ) * ((p->nx + TH_OI - 1) / TH_OI);
-        ALLOC(ctx->therm_border, 8 * std::max(nb, nt));
+        ALLOC(ctx->therm_border, 8 * (size_t)g.nr * g.ns * TS_NB(g.w));
     }
     ctx->a.tbord = ctx->therm_border;
     ALLOC(ctx->a.tpre, 8 * (size_t)GF_NPRE * 2 * (p->nx + p->nz));
@@ -791,6 +794,7 @@ static void therm_forget(gf_ctx *ctx)
 {
     ctx->temp0_prev = false;
     ctx->therm_hist = 0;
+    ctx->therm_batch = nullptr;
 }
 
 extern "C" int gf_upload(gf_ctx *ctx, uint32_t mask)
@@ -1208,15 +1212,20 @@ static int enq_therm(gf_ctx *ctx, int ops = 0, bool defer = false)
     // the flags of the passes start at 0: the last step's fl_node cleared them, or this
     if (!ctx->therm_clean && (rc = enq_clock(ctx, CK_THERM_BEGIN))) return rc;
     ctx->therm_clean = false;
+    if (ctx->therm_batch) {  // (the batch numbers its own calls)
+        ctx->therm_batch = nullptr;
+        ctx->therm_hist = 0;
+    }
     const bool dis = ctx->p.ishearh == 1 && ctx->p.itherm != 2;
     const int arp = ctx->area_pending ? 1 : 0;
     if (!ctx->therm_proof) {
         // FP32-arithmetic mode: one tile pass, whose result (which depends on the sweeps
-        // it made) is taken as it is, then the boundary conditions
-        auto kern = dis ? k_therm_pipe<0, true> : k_therm_pipe<0, false>;
-        LAUNCH_DIM("k_therm_pipe", kern, ctx->therm_grid, TH_J * TH_I, ctx->dp, ctx->dck, ctx->a, 0, GF_THERM_STOL,
-                   arp, 0, ops);
-        LAUNCH(k_therm_bc, 2L * (ctx->p.nx + ctx->p.nz), ctx->dp, ctx->dck, ctx->a);
+        // it made) is taken as it is
+        auto kern = dis ? k_therm_pipe<true> : k_therm_pipe<false>;
+        const int fold = ctx->p.itemp_bc != 2;
+        LAUNCH_DIM("k_therm_pipe", kern, ctx->therm_grid, TH_J * TH_I, ctx->dp, ctx->dck, ctx->a, GF_THERM_STOL, arp,
+                   fold, ops);
+        if (!fold) LAUNCH(k_therm_bc, 2L * (ctx->p.nx + ctx->p.nz), ctx->dp, ctx->a);
         return enq_therm_rest(ctx);
     }
     const ThermGeo g = therm_geo_host(ctx->p, ctx->therm_w);
@@ -2386,28 +2395,29 @@ struct gf_batch {
     bool shearh = false, no_mech = false;
     gf_params p0{};  // frequencies and switches shared by all models
     BatchEntry *dtab = nullptr;
+    std::vector<BatchEntry> tab;  // the table as the device holds it between calls
+    bool tab_valid = false;
     int *dmap = nullptr;  // chunk -> model tables (BatchMap)
-    unsigned therm_grid = 8;  // workgroups of the thermal pipeline (the CUs)
+    double *border = nullptr;  // the thermal strips' border values
+    int therm_w = 2;      // output columns of a strip
+    bool fold = true;     // FP32-arithmetic mode: the tiles apply the boundary conditions
+    unsigned therm_grid = 8;  // workgroups of the thermal kernels with one per CU
     BatchMap map{};
     int nm = 0;
     long tot_e = 0, tot_n = 0, tot_t = 0, tot_b = 0, tot_m = 0;
     bool markers = false;   // some model has markers (change_phase runs)
     // every model's temp0 holds the temperature at the start of its previous thermal
     // step: pass 0 starts from the extrapolation 2 temp - temp0, as a model alone does
-    bool temp0_prev = false, g_t0prev = false, noguess = false;
+    bool temp0_prev = false, noguess = false;
     bool movegrid = true;   // the models move their grids (all or none)
     hipStream_t stream = nullptr;
     int32_t nloop = 0, nsrate = 0;
-    int bs[3] = {256, 256, 256};  // threads per workgroup of the rheology, node and element-area kernels
+    int pend_ops = 0;       // clock updates left to the next launch that makes them
+    int bs[3] = {256, 256, 256};  // threads per workgroup of the rheology and node kernels (the third is unused)
     bool use_graph = false;
-    // the batch's last element move left its rotation to the next kb_rheol (kb_visc and
-    // kb_dens rotate what they read themselves); g_rot0: the same at the start of the
-    // captured cycle
-    bool rot_pending = false, g_rot0 = false;
-    // ... and its areas and dvol to the next kb_rheol (the thermal tiles before it form
-    // the areas they need), in FP32-arithmetic mode, whose thermal step has no fallback
-    // passes; g_area0: the same at the start of the captured cycle
-    bool area_pending = false, g_area0 = false, g_area_end = false, g_rot_end = false;
+    // the batch's last element move left its rotation, its areas and dvol to the next
+    // kb_rheol (the kernels between form what they read of them)
+    bool rot_pending = false, area_pending = false;
     hipGraphExec_t gexec = nullptr;
     int32_t g_nsrate0 = -99, g_nsrate1 = 0;  // nsrate before and after the captured 10 steps
     // optional per-kernel timing (autotuner)
@@ -2445,6 +2455,7 @@ extern "C" void gf_batch_destroy(gf_batch *b)
         if (e) (void)hipEventDestroy(e);
     if (b->dtab) (void)hipFree(b->dtab);
     if (b->dmap) (void)hipFree(b->dmap);
+    if (b->border) (void)hipFree(b->border);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     if (b->pinned)
         for (gf_ctx *c : b->m) c->in_batch--;
@@ -2463,6 +2474,14 @@ extern "C" int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out)
     };
     const gf_ctx *c0 = models[0];
     if (!c0) return fail(GF_ERR_ARG, "null model");
+    {
+        std::vector<const gf_params *> ps;
+        for (int k = 0; k < n; k++) {
+            if (!models[k]) return fail(GF_ERR_ARG, "null model");
+            ps.push_back(&models[k]->p);
+        }
+        b->therm_w = therm_strip_width(ps);
+    }
     std::vector<BatchEntry> tab(n + 1);
     long pe = 0, pn = 0, pt = 0, pb = 0, pm = 0;
     auto align = [](long v) { return (v + BATCH_ALIGN - 1) / BATCH_ALIGN * BATCH_ALIGN; };
@@ -2480,23 +2499,29 @@ extern "C" int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out)
                         "models of a batch share precision, switches, frequencies, movegrid and loop counters "
                         "(and run without stress boundaries and surface processes)");
         if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(GF_ERR_HIP, "sync");
-        const long ntiles = (long)((q.nz + TH_OJ - 1) / TH_OJ) * ((q.nx + TH_OI - 1) / TH_OI);
+        // thermal strips of the proven step (and their border values), or the tiles of
+        // FP32-arithmetic mode
+        const ThermGeo tg = therm_geo_host(q, b->therm_w);
+        const long ntiles = c0->therm_proof ? (long)tg.nr * tg.ns
+                                            : (long)((q.nz + TH_OJ - 1) / TH_OJ) * ((q.nx + TH_OI - 1) / TH_OI);
+        const long nbord = c0->therm_proof ? ntiles * TS_NB(b->therm_w) : 0;
         const long nmk = c->markers_uploaded ? c->a.nmarkers : 0;
-        tab[k] = BatchEntry{c->dp, c->dck, c->a, pe, pn, pt, pb, pm, c->ne, c->nn, ntiles, ntiles * TH_NB, nmk};
+        tab[k] = BatchEntry{c->dp, c->dck, c->a, nullptr, nullptr, pe, pn, pt, pb, pm, c->ne, c->nn, ntiles, nbord, nmk};
+        b->fold = b->fold && q.itemp_bc != 2;
         if (nmk > 0) b->markers = true;
         mm.insert(mm.end(), align(nmk) / BATCH_ALIGN, k);
         pm += align(nmk);
         me.insert(me.end(), align(c->ne) / BATCH_ALIGN, k);
         mn.insert(mn.end(), align(c->nn) / BATCH_ALIGN, k);
-        mb.insert(mb.end(), align(ntiles * TH_NB) / BATCH_ALIGN, k);
+        mb.insert(mb.end(), align(nbord) / BATCH_ALIGN, k);
         mt.insert(mt.end(), ntiles, k);
         pe += align(c->ne);
         pn += align(c->nn);
         pt += ntiles;
-        pb += align(ntiles * TH_NB);
+        pb += align(nbord);
         b->m.push_back(c);
     }
-    tab[n] = BatchEntry{nullptr, nullptr, GfDevArrays{}, pe, pn, pt, pb, pm, 0, 0, 0, 0, 0};
+    tab[n] = BatchEntry{nullptr, nullptr, GfDevArrays{}, nullptr, nullptr, pe, pn, pt, pb, pm, 0, 0, 0, 0, 0};
     b->nm = n;
     b->tot_e = pe; b->tot_n = pn; b->tot_t = pt; b->tot_b = pb; b->tot_m = pm;
     b->movegrid = c0->p.movegrid != 0;
@@ -2527,8 +2552,12 @@ extern "C" int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out)
     b->p0 = c0->p;
     b->nloop = c0->nloop;
     b->nsrate = c0->nsrate;
+    if (pb > 0) {  // (the batch's strips may be narrower than a model's own)
+        if (hipMalloc((void **)&b->border, sizeof(double) * pb) != hipSuccess) return fail(GF_ERR_HIP, "allocation");
+        for (int k = 0; k < n; k++) tab[k].A.tbord = b->border + tab[k].pb;
+    }
+    b->tab = tab;
     if (hipMalloc((void **)&b->dtab, sizeof(BatchEntry) * (n + 1)) != hipSuccess ||
-        hipMemcpy(b->dtab, tab.data(), sizeof(BatchEntry) * (n + 1), hipMemcpyHostToDevice) != hipSuccess ||
         hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&b->ev[0]) != hipSuccess || hipEventCreate(&b->ev[1]) != hipSuccess)
         return fail(GF_ERR_HIP, "allocation");
@@ -2569,36 +2598,41 @@ static int enq_batch_flac(gf_batch *b)
     const int nm = b->nm;
     const BatchMap map = b->map;
     const unsigned gm = bgrid(nm, 64);
-    // fl_therm's and fl_rheol's clock updates in one launch
-    BLAUNCH(kb_clock, gm, 64, b->dtab, map, (int)(CK_THERM_BEGIN | (b->no_mech ? 0 : CK_DTAVG_ADD)));
-    const bool dis = b->p0.ishearh == 1 && b->p0.itherm != 2;
-    const int npass = b->m[0]->therm_passes;
-    const bool proof = b->m[0]->therm_proof;
-    for (int pass = 0; pass < npass; pass++) {
-        // pass 0 through the pipeline; a fallback pass, which only some models need,
-        // with one workgroup per tile that returns at once for a proven model
-        const bool ex = b->temp0_prev && !b->noguess && proof;  // (as a model alone, enq_therm)
-        if (pass == 0 && ex)
-            BLAUNCH((dis ? kb_therm_pipe<2, true> : kb_therm_pipe<2, false>), b->therm_grid, TH_J * TH_I,
-                    b->dtab, map, b->tot_t, pass, proof ? 0.0 : GF_THERM_STOL, b->area_pending ? 1 : 0);
-        else if (pass == 0)
-            BLAUNCH((dis ? kb_therm_pipe<0, true> : kb_therm_pipe<0, false>), b->therm_grid, TH_J * TH_I,
-                    b->dtab, map, b->tot_t, pass, proof ? 0.0 : GF_THERM_STOL, b->area_pending ? 1 : 0);
+    const gf_params &p = b->p0;
+    const bool rm = !b->no_mech && b->nloop % p.ifreq_rmasses == 0, im = !b->no_mech && b->nloop % p.ifreq_imasses == 0;
+    // fl_therm's, fl_rheol's and dt_mass's clock updates and the last step's time advance
+    // in one launch, which also turns the buffers over
+    BLAUNCH(kb_begin, gm, 64, b->dtab, map,
+            b->pend_ops | (int)(CK_THERM_BEGIN | (b->no_mech ? 0 : CK_DTAVG_ADD) | (im ? CK_DT_BEGIN : 0)),
+            b->movegrid && !b->no_mech ? 1 : 0);
+    b->pend_ops = 0;
+    const bool dis = p.ishearh == 1 && p.itherm != 2;
+    const int npass = b->m[0]->therm_passes, arp = b->area_pending ? 1 : 0;
+    if (!b->m[0]->therm_proof) {
+        BLAUNCH((dis ? kb_therm_pipe<true> : kb_therm_pipe<false>), b->therm_grid, TH_J * TH_I, b->dtab, map, b->tot_t,
+                GF_THERM_STOL, arp, b->fold ? 1 : 0);
+        if (!b->fold) BLAUNCH(kb_therm_bc, bgrid(b->tot_n, 256), 256, b->dtab, map);
+    } else {
+        const int total = (int)b->tot_t, w = b->therm_w;
+        const bool ex = b->temp0_prev && !b->noguess;  // (as a model alone, enq_therm)
+        const unsigned grid = 8u * (unsigned)((total + 7) / 8);
+        if (ex)
+            BLAUNCH((dis ? kb_therm_strip<true, 2> : kb_therm_strip<false, 2>), grid, 64, b->dtab, map, total, w, arp);
         else
-            BLAUNCH(kb_therm_tile, (unsigned)std::min<long>(b->tot_t, 512), TH_J * TH_I, b->dtab, map, b->tot_t, pass);
-        if (proof) BLAUNCH(kb_therm_check, bgrid(b->tot_b, 256), 256, b->dtab, map, pass);
+            BLAUNCH((dis ? kb_therm_strip<true, 0> : kb_therm_strip<false, 0>), grid, 64, b->dtab, map, total, w, arp);
+        BLAUNCH(kb_therm_check, bgrid(b->tot_b, 256), 256, b->dtab, map, w, arp);
+        BLAUNCH((dis ? kb_therm_rest<true> : kb_therm_rest<false>), b->therm_grid, 256, b->dtab, map, total, w, b->tot_b,
+                arp, npass);
     }
-    BLAUNCH(kb_therm_bc, bgrid(b->tot_n, 256), 256, b->dtab, map, npass, proof ? 1 : 0);
     b->temp0_prev = true;
     if (!b->no_mech) {
-        const gf_params &p = b->p0;
         const int do_visc = (b->nloop % p.ifreq_visc) == 0;
         int avgsr = 0;
         if (b->nsrate == p.ifreq_avgsr)
             avgsr = 1;
         else if (b->nsrate == -1)
             avgsr = 2;
-        if (b->markers && b->nloop % p.ifreq_rmasses == 0) {  // change_phase
+        if (b->markers && rm) {  // change_phase
             if (b->tot_m > 0) BLAUNCH(kb_phase_rules, bgrid(b->tot_m, 256), 256, b->dtab, map);
             BLAUNCH(kb_phase_plan, gm, 64, b->dtab, map);
             BLAUNCH(kb_phase_update, bgrid(b->tot_e, 256), 256, b->dtab, map);
@@ -2613,29 +2647,25 @@ static int enq_batch_flac(gf_batch *b)
             b->nsrate = 0;
         }
         b->nsrate = b->nsrate + 1;
-        BTIMED(1, BLAUNCH(kb_node<M>, bgrid(b->tot_n, b->bs[1]), b->bs[1], b->dtab, map));
-        if (b->movegrid) {  // fl_move returns at once without movegrid (src/fl_move.f90:16)
-            BLAUNCH(kb_move_cord<SV>, bgrid(b->tot_n, 256), 256, b->dtab, map);
-            const bool masses = b->nloop % p.ifreq_rmasses == 0 || b->nloop % p.ifreq_imasses == 0;
-            if (npass == 1 && !masses)
-                b->area_pending = true;
-            else
-                BTIMED(2, BLAUNCH(kb_move_area, bgrid(b->tot_e, b->bs[2]), b->bs[2], b->dtab, map));
-            b->rot_pending = true;
-        }
-        if (b->nloop % p.ifreq_rmasses == 0) {
-            BLAUNCH(kb_dens<M>, bgrid(b->tot_e, 256), 256, b->dtab, map, b->rot_pending ? 1 : 0);
-            BLAUNCH(kb_rmass, bgrid(b->tot_n, 256), 256, b->dtab, map);
-        }
-        if (b->nloop % p.ifreq_imasses == 0) {
-            BLAUNCH(kb_clock, gm, 64, b->dtab, map, (int)CK_DT_BEGIN);
-            BLAUNCH(kb_dt_reduce<SV>, (unsigned)(nm * BATCH_DT_BLOCKS), 256, b->dtab, map);
-            BLAUNCH(kb_dt_scalars, gm, 64, b->dtab, map);
-            BLAUNCH(kb_amass, bgrid(b->tot_n, 256), 256, b->dtab, map);
+        // fl_move returns at once without movegrid (src/fl_move.f90:16); its areas and
+        // rotation wait for the next kb_rheol (the kernels between form what they read)
+        BTIMED(1, BLAUNCH(kb_node<M>, bgrid(b->tot_n, b->bs[1]), b->bs[1], b->dtab, map, b->movegrid ? 1 : 0));
+        b->rot_pending = b->area_pending = b->movegrid;
+        const int arm = b->area_pending ? 1 : 0;
+        if (rm) BLAUNCH(kb_dens<M>, bgrid(b->tot_e, 256), 256, b->dtab, map, b->rot_pending ? 1 : 0);
+        if (im) BLAUNCH(kb_dt_reduce<SV>, (unsigned)(nm * BATCH_DT_BLOCKS), 256, b->dtab, map, arm);
+        if (rm && im) {
+            BLAUNCH(kb_masses, bgrid(b->tot_n, 256), 256, b->dtab, map, arm);
+        } else {
+            if (rm) BLAUNCH(kb_rmass, bgrid(b->tot_n, 256), 256, b->dtab, map, arm);
+            if (im) {
+                BLAUNCH(kb_dt_scalars, gm, 64, b->dtab, map);
+                BLAUNCH(kb_amass, bgrid(b->tot_n, 256), 256, b->dtab, map, arm);
+            }
         }
     }
     b->nloop = b->nloop + 1;
-    BLAUNCH(kb_clock, gm, 64, b->dtab, map, (int)CK_TIME_ADVANCE);
+    b->pend_ops = CK_TIME_ADVANCE;  // (with the next step's first launch, or batch_time)
     return GF_OK;
 }
 
@@ -2649,6 +2679,64 @@ static int enq_batch_step(gf_batch *b)
     }
 }
 
+// the time advance of the last step, on its own
+static int batch_time(gf_batch *b)
+{
+    if (b->pend_ops) BLAUNCH(kb_clock, bgrid(b->nm, 64), 64, b->dtab, b->map, b->pend_ops);
+    b->pend_ops = 0;
+    return GF_OK;
+}
+
+// The table takes the contexts' buffers over where they have changed since the last call
+// (their own steps, uploads, another batch), in the order that kb_begin's next turn
+// expects
+static bool batch_turns_cord(const gf_batch *b) { return b->movegrid && !b->no_mech; }
+static int batch_pointers(gf_batch *b)
+{
+    bool same = b->tab_valid, mine = true;
+    for (int k = 0; k < b->nm; k++) {
+        gf_ctx *c = b->m[k];
+        BatchEntry e = b->tab[k];
+        double *const tbord = e.A.tbord;
+        e.A = c->a;
+        e.A.tbord = tbord;
+        e.tprev = c->a.xa;
+        e.cord_next = c->cord_alt;
+        if (batch_turns_cord(b)) std::swap(e.A.cord, e.cord_next);
+        same = same && memcmp(&e, &b->tab[k], sizeof e) == 0;
+        mine = mine && c->therm_batch == b;
+        c->therm_batch = b;
+        b->tab[k] = e;
+    }
+    if (!same) BCHK(hipMemcpy(b->dtab, b->tab.data(), sizeof(BatchEntry) * (b->nm + 1), hipMemcpyHostToDevice));
+    if (!mine) BLAUNCH(kb_fresh, bgrid(b->nm, 64), 64, b->dtab, b->map);
+    b->tab_valid = false;  // (until the call's end)
+    return GF_OK;
+}
+// the contexts' buffers after `steps` steps (as many of kb_begin's turns)
+static void batch_turn(gf_batch *b, int32_t steps)
+{
+    for (int k = 0; k < b->nm; k++) {
+        gf_ctx *c = b->m[k];
+        BatchEntry &e = b->tab[k];
+        for (int32_t n = 0; n < steps % 3; n++) {
+            double *t = e.tprev;
+            e.tprev = e.A.temp0;
+            e.A.temp0 = e.A.temp;
+            e.A.temp = t;
+        }
+        const bool cord = batch_turns_cord(b);
+        if (cord && steps % 2 != 0) std::swap(e.A.cord, e.cord_next);
+        c->a.temp = e.A.temp;
+        c->a.temp0 = e.A.temp0;
+        c->a.xa = e.tprev;
+        c->a.cord = cord ? e.cord_next : e.A.cord;
+        c->cord_alt = cord ? e.A.cord : e.cord_next;
+        e.A.xa = c->a.xa;  // (as batch_pointers finds it; the kernels use the names above)
+    }
+    b->tab_valid = true;
+}
+
 extern "C" int gf_batch_set_graph(gf_batch *b, int32_t on)
 {
     if (!b) return GF_ERR_ARG;
@@ -2658,11 +2746,15 @@ extern "C" int gf_batch_set_graph(gf_batch *b, int32_t on)
 
 // Steps in cycles of 10 starting at a multiple of 10 repeat the same launches when
 // every frequency divides 10 and the strain-rate average counter starts the cycle
-// at the same value: such cycles replay one captured graph.
+// at the same value: such cycles replay one captured graph.  A cycle also starts with the
+// move of a step before it pending and its start extrapolated, as it ends: a call's first
+// cycle, whose moves are completed, is launched step by step instead of being captured
+// for itself.
 static bool graph_cycle_ok(const gf_batch *b)
 {
     const gf_params &p = b->p0;
-    return b->nloop % 10 == 0 && b->nsrate >= 0 && 10 % p.ifreq_visc == 0 && 10 % p.ifreq_rmasses == 0 &&
+    const bool steady = b->no_mech || (b->rot_pending == b->movegrid && b->area_pending == b->movegrid);
+    return steady && b->temp0_prev && b->nloop % 10 == 0 && b->nsrate >= 0 && 10 % p.ifreq_visc == 0 && 10 % p.ifreq_rmasses == 0 &&
            10 % p.ifreq_imasses == 0 && p.ifreq_avgsr == 10;
 }
 
@@ -2686,53 +2778,47 @@ extern "C" int gf_batch_step(gf_batch *b, int32_t nsteps)
     if (!b || nsteps < 0) return GF_ERR_ARG;
     int rc;
     if ((rc = batch_flush(b))) return rc;
+    if (nsteps == 0) return GF_OK;
+    if ((rc = batch_pointers(b))) return rc;
     for (int32_t n = 0; n < nsteps;) {
         if (b->use_graph && !b->timing && nsteps - n >= 10 && graph_cycle_ok(b)) {
-            if (!b->gexec || b->g_nsrate0 != b->nsrate || b->g_rot0 != b->rot_pending ||
-                b->g_area0 != b->area_pending || b->g_t0prev != b->temp0_prev) {
+            if ((rc = batch_time(b))) return rc;
+            if (!b->gexec || b->g_nsrate0 != b->nsrate) {
                 if (b->gexec) {
                     BCHK(hipGraphExecDestroy(b->gexec));
                     b->gexec = nullptr;
                 }
                 const int32_t ns0 = b->nsrate, nl0 = b->nloop;
-                const bool rot0 = b->rot_pending, area0 = b->area_pending, t0p = b->temp0_prev;
                 hipGraph_t g = nullptr;
                 BCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-                for (int k = 0; k < 10; k++)
-                    if ((rc = enq_batch_step(b))) {
-                        (void)hipStreamEndCapture(b->stream, &g);
-                        if (g) (void)hipGraphDestroy(g);
-                        return rc;
-                    }
+                rc = GF_OK;
+                for (int k = 0; k < 10 && rc == GF_OK; k++) rc = enq_batch_step(b);
+                if (rc == GF_OK) rc = batch_time(b);
+                if (rc) {
+                    (void)hipStreamEndCapture(b->stream, &g);
+                    if (g) (void)hipGraphDestroy(g);
+                    return rc;
+                }
                 BCHK(hipStreamEndCapture(b->stream, &g));
                 hipError_t ie = hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(g);
                 if (ie != hipSuccess) return bset_err(b, GF_ERR_HIP, "hipGraphInstantiate failed");
                 b->g_nsrate0 = ns0;
                 b->g_nsrate1 = b->nsrate;
-                b->g_area_end = b->area_pending;
-                b->g_rot_end = b->rot_pending;
-                b->g_rot0 = rot0;
-                b->g_area0 = area0;
-                b->g_t0prev = t0p;
                 b->nloop = nl0;  // the capture only recorded the launches
                 b->nsrate = ns0;
-                b->rot_pending = rot0;
-                b->area_pending = area0;
-                b->temp0_prev = t0p;
             }
             BCHK(hipGraphLaunch(b->gexec, b->stream));
             b->nloop += 10;
             b->nsrate = b->g_nsrate1;
-            b->rot_pending = b->g_rot_end;  // the cycle ends with a move when the models move
-            b->area_pending = b->g_area_end;
-            b->temp0_prev = true;
             n += 10;
             continue;
         }
         if ((rc = enq_batch_step(b))) return rc;
         n++;
     }
+    if ((rc = batch_time(b))) return rc;
+    batch_turn(b, nsteps);
     if (b->area_pending)  // the negative-area STOP of the last move, now
         BLAUNCH(kb_area_check, bgrid(b->tot_e, 256), 256, b->dtab, b->map);
     BCHK(hipStreamSynchronize(b->stream));
@@ -2743,7 +2829,6 @@ extern "C" int gf_batch_step(gf_batch *b, int32_t nsteps)
         c->rot_pending = b->rot_pending;  // completed by the model's own k_move_rot where needed
         c->area_pending = b->area_pending;
         c->temp0_prev = b->temp0_prev;
-        c->therm_hist = 0;  // (the batch keeps no boundary values)
         c->therm_clean = false;
         int r = fetch_clock(c, nullptr);
         if (r && first == GF_OK) first = r;
@@ -2758,6 +2843,7 @@ extern "C" int gf_batch_autotune(gf_batch *b, int32_t steps, int32_t chosen[3])
 {
     if (!b || steps < 1) return GF_ERR_ARG;
     if (int frc = batch_flush(b)) return frc;
+    if (int prc = batch_pointers(b)) return prc;
     const int cand[3] = {64, 128, 256};
     double best[3] = {1e30, 1e30, 1e30};
     int pick[3] = {256, 256, 256};
@@ -2777,12 +2863,16 @@ extern "C" int gf_batch_autotune(gf_batch *b, int32_t steps, int32_t chosen[3])
                 pick[q] = cand[c];
             }
     }
+    if (int trc = batch_time(b)) return trc;
     BCHK(hipStreamSynchronize(b->stream));
+    batch_turn(b, 3 * steps);
     for (gf_ctx *c : b->m) {
         c->nloop = b->nloop;
         c->nsrate = b->nsrate;
         c->rot_pending = b->rot_pending;
         c->area_pending = b->area_pending;
+        c->temp0_prev = b->temp0_prev;
+        c->therm_clean = false;
     }
     for (int q = 0; q < 3; q++) {
         b->bs[q] = pick[q];

@@ -402,15 +402,20 @@ GF_DEV void therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, const
     if (!still && lane == 0) atomicOr(&ck->therm_pass_changed[it.pass], 2u);
 }
 
+// by the lanes of one wave, for that wave
 GF_DEV void therm_phase_table(const GfDevParams *__restrict__ P, double (*sPh)[GF_MAXPH])
 {
-    for (int q = threadIdx.x; q < GF_MAXPH; q += blockDim.x) {
+    const int q = threadIdx.x % 64;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // (the wave's reads of another model's table are done)
+    if (q < GF_MAXPH) {
         sPh[0][q] = P->ph[q].den;
         sPh[1][q] = P->ph[q].cp;
         sPh[2][q] = 0.5 * P->ph[q].diff;
         sPh[3][q] = 1.0 / P->ph[q].cp;
     }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // pass 0 (mode 0 or 2) or, with launches per phase, a fallback pass: one wave a strip
@@ -549,7 +554,8 @@ __global__ void __launch_bounds__(256) k_therm_rest(const GfDevParams *__restric
                                                     int w, int arp, ThermSlots sl, int npass)
 {
     if (ck->therm_pass_changed[0] == 0u) return;
-    __shared__ double sPh[4][GF_MAXPH];
+    __shared__ double sPhw[4][4][GF_MAXPH];  // (a table a wave)
+    double(*sPh)[GF_MAXPH] = sPhw[threadIdx.x / 64];
     therm_phase_table(P, sPh);
     const ThermGeo g = therm_geo(P, w);
     const int nt = g.nr * g.ns;

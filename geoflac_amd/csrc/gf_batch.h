@@ -24,6 +24,7 @@ struct BatchEntry {
     GfDevArrays A;
     double *tprev;      // the starting temperature of the call before (the next call's result)
     double *cord_next;
+    ThermGeo tg;        // thermal strips
     long pe, pn, pt, pb, pm;  // first global index: elements, nodes, thermal tiles, border entries, markers
     long ce, cn, ct, cb, cm;  // counts of the same
 };
@@ -135,7 +136,7 @@ GF_DEV ThermSlots bslots(const BatchEntry &b) { return therm_slots(b.ck->th_call
 // one wave a strip over the strips of all models
 template <bool DIS, int MODE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
-kb_therm_strip(const BatchEntry *__restrict__ tab, BatchMap map, int total, int w, int arp)
+kb_therm_strip(const BatchEntry *__restrict__ tab, BatchMap map, int total, int arp)
 {
     __shared__ double sPh[4][GF_MAXPH];
     const int q = (total + 7) / 8, g = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
@@ -145,20 +146,20 @@ kb_therm_strip(const BatchEntry *__restrict__ tab, BatchMap map, int total, int 
     therm_phase_table(b.P, sPh);
     const ThermIter it{A.xb, A.xa, arp, 0};
     const int t = g - (int)b.pt;
-    therm_strip<DIS, MODE>(b.P, b.ck, A, therm_geo(b.P, w), t, it, bslots(b), A.tbord + (long)t * TS_NB(w), b.ck->dt,
+    therm_strip<DIS, MODE>(b.P, b.ck, A, b.tg, t, it, bslots(b), A.tbord + (long)t * TS_NB(b.tg.w), b.ck->dt,
                            sPh);
 }
-__global__ void __launch_bounds__(256) kb_therm_check(const BatchEntry *__restrict__ tab, BatchMap map, int w, int arp)
+__global__ void __launch_bounds__(256) kb_therm_check(const BatchEntry *__restrict__ tab, BatchMap map, int arp)
 {
     batch_apply<BK_BORD>(tab, map, [&](const BatchEntry &b, long t) {
-        therm_check_one(b.P, b.ck, bthermal(b), therm_geo(b.P, w), t, 0, arp, bslots(b));
+        therm_check_one(b.P, b.ck, bthermal(b), b.tg, t, 0, arp, bslots(b));
     });
 }
 // Returns at once when every model's pass 0 is proven.  Otherwise the further passes of
 // the models that are not, with grid barriers on the first model's counters (one workgroup
 // per CU at most, as k_therm_rest).
 template <bool DIS>
-__global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restrict__ tab, BatchMap map, int total, int w,
+__global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restrict__ tab, BatchMap map, int total,
                                                      long border, int arp, int npass)
 {
     auto flag = [&](int m, int pass) {  // written by other workgroups of this launch too
@@ -184,7 +185,7 @@ __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restric
             therm_phase_table(b.P, sPh);
             const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, arp, pass};
             const int t = g - (int)b.pt;
-            therm_strip<DIS, 1>(b.P, b.ck, A, therm_geo(b.P, w), t, it, bslots(b), A.tbord + (long)t * TS_NB(w),
+            therm_strip<DIS, 1>(b.P, b.ck, A, b.tg, t, it, bslots(b), A.tbord + (long)t * TS_NB(b.tg.w),
                                 b.ck->dt, sPh);
         }
         if (!grid_sync(bar)) return;  // every strip's iterate is written
@@ -193,7 +194,7 @@ __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restric
             const long t = g + threadIdx.x - b.pb;
             if (t < b.cb &&
                 __hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)
-                therm_check_one(b.P, b.ck, bthermal(b), therm_geo(b.P, w), t, pass, arp, bslots(b));
+                therm_check_one(b.P, b.ck, bthermal(b), b.tg, t, pass, arp, bslots(b));
         }
         if (!grid_sync(bar)) return;  // every border is checked
         if (!open_after(pass)) break;

@@ -14,6 +14,7 @@
 #include "gf_ddmath.h"
 
 #define GF_DEV static __device__ __forceinline__
+#define GF_DEVM __device__ __forceinline__  // (members)
 
 // Per-phase constants (phase id k stored at index k-1).
 struct GfPhase {

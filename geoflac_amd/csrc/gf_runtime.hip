@@ -101,10 +101,12 @@ struct gf_ctx {
     // fit on every CU)
     bool therm_rest = false;
     int therm_w = 0;     // output columns of a thermal strip
+    bool therm_cols = false;  // pass 0 by a workgroup a strip (k_therm_cols)
     int therm_call = 0;  // thermal calls, modulo 3: the slot of a.tpre this call writes
     ThermChk chk{};      // the border check of the thermal call under way
     int node_ops = 0;    // clock updates left to the step's fl_node
     bool therm_clean = true;  // the flags of the thermal passes are 0 on the device
+    double dt_seen = 0.0;  // the clock's dt at the last read-back (a hint for the thermal halo)
     void *therm_batch = nullptr;  // the batch whose steps were the model's last thermal calls
     int therm_hist = 0;  // calls before it (at most 2) whose slots hold their boundary values
     // per-kernel event timing
@@ -133,20 +135,10 @@ static int set_err(gf_ctx *c, int code, const char *fmt, ...)
             return set_err(ctx, GF_ERR_HIP, "%s failed: %s", #call, hipGetErrorString(e_));   \
     } while (0)
 
-static ThermGeo therm_geo_host(const gf_params &p, int w)
-{
-    ThermGeo g;
-    g.nz = p.nz;
-    g.nx = p.nx;
-    g.w = w;
-    g.nr = g.nz <= 64 ? 1 : (g.nz - 2 * TS_HB + TS_OJ - 1) / TS_OJ;
-    g.ns = (g.nx + w - 1) / w;
-    return g;
-}
-// Output columns of the thermal strips of one or more meshes in a launch.  A strip of w columns takes some w + 6 column times
-// (halo, ring, start); a column takes a wave alone on its SIMD 1.3 us (latency), n waves
-// 0.6 us more each, 0.9 us each where issue bounds.  The width of least time over the
-// 1024 SIMDs.  Measured, us a step (whole step) at widths 2, 4, 8, 16, 24: 401x101 nodes
+// Output columns of the thermal strips of one or more meshes that a launch marches over.  A
+// strip of w columns takes some w + 6 column times (halo, ring, start); a column takes a
+// wave alone on its SIMD 1.3 us (latency), n waves 0.6 us more each, 0.9 us each where
+// issue bounds.  The width of least time over the 1024 SIMDs.  Measured, us a step (whole step) at widths 2, 4, 8, 16, 24: 401x101 nodes
 // 38, 41, 47, 59, 70; 902x302 101, 97, 102, 110, 121; 2001x1001 541, 508, 492, 493, 497.
 static int therm_strip_width(const std::vector<const gf_params *> &ps)
 {
@@ -155,7 +147,7 @@ static int therm_strip_width(const std::vector<const gf_params *> &ps)
     for (int w = 2; w <= 32; w++) {
         long strips = 0;
         for (const gf_params *p : ps) {
-            const ThermGeo g = therm_geo_host(*p, w);
+            const ThermGeo g = therm_geo(p->nz, p->nx, w);
             strips += (long)g.nr * g.ns;
         }
         const double n = (double)strips / 1024.0;
@@ -335,7 +327,10 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
         const char *tm = getenv("GF_THERM");
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_therm_rest<true>, 256, 0) != hipSuccess) nb = 0;
         ctx->therm_rest = nb >= 1 && ncu >= 8 && !(tm && strcmp(tm, "multi") == 0);
-        ctx->therm_w = therm_strip_width({p});
+        // a workgroup a strip where every strip then has a CU of its own
+        const ThermGeo gc = therm_geo(p->nz, p->nx, TC_W - 1 - TC_HI);
+        ctx->therm_cols = gc.nr * gc.ns <= ncu;
+        ctx->therm_w = ctx->therm_cols ? gc.w : therm_strip_width({p});
         (void)hipGetLastError();
     }
     ALLOC(ctx->dp, sizeof(GfDevParams));
@@ -374,7 +369,7 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
     ALLOC(ctx->a.xa, 8 * nn);
     ALLOC(ctx->a.xb, 8 * nn);
     {
-        const ThermGeo g = therm_geo_host(*p, ctx->therm_w);
+        const ThermGeo g = therm_geo(p->nz, p->nx, ctx->therm_w);
         ALLOC(ctx->therm_border, 8 * (size_t)g.nr * g.ns * TS_NB(g.w));
     }
     ctx->a.tbord = ctx->therm_border;
@@ -1051,6 +1046,7 @@ extern "C" int gf_set_clock(gf_ctx *ctx, const gf_clock *c)
     HIPCHK(hipMemcpy(ctx->dck, &ck, sizeof(ck), hipMemcpyHostToDevice));
     ctx->nloop = c->nloop;
     ctx->nsrate = c->nsrate;
+    ctx->dt_seen = c->dt;
     return GF_OK;
 }
 
@@ -1060,6 +1056,7 @@ static int fetch_clock(gf_ctx *ctx, gf_clock *c)
     GfDevClock ck;
     HIPCHK(hipStreamSynchronize(ctx->stream));
     HIPCHK(hipMemcpy(&ck, ctx->dck, sizeof(ck), hipMemcpyDeviceToHost));
+    ctx->dt_seen = ck.dt;
     if (ctx->markers_uploaded && ctx->p.topo_kappa > 0.0) ctx->a.nmarkers = ck.nmarkers;  // (resurface appends)
     if (ck.bar_timeout != 0) {  // (not expected: every workgroup of the launch is resident)
         GfDevClock z = ck;
@@ -1228,18 +1225,25 @@ static int enq_therm(gf_ctx *ctx, int ops = 0, bool defer = false)
         if (!fold) LAUNCH(k_therm_bc, 2L * (ctx->p.nx + ctx->p.nz), ctx->dp, ctx->a);
         return enq_therm_rest(ctx);
     }
-    const ThermGeo g = therm_geo_host(ctx->p, ctx->therm_w);
+    const ThermGeo g = therm_geo(ctx->p.nz, ctx->p.nx, ctx->therm_w);
     const unsigned grid = 8u * (unsigned)((g.nr * g.ns + 7) / 8);
     const long nb = (long)g.nr * g.ns * TS_NB(g.w);
-    ctx->chk = ThermChk{(int)nblk(nb), g.w, arp, therm_slots(ctx->therm_call, ctx->therm_hist), ctx->a.temp, ctx->a.xa};
+    ctx->chk = ThermChk{(int)nblk(nb), arp, g, therm_slots(ctx->therm_call, ctx->therm_hist), ctx->a.temp, ctx->a.xa};
     // pass 0 starts from the extrapolation 2 temp - temp0 once temp0 holds the
     // previous step's starting temperature
     const bool ex = ctx->temp0_prev && !ctx->therm_noguess;
-    auto kern = ex ? (dis ? k_therm_strip<true, 2> : k_therm_strip<false, 2>)
-                   : (dis ? k_therm_strip<true, 0> : k_therm_strip<false, 0>);
-    LAUNCH_DIM("k_therm_strip", kern, grid, 64, ctx->dp, ctx->dck, ctx->a, g.w, 0, arp, ctx->chk.sl, ops);
+    // (a mesh whose columns couple more strongly than TC_HI halo columns damp is marched)
+    if (ctx->therm_cols && therm_halo(ctx->hp.diff_max, ctx->hp.rxbo, g.nx, ctx->dt_seen) <= TC_HI) {
+        auto kern = ex ? (dis ? k_therm_cols<true, 2> : k_therm_cols<false, 2>)
+                       : (dis ? k_therm_cols<true, 0> : k_therm_cols<false, 0>);
+        LAUNCH_DIM("k_therm_cols", kern, grid, 64 * TC_W, ctx->dp, ctx->dck, ctx->a, g, arp, ctx->chk.sl, ops);
+    } else {
+        auto kern = ex ? (dis ? k_therm_strip<true, 2> : k_therm_strip<false, 2>)
+                       : (dis ? k_therm_strip<true, 0> : k_therm_strip<false, 0>);
+        LAUNCH_DIM("k_therm_strip", kern, grid, 64, ctx->dp, ctx->dck, ctx->a, g, 0, arp, ctx->chk.sl, ops);
+    }
     if (defer) return GF_OK;
-    LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, g.w, 0, arp, ctx->chk.sl, nb);
+    LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, g, 0, arp, ctx->chk.sl, nb);
     return enq_therm_rest(ctx);
 }
 
@@ -1248,7 +1252,8 @@ static int enq_therm_rest(gf_ctx *ctx)
 {
     if (ctx->therm_proof) {
         const bool dis = ctx->p.ishearh == 1 && ctx->p.itherm != 2;
-        const int npass = ctx->therm_passes, w = ctx->chk.w, arp = ctx->chk.arp;
+        const int npass = ctx->therm_passes, arp = ctx->chk.arp;
+        const ThermGeo g = ctx->chk.g;
         const ThermSlots sl = ctx->chk.sl;
         if (ctx->therm_rest) {
             // A plain launch: its grid (one workgroup per CU, at most the CUs) is resident
@@ -1258,15 +1263,14 @@ static int enq_therm_rest(gf_ctx *ctx)
             // waiting for ever.  (A cooperative launch guarantees residency but costs
             // ~16 us more per launch on MI355X, more than the launches it replaces.)
             auto rest = dis ? k_therm_rest<true> : k_therm_rest<false>;
-            LAUNCH_DIM("k_therm_rest", rest, ctx->therm_grid, 256, ctx->dp, ctx->dck, ctx->a, w, arp, sl, npass);
+            LAUNCH_DIM("k_therm_rest", rest, ctx->therm_grid, 256, ctx->dp, ctx->dck, ctx->a, g, arp, sl, npass);
         } else {
-            const ThermGeo g = therm_geo_host(ctx->p, w);
             const unsigned grid = 8u * (unsigned)((g.nr * g.ns + 7) / 8);
-            const long nb = (long)g.nr * g.ns * TS_NB(w);
+            const long nb = (long)g.nr * g.ns * TS_NB(g.w);
             auto extra = dis ? k_therm_strip<true, 1> : k_therm_strip<false, 1>;
             for (int pass = 1; pass < npass; pass++) {
-                LAUNCH_DIM("k_therm_strip_extra", extra, grid, 64, ctx->dp, ctx->dck, ctx->a, w, pass, arp, sl, 0);
-                LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, w, pass, arp, sl, nb);
+                LAUNCH_DIM("k_therm_strip_extra", extra, grid, 64, ctx->dp, ctx->dck, ctx->a, g, pass, arp, sl, 0);
+                LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, g, pass, arp, sl, nb);
             }
             LAUNCH_DIM("k_therm_last", k_therm_last, ctx->therm_grid, 256, ctx->dp, ctx->dck, ctx->a, sl, npass);
         }
@@ -2501,12 +2505,12 @@ extern "C" int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out)
         if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(GF_ERR_HIP, "sync");
         // thermal strips of the proven step (and their border values), or the tiles of
         // FP32-arithmetic mode
-        const ThermGeo tg = therm_geo_host(q, b->therm_w);
+        const ThermGeo tg = therm_geo(q.nz, q.nx, b->therm_w);
         const long ntiles = c0->therm_proof ? (long)tg.nr * tg.ns
                                             : (long)((q.nz + TH_OJ - 1) / TH_OJ) * ((q.nx + TH_OI - 1) / TH_OI);
         const long nbord = c0->therm_proof ? ntiles * TS_NB(b->therm_w) : 0;
         const long nmk = c->markers_uploaded ? c->a.nmarkers : 0;
-        tab[k] = BatchEntry{c->dp, c->dck, c->a, nullptr, nullptr, pe, pn, pt, pb, pm, c->ne, c->nn, ntiles, nbord, nmk};
+        tab[k] = BatchEntry{c->dp, c->dck, c->a, nullptr, nullptr, tg, pe, pn, pt, pb, pm, c->ne, c->nn, ntiles, nbord, nmk};
         b->fold = b->fold && q.itemp_bc != 2;
         if (nmk > 0) b->markers = true;
         mm.insert(mm.end(), align(nmk) / BATCH_ALIGN, k);
@@ -2521,7 +2525,7 @@ extern "C" int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out)
         pb += align(nbord);
         b->m.push_back(c);
     }
-    tab[n] = BatchEntry{nullptr, nullptr, GfDevArrays{}, nullptr, nullptr, pe, pn, pt, pb, pm, 0, 0, 0, 0, 0};
+    tab[n] = BatchEntry{nullptr, nullptr, GfDevArrays{}, nullptr, nullptr, ThermGeo{}, pe, pn, pt, pb, pm, 0, 0, 0, 0, 0};
     b->nm = n;
     b->tot_e = pe; b->tot_n = pn; b->tot_t = pt; b->tot_b = pb; b->tot_m = pm;
     b->movegrid = c0->p.movegrid != 0;
@@ -2613,15 +2617,15 @@ static int enq_batch_flac(gf_batch *b)
                 GF_THERM_STOL, arp, b->fold ? 1 : 0);
         if (!b->fold) BLAUNCH(kb_therm_bc, bgrid(b->tot_n, 256), 256, b->dtab, map);
     } else {
-        const int total = (int)b->tot_t, w = b->therm_w;
+        const int total = (int)b->tot_t;
         const bool ex = b->temp0_prev && !b->noguess;  // (as a model alone, enq_therm)
         const unsigned grid = 8u * (unsigned)((total + 7) / 8);
         if (ex)
-            BLAUNCH((dis ? kb_therm_strip<true, 2> : kb_therm_strip<false, 2>), grid, 64, b->dtab, map, total, w, arp);
+            BLAUNCH((dis ? kb_therm_strip<true, 2> : kb_therm_strip<false, 2>), grid, 64, b->dtab, map, total, arp);
         else
-            BLAUNCH((dis ? kb_therm_strip<true, 0> : kb_therm_strip<false, 0>), grid, 64, b->dtab, map, total, w, arp);
-        BLAUNCH(kb_therm_check, bgrid(b->tot_b, 256), 256, b->dtab, map, w, arp);
-        BLAUNCH((dis ? kb_therm_rest<true> : kb_therm_rest<false>), b->therm_grid, 256, b->dtab, map, total, w, b->tot_b,
+            BLAUNCH((dis ? kb_therm_strip<true, 0> : kb_therm_strip<false, 0>), grid, 64, b->dtab, map, total, arp);
+        BLAUNCH(kb_therm_check, bgrid(b->tot_b, 256), 256, b->dtab, map, arp);
+        BLAUNCH((dis ? kb_therm_rest<true> : kb_therm_rest<false>), b->therm_grid, 256, b->dtab, map, total, b->tot_b,
                 arp, npass);
     }
     b->temp0_prev = true;

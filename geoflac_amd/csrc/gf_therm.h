@@ -55,34 +55,32 @@ GF_DEV double *therm_pre(const GfDevParams *P, const GfDevArrays &A, int slot)
     return A.tpre + (long)slot * 2 * (P->nx + P->nz);
 }
 
-// Halo columns of a strip: each damps what the ring's start leaves by the coupling of
-// columns c = diff dt / dx^2, and that error is some 1e-5 of a value's change (rows 1
-// and nz, whose start follows the last two calls).  Enough of them that c^hi <= 1e-11
-// (at least 2): at c = 1.3e-2 (901x301 cells of 333 m) 4, 5 and 6 columns need a further
-// pass in 45%, 2% and none of the steps; more columns only cost their own time, and
-// what a strip leaves unsettled the border check finds.
-GF_DEV int therm_halo(const GfDevParams *P, double dt)
+struct ThermGeo {
+    int nz, nx, w, nr, ns;  // row strips, column strips
+};
+__host__ __device__ inline ThermGeo therm_geo(int nz, int nx, int w)
 {
-    const double dx = P->rxbo / (double)(P->nx - 1), c = P->diff_max * dt / (dx * dx);
+    ThermGeo g;
+    g.nz = nz;
+    g.nx = nx;
+    g.w = w;
+    g.nr = nz <= 64 ? 1 : (nz - 2 * TS_HB + TS_OJ - 1) / TS_OJ;
+    g.ns = (nx + w - 1) / w;
+    return g;
+}
+// Halo columns of a strip: each damps what the ring's start leaves by the coupling of
+// columns c = diff dt / dx^2, and that error is some 1e-5 of a value's change (rows 1 and
+// nz, whose start follows the last two calls).  Enough of them that c^hi <= 1e-11 (at
+// least 2): at c = 1.3e-2 (901x301 cells of 333 m) 4, 5 and 6 columns need a further pass
+// in 45%, 2% and none of the steps; more columns only cost their own time, and what a
+// strip leaves unsettled the border check finds.
+__host__ __device__ inline int therm_halo(double diff_max, double rxbo, int nx, double dt)
+{
+    const double dx = rxbo / (double)(nx - 1), c = diff_max * dt / (dx * dx);
     int hi = 2;
     for (double v = c * c; v > 1.0e-11 && hi < TS_HI_MAX; v *= c) hi++;
     return hi;
 }
-
-struct ThermGeo {
-    int nz, nx, w, nr, ns;  // row strips, column strips
-};
-GF_DEV ThermGeo therm_geo(const GfDevParams *P, int w)
-{
-    ThermGeo g;
-    g.nz = P->nz;
-    g.nx = P->nx;
-    g.w = w;
-    g.nr = g.nz <= 64 ? 1 : (g.nz - 2 * TS_HB + TS_OJ - 1) / TS_OJ;
-    g.ns = (g.nx + w - 1) / w;
-    return g;
-}
-// strip t (row strips fastest): row of lane 0, first and last output lane, output columns
 struct ThermStrip {
     int jb, fo, lo, c0, c1;
     bool top, bot;  // it holds the mesh's first, last row
@@ -157,47 +155,76 @@ struct ThermIter {
     int pass;
 };
 
-// One strip.  MODE, the start: 0 the old temperature, 1 xin, 2 the extrapolation
-// 2 temp - temp0.  sPh: den, cp, 0.5 diff, 1 / cp per phase (LDS).
+// What a wave knows of its strip, and its loads and stores.  MODE, the start: 0 the old
+// temperature, 1 xin, 2 the extrapolation 2 temp - temp0.
 template <bool DIS, int MODE>
-GF_DEV void therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, const ThermGeo &g,
-                        int t, const ThermIter &it, const ThermSlots &sl, double *bord, double dt,
-                        const double (*sPh)[GF_MAXPH])
-{
-    t = __builtin_amdgcn_readfirstlane(t);
-    const int lane = threadIdx.x % 64;
-    const ThermStrip s = therm_strip_of(g, t);
-    const int nz = g.nz, nx = g.nx, row = s.jb + lane;
-    const unsigned nn = (unsigned)nz * nx, ne = (unsigned)(nz - 1) * (nx - 1);
-    constexpr unsigned OOB = 0x80000000u;  // past every array: loads read 0, stores are dropped
-    const unsigned nvo = row <= nz ? (unsigned)(row - 1) * 8u : OOB;
-    const bool erow = row < nz && lane < 63;
-    const unsigned evo = erow ? (unsigned)(row - 1) * 8u : OOB, evi = erow ? (unsigned)(row - 1) * 4u : OOB;
-    const Buf bT = mkbuf(A.temp, 8ull * nn), bC = mkbuf(A.cord, 16ull * nn),
-              bG = mkbuf(MODE == 1 ? it.xin : A.temp0, 8ull * nn), bX = mkbuf(it.xout, 8ull * nn),
-              bA = mkbuf(A.area, 16ull * ne), bS = mkbuf(A.source, 8ull * ne), bI = mkbuf(A.iphase, 4ull * ne),
-              bH = mkbuf(A.shrheat, 8ull * ne);
-    const unsigned npre = 2u * (nx + nz);
-    const bool edge = s.top || s.bot;  // (uniform)
-    const bool erow1 = row == 1, erown = row == nz;
-    // start of rows 1 and nz: the values before the boundary conditions of the last two
-    // calls, carried on (pass 0), or those of the last pass (the iterate's own boundary
-    // rows hold the conditions)
-    const int pslot = MODE == 1 ? sl.cur[(it.pass - 1) & 1] : sl.prev;
-    const Buf bP = mkbuf(A.tpre + (long)pslot * npre, 8ull * npre),
-              bP2 = mkbuf(A.tpre + (long)sl.prev2 * npre, 8ull * npre),
-              bW = mkbuf(A.tpre + (long)sl.cur[it.pass & 1] * npre, 8ull * npre);
-    const unsigned pvo = erow1 ? 0u : erown ? 8u * nx : OOB;  // row arrays, + 8 (i - 1)
-    const unsigned pco = row <= nz ? 8u * (2 * nx + row - 1) : OOB;  // column arrays, + 8 nz for column nx
-    const bool pedge = edge && (MODE == 1 || (MODE == 2 && sl.hist > 0));
-    const bool plin = MODE == 2 && sl.hist > 1;
+struct ThermWave {
+    const GfDevParams *__restrict__ P;
+    ThermGeo g;
+    ThermStrip s;
+    int hi, lane, row, nz, nx, arp;
+    unsigned nn, ne, nvo, evo, evi, pvo, pco;
+    bool erow, edge, erow1, erown, pedge, plin;
+    // lanes that hold the start in every column (the ring rows), or no node
+    bool hold;
+    Buf bT, bC, bG, bX, bA, bS, bI, bH, bP, bP2, bW;
+    double *bord;
 
+    static constexpr unsigned OOB = 0x80000000u;  // past every array: loads read 0, stores are dropped
     struct Node {
         double x, y, t, g, p, p2;
     };
-    auto load_node = [&](int i) {
+    struct Elem {
+        double a0, a1, src, sh;
+        int ph;
+    };
+
+    GF_DEVM ThermWave(const GfDevParams *__restrict__ P_, const GfDevArrays &A, const ThermGeo &g_, int t,
+                      const ThermIter &it, const ThermSlots &sl, double *bord_, int hi_)
+        : P(P_), g(g_), hi(hi_), bord(bord_)
+    {
+        s = therm_strip_of(g, t);
+        lane = threadIdx.x % 64;
+        nz = g.nz;
+        nx = g.nx;
+        arp = it.arp;
+        row = s.jb + lane;
+        nn = (unsigned)nz * nx;
+        ne = (unsigned)(nz - 1) * (nx - 1);
+        nvo = row <= nz ? (unsigned)(row - 1) * 8u : OOB;
+        erow = row < nz && lane < 63;
+        evo = erow ? (unsigned)(row - 1) * 8u : OOB;
+        evi = erow ? (unsigned)(row - 1) * 4u : OOB;
+        edge = s.top || s.bot;  // (uniform)
+        erow1 = row == 1;
+        erown = row == nz;
+        hold = (lane == 0 && !s.top) || (lane == 63 && !s.bot) || row > nz;
+        bT = mkbuf(A.temp, 8ull * nn);
+        bC = mkbuf(A.cord, 16ull * nn);
+        bG = mkbuf(MODE == 1 ? it.xin : A.temp0, 8ull * nn);
+        bX = mkbuf(it.xout, 8ull * nn);
+        bA = mkbuf(A.area, 16ull * ne);
+        bS = mkbuf(A.source, 8ull * ne);
+        bI = mkbuf(A.iphase, 4ull * ne);
+        bH = mkbuf(A.shrheat, 8ull * ne);
+        // start of rows 1 and nz: the values before the boundary conditions of the last two
+        // calls, carried on (pass 0), or those of the last pass (the iterate's own boundary
+        // rows hold the conditions)
+        const unsigned npre = 2u * (nx + nz);
+        const int pslot = MODE == 1 ? sl.cur[(it.pass - 1) & 1] : sl.prev;
+        bP = mkbuf(A.tpre + (long)pslot * npre, 8ull * npre);
+        bP2 = mkbuf(A.tpre + (long)sl.prev2 * npre, 8ull * npre);
+        bW = mkbuf(A.tpre + (long)sl.cur[it.pass & 1] * npre, 8ull * npre);
+        pvo = erow1 ? 0u : erown ? 8u * nx : OOB;               // row arrays, + 8 (i - 1)
+        pco = row <= nz ? 8u * (2 * nx + row - 1) : OOB;        // column arrays, + 8 nz for column nx
+        pedge = edge && (MODE == 1 || (MODE == 2 && sl.hist > 0));
+        plin = MODE == 2 && sl.hist > 1;
+    }
+    // node column i (i >= 1; 0 past the mesh and past the strip's last neighbours)
+    GF_DEVM Node node(int i) const
+    {
         Node n{0, 0, 0, 0, 0, 0};
-        if (i <= min(nx, s.c1 + 1)) {  // (uniform; i >= 1)
+        if (i <= min(nx, s.c1 + 1)) {  // (uniform)
             const unsigned so = (unsigned)nz * (unsigned)(i - 1) * 8u;
             n.x = bld(bC, nvo, so);
             n.y = bld(bC, nvo, so + 8u * nn);
@@ -207,130 +234,197 @@ GF_DEV void therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, const
                 n.p = bld(bP, pvo, 8u * (i - 1));
                 if (plin) n.p2 = bld(bP2, pvo, 8u * (i - 1));
             }
-            if (MODE == 1 && (i == 1 || i == nx)) {  // (the iterate's boundary columns, likewise)
+            if (MODE == 1 && (i == 1 || i == nx))  // (the iterate's boundary columns, likewise)
                 n.g = bld(bP, pco, i == 1 ? 0u : 8u * nz);
-            }
         }
         return n;
-    };
-    struct Elem {
-        double a0, a1, src, sh;
-        int ph;
-    };
-    auto load_elem = [&](int i) {
+    }
+    GF_DEVM Elem elem(int i) const
+    {
         Elem e{0, 0, 0, 0, 1};
         if (i <= min(nx - 1, s.c1)) {
             const unsigned ec = (unsigned)(nz - 1) * (unsigned)(i - 1);
             e.src = bld(bS, evo, ec * 8u);
             e.ph = bldi(bI, evi, ec * 4u);
-            if (!it.arp) {
+            if (!arp) {
                 e.a0 = bld(bA, evo, ec * 8u);
                 e.a1 = bld(bA, evo, (ec + ne) * 8u);
             }
             if (DIS) e.sh = bld(bH, evo, ec * 8u);
         }
         return e;
-    };
-    auto start_of = [&](const Node &n) {
+    }
+    GF_DEVM double start(const Node &n) const
+    {
         double v = MODE == 0 ? n.t : MODE == 1 ? n.g : 2.0 * n.t - n.g;
         if (pedge && (erow1 || erown)) v = plin ? 2.0 * n.p - n.p2 : n.p;
         return v;
-    };
-
-    const int hi = __builtin_amdgcn_readfirstlane(therm_halo(P, dt));
-    const int ib = max(1, s.c0 - hi - 1);
-    const bool has_ring = s.c0 - hi > 1;  // column ib only holds the start
-    // lanes that hold the start in every column (the ring rows), or no node
-    const bool hold = (lane == 0 && !s.top) || (lane == 63 && !s.bot) || row > nz;
-
-    Node n0 = load_node(ib), n1 = load_node(ib + 1);
-    Elem e0 = load_elem(ib);
-    double ydn0 = lane_dn(n0.y), xdn0 = lane_dn(n0.x), tdn0 = lane_dn(n0.t);
-    double xl = 0.0, xd = 0.0;  // X(j, i-1), X(j+1, i-1)
-    // element column i-1: triangle B one row up, A and B of this row
-    double lB13 = 0, lB23 = 0, lB33 = 0, lBp = 0, lBq = 0, lBr = 0;
-    double mA13 = 0, mA23 = 0, mA33 = 0, mAp = 0, mAq = 0, mAr = 0;
-    double mB11 = 0, mB12 = 0, mB13 = 0, mBp = 0, mBq = 0, mBr = 0;
-    bool still = true;
-    for (int i = ib; i <= s.c1; i++) {
-        // the loads of the columns ahead
-        const Node n2 = load_node(i + 2);
-        const Elem e1 = load_elem(i + 1);
-        // ---- element column i (between node columns i and i+1)
-        const double ydn1 = lane_dn(n1.y), xdn1 = lane_dn(n1.x), tdn1 = lane_dn(n1.t);
-        const int phs = e0.ph >= 1 && e0.ph <= GF_MAXPH ? e0.ph - 1 : 0;  // (0 where there is no element)
+    }
+    // Element column i between node columns n0 and n1 (yd, xd: their rows below).
+    // sPh: den, cp, 0.5 diff, 1 / cp per phase (LDS).
+    GF_DEVM void tris(int i, const Node &n0, const Node &n1, double xd0, double yd0, double xd1, double yd1,
+                      const Elem &e, int phs, const double (*sPh)[GF_MAXPH], ThermTri &ta, ThermTri &tb) const
+    {
         const bool eok = erow && i < nx;
-        ThermTri ta, tb;
-        {
-            double ar0 = e0.a0, ar1 = e0.a1, inv0, inv1;
-            if (it.arp) {
-                const double xc[5] = {0.0, n0.x, xdn0, n1.x, xdn1}, yc[5] = {0.0, n0.y, ydn0, n1.y, ydn1};
-                const double det0 = move_det(xc, yc, 0), det1 = move_det(xc, yc, 1);
-                ar0 = rcp_core(det0);
-                ar1 = rcp_core(det1);
-                inv0 = rcp_back(ar0, det0);
-                inv1 = rcp_back(ar1, det1);
-                if (__any(eok && !(rcp_safe(det0) && rcp_safe(det1) && rcp_safe(ar0) && rcp_safe(ar1)))) {
-                    ar0 = 1.0 / det0;
-                    ar1 = 1.0 / det1;
-                    inv0 = 1.0 / ar0;
-                    inv1 = 1.0 / ar1;
-                }
-            } else {
-                inv0 = rcp_core(ar0);
-                inv1 = rcp_core(ar1);
-                if (__any(eok && !(rcp_safe(ar0) && rcp_safe(ar1)))) {
-                    inv0 = 1.0 / ar0;
-                    inv1 = 1.0 / ar1;
+        double ar0 = e.a0, ar1 = e.a1, inv0, inv1;
+        if (arp) {
+            const double xc[5] = {0.0, n0.x, xd0, n1.x, xd1}, yc[5] = {0.0, n0.y, yd0, n1.y, yd1};
+            const double det0 = move_det(xc, yc, 0), det1 = move_det(xc, yc, 1);
+            ar0 = rcp_core(det0);
+            ar1 = rcp_core(det1);
+            inv0 = rcp_back(ar0, det0);
+            inv1 = rcp_back(ar1, det1);
+            if (__any(eok && !(rcp_safe(det0) && rcp_safe(det1) && rcp_safe(ar0) && rcp_safe(ar1)))) {
+                ar0 = 1.0 / det0;
+                ar1 = 1.0 / det1;
+                inv0 = 1.0 / ar0;
+                inv1 = 1.0 / ar1;
+            }
+        } else {
+            inv0 = rcp_core(ar0);
+            inv1 = rcp_core(ar1);
+            if (__any(eok && !(rcp_safe(ar0) && rcp_safe(ar1)))) {
+                inv0 = 1.0 / ar0;
+                inv1 = 1.0 / ar1;
+            }
+        }
+        ar0 = eok ? ar0 : 0.0;
+        ar1 = eok ? ar1 : 0.0;
+        inv0 = eok ? inv0 : 0.0;
+        inv1 = eok ? inv1 : 0.0;
+        // dummye = (source + dissip / den) / cp (:405-414; + 0 without shear heating)
+        const double sd = DIS ? e.src + e.sh / sPh[0][phs] : e.src + 0.0, cp = sPh[1][phs];
+        double dm = div_fma(sd, cp, sPh[3][phs]);
+        if (__any(eok && sd != 0.0 && !(rcp_safe(sd) && rcp_safe(cp)))) dm = sd / cp;
+        dm = eok ? dm : 0.0;
+        const double hdf = sPh[2][phs];
+        const double y1 = n0.y, y2 = yd0, y3 = n1.y, y4 = yd1, x1 = n0.x, x2 = xd0, x3 = n1.x, x4 = xd1;
+        const double da[6] = {(y2 - y3) * ar0, (y3 - y1) * ar0, (y1 - y2) * ar0,
+                              (x3 - x2) * ar0, (x1 - x3) * ar0, (x2 - x1) * ar0};
+        const double db[6] = {(y2 - y4) * ar1, (y4 - y3) * ar1, (y3 - y2) * ar1,
+                              (x4 - x2) * ar1, (x3 - x4) * ar1, (x2 - x3) * ar1};
+        ta = therm_tri(da, inv0, dm, hdf);
+        tb = therm_tri(db, inv1, dm, hdf);
+    }
+    // 1 / area of a node, 0 in the lanes that hold their start (a zero increment)
+    GF_DEVM double rarea(double area_n) const
+    {
+        double r = rcp_core(area_n);
+        if (__any(!hold && !rcp_safe(area_n))) r = 1.0 / area_n;
+        return hold ? 0.0 : r;
+    }
+    // the result x of column i and the border values it holds
+    GF_DEVM void store(int i, double x, double y, int phs) const
+    {
+        if (i < s.c0) {
+            if (i == s.c0 - 1) bord[2 * g.w + lane] = x;
+            return;
+        }
+        const bool out = lane >= s.fo && lane <= s.lo;
+        const unsigned so = (unsigned)nz * (unsigned)(i - 1) * 8u;
+        const unsigned vo = out ? nvo : OOB;
+        double v = x;
+        if (edge) {
+            // before the conditions: kept apart
+            bst(bW, out ? pvo : OOB, 8u * (i - 1), x);
+            double vb = P->bot_bc;
+            if (P->itemp_bc != 1) {
+                vb = x;
+                if (P->itemp_bc == 2) {
+                    const int phu = lane_up(phs);
+                    vb = lane_up(x) + P->bot_bc * (lane_up(y) - y) / PHASE(phu + 1).conduct;
                 }
             }
-            ar0 = eok ? ar0 : 0.0;
-            ar1 = eok ? ar1 : 0.0;
-            inv0 = eok ? inv0 : 0.0;
-            inv1 = eok ? inv1 : 0.0;
-            // dummye = (source + dissip / den) / cp (:405-414; + 0 without shear heating)
-            const double sd = DIS ? e0.src + e0.sh / sPh[0][phs] : e0.src + 0.0, cp = sPh[1][phs];
-            double dm = div_fma(sd, cp, sPh[3][phs]);
-            if (__any(eok && sd != 0.0 && !(rcp_safe(sd) && rcp_safe(cp)))) dm = sd / cp;
-            dm = eok ? dm : 0.0;
-            const double hdf = sPh[2][phs];
-            const double y1 = n0.y, y2 = ydn0, y3 = n1.y, y4 = ydn1, x1 = n0.x, x2 = xdn0, x3 = n1.x, x4 = xdn1;
-            const double da[6] = {(y2 - y3) * ar0, (y3 - y1) * ar0, (y1 - y2) * ar0,
-                                  (x3 - x2) * ar0, (x1 - x3) * ar0, (x2 - x1) * ar0};
-            const double db[6] = {(y2 - y4) * ar1, (y4 - y3) * ar1, (y3 - y2) * ar1,
-                                  (x4 - x2) * ar1, (x3 - x4) * ar1, (x2 - x3) * ar1};
-            ta = therm_tri(da, inv0, dm, hdf);
-            tb = therm_tri(db, inv1, dm, hdf);
+            if (erown) v = vb;
+            if (erow1) v = P->t_top;
         }
-        // one row up: element row j-1 for node row j
-        const double uA12 = lane_up(ta.k12), uA22 = lane_up(ta.k22), uA23 = lane_up(ta.k23);
-        const double uAp = lane_up(ta.p), uAq = lane_up(ta.q), uAr = lane_up(ta.ra);
-        const double uB12 = lane_up(tb.k12), uB22 = lane_up(tb.k22), uB23 = lane_up(tb.k23);
-        const double uBp = lane_up(tb.p), uBq = lane_up(tb.q), uBr = lane_up(tb.ra);
-        double x = start_of(n0);
+        // the side columns take their neighbours' values (:590-598)
+        if (i == 1 || i == nx) {
+            bst(bW, out ? pco : OOB, i == 1 ? 0u : 8u * nz, x);
+        } else {
+            bst(bX, vo, so, v);
+            if (i == 2) bst(bX, vo, 0u, v);
+            if (i == nx - 1) bst(bX, vo, so + 8u * nz, v);
+        }
+        // border: the row above the output rows, the row below them
+        if (g.nr > 1) {
+            const unsigned k = (unsigned)(i - s.c0);
+            const int b = lane == s.fo - 1 ? 0 : lane == s.lo + 1 ? 1 : -1;
+            if (b >= 0 && !(b == 0 && s.top) && !(b == 1 && s.bot)) bord[b * g.w + k] = x;
+        }
+    }
+};
+GF_DEV int therm_phs(int ph) { return ph >= 1 && ph <= GF_MAXPH ? ph - 1 : 0; }  // (0 where there is no element)
+
+// What node column i+1 takes of element column i: triangle B one row up (t1), A and B of
+// its own row (t4, t5)
+struct ThermLeft {
+    double b13, b23, b33, bp, bq, br;
+    double a13, a23, a33, ap, aq, ar;
+    double c11, c12, c13, cp, cq, cr;
+};
+// What node column i takes of element column i from the row above (t2 A, t3 B)
+struct ThermUp {
+    double a12, a22, a23, ap, aq, ar, b12, b22, b23, bp, bq, br;
+};
+GF_DEV ThermUp therm_up(const ThermTri &ta, const ThermTri &tb)
+{
+    return ThermUp{lane_up(ta.k12), lane_up(ta.k22), lane_up(ta.k23), lane_up(ta.p), lane_up(ta.q), lane_up(ta.ra),
+                   lane_up(tb.k12), lane_up(tb.k22), lane_up(tb.k23), lane_up(tb.p), lane_up(tb.q), lane_up(tb.ra)};
+}
+GF_DEV ThermLeft therm_left(const ThermTri &ta, const ThermTri &tb, const ThermUp &u)
+{
+    return ThermLeft{lane_up(tb.k13), u.b23, lane_up(tb.k33), u.bp, u.bq, u.br, ta.k13, ta.k23, ta.k33,
+                     ta.p, ta.q, ta.ra, tb.k11, tb.k12, tb.k13, tb.p, tb.q, tb.ra};
+}
+
+// One strip by one wave.
+template <bool DIS, int MODE>
+GF_DEV void therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, const ThermGeo &g,
+                        int t, const ThermIter &it, const ThermSlots &sl, double *bord, double dt,
+                        const double (*sPh)[GF_MAXPH])
+{
+    typedef ThermWave<DIS, MODE> W;
+    const W w(P, A, g, __builtin_amdgcn_readfirstlane(t), it, sl, bord,
+              __builtin_amdgcn_readfirstlane(therm_halo(P->diff_max, P->rxbo, P->nx, dt)));
+    const int ib = max(1, w.s.c0 - w.hi - 1);
+    const bool has_ring = w.s.c0 - w.hi > 1;  // column ib only holds the start
+    typename W::Node n0 = w.node(ib), n1 = w.node(ib + 1);
+    typename W::Elem e0 = w.elem(ib);
+    double ydn0 = lane_dn(n0.y), xdn0 = lane_dn(n0.x), tdn0 = lane_dn(n0.t);
+    double xl = 0.0, xd = 0.0;  // X(j, i-1), X(j+1, i-1)
+    ThermLeft l{};              // of element column i-1 (none at the mesh's left)
+    bool still = true;
+    for (int i = ib; i <= w.s.c1; i++) {
+        // the loads of the columns ahead
+        const typename W::Node n2 = w.node(i + 2);
+        const typename W::Elem e1 = w.elem(i + 1);
+        const double ydn1 = lane_dn(n1.y), xdn1 = lane_dn(n1.x), tdn1 = lane_dn(n1.t);
+        const int phs = therm_phs(e0.ph);
+        ThermTri ta, tb;
+        w.tris(i, n0, n1, xdn0, ydn0, xdn1, ydn1, e0, phs, sPh, ta, tb);
+        const ThermUp u = therm_up(ta, tb);
+        double x = w.start(n0);
         if (!(has_ring && i == ib)) {  // (uniform)
-            // ---- node column i: t1 B of (j-1,i-1), t2 A of (j-1,i), t3 B of (j-1,i),
-            // t4 A of (j,i-1), t5 B of (j,i-1), t6 A of (j,i)
+            // t1 B of (j-1,i-1), t2 A of (j-1,i), t3 B of (j-1,i), t4 A of (j,i-1),
+            // t5 B of (j,i-1), t6 A of (j,i)
             const double tme = n0.t, tur = lane_up(n1.t);  // T(j,i), T(j-1,i+1)
-            const double area_n = (((((0.0 + lBr) + uAr) + uBr) + mAr) + mBr) + ta.ra;
-            // a lane that holds its start: told = start, 1/area = 0 (a zero increment)
-            double rarea = rcp_core(area_n);
-            if (__any(!hold && !rcp_safe(area_n))) rarea = 1.0 / area_n;
-            rarea = hold ? 0.0 : rarea;
-            const double told = hold ? x : tme;
-            const double xl12 = xl * lB23, c13 = tme * lB33;             // t1: K13 K23 K33
-            const double c22 = tme * uA22, c23 = tur * uA23;             // t2
-            const double qs3 = uBq * (tur * uB12 + tme * uB22 + n1.t * uB23);
-            const double qs4 = mAq * ((xl * mA13 + xd * mA23) + tme * mA33);
-            const double qs5 = mBq * ((tme * mB11 + xd * mB12) + tdn0 * mB13);
+            const double area_n = (((((0.0 + l.br) + u.ar) + u.br) + l.ar) + l.cr) + ta.ra;
+            const double rarea = w.rarea(area_n);
+            const double told = w.hold ? x : tme;
+            const double xl12 = xl * l.b23, c13 = tme * l.b33;           // t1: K13 K23 K33
+            const double c22 = tme * u.a22, c23 = tur * u.a23;           // t2
+            const double qs3 = u.bq * (tur * u.b12 + tme * u.b22 + n1.t * u.b23);
+            const double qs4 = l.aq * ((xl * l.a13 + xd * l.a23) + tme * l.a33);
+            const double qs5 = l.cq * ((tme * l.c11 + xd * l.c12) + tdn0 * l.c13);
             const double qs6 = ta.q * (tme * ta.k11 + tdn0 * ta.k12 + n1.t * ta.k13);
             auto eval = [&](double xu) {
                 double rhs = 0.0;
-                rhs = rhs + lBp - lBq * ((xu * lB13 + xl12) + c13);
-                rhs = rhs + uAp - uAq * ((xu * uA12 + c22) + c23);
-                rhs = rhs + uBp - qs3;
-                rhs = rhs + mAp - qs4;
-                rhs = rhs + mBp - qs5;
+                rhs = rhs + l.bp - l.bq * ((xu * l.b13 + xl12) + c13);
+                rhs = rhs + u.ap - u.aq * ((xu * u.a12 + c22) + c23);
+                rhs = rhs + u.bp - qs3;
+                rhs = rhs + l.ap - qs4;
+                rhs = rhs + l.cp - qs5;
                 rhs = rhs + ta.p - qs6;
                 return told + div_fma(rhs * dt, area_n, rarea);
             };
@@ -349,49 +443,11 @@ GF_DEV void therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, const
                 }
             }
         }
-        // ---- results of column i
-        if (i >= s.c0) {
-            const bool out = lane >= s.fo && lane <= s.lo;
-            const unsigned so = (unsigned)nz * (unsigned)(i - 1) * 8u;
-            const unsigned vo = out ? nvo : OOB;
-            double v = x;
-            if (edge) {
-                // before the conditions: kept apart
-                bst(bW, out ? pvo : OOB, 8u * (i - 1), x);
-                double vb = P->bot_bc;
-                if (P->itemp_bc != 1) {
-                    vb = x;
-                    if (P->itemp_bc == 2) {
-                        const int phu = lane_up(phs);
-                        vb = lane_up(x) + P->bot_bc * (lane_up(n0.y) - n0.y) / PHASE(phu + 1).conduct;
-                    }
-                }
-                if (erown) v = vb;
-                if (erow1) v = P->t_top;
-            }
-            // the side columns take their neighbours' values (:590-598)
-            if (i == 1 || i == nx) {
-                bst(bW, out ? pco : OOB, i == 1 ? 0u : 8u * nz, x);
-            } else {
-                bst(bX, vo, so, v);
-                if (i == 2) bst(bX, vo, 0u, v);
-                if (i == nx - 1) bst(bX, vo, so + 8u * nz, v);
-            }
-            // border: the row above the output rows, the row below them
-            if (g.nr > 1) {
-                const unsigned k = (unsigned)(i - s.c0);
-                const int b = lane == s.fo - 1 ? 0 : lane == s.lo + 1 ? 1 : -1;
-                if (b >= 0 && !(b == 0 && s.top) && !(b == 1 && s.bot)) bord[b * g.w + k] = x;
-            }
-        } else if (i == s.c0 - 1) {
-            bord[2 * g.w + lane] = x;
-        }
-        // ---- on to column i+1
+        w.store(i, x, n0.y, phs);
+        // on to column i+1
         xl = x;
         xd = lane_dn(x);
-        lB13 = lane_up(tb.k13); lB23 = uB23; lB33 = lane_up(tb.k33); lBp = uBp; lBq = uBq; lBr = uBr;
-        mA13 = ta.k13; mA23 = ta.k23; mA33 = ta.k33; mAp = ta.p; mAq = ta.q; mAr = ta.ra;
-        mB11 = tb.k11; mB12 = tb.k12; mB13 = tb.k13; mBp = tb.p; mBq = tb.q; mBr = tb.ra;
+        l = therm_left(ta, tb, u);
         n0 = n1;
         n1 = n2;
         e0 = e1;
@@ -399,7 +455,124 @@ GF_DEV void therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, const
         ydn0 = ydn1;
         tdn0 = tdn1;
     }
-    if (!still && lane == 0) atomicOr(&ck->therm_pass_changed[it.pass], 2u);
+    if (!still && w.lane == 0) atomicOr(&ck->therm_pass_changed[it.pass], 2u);
+}
+
+// One strip by one workgroup, a wave a column, for meshes of so few strips that each has a
+// CU of its own: a wave's march from column to column (1.3 us each) leaves 3 of a CU's 4
+// SIMDs idle there.  Column
+// c0 - hi - 1 + q is wave q's.  The waves form their element columns at the same time, hand
+// the next column its share through LDS, and apply the update together from the last
+// iterate of the column to the left (a barrier each time) until no bit of the strip changes:
+// more applications than the march takes, but all columns in one of them.  The same fixed
+// point, borders and proof.  Bound by latency: the loads and element columns some 3 us, 6 to
+// 8 applications 0.4 us each.  At 4 + 4 columns the kernel takes 6.9 us where the march took
+// 12 (60x20 cells), 7.4 for 12 (151x47) and 9.3 for 13 (400x100); a step there 39.3 -> 36.2,
+// 49.4 -> 44.9 and 37.1 -> 33.2 us.  2, 3 and 4 output columns are within 2% at the two
+// smaller meshes; 400x100 cells take 34.8, 34.3 and 33.2 us a step (400 workgroups to 200).
+#define TC_W 9   // waves (columns) of a workgroup: output columns, halo columns, the ring
+#define TC_HI 4  // most halo columns (fewer are used where therm_halo says so)
+struct ThermColLds {
+    double ph[4][GF_MAXPH];
+    double left[TC_W - 1][18][64];
+    double x[2][TC_W][64];
+    int flag[3];
+};
+template <bool DIS, int MODE>
+GF_DEV void therm_cols(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, const ThermGeo &g,
+                       int t, const ThermIter &it, const ThermSlots &sl, double *bord, ThermColLds &L)
+{
+    typedef ThermWave<DIS, MODE> W;
+    const int q = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
+    const W w(P, A, g, t, it, sl, bord, TC_W - 1 - g.w);
+    const int i = w.s.c0 - w.hi - 1 + q;
+    const bool in = i >= 1 && i <= w.s.c1;  // (uniform in a wave; the others only keep the barriers)
+    const double dt = ck->dt;
+    typename W::Node n0{}, n1{};
+    typename W::Elem e0{};
+    if (in) {
+        n0 = w.node(i);
+        n1 = w.node(i + 1);
+        e0 = w.elem(i);
+    }
+    if (threadIdx.x < GF_MAXPH) {
+        const int k = threadIdx.x;
+        L.ph[0][k] = P->ph[k].den;
+        L.ph[1][k] = P->ph[k].cp;
+        L.ph[2][k] = 0.5 * P->ph[k].diff;
+        L.ph[3][k] = 1.0 / P->ph[k].cp;
+    }
+    if (threadIdx.x < 3) L.flag[threadIdx.x] = 0;
+    // (dt, and so the halo, come after the loads on purpose: columns beyond it are let go)
+    const int hi = min(w.hi, __builtin_amdgcn_readfirstlane(therm_halo(P->diff_max, P->rxbo, P->nx, dt)));
+    const bool work = in && i >= w.s.c0 - hi;  // (the ring and what is beyond it only hold the start)
+    __syncthreads();
+    const double ydn0 = lane_dn(n0.y), xdn0 = lane_dn(n0.x), tdn0 = lane_dn(n0.t);
+    const int phs = therm_phs(e0.ph);
+    ThermTri ta, tb;
+    w.tris(i, n0, n1, xdn0, ydn0, lane_dn(n1.x), lane_dn(n1.y), e0, phs, L.ph, ta, tb);
+    const ThermUp u = therm_up(ta, tb);
+    double x = w.start(n0);
+    {
+        const ThermLeft l = therm_left(ta, tb, u);
+        const double v[18] = {l.b13, l.b23, l.b33, l.bp, l.bq, l.br, l.a13, l.a23, l.a33,
+                              l.ap, l.aq, l.ar, l.c11, l.c12, l.c13, l.cp, l.cq, l.cr};
+        if (q < TC_W - 1) {
+#pragma unroll
+            for (int k = 0; k < 18; k++) L.left[q][k][w.lane] = v[k];
+        }
+        L.x[0][q][w.lane] = x;
+        L.x[1][q][w.lane] = x;
+    }
+    lds_barrier();
+    ThermLeft l{};
+    if (q > 0 && i > 1) {
+        double v[18];
+#pragma unroll
+        for (int k = 0; k < 18; k++) v[k] = L.left[q - 1][k][w.lane];
+        l = ThermLeft{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8],
+                      v[9], v[10], v[11], v[12], v[13], v[14], v[15], v[16], v[17]};
+    }
+    const double tme = n0.t, tur = lane_up(n1.t);
+    const double area_n = (((((0.0 + l.br) + u.ar) + u.br) + l.ar) + l.cr) + ta.ra;
+    const double rarea = w.rarea(work ? area_n : 1.0);
+    const double told = w.hold ? x : tme;
+    const double c13 = tme * l.b33, c22 = tme * u.a22, c23 = tur * u.a23, c43 = tme * l.a33, c51 = tme * l.c11,
+                 c53 = tdn0 * l.c13;
+    const double qs3 = u.bq * (tur * u.b12 + tme * u.b22 + n1.t * u.b23);
+    const double qs6 = ta.q * (tme * ta.k11 + tdn0 * ta.k12 + n1.t * ta.k13);
+    int cur = 0, nsweep = 0;
+    bool still = false;
+    while (nsweep < TS_MAXSWEEP) {
+        if (work) {
+            const double xl = q > 0 ? L.x[cur][q - 1][w.lane] : 0.0, xd = lane_dn(xl), xu = lane_up(x);
+            double rhs = 0.0;
+            rhs = rhs + l.bp - l.bq * ((xu * l.b13 + xl * l.b23) + c13);
+            rhs = rhs + u.ap - u.aq * ((xu * u.a12 + c22) + c23);
+            rhs = rhs + u.bp - qs3;
+            rhs = rhs + l.ap - l.aq * ((xl * l.a13 + xd * l.a23) + c43);
+            rhs = rhs + l.cp - l.cq * ((c51 + xd * l.c12) + c53);
+            rhs = rhs + ta.p - qs6;
+            const double xn = told + div_fma(rhs * dt, area_n, rarea);
+            if (nsweep >= TS_SWEEP0 && __any(__double_as_longlong(xn) != __double_as_longlong(x)) && w.lane == 0)
+                L.flag[nsweep % 3] = 1;
+            x = xn;
+            L.x[cur ^ 1][q][w.lane] = x;
+        }
+        lds_barrier();
+        // (flag nsweep % 3 is raised before the barrier and read after it; the one of two
+        // applications on is cleared meanwhile)
+        const int any = nsweep < TS_SWEEP0 ? 1 : L.flag[nsweep % 3];
+        if (threadIdx.x == 0) L.flag[(nsweep + 2) % 3] = 0;
+        cur ^= 1;
+        nsweep++;
+        if (!any) {
+            still = true;
+            break;
+        }
+    }
+    if (in) w.store(i, x, n0.y, phs);
+    if (!still && threadIdx.x == 0) atomicOr(&ck->therm_pass_changed[it.pass], 2u);
 }
 
 // by the lanes of one wave, for that wave
@@ -421,19 +594,31 @@ GF_DEV void therm_phase_table(const GfDevParams *__restrict__ P, double (*sPh)[G
 // pass 0 (mode 0 or 2) or, with launches per phase, a fallback pass: one wave a strip
 template <bool DIS, int MODE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
-k_therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, int w, int pass, int arp, ThermSlots sl,
-              int ops)
+k_therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, ThermGeo g, int pass, int arp,
+              ThermSlots sl, int ops)
 {
     if (ops && blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
     __shared__ double sPh[4][GF_MAXPH];
     if (pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) return;  // already proven
-    const ThermGeo g = therm_geo(P, w);
     const int nt = g.nr * g.ns, q = (nt + 7) / 8;  // XCD x runs strips [x q, (x+1) q)
     const int t = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
     if ((int)(blockIdx.x / 8) >= q || t >= nt) return;
     therm_phase_table(P, sPh);
     const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, arp, pass};
-    therm_strip<DIS, MODE>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(w), ck->dt, sPh);
+    therm_strip<DIS, MODE>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(g.w), ck->dt, sPh);
+}
+// pass 0, one workgroup a strip
+template <bool DIS, int MODE>
+__global__ void __launch_bounds__(64 * TC_W)
+k_therm_cols(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, ThermGeo g, int arp, ThermSlots sl,
+             int ops)
+{
+    if (ops && blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
+    __shared__ ThermColLds L;
+    const int nt = g.nr * g.ns, q = (nt + 7) / 8, t = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= q || t >= nt) return;
+    const ThermIter it{A.xb, A.xa, arp, 0};
+    therm_cols<DIS, MODE>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(g.w), L);
 }
 
 // Compares border value t of the strips with the value its owner wrote.  A node whose
@@ -499,10 +684,9 @@ GF_DEV void therm_check_one(const GfDevParams *__restrict__ P, GfDevClock *ck, c
 }
 
 __global__ void __launch_bounds__(256) k_therm_check(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                    int w, int pass, int arp, ThermSlots sl, long total)
+                                                    ThermGeo g, int pass, int arp, ThermSlots sl, long total)
 {
     if (pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) return;  // that pass did not run
-    const ThermGeo g = therm_geo(P, w);
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
     if (t < total) therm_check_one(P, ck, A, g, t, pass, arp, sl);
 }
@@ -510,7 +694,8 @@ __global__ void __launch_bounds__(256) k_therm_check(const GfDevParams *__restri
 // temperature nor writes what the check reads (grid 0: none; a multiple of 8, so that the
 // others keep their XCDs)
 struct ThermChk {
-    int grid, w, arp;
+    int grid, arp;
+    ThermGeo g;
     ThermSlots sl;
     double *temp, *xa;  // the call's old temperature and its result
 };
@@ -518,8 +703,7 @@ GF_DEV void therm_chk_block(const GfDevParams *__restrict__ P, GfDevClock *ck, G
 {
     A.temp = c.temp;
     A.xa = c.xa;
-    const ThermGeo g = therm_geo(P, c.w);
-    therm_check_one(P, ck, A, g, (long)blockIdx.x * 256 + threadIdx.x, 0, c.arp, c.sl);
+    therm_check_one(P, ck, A, c.g, (long)blockIdx.x * 256 + threadIdx.x, 0, c.arp, c.sl);
 }
 
 // The call's outcome, once: statistics, and GF_ERR_THERM_SWEEPS where no pass was proven
@@ -551,21 +735,20 @@ GF_DEV void therm_settle(const GfDevParams *__restrict__ P, const GfDevArrays &A
 // the same decision; flag 0 was written by earlier launches.
 template <bool DIS>
 __global__ void __launch_bounds__(256) k_therm_rest(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                    int w, int arp, ThermSlots sl, int npass)
+                                                    ThermGeo g, int arp, ThermSlots sl, int npass)
 {
     if (ck->therm_pass_changed[0] == 0u) return;
     __shared__ double sPhw[4][4][GF_MAXPH];  // (a table a wave)
     double(*sPh)[GF_MAXPH] = sPhw[threadIdx.x / 64];
     therm_phase_table(P, sPh);
-    const ThermGeo g = therm_geo(P, w);
     const int nt = g.nr * g.ns;
-    const long nb = (long)nt * TS_NB(w);
+    const long nb = (long)nt * TS_NB(g.w);
     const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x, nthr = (long)gridDim.x * blockDim.x;
     int proven = -1, pass = 1;
     for (; pass < npass; pass++) {
         const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, arp, pass};
         for (int t = (int)(tid / 64); t < nt; t += (int)(nthr / 64))
-            therm_strip<DIS, 1>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(w), ck->dt, sPh);
+            therm_strip<DIS, 1>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(g.w), ck->dt, sPh);
         if (!grid_sync(ck)) return;  // every strip's iterate is written
         for (long t = tid; t < nb; t += nthr) therm_check_one(P, ck, A, g, t, pass, arp, sl);
         if (!grid_sync(ck)) return;  // every border is checked

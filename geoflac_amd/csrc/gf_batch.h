@@ -252,9 +252,16 @@ template <bool SHEARH, int M>
 __global__ void __launch_bounds__(256) kb_rheol(const BatchEntry *__restrict__ tab, BatchMap map, int avgsr,
                                                 int rot)
 {
-    batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) {
-        rheol_single<SHEARH, typename Prec<M>::SV, typename Prec<M>::AT>(b.P, b.P->ph, b.ck, b.A, e, avgsr, rot);
-    });
+    __shared__ RheolPhases phs;
+    const long g0 = (long)xcd_block() * blockDim.x;
+    const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_ELEM][g0 / BATCH_ALIGN]));
+    const long e = g0 + threadIdx.x - b.pe;
+    rheol_single<SHEARH, typename Prec<M>::SV, typename Prec<M>::AT>(
+        b.P, phs, b.ck, b.A, min(e, b.ce - 1), avgsr, rot, e < b.ce, [&]() {
+            for (int k = threadIdx.x; k < RP_N * GF_MAXPH; k += blockDim.x)
+                (&phs.f[0][0])[k] = rheol_phase_value(b.P, k);
+            lds_barrier();
+        });
 }
 
 // move: the coordinates move into cord_next as the node has its velocity (and the move's

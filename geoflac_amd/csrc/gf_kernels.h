@@ -850,7 +850,10 @@ GF_DEV void dev_pre_plast(const GfDevParams *P, const GfPhase *phs, double aps, 
                           double &phi, double &psi, double &hardn)
 {
     phi = 0; coh = 0; psi = 0; hardn = 0;
-    for (int a = 0; a < P->nactive; a++) {
+    const int na = P->nactive;
+#pragma unroll
+    for (int a = 0; a < GF_MAXACT; a++) {  // (unrolled: prv stays in registers)
+        if (a >= na) break;
         double r = prv[a];
         if (r < 0.01) continue;
         const GfPhase &ph = phs[P->active[a] - 1];
@@ -1143,16 +1146,52 @@ static __device__ __noinline__ SinSinTan cr_sin_sin_tan(double phi, double psi)
     return r;
 }
 
-// the phase constants fl_rheol reads, fetched together as soon as the phase index
-// is known (one cache round trip instead of one per use)
-struct RheolPhase {
-    int irheol;
-    double bulkm, rm, phi0, psi0, sphi0, spsi0, tphi0;
+// the phase constants fl_rheol reads: a workgroup's copy in LDS, a field a row
+enum {
+    RP_IRHEOL, RP_BULKM, RP_RM, RP_PHI0, RP_PSI0, RP_SPHI0, RP_SPSI0, RP_TPHI0,
+    RP_PLS1, RP_PLS2, RP_FRIC1, RP_FRIC2, RP_COH1, RP_COH2, RP_DIL1, RP_DIL2, RP_N
 };
-GF_DEV RheolPhase rheol_phase(const GfPhase *__restrict__ phs, int iph)
+struct RheolPhases {
+    double f[RP_N][GF_MAXPH];
+};
+// (irheol: the bits of the first 8 bytes)
+GF_DEV double rheol_phase_value(const GfDevParams *__restrict__ P, int k)
 {
-    const GfPhase &ph = phs[iph - 1];
-    return {ph.irheol, ph.bulkm, ph.rm, ph.phi0, ph.psi0, ph.sphi0, ph.spsi0, ph.tphi0};
+    const int f = k / GF_MAXPH;
+    const size_t o = f == RP_IRHEOL ? offsetof(GfPhase, irheol)
+                     : f == RP_BULKM ? offsetof(GfPhase, bulkm)
+                     : f == RP_RM ? offsetof(GfPhase, rm)
+                     : f <= RP_TPHI0 ? offsetof(GfPhase, phi0) + 8 * (size_t)(f - RP_PHI0)
+                                     : offsetof(GfPhase, plstrain1) + 8 * (size_t)(f - RP_PLS1);
+    return *(const double *)((const char *)&P->ph[k % GF_MAXPH] + o);
+}
+static_assert(offsetof(GfPhase, irheol) == 0, "irheol in the low half");
+static_assert(offsetof(GfPhase, tphi0) == offsetof(GfPhase, phi0) + 8 * (RP_TPHI0 - RP_PHI0), "phi0 .. tphi0 in a row");
+static_assert(offsetof(GfPhase, dilat2) == offsetof(GfPhase, plstrain1) + 8 * (RP_DIL2 - RP_PLS1),
+              "plstrain1 .. dilat2 in a row");
+// pre_plast of an element of phase iph alone (ratio 1): dev_pre_plast's one term
+GF_DEV void dev_pre_plast_pure(const RheolPhases &L, int iph, double aps, double &coh, double &phi, double &psi,
+                               double &hardn)
+{
+    const int m = iph - 1;
+    const double p1 = L.f[RP_PLS1][m], p2 = L.f[RP_PLS2][m], f1 = L.f[RP_FRIC1][m], f2 = L.f[RP_FRIC2][m];
+    const double c1 = L.f[RP_COH1][m], c2 = L.f[RP_COH2][m], d1 = L.f[RP_DIL1][m], d2 = L.f[RP_DIL2][m];
+    double f, c, d, h;
+    if (aps < p1) {
+        f = f1; c = c1; d = d1; h = 0;
+    } else if (aps < p2) {
+        const double dpl = (aps - p1) / (p2 - p1);
+        f = f1 + (f2 - f1) * dpl;
+        d = d1 + (d2 - d1) * dpl;
+        c = c1 + (c2 - c1) * dpl;
+        h = (c2 - c1) / (p2 - p1);
+    } else {
+        f = f2; c = c2; d = d2; h = 0;
+    }
+    phi = 1 / (0.0 + 1.0 / f);
+    coh = 1 / (0.0 + 1.0 / c);
+    psi = 0.0 + 1.0 * d;
+    hardn = 0.0 + 1.0 * h;
 }
 
 // the constitutive update of one triangle for rheology irh (:216-264), in arithmetic T;
@@ -1241,9 +1280,13 @@ GF_DEV void move_rotate(T &s11, T &s22, T &s12, T w)
 // k_move_area ran): they are formed here from the moved coordinates the kernel loads
 // anyway, with k_move_area's arithmetic, used, and stored (src/fl_move.f90:108-126).
 //
-// phs: the phase table (a workgroup's LDS copy of P->ph, or P->ph itself).  Every
-// per-element load is issued before the first use, so that a wave pays one memory
-// round trip for its inputs instead of a chain of them.
+// Every per-element load is issued before the first use of any, the phase index's
+// included, so that a wave pays one memory round trip for its inputs; what depends on the
+// phase index is read from a workgroup's copy of the phase constants in LDS, and only an
+// element of several phases loads its ratios, in a second trip.  (With the index waited
+// for first, and constants and softening means fetched per phase through scalar loads, a
+// wave of a small mesh spent 6000 of 17000 cycles on those chains; 2000x1000 elements
+// took 223 us, now 205, where passing the planes through unchanged takes 167.)
 // the LDS rows of rheol_single's two branch results (see there): one column per
 // thread of a workgroup of at most GF_RHEOL_WG threads
 #define GF_RHEOL_WG 256
@@ -1256,9 +1299,12 @@ GF_DEV AT (*rheol_branch_lds())[GF_RHEOL_WG]
 #define RH_ROT 1
 #define RH_AREA 2
 #define RH_NODVOL 4  // (with RH_AREA) dvol is formed and used but not stored: nothing reads it back
-template <bool SHEARH, typename SV, typename AT>
-GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__restrict__ phs, GfDevClock *ck,
-                         const GfDevArrays &A, long e, int avgsr, int rot)
+// ready(): fills phs and synchronizes the workgroup, between the issue of the loads and
+// their first use; live: false in a thread past the last element, which comes along so far
+// with e the last one.
+template <bool SHEARH, typename SV, typename AT, typename Ready>
+GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const RheolPhases &phs, GfDevClock *ck,
+                         const GfDevArrays &A, long e, int avgsr, int rot, bool live, Ready ready)
 {
     const unsigned nzm = (unsigned)(NZ - 1);
     const unsigned ne = (unsigned)NE, nn = (unsigned)NN, nzu = (unsigned)NZ;
@@ -1281,18 +1327,11 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
     // phase ratios: GF_MAXACT planes are read; those past nactive lie outside the
     // buffer and read 0 without touching memory
     const Buf bPR = mkbuf(A.pr, (unsigned long long)P->nactive * pe);
-    const int iphx = bldi(bIP, (unsigned)e * 4u, 0), iph = iphx & IPHX_PHASE;
-    // an element of one phase (ratio exactly 1, the others 0) reads no ratio plane
-    double prv[GF_MAXACT];
-    if (iphx & IPHX_PURE) {
-#pragma unroll
-        for (int a = 0; a < GF_MAXACT; a++) prv[a] = P->active[a] == iph ? 1.0 : 0.0;
-    } else {
-#pragma unroll
-        for (int a = 0; a < GF_MAXACT; a++) prv[a] = bld(bPR, eo, a * pe);
-    }
+    const int iphx = bldi(bIP, (unsigned)e * 4u, 0);
+    const double dt = ck->dt, dtm = ck->dt_move;
+    const double pref = ref_press<SV>(A, e);
     double aps = bld(bAPS, eo, 0);
-    const float csc = A.coh_scale ? A.coh_scale[e] : 1.0f;
+    const float csc = bldf(mkbuf(A.coh_scale, A.coh_scale ? 4ull * ne : 0ull), (unsigned)e * 4u, 0);  // (0 without)
     const double vis = bld(bVIS, eo, 0);  // refreshed by k_visc on viscosity-update steps
     double se_in[3], sshr_in, str_in[3];
     for (int c = 0; c < 3; c++) se_in[c] = bld(bSE, eo, c * pe);
@@ -1306,20 +1345,35 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
         for (int k = 0; k < 4; k++) dvl[k] = bld(bD, eo, k * pe);
     double ar[4];  // (the areas before the move when they are pending)
     for (int k = 0; k < 4; k++) ar[k] = bld(bA, eo, k * pe);
-    const RheolPhase rp = rheol_phase(phs, iph);
-    const double dt = ck->dt;
+    // corners 1 (j,i), 2 (j+1,i), 3 (j,i+1), 4 (j+1,i+1)
+    SV vin[8];
+    double cin[8];
+    for (int k = 0; k < 4; k++) {
+        vin[k] = bldt<SV>(bV, nov, (k & 1) * W + (k >> 1) * colv);
+        vin[4 + k] = bldt<SV>(bV, nov, pnv + (k & 1) * W + (k >> 1) * colv);
+        cin[k] = bld(bC, no, (k & 1) * 8u + (k >> 1) * col);
+        cin[4 + k] = bld(bC, no, pn + (k & 1) * 8u + (k >> 1) * col);
+    }
+    SB();  // (the loads above are issued before the first wait)
+    ready();
+    if (!live) return;
+    const int iph = iphx & IPHX_PHASE;
+    const bool pure = (iphx & IPHX_PURE) != 0;
+    double prv[GF_MAXACT];
+    if (!pure) {
+#pragma unroll
+        for (int a = 0; a < GF_MAXACT; a++) prv[a] = bld(bPR, eo, a * pe);
+    }
+    const int irh = __double2loint(phs.f[RP_IRHEOL][iph - 1]);
+    const double rbulkm = phs.f[RP_BULKM][iph - 1], rrm = phs.f[RP_RM][iph - 1];
     const AT dtS = AT(dt);
     AT sr[4][3];
     double dw[4] = {0.0, 0.0, 0.0, 0.0};  // pending rotation increments
     {
-        // corners 1 (j,i), 2 (j+1,i), 3 (j,i+1), 4 (j+1,i+1)
-        const AT vx1 = AT(bldt<SV>(bV, nov, 0)), vy1 = AT(bldt<SV>(bV, nov, pnv)), vx2 = AT(bldt<SV>(bV, nov, W)),
-                 vy2 = AT(bldt<SV>(bV, nov, pnv + W));
-        const AT vx3 = AT(bldt<SV>(bV, nov, colv)), vy3 = AT(bldt<SV>(bV, nov, pnv + colv)),
-                 vx4 = AT(bldt<SV>(bV, nov, colv + W)), vy4 = AT(bldt<SV>(bV, nov, pnv + colv + W));
-        const double x1 = bld(bC, no, 0), y1 = bld(bC, no, pn), x2 = bld(bC, no, 8), y2 = bld(bC, no, pn + 8);
-        const double x3 = bld(bC, no, col), y3 = bld(bC, no, pn + col), x4 = bld(bC, no, col + 8),
-                     y4 = bld(bC, no, pn + col + 8);
+        const AT vx1 = AT(vin[0]), vx2 = AT(vin[1]), vx3 = AT(vin[2]), vx4 = AT(vin[3]);
+        const AT vy1 = AT(vin[4]), vy2 = AT(vin[5]), vy3 = AT(vin[6]), vy4 = AT(vin[7]);
+        const double x1 = cin[0], x2 = cin[1], x3 = cin[2], x4 = cin[3];
+        const double y1 = cin[4], y2 = cin[5], y3 = cin[6], y4 = cin[7];
         if (areas) {  // the move's areas and dvol (move_area_body)
             const double xc[5] = {0.0, x1, x2, x3, x4}, yc[5] = {0.0, y1, y2, y3, y4};
             bool bad = false;
@@ -1355,7 +1409,6 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
             const double xc[5] = {0.0, x1, x2, x3, x4}, yc[5] = {0.0, y1, y2, y3, y4};
             const double xv[5] = {0.0, (double)vx1, (double)vx2, (double)vx3, (double)vx4};
             const double yv[5] = {0.0, (double)vy1, (double)vy2, (double)vy3, (double)vy4};
-            const double dtm = ck->dt_move;
 #pragma unroll
             for (int k = 0; k < 4; k++) dw[k] = move_dw12(xc, yc, xv, yv, k, move_det(xc, yc, k), dtm);
         }
@@ -1379,7 +1432,6 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
             move_rotate<AT>(st[k][0], st[k][1], st[k][2], AT(dw[k]));
             for (int c = 0; c < 3; c++) st[k][c] = AT(SV(st[k][c]));  // as k_move_rot stores them
         }
-    const double pref = ref_press<SV>(A, e);
     if (conv)
         for (int k = 0; k < 4; k++) {
             st[k][0] = st[k][0] - pref;
@@ -1406,10 +1458,9 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
         sshr = sshr_in;
         if (srII != AT(0.0)) sshr = sshr + adiv(stII, srII) * srs2 * dt;
     }
-    const GfPhase &ph = phs[iph - 1];
-    const int irh = rp.irheol;
-    const AT bulkm = AT(rp.bulkm), rmu = AT(rp.rm);
+    const AT bulkm = AT(rbulkm), rmu = AT(rrm);
     AT stherm = AT(0.0);
+    const GfPhase &ph = PHASE(iph);
     if (P->istress_therm > 0) stherm = AT(-ph.alfa * ph.bulkm * (A.temp[IN(j, i)] - A.temp0[IN(j, i)]));
     const bool plas_law = irh == 6 || irh >= 11;
     PlasticConstT<AT> pc{};
@@ -1417,13 +1468,16 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
     AT hardn = AT(0);
     if (plas_law) {
         double coh, phi, psi, hd;
-        dev_pre_plast(P, phs, aps, prv, coh, phi, psi, hd);
+        if (pure)
+            dev_pre_plast_pure(phs, iph, aps, coh, phi, psi, hd);
+        else
+            dev_pre_plast(P, P->ph, aps, prv, coh, phi, psi, hd);
         if (A.coh_scale) coh = coh * (double)csc;
         double sphi, spsi, tphi;
-        if (phi == rp.phi0 && psi == rp.psi0) {
-            sphi = rp.sphi0;
-            spsi = rp.spsi0;
-            tphi = rp.tphi0;
+        if (phi == phs.f[RP_PHI0][iph - 1] && psi == phs.f[RP_PSI0][iph - 1]) {
+            sphi = phs.f[RP_SPHI0][iph - 1];
+            spsi = phs.f[RP_SPSI0][iph - 1];
+            tphi = phs.f[RP_TPHI0][iph - 1];
         } else if (!dev_form) {
             const SinSinTan t = cr_sin_sin_tan(phi, psi);
             sphi = t.sphi;
@@ -1439,8 +1493,8 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
         const double c4d3 = 4.0 / 3.0, c2d3 = 2.0 / 3.0;
         const double anphi = (1.0 + sphi) / (1.0 - sphi);
         const double anpsi = (1.0 + spsi) / (1.0 - spsi);
-        const double e1 = rp.bulkm + c4d3 * rp.rm;
-        const double e2 = rp.bulkm - c2d3 * rp.rm;
+        const double e1 = rbulkm + c4d3 * rrm;
+        const double e2 = rbulkm - c2d3 * rrm;
         pc.anphi = AT(anphi);
         pc.anpsi = AT(anpsi);
         pc.amc = AT(2.0 * coh * sqrt(anphi));
@@ -1464,7 +1518,7 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
     // while the choice is made, so that neither is evaluated twice
     AT(*const brs)[GF_RHEOL_WG] = rheol_branch_lds<AT>();
     // src/rh_maxwell.f90:16-30, the same for the element's four triangles
-    const MaxwellConst mc = maxwell_const(rp.rm, vis, dt);
+    const MaxwellConst mc = maxwell_const(rrm, vis, dt);
     const int lt = threadIdx.x;
     if (irh >= 11) {
         AT s11p = 0, s12p = 0, s11v = 0, s12v = 0, s22p[4], s22v[4];
@@ -1603,43 +1657,47 @@ GF_DEV void rheol_single(const GfDevParams *__restrict__ P, const GfPhase *__res
     bst(bSH, eo, 0, sshr);
 }
 
-template <bool SHEARH>
-__global__ void __launch_bounds__(256) k_rheol1(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                int avgsr, int rot, ThermChk chk)
+// the element update as a launch: its first chk.grid workgroups run a thermal border check
+template <bool SHEARH, typename SV, typename AT>
+GF_DEV void rheol_block(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, int avgsr, int rot,
+                        const ThermChk &chk)
 {
     if (blockIdx.x < (unsigned)chk.grid) {
         therm_chk_block(P, ck, A, chk);
         return;
     }
-    long e = xcd_lin((unsigned)chk.grid);
-    if (e >= NE) return;
-    rheol_single<SHEARH, double, double>(P, P->ph, ck, A, e, avgsr, rot);
+    __shared__ RheolPhases phs;
+    constexpr int N = RP_N * GF_MAXPH;
+    static_assert(N <= 2 * GF_BLOCK, "two values a thread");
+    double *const lp = &phs.f[0][0];
+    const int t0 = threadIdx.x, t1 = t0 + GF_BLOCK;
+    const double v0 = rheol_phase_value(P, t0), v1 = rheol_phase_value(P, min(t1, N - 1));
+    const long e = xcd_lin((unsigned)chk.grid), last = NE - 1;
+    rheol_single<SHEARH, SV, AT>(P, phs, ck, A, min(e, last), avgsr, rot, e <= last, [&]() {
+        lp[t0] = v0;
+        if (t1 < N) lp[t1] = v1;
+        lds_barrier();
+    });
+}
+template <bool SHEARH>
+__global__ void __launch_bounds__(256) k_rheol1(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
+                                                int avgsr, int rot, ThermChk chk)
+{
+    rheol_block<SHEARH, double, double>(P, ck, A, avgsr, rot, chk);
 }
 // mixed precision: FP32 strain rate and stress
 template <bool SHEARH>
 __global__ void __launch_bounds__(256) k_rheol1m(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
                                                  int avgsr, int rot, ThermChk chk)
 {
-    if (blockIdx.x < (unsigned)chk.grid) {
-        therm_chk_block(P, ck, A, chk);
-        return;
-    }
-    long e = xcd_lin((unsigned)chk.grid);
-    if (e >= NE) return;
-    rheol_single<SHEARH, float, float>(P, P->ph, ck, A, e, avgsr, rot);
+    rheol_block<SHEARH, float, float>(P, ck, A, avgsr, rot, chk);
 }
 // FP32 storage, FP64 arithmetic
 template <bool SHEARH>
 __global__ void __launch_bounds__(256) k_rheol1s(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
                                                  int avgsr, int rot, ThermChk chk)
 {
-    if (blockIdx.x < (unsigned)chk.grid) {
-        therm_chk_block(P, ck, A, chk);
-        return;
-    }
-    long e = xcd_lin((unsigned)chk.grid);
-    if (e >= NE) return;
-    rheol_single<SHEARH, float, double>(P, P->ph, ck, A, e, avgsr, rot);
+    rheol_block<SHEARH, float, double>(P, ck, A, avgsr, rot, chk);
 }
 
 // Eff_visc of src/fl_rheol.f90:203-206 on viscosity-update steps (mod(nloop,

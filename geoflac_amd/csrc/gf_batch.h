@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restric
             therm_strip<DIS, 1>(b.P, b.ck, A, b.tg, t, it, bslots(b), A.tbord + (long)t * TS_NB(b.tg.w),
                                 b.ck->dt, sPh);
         }
-        if (!grid_sync(bar)) return;  // every strip's iterate is written
+        if (!grid_sync(bar, gridDim.x)) return;  // every strip's iterate is written
         for (long g = (long)blockIdx.x * 256; g < border; g += nthr) {
             const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_BORD][g / BATCH_ALIGN]));
             const long t = g + threadIdx.x - b.pb;
@@ -196,7 +196,7 @@ __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restric
                 __hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)
                 therm_check_one(b.P, b.ck, bthermal(b), b.tg, t, pass, arp, bslots(b));
         }
-        if (!grid_sync(bar)) return;  // every border is checked
+        if (!grid_sync(bar, gridDim.x)) return;  // every border is checked
         if (!open_after(pass)) break;
     }
     for (int m = 0; m < map.nm; m++) {

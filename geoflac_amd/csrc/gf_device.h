@@ -63,7 +63,9 @@ struct GfDevClock {
     int error_code, pad;
     long long error_index;      // smallest linear index (reference loop order) that failed
     unsigned long long therm_unconverged, therm_extra_passes, therm_mismatch, therm_mismatch_ulp;
-    unsigned int therm_pass_changed[GF_MAX_SWEEPS];  // bit 0: a tile border differs from its owner; bit 1: a tile did not settle
+    // flags of a thermal call's passes: bit 0: a border differs from its owner; bit 1: a
+    // strip (tile) did not settle.  Two sets, used in turn (ThermSlots)
+    unsigned int therm_pass_changed[2 * GF_MAX_SWEEPS];
     double dt_move;             // dt of the last element move (its stress rotation may still be pending)
     // change_phase (src/change_phase.f90:1-260) on the device
     unsigned int ph_newmask;    // phases (bit id-1) that markers turned into in the current call

@@ -124,7 +124,7 @@ GF_DEV void clock_op(GfDevClock *ck, int op)
 {
     if (op & CK_TIME_ADVANCE) ck->time = ck->time + ck->dt;
     if (op & CK_THERM_BEGIN)
-        for (int k = 0; k < GF_MAX_SWEEPS; k++) ck->therm_pass_changed[k] = 0u;
+        for (int k = 0; k < 2 * GF_MAX_SWEEPS; k++) ck->therm_pass_changed[k] = 0u;
     if (op & CK_DTAVG_ADD) ck->dtavg = ck->dtavg + ck->dt;
     if (op & CK_DTAVG_RESET) ck->dtavg = 0.0;
     if (op & CK_DT_BEGIN) {
@@ -748,7 +748,7 @@ __global__ void __launch_bounds__(256) k_therm_bc(const GfDevParams *__restrict_
 // times raises bar_timeout and returns false, so the launch always ends (the host
 // then reports the call as failed).
 #define GF_BAR_SPIN (1 << 22)
-GF_DEV bool grid_sync(GfDevClock *ck)
+GF_DEV bool grid_sync(GfDevClock *ck, unsigned nblocks)
 {
     __shared__ int s_ok;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -759,7 +759,7 @@ GF_DEV bool grid_sync(GfDevClock *ck)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         const unsigned arrived =
             __hip_atomic_fetch_add(&ck->bar_cnt, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-        if (arrived == gridDim.x) {
+        if (arrived == nblocks) {
             __hip_atomic_store(&ck->bar_cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_fetch_add(&ck->bar_gen, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         } else {
@@ -2293,25 +2293,51 @@ GF_DEV void node_tile_update(const GfDevParams *__restrict__ P, GfDevClock *ck, 
 // of tiles by column).  (Persistent workgroups that load the next tile into registers
 // while computing the current one ran slower: two workgroups per CU instead of three.)
 template <int M, bool MOVE>
-__global__ void __launch_bounds__(256) k_node_t(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                double *cord_out, int ops)
+GF_DEV void node_block(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, NodeLds<M> &L,
+                       double *cord_out, int ops, unsigned block)
 {
-    __shared__ NodeLds<M> L;
     const int ntiles = node_ntj(P) * node_nti(P);
-    const int q = (ntiles + 7) / 8, tile = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
+    const int q = (ntiles + 7) / 8, tile = (int)(block % 8) * q + (int)(block / 8);
     if (tile >= ntiles) return;  // the whole workgroup
     const NodeClk kc = node_clk(ck);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (block == 0 && threadIdx.x == 0) {
         if (MOVE) ck->dt_move = kc.dt;  // the move's dt (no other reader here)
         if (ops) clock_op(ck, ops);     // (fields nothing here reads)
     }
     // dt_mass's maxima of this step start at 0 (k_dens)
-    if ((ops & CK_DT_BEGIN) && blockIdx.x == 0 && threadIdx.x < 2 * DTR_SLOTS)
+    if ((ops & CK_DT_BEGIN) && block == 0 && threadIdx.x < 2 * DTR_SLOTS)
         A.dtred[(threadIdx.x >> 1) * DTR_PAD + (threadIdx.x & 1)] = 0ull;
     const NodePf<M> pf = node_prefetch<M>(P, A, tile);
     node_stage<M>(pf, L);
     __syncthreads();
     node_tile_update<M, MOVE>(P, ck, A, tile, L, pf.own, pf.ar, kc, cord_out);
+}
+template <int M, bool MOVE>
+__global__ void __launch_bounds__(256) k_node_t(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
+                                                double *cord_out, int ops)
+{
+    __shared__ NodeLds<M> L;
+    node_block<M, MOVE>(P, ck, A, L, cord_out, ops, blockIdx.x);
+}
+// ... with the end of the step's thermal call (k_therm_rest) in its first workgroups, which
+// find pass 0 proven in nearly every step and return: a launch of its own takes 3 us for
+// that answer.  They are the launch's first, so all of them are resident when they need
+// their barriers.  (At 128 VGPRs, four workgroups per CU, a further pass spills.)
+template <int M>
+__global__ void __launch_bounds__(256, 4) k_node_rest(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
+                                                      double *cord_out, int ops, ThermRest R)
+{
+    __shared__ NodeLds<M> L;
+    if (blockIdx.x >= (unsigned)R.grid) {
+        node_block<M, true>(P, ck, A, L, cord_out, ops, blockIdx.x - (unsigned)R.grid);
+        return;
+    }
+    // (the buffers have turned over since)
+    GfDevArrays B = A;
+    B.temp = A.temp0;
+    B.xa = A.temp;
+    B.temp0 = A.xa;
+    therm_rest_body<false>(P, ck, B, R, blockIdx.x);
 }
 
 // ------------------------------------------------------------------ fl_move

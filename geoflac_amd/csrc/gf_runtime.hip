@@ -103,6 +103,8 @@ struct gf_ctx {
     int therm_w = 0;     // output columns of a thermal strip
     bool therm_cols = false;  // pass 0 by a workgroup a strip (k_therm_cols)
     int therm_call = 0;  // thermal calls, modulo 3: the slot of a.tpre this call writes
+    ThermRest rest{};    // the end of a thermal call that the next fl_node launches (grid > 0)
+    int therm_set = 0;   // the next call's set of flags
     ThermChk chk{};      // the border check of the thermal call under way
     int node_ops = 0;    // clock updates left to the step's fl_node
     bool therm_clean = true;  // the flags of the thermal passes are 0 on the device
@@ -1202,11 +1204,12 @@ static int flush_rot(gf_ctx *ctx)
 // ops: clock updates for the first kernel of the call to make (or a launch of their own);
 // defer: the border check of pass 0 goes into the launch of fl_rheol (ctx->chk), after
 // which enq_therm_rest ends the call
-static int enq_therm_rest(gf_ctx *ctx);
+static int enq_therm_rest(gf_ctx *ctx, bool with_node = false);
 static int enq_therm(gf_ctx *ctx, int ops = 0, bool defer = false)
 {
     int rc;
-    // the flags of the passes start at 0: the last step's fl_node cleared them, or this
+    ctx->rest.grid = 0;
+    // the flags of the passes start at 0: the call before cleared them, or this
     if (!ctx->therm_clean && (rc = enq_clock(ctx, CK_THERM_BEGIN))) return rc;
     ctx->therm_clean = false;
     if (ctx->therm_batch) {  // (the batch numbers its own calls)
@@ -1228,7 +1231,7 @@ static int enq_therm(gf_ctx *ctx, int ops = 0, bool defer = false)
     const ThermGeo g = therm_geo(ctx->p.nz, ctx->p.nx, ctx->therm_w);
     const unsigned grid = 8u * (unsigned)((g.nr * g.ns + 7) / 8);
     const long nb = (long)g.nr * g.ns * TS_NB(g.w);
-    ctx->chk = ThermChk{(int)nblk(nb), arp, g, therm_slots(ctx->therm_call, ctx->therm_hist), ctx->a.temp, ctx->a.xa};
+    ctx->chk = ThermChk{(int)nblk(nb), arp, g, therm_slots(ctx->therm_call, ctx->therm_hist, ctx->therm_set), ctx->a.temp, ctx->a.xa};
     // pass 0 starts from the extrapolation 2 temp - temp0 once temp0 holds the
     // previous step's starting temperature
     const bool ex = ctx->temp0_prev && !ctx->therm_noguess;
@@ -1247,8 +1250,9 @@ static int enq_therm(gf_ctx *ctx, int ops = 0, bool defer = false)
     return enq_therm_rest(ctx);
 }
 
-// the further passes, if pass 0 was not proven, and the end of the call
-static int enq_therm_rest(gf_ctx *ctx)
+// the further passes, if pass 0 was not proven, and the end of the call; with_node: the
+// fl_node that follows launches them (k_node_rest)
+static int enq_therm_rest(gf_ctx *ctx, bool with_node)
 {
     if (ctx->therm_proof) {
         const bool dis = ctx->p.ishearh == 1 && ctx->p.itherm != 2;
@@ -1262,8 +1266,13 @@ static int enq_therm_rest(gf_ctx *ctx)
             // wait boundedly, so a launch that is not resident reports an error instead of
             // waiting for ever.  (A cooperative launch guarantees residency but costs
             // ~16 us more per launch on MI355X, more than the launches it replaces.)
-            auto rest = dis ? k_therm_rest<true> : k_therm_rest<false>;
-            LAUNCH_DIM("k_therm_rest", rest, ctx->therm_grid, 256, ctx->dp, ctx->dck, ctx->a, g, arp, sl, npass);
+            // Fewer where there are fewer strips than waves.
+            ctx->rest = ThermRest{(int)std::min<long>(ctx->therm_grid, ((long)g.nr * g.ns + 31) / 32 * 8), arp, npass, g, sl};
+            if (!with_node) {
+                auto rest = dis ? k_therm_rest<true> : k_therm_rest<false>;
+                LAUNCH_DIM("k_therm_rest", rest, ctx->rest.grid, 256, ctx->dp, ctx->dck, ctx->a, ctx->rest);
+                ctx->rest.grid = 0;
+            }
         } else {
             const unsigned grid = 8u * (unsigned)((g.nr * g.ns + 7) / 8);
             const long nb = (long)g.nr * g.ns * TS_NB(g.w);
@@ -1275,6 +1284,8 @@ static int enq_therm_rest(gf_ctx *ctx)
             LAUNCH_DIM("k_therm_last", k_therm_last, ctx->therm_grid, 256, ctx->dp, ctx->dck, ctx->a, sl, npass);
         }
         ctx->therm_call = (ctx->therm_call + 1) % 3;
+        ctx->therm_set ^= 1;
+        ctx->therm_clean = true;  // (pass 0 cleared the other set)
         ctx->therm_hist = std::min(ctx->therm_hist + 1, 2);
         ctx->chk.grid = 0;
     }
@@ -1373,6 +1384,12 @@ static int enq_rheol(gf_ctx *ctx, bool clock_done = false, bool last = true)
     return GF_OK;
 }
 
+// fl_node's tiles, ND_TJ x ND_TI nodes each
+static long node_tiles(const gf_ctx *ctx)
+{
+    return (long)((ctx->p.nz + ND_TJ - 1) / ND_TJ) * ((ctx->p.nx + ND_TI - 1) / ND_TI);
+}
+
 // move: the step's fl_move follows at once, so that the coordinate update may run here
 static int enq_node(gf_ctx *ctx, bool move)
 {
@@ -1382,17 +1399,27 @@ static int enq_node(gf_ctx *ctx, bool move)
         LAUNCH_M(k_node, ctx->nn, ctx->dp, ctx->dck, ctx->a);
         return GF_OK;
     }
-    // tiles of ND_TJ x ND_TI nodes, a multiple of 8 workgroups
-    const long ntiles = (long)((ctx->p.nz + ND_TJ - 1) / ND_TJ) * ((ctx->p.nx + ND_TI - 1) / ND_TI);
-    const long n = (ntiles + 7) / 8 * 8 * 256;
+    const long n = (node_tiles(ctx) + 7) / 8 * 8 * 256;  // a multiple of 8 workgroups
     const bool fuse = move && ctx->p.movegrid != 0 && ctx->in_batch == 0;
     const int M = ctx->precision == GF_PREC_MIXED ? 1 : ctx->precision == GF_PREC_MIXED_STORAGE ? 2 : 0;
     double *out = fuse ? ctx->cord_alt : nullptr;
     // in the step also the clock updates that no kernel up to here could make
-    const int ops = move ? ctx->node_ops | CK_THERM_BEGIN : 0;
+    const int ops = move ? ctx->node_ops | (ctx->therm_proof ? 0 : CK_THERM_BEGIN) : 0;
     if (move) {
         ctx->node_ops = 0;
         ctx->therm_clean = true;
+    }
+    if (ctx->rest.grid > 0) {  // (the moving FP64-arithmetic forms, enq_flac)
+        const ThermRest rest = ctx->rest;
+        ctx->rest.grid = 0;
+        const unsigned grid = nblk(n) + (unsigned)rest.grid;
+        if (M == 2)
+            LAUNCH_DIM("k_node_t<2>", k_node_rest<2>, grid, 256, ctx->dp, ctx->dck, ctx->a, out, ops, rest);
+        else
+            LAUNCH_DIM("k_node_t<0>", k_node_rest<0>, grid, 256, ctx->dp, ctx->dck, ctx->a, out, ops, rest);
+        std::swap(ctx->a.cord, ctx->cord_alt);
+        ctx->cord_moved = true;
+        return GF_OK;
     }
     // (timed under one name per precision, with or without the move)
     if (M == 1 && fuse) LAUNCH_NAMED("k_node_t<1>", (k_node_t<1, true>), n, ctx->dp, ctx->dck, ctx->a, out, ops);
@@ -1594,7 +1621,15 @@ static int enq_flac(gf_ctx *ctx, int pending = 0, bool last = true)
     if (mech) {
         if (phases && (rc = enq_change_phase(ctx))) return rc;
         if ((rc = enq_rheol(ctx, true, last))) return rc;
-        if (defer && (rc = enq_therm_rest(ctx))) return rc;
+        // fl_node's launch also ends the thermal call where it reads no temperature that a
+        // further pass could still change (the Winkler support reads the bottom row's), on
+        // meshes whose tiles are all resident at once: a step 33.1 -> 31.4 us at 400x100
+        // cells, 35.7 -> 34.1 at 60x20, 44.0 -> 42.3 at 151x47.  Where they are not, the
+        // registers of the further passes cost fl_node waves: 0.6 us more at 901x301, 1 us at
+        // 1200x500 with FP32 storage (3 us less at 2000x1000).
+        const bool with_node = ctx->therm_rest && !ctx->node_direct && ctx->p.movegrid != 0 && ctx->in_batch == 0 &&
+                               (ctx->p.nyhydro <= 0 || ctx->p.itemp_bc == 1) && node_tiles(ctx) <= 3L * ctx->therm_grid;
+        if (defer && (rc = enq_therm_rest(ctx, with_node))) return rc;
         if (ctx->p.nystressbc == 1 && (rc = enq_bc_update(ctx))) return rc;
         const bool rm = phases, im = ctx->nloop % ctx->p.ifreq_imasses == 0;
         const bool both = rm && im && !ctx->node_direct;

@@ -39,16 +39,24 @@
 // next call's rows 1 and nz start from; they go to a ring buffer of GF_NPRE slots of
 // 2 nx + 2 nz values: row 1, row nz, column 1, column nx.
 #define GF_NPRE 4
-// slots of a call: pass p writes slot[p & 1]; the last two calls' final values (hist of
-// them are valid)
+// slots of a call: pass p writes of(p); the last two calls' final values (hist of them are
+// valid)
 struct ThermSlots {
-    int cur[2], prev, prev2, hist;
+    int cur, prev, prev2, hist;
+    int flag;  // first flag of the call's passes; the other set's are cleared by pass 0
+    GF_DEVM int of(int pass) const { return pass & 1 ? GF_NPRE - 1 : cur; }
 };
 // consecutive calls number `call` turn three slots over; an odd pass uses the fourth
-__host__ __device__ inline ThermSlots therm_slots(int call, int hist)
+__host__ __device__ inline ThermSlots therm_slots(int call, int hist, int set = 0)
 {
     const int c = call % 3;
-    return ThermSlots{{c, 3}, (c + 2) % 3, (c + 1) % 3, hist};
+    return ThermSlots{c, (c + 2) % 3, (c + 1) % 3, hist, set ? GF_MAX_SWEEPS : 0};
+}
+// the flags of the next call (those of the one before this, whose passes are over)
+GF_DEV void therm_clear_other(GfDevClock *ck, const ThermSlots &sl)
+{
+    if (blockIdx.x == 0 && threadIdx.x < GF_MAX_SWEEPS)
+        ck->therm_pass_changed[(sl.flag ^ GF_MAX_SWEEPS) + threadIdx.x] = 0u;
 }
 GF_DEV double *therm_pre(const GfDevParams *P, const GfDevArrays &A, int slot)
 {
@@ -211,10 +219,10 @@ struct ThermWave {
         // calls, carried on (pass 0), or those of the last pass (the iterate's own boundary
         // rows hold the conditions)
         const unsigned npre = 2u * (nx + nz);
-        const int pslot = MODE == 1 ? sl.cur[(it.pass - 1) & 1] : sl.prev;
+        const int pslot = MODE == 1 ? sl.of(it.pass - 1) : sl.prev;
         bP = mkbuf(A.tpre + (long)pslot * npre, 8ull * npre);
         bP2 = mkbuf(A.tpre + (long)sl.prev2 * npre, 8ull * npre);
-        bW = mkbuf(A.tpre + (long)sl.cur[it.pass & 1] * npre, 8ull * npre);
+        bW = mkbuf(A.tpre + (long)sl.of(it.pass) * npre, 8ull * npre);
         pvo = erow1 ? 0u : erown ? 8u * nx : OOB;               // row arrays, + 8 (i - 1)
         pco = row <= nz ? 8u * (2 * nx + row - 1) : OOB;        // column arrays, + 8 nz for column nx
         pedge = edge && (MODE == 1 || (MODE == 2 && sl.hist > 0));
@@ -455,7 +463,7 @@ GF_DEV void therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, const
         ydn0 = ydn1;
         tdn0 = tdn1;
     }
-    if (!still && w.lane == 0) atomicOr(&ck->therm_pass_changed[it.pass], 2u);
+    if (!still && w.lane == 0) atomicOr(&ck->therm_pass_changed[sl.flag + it.pass], 2u);
 }
 
 // One strip by one workgroup, a wave a column, for meshes of so few strips that each has a
@@ -572,7 +580,7 @@ GF_DEV void therm_cols(const GfDevParams *__restrict__ P, GfDevClock *ck, const 
         }
     }
     if (in) w.store(i, x, n0.y, phs);
-    if (!still && threadIdx.x == 0) atomicOr(&ck->therm_pass_changed[it.pass], 2u);
+    if (!still && threadIdx.x == 0) atomicOr(&ck->therm_pass_changed[sl.flag + it.pass], 2u);
 }
 
 // by the lanes of one wave, for that wave
@@ -597,9 +605,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 k_therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, ThermGeo g, int pass, int arp,
               ThermSlots sl, int ops)
 {
+    if (pass == 0) therm_clear_other(ck, sl);
     if (ops && blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
     __shared__ double sPh[4][GF_MAXPH];
-    if (pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) return;  // already proven
+    if (pass > 0 && ck->therm_pass_changed[sl.flag + pass - 1] == 0u) return;  // already proven
     const int nt = g.nr * g.ns, q = (nt + 7) / 8;  // XCD x runs strips [x q, (x+1) q)
     const int t = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
     if ((int)(blockIdx.x / 8) >= q || t >= nt) return;
@@ -613,6 +622,7 @@ __global__ void __launch_bounds__(64 * TC_W)
 k_therm_cols(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, ThermGeo g, int arp, ThermSlots sl,
              int ops)
 {
+    therm_clear_other(ck, sl);
     if (ops && blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
     __shared__ ThermColLds L;
     const int nt = g.nr * g.ns, q = (nt + 7) / 8, t = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
@@ -651,7 +661,7 @@ GF_DEV void therm_check_one(const GfDevParams *__restrict__ P, GfDevClock *ck, c
     if (i > s.c1) return;
     const int nz = g.nz, nx = g.nx, j = s.jb + lane;
     const double *__restrict__ x = (pass % 2 == 0) ? A.xa : A.xb;
-    const double *__restrict__ pre = therm_pre(P, A, sl.cur[pass & 1]);
+    const double *__restrict__ pre = therm_pre(P, A, sl.of(pass));
     // the pass's value before the boundary conditions
     auto X = [&](int jj, int ii) -> double {
         if (jj == 1) return pre[ii - 1];
@@ -680,13 +690,13 @@ GF_DEV void therm_check_one(const GfDevParams *__restrict__ P, GfDevClock *ck, c
     }
     atomicAdd(&ck->therm_mismatch, 1ull);  // (statistics)
     atomicMax(&ck->therm_mismatch_ulp, (unsigned long long)(a > b ? a - b : b - a));
-    if (bad) atomicOr(&ck->therm_pass_changed[pass], 1u);
+    if (bad) atomicOr(&ck->therm_pass_changed[sl.flag + pass], 1u);
 }
 
 __global__ void __launch_bounds__(256) k_therm_check(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
                                                     ThermGeo g, int pass, int arp, ThermSlots sl, long total)
 {
-    if (pass > 0 && ck->therm_pass_changed[pass - 1] == 0u) return;  // that pass did not run
+    if (pass > 0 && ck->therm_pass_changed[sl.flag + pass - 1] == 0u) return;  // that pass did not run
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
     if (t < total) therm_check_one(P, ck, A, g, t, pass, arp, sl);
 }
@@ -722,8 +732,8 @@ GF_DEV void therm_settle(const GfDevParams *__restrict__ P, const GfDevArrays &A
 {
     if (last % 2 == 0) return;
     for (long t = tid; t < NN; t += nthr) A.xa[t] = A.xb[t];
-    const double *from = therm_pre(P, A, sl.cur[1]);
-    double *to = therm_pre(P, A, sl.cur[0]);
+    const double *from = therm_pre(P, A, sl.of(1));
+    double *to = therm_pre(P, A, sl.of(0));
     for (long t = tid; t < 2L * (P->nx + P->nz); t += nthr) to[t] = from[t];
 }
 
@@ -733,32 +743,48 @@ GF_DEV void therm_settle(const GfDevParams *__restrict__ P, const GfDevArrays &A
 // barriers between the phases, until one is proven or npass ran.  The flags that decide
 // another pass are read with coherent loads after a barrier, so every workgroup takes
 // the same decision; flag 0 was written by earlier launches.
+struct ThermRest {
+    int grid, arp, npass;
+    ThermGeo g;
+    ThermSlots sl;
+};
+// (workgroup `block` of R.grid of 256 threads)
 template <bool DIS>
-__global__ void __launch_bounds__(256) k_therm_rest(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                    ThermGeo g, int arp, ThermSlots sl, int npass)
+GF_DEV void therm_rest_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, const ThermRest &R,
+                            unsigned block)
 {
-    if (ck->therm_pass_changed[0] == 0u) return;
+    const ThermSlots sl = R.sl;
+    if (ck->therm_pass_changed[sl.flag] == 0u) return;
+    const ThermGeo g = R.g;
+    const int npass = R.npass;
     __shared__ double sPhw[4][4][GF_MAXPH];  // (a table a wave)
     double(*sPh)[GF_MAXPH] = sPhw[threadIdx.x / 64];
     therm_phase_table(P, sPh);
     const int nt = g.nr * g.ns;
     const long nb = (long)nt * TS_NB(g.w);
-    const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x, nthr = (long)gridDim.x * blockDim.x;
+    const long tid = (long)block * 256 + threadIdx.x, nthr = (long)R.grid * 256;
     int proven = -1, pass = 1;
     for (; pass < npass; pass++) {
-        const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, arp, pass};
+        const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, R.arp, pass};
         for (int t = (int)(tid / 64); t < nt; t += (int)(nthr / 64))
             therm_strip<DIS, 1>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(g.w), ck->dt, sPh);
-        if (!grid_sync(ck)) return;  // every strip's iterate is written
-        for (long t = tid; t < nb; t += nthr) therm_check_one(P, ck, A, g, t, pass, arp, sl);
-        if (!grid_sync(ck)) return;  // every border is checked
-        if (__hip_atomic_load(&ck->therm_pass_changed[pass], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
+        if (!grid_sync(ck, R.grid)) return;  // every strip's iterate is written
+        for (long t = tid; t < nb; t += nthr) therm_check_one(P, ck, A, g, t, pass, R.arp, sl);
+        if (!grid_sync(ck, R.grid)) return;  // every border is checked
+        if (__hip_atomic_load(&ck->therm_pass_changed[sl.flag + pass], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+            0u) {
             proven = pass;
             break;
         }
     }
     if (tid == 0) therm_outcome(ck, proven);
     therm_settle(P, A, sl, proven < 0 ? npass - 1 : proven, tid, nthr);
+}
+template <bool DIS>
+__global__ void __launch_bounds__(256) k_therm_rest(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
+                                                    ThermRest R)
+{
+    therm_rest_body<DIS>(P, ck, A, R, blockIdx.x);
 }
 
 // the end of a call whose further passes ran as launches of their own
@@ -767,7 +793,7 @@ __global__ void __launch_bounds__(256) k_therm_last(const GfDevParams *__restric
 {
     int proven = -1;
     for (int k = npass - 1; k >= 0; k--)
-        if (ck->therm_pass_changed[k] == 0u) proven = k;
+        if (ck->therm_pass_changed[sl.flag + k] == 0u) proven = k;
     const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x, nthr = (long)gridDim.x * blockDim.x;
     if (tid == 0) therm_outcome(ck, proven);
     therm_settle(P, A, sl, proven < 0 ? npass - 1 : proven, tid, nthr);

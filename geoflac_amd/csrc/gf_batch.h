@@ -25,6 +25,7 @@ struct BatchEntry {
     double *tprev;      // the starting temperature of the call before (the next call's result)
     double *cord_next;
     ThermGeo tg;        // thermal strips
+    GfDevClock *host;   // the model's clock in page-locked memory
     long pe, pn, pt, pb, pm;  // first global index: elements, nodes, thermal tiles, border entries, markers
     long ce, cn, ct, cb, cm;  // counts of the same
 };
@@ -279,6 +280,8 @@ __global__ void __launch_bounds__(256) kb_area_check(const BatchEntry *__restric
 {
     batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) { area_check_body(b.P, b.ck, bmoved(b), e); });
 }
+
+__global__ void kb_clock_out(const BatchEntry *__restrict__ tab) { clock_out(tab[blockIdx.x].ck, tab[blockIdx.x].host); }
 
 // the masses and dt minima after the step's move (arp: its areas are pending)
 template <int M>

@@ -88,6 +88,7 @@ struct GfDevClock {
     int th_call, th_hist;
     // itest_mesh's smallest triangle angle, as an order-preserving key (rem_angle_key)
     unsigned long long rem_key;
+    unsigned int out_cnt, out_pad;  // workgroups of a launch that ends with clock_out and are done
 };
 
 // ---------------------------------------------------------------- buffer access

@@ -138,6 +138,45 @@ __global__ void k_clock(GfDevClock *ck, int op)
 {
     if (threadIdx.x == 0) clock_op(ck, op);
 }
+// ... and in a launch that may set the caller's time first
+struct ClockOps {
+    int ops, set_time;
+    double time;
+};
+GF_DEV void clock_op(GfDevClock *ck, const ClockOps &o)
+{
+    if (o.set_time) ck->time = o.time;
+    clock_op(ck, o.ops);
+}
+
+// The clock goes to page-locked host memory from the call's last launch, so that the host
+// waits once and copies nothing: a call of gf_flac at 60x20 cells, with a tenth of an
+// itest_mesh, took 87 us with copies of pageable memory both ways and takes 58 (34 of them
+// in the kernels).
+// (the threads of one workgroup; the values other workgroups of the launch wrote are read
+// past the caches)
+GF_DEV void clock_out(const GfDevClock *ck, GfDevClock *host)
+{
+    const unsigned *w = (const unsigned *)ck;
+    for (int k = threadIdx.x; k < (int)(sizeof(GfDevClock) / 4); k += blockDim.x)
+        ((unsigned *)host)[k] = __hip_atomic_load(w + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__global__ void k_clock_out(const GfDevClock *ck, GfDevClock *host) { clock_out(ck, host); }
+// true in the workgroup of the launch that gets here last, for all its threads
+GF_DEV bool last_block(GfDevClock *ck)
+{
+    __shared__ int s_last;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence();
+        const unsigned done = __hip_atomic_fetch_add(&ck->out_cnt, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = done + 1 == gridDim.x;
+        if (s_last) __hip_atomic_store(&ck->out_cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __threadfence();
+    }
+    __syncthreads();
+    return s_last != 0;
+}
 
 // correctly rounded math of the FP64 path, evaluated for a list of arguments
 // (fn: 0 sin, 1 tan, 2 exp, 3 pow with y = args2)
@@ -676,9 +715,9 @@ GF_DEV void therm_tile_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, c
 // arp: the element areas of the last move are pending (formed from the coordinates)
 template <bool DIS>
 __global__ void __launch_bounds__(1024) k_therm_pipe(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                     double stol, int arp, int fold, int ops)
+                                                     double stol, int arp, int fold, ClockOps ops)
 {
-    if (ops && blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
+    if (blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
     __shared__ ThermRaw raw;
     __shared__ double sU[TH_NF * TH_NE];
     __shared__ int sFlag[3];
@@ -2443,11 +2482,13 @@ GF_DEV void area_check_body(const GfDevParams *__restrict__ P, GfDevClock *ck, c
     for (int k = 0; k < 4; k++) bad |= (1.0 / move_det(xc, yc, k) <= 0);
     if (bad) raise_error(ck, GF_STOP_NEGATIVE_AREA, e);
 }
-__global__ void __launch_bounds__(256) k_area_check(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A)
+// (the call's last launch: it also hands the clock over)
+__global__ void __launch_bounds__(256) k_area_check(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
+                                                    GfDevClock *host)
 {
     long e = xcd_lin();
-    if (e >= NE) return;
-    area_check_body(P, ck, A, e);
+    if (e < NE) area_check_body(P, ck, A, e);
+    if (last_block(ck)) clock_out(ck, host);
 }
 // rec_dt: record the move's dt (0 when completing a move whose dt is recorded already)
 __global__ void __launch_bounds__(256) k_move_area(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
@@ -2835,7 +2876,15 @@ GF_DEV double rem_elem_angle(const GfDevParams *__restrict__ P, const GfDevArray
     }
     return amin;
 }
-__global__ void __launch_bounds__(256) k_rem_angle(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A)
+// What itest_mesh reads: the smallest angle's key (left at the largest for the next call)
+// and the corner coordinates of its other tests
+struct RemOut {
+    unsigned long long key;
+    double x11, x1n, y11, y21;
+};
+#define REM_KEY_180 0xc066800000000000ull  // of 180 degrees
+__global__ void __launch_bounds__(256) k_rem_angle(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
+                                                   RemOut *host)
 {
     __shared__ double s_min[4];
     const long e = xcd_lin();
@@ -2850,6 +2899,9 @@ __global__ void __launch_bounds__(256) k_rem_angle(const GfDevParams *__restrict
     if (threadIdx.x == 0) {
         for (int q = 1; q < (int)(blockDim.x >> 6); q++) amin = fmin(amin, s_min[q]);
         atomicMin(&ck->rem_key, rem_angle_key(amin));
+    }
+    if (last_block(ck) && threadIdx.x == 0) {
+        *host = RemOut{atomicExch(&ck->rem_key, REM_KEY_180), CORD(1, 1, 1), CORD(1, NX, 1), CORD(1, 1, 2), CORD(2, 1, 2)};
     }
 }
 

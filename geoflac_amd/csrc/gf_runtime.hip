@@ -103,6 +103,13 @@ struct gf_ctx {
     int therm_w = 0;     // output columns of a thermal strip
     bool therm_cols = false;  // pass 0 by a workgroup a strip (k_therm_cols)
     int therm_call = 0;  // thermal calls, modulo 3: the slot of a.tpre this call writes
+    bool set_time = false;  // the next thermal launch sets the device's time to `time`
+    double time = 0.0;
+    // page-locked: what launches hand to the host
+    struct HostOut {
+        GfDevClock ck;
+        RemOut rem;
+    } *hout = nullptr;
     ThermRest rest{};    // the end of a thermal call that the next fl_node launches (grid > 0)
     int therm_set = 0;   // the next call's set of flags
     ThermChk chk{};      // the border check of the thermal call under way
@@ -337,6 +344,10 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
     }
     ALLOC(ctx->dp, sizeof(GfDevParams));
     ALLOC(ctx->dck, sizeof(GfDevClock));
+    if (hipHostMalloc((void **)&ctx->hout, sizeof(*ctx->hout), hipHostMallocDefault) != hipSuccess) {
+        rc = set_err(ctx, GF_ERR_HIP, "hipHostMalloc failed");
+        goto fail;
+    }
     ALLOC(ctx->a.cord, 8 * nn * 2);
     ALLOC(ctx->cord_alt, 8 * nn * 2);
     // stress, velocity and force in the path's precision (FP32 planes when mixed)
@@ -398,6 +409,7 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
     {
         GfDevClock ck{};
         ck.error_index = (long long)1 << 62;
+        ck.rem_key = REM_KEY_180;
         if (hipMemcpy(ctx->dck, &ck, sizeof(ck), hipMemcpyHostToDevice) != hipSuccess) {
             rc = set_err(ctx, GF_ERR_HIP, "clock init failed");
             goto fail;
@@ -430,6 +442,7 @@ extern "C" void gf_destroy(gf_ctx *ctx)
                     ctx->a.dtopo, ctx->a.dhacc, ctx->a.dhacc_corr, ctx->a.topo_tmp, ctx->a.iphx};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    if (ctx->hout) (void)hipHostFree(ctx->hout);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -977,16 +990,15 @@ extern "C" int gf_itest_mesh(gf_ctx *ctx, int32_t mode_rem, double dx_rem, doubl
     *need_remeshing = 0;
     *anglemin = 180.0;
     *value = 0.0;
-    const long nz = ctx->p.nz, nx = ctx->p.nx, nn = nz * nx;
+    const long nx = ctx->p.nx;
+    // one launch for the smallest angle (:51-129) and the coordinates the other tests read
+    hipLaunchKernelGGL(k_rem_angle, dim3(nblk(ctx->ne)), dim3(256), 0, ctx->stream, ctx->dp, ctx->dck, ctx->a,
+                       &ctx->hout->rem);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    auto cord = [&](long j, long i, int d, double &v) {  // one coordinate from the device
-        return hipMemcpy(&v, ctx->a.cord + (j - 1) + nz * (i - 1) + nn * (d - 1), sizeof(double),
-                         hipMemcpyDeviceToHost);
-    };
+    const RemOut rem = ctx->hout->rem;
     if (mode_rem == 11 || mode_rem == 3) {  // :15-29
-        double x1 = 0.0, xn = 0.0;
-        HIPCHK(cord(1, 1, 1, x1));
-        HIPCHK(cord(1, nx, 1, xn));
+        const double x1 = rem.x11, xn = rem.x1n;
         const double testcr = dx_rem * ctx->p.rxbo / (nx - 1);
         const double shortening = fabs(xn - x1 - ctx->p.rxbo);
         if (shortening > testcr) {
@@ -997,10 +1009,7 @@ extern "C" int gf_itest_mesh(gf_ctx *ctx, int32_t mode_rem, double dx_rem, doubl
     }
     const double arc_extrusion_rate = 1.0 - ratio_mantle_mzone;  // :31-49
     if (ctx->p.topo_kappa > 0 || arc_extrusion_rate > 0) {
-        double y11 = 0.0, y21 = 0.0;
-        HIPCHK(cord(1, 1, 2, y11));
-        HIPCHK(cord(2, 1, 2, y21));
-        const double testcr = (y11 - y21) * 0.3333;
+        const double testcr = (rem.y11 - rem.y21) * 0.3333;
         // dhacc (diff_topo's accumulated change; zero where diff_topo does not run);
         // extr_acc is zero without melting (refused at gf_create)
         std::vector<double> dh(nx - 1, 0.0);
@@ -1015,22 +1024,7 @@ extern "C" int gf_itest_mesh(gf_ctx *ctx, int32_t mode_rem, double dx_rem, doubl
             return GF_OK;
         }
     }
-    // :51-129, the smallest angle
-    const GfDevClock init_key = [] {
-        GfDevClock z{};
-        const double a = 180.0;
-        unsigned long long u;
-        memcpy(&u, &a, sizeof u);
-        z.rem_key = (u >> 63) ? ~u : (u | 0x8000000000000000ull);
-        return z;
-    }();
-    HIPCHK(hipMemcpy((char *)ctx->dck + offsetof(GfDevClock, rem_key), &init_key.rem_key, sizeof init_key.rem_key,
-                     hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_rem_angle, dim3(nblk(ctx->ne)), dim3(256), 0, ctx->stream, ctx->dp, ctx->dck, ctx->a);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    unsigned long long key = 0;
-    HIPCHK(hipMemcpy(&key, (char *)ctx->dck + offsetof(GfDevClock, rem_key), sizeof key, hipMemcpyDeviceToHost));
+    const unsigned long long key = rem.key;
     const unsigned long long u = (key >> 63) ? (key & 0x7fffffffffffffffull) : ~key;
     memcpy(anglemin, &u, sizeof u);
     if (*anglemin <= angle_rem) *need_remeshing = 1;
@@ -1052,12 +1046,11 @@ extern "C" int gf_set_clock(gf_ctx *ctx, const gf_clock *c)
     return GF_OK;
 }
 
-// read the clock back and turn a device-side STOP into its status code
-static int fetch_clock(gf_ctx *ctx, gf_clock *c)
+// the clock as a launch left it in host memory (clock_out), once the stream is done; turns
+// a device-side STOP into its status code
+static int read_clock(gf_ctx *ctx, gf_clock *c)
 {
-    GfDevClock ck;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(&ck, ctx->dck, sizeof(ck), hipMemcpyDeviceToHost));
+    const GfDevClock ck = ctx->hout->ck;
     ctx->dt_seen = ck.dt;
     if (ctx->markers_uploaded && ctx->p.topo_kappa > 0.0) ctx->a.nmarkers = ck.nmarkers;  // (resurface appends)
     if (ck.bar_timeout != 0) {  // (not expected: every workgroup of the launch is resident)
@@ -1088,6 +1081,10 @@ static int fetch_clock(gf_ctx *ctx, gf_clock *c)
     }
     return GF_OK;
 }
+
+// check: the last launch looks for the negative areas of a move that is pending still, so
+// that the call that moved the grid reports them
+static int fetch_clock(gf_ctx *ctx, gf_clock *c, bool check = false);
 
 extern "C" int gf_get_clock(gf_ctx *ctx, gf_clock *c)
 {
@@ -1205,9 +1202,11 @@ static int flush_rot(gf_ctx *ctx)
 // defer: the border check of pass 0 goes into the launch of fl_rheol (ctx->chk), after
 // which enq_therm_rest ends the call
 static int enq_therm_rest(gf_ctx *ctx, bool with_node = false);
-static int enq_therm(gf_ctx *ctx, int ops = 0, bool defer = false)
+static int enq_therm(gf_ctx *ctx, int clock_ops = 0, bool defer = false)
 {
     int rc;
+    const ClockOps ops{clock_ops, ctx->set_time ? 1 : 0, ctx->time};
+    ctx->set_time = false;
     ctx->rest.grid = 0;
     // the flags of the passes start at 0: the call before cleared them, or this
     if (!ctx->therm_clean && (rc = enq_clock(ctx, CK_THERM_BEGIN))) return rc;
@@ -1278,7 +1277,7 @@ static int enq_therm_rest(gf_ctx *ctx, bool with_node)
             const long nb = (long)g.nr * g.ns * TS_NB(g.w);
             auto extra = dis ? k_therm_strip<true, 1> : k_therm_strip<false, 1>;
             for (int pass = 1; pass < npass; pass++) {
-                LAUNCH_DIM("k_therm_strip_extra", extra, grid, 64, ctx->dp, ctx->dck, ctx->a, g, pass, arp, sl, 0);
+                LAUNCH_DIM("k_therm_strip_extra", extra, grid, 64, ctx->dp, ctx->dck, ctx->a, g, pass, arp, sl, ClockOps{});
                 LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, g, pass, arp, sl, nb);
             }
             LAUNCH_DIM("k_therm_last", k_therm_last, ctx->therm_grid, 256, ctx->dp, ctx->dck, ctx->a, sl, npass);
@@ -1595,13 +1594,17 @@ static int enq_diff_topo(gf_ctx *ctx)
     return GF_OK;
 }
 
-// Before a call returns: a move whose areas are still pending is checked for the
-// negative-area STOP now (the areas come with the next fl_rheol), so that the call
-// that moved the grid reports it.
-static int enq_area_check(gf_ctx *ctx)
+static int fetch_clock(gf_ctx *ctx, gf_clock *c, bool check)
 {
-    if (ctx->area_pending) LAUNCH(k_area_check, ctx->ne, ctx->dp, ctx->dck, ctx->a);
-    return GF_OK;
+    if (check && ctx->area_pending) {
+        LAUNCH(k_area_check, ctx->ne, ctx->dp, ctx->dck, ctx->a, &ctx->hout->ck);
+    } else {
+        hipLaunchKernelGGL(k_clock_out, dim3(1), dim3(256), 0, ctx->stream, ctx->dck, &ctx->hout->ck);
+        int rc = launch_check(ctx, "k_clock_out");
+        if (rc) return rc;
+    }
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return read_clock(ctx, c);
 }
 
 // one call of subroutine flac, src/flac.f90:18-83; pending: clock updates left by the
@@ -1657,8 +1660,7 @@ extern "C" int gf_step(gf_ctx *ctx, int32_t nsteps, gf_clock *clock)
         ctx->nloop = ctx->nloop + 1;
     }
     if (nsteps > 0 && (rc = enq_clock(ctx, CK_TIME_ADVANCE))) return rc;
-    if ((rc = enq_area_check(ctx))) return rc;
-    return fetch_clock(ctx, clock);
+    return fetch_clock(ctx, clock, true);
 }
 
 extern "C" int gf_flac(gf_ctx *ctx, gf_clock *clock)
@@ -1669,11 +1671,10 @@ extern "C" int gf_flac(gf_ctx *ctx, gf_clock *clock)
     // the caller owns nloop and time between calls (src/par.f90:83-86)
     ctx->nloop = clock->nloop;
     ctx->nsrate = clock->nsrate;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(&ctx->dck->time, &clock->time, sizeof(double), hipMemcpyHostToDevice));
+    ctx->set_time = true;  // (the thermal launch sets it)
+    ctx->time = clock->time;
     if ((rc = enq_flac(ctx))) return rc;
-    if ((rc = enq_area_check(ctx))) return rc;
-    return fetch_clock(ctx, clock);
+    return fetch_clock(ctx, clock, true);
 }
 
 #define SINGLE(name, body)                                                \
@@ -2545,7 +2546,7 @@ extern "C" int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out)
                                             : (long)((q.nz + TH_OJ - 1) / TH_OJ) * ((q.nx + TH_OI - 1) / TH_OI);
         const long nbord = c0->therm_proof ? ntiles * TS_NB(b->therm_w) : 0;
         const long nmk = c->markers_uploaded ? c->a.nmarkers : 0;
-        tab[k] = BatchEntry{c->dp, c->dck, c->a, nullptr, nullptr, tg, pe, pn, pt, pb, pm, c->ne, c->nn, ntiles, nbord, nmk};
+        tab[k] = BatchEntry{c->dp, c->dck, c->a, nullptr, nullptr, tg, &c->hout->ck, pe, pn, pt, pb, pm, c->ne, c->nn, ntiles, nbord, nmk};
         b->fold = b->fold && q.itemp_bc != 2;
         if (nmk > 0) b->markers = true;
         mm.insert(mm.end(), align(nmk) / BATCH_ALIGN, k);
@@ -2560,7 +2561,7 @@ extern "C" int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out)
         pb += align(nbord);
         b->m.push_back(c);
     }
-    tab[n] = BatchEntry{nullptr, nullptr, GfDevArrays{}, nullptr, nullptr, ThermGeo{}, pe, pn, pt, pb, pm, 0, 0, 0, 0, 0};
+    tab[n] = BatchEntry{nullptr, nullptr, GfDevArrays{}, nullptr, nullptr, ThermGeo{}, nullptr, pe, pn, pt, pb, pm, 0, 0, 0, 0, 0};
     b->nm = n;
     b->tot_e = pe; b->tot_n = pn; b->tot_t = pt; b->tot_b = pb; b->tot_m = pm;
     b->movegrid = c0->p.movegrid != 0;
@@ -2860,6 +2861,7 @@ extern "C" int gf_batch_step(gf_batch *b, int32_t nsteps)
     batch_turn(b, nsteps);
     if (b->area_pending)  // the negative-area STOP of the last move, now
         BLAUNCH(kb_area_check, bgrid(b->tot_e, 256), 256, b->dtab, b->map);
+    BLAUNCH(kb_clock_out, (unsigned)b->nm, 256, b->dtab);
     BCHK(hipStreamSynchronize(b->stream));
     int first = GF_OK;
     for (gf_ctx *c : b->m) {
@@ -2869,7 +2871,7 @@ extern "C" int gf_batch_step(gf_batch *b, int32_t nsteps)
         c->area_pending = b->area_pending;
         c->temp0_prev = b->temp0_prev;
         c->therm_clean = false;
-        int r = fetch_clock(c, nullptr);
+        int r = read_clock(c, nullptr);
         if (r && first == GF_OK) first = r;
     }
     if (first) snprintf(b->msg, sizeof(b->msg), "a model stopped with code %d (see its context)", first);

@@ -603,10 +603,10 @@ GF_DEV void therm_phase_table(const GfDevParams *__restrict__ P, double (*sPh)[G
 template <bool DIS, int MODE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 k_therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, ThermGeo g, int pass, int arp,
-              ThermSlots sl, int ops)
+              ThermSlots sl, ClockOps ops)
 {
     if (pass == 0) therm_clear_other(ck, sl);
-    if (ops && blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
+    if (blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
     __shared__ double sPh[4][GF_MAXPH];
     if (pass > 0 && ck->therm_pass_changed[sl.flag + pass - 1] == 0u) return;  // already proven
     const int nt = g.nr * g.ns, q = (nt + 7) / 8;  // XCD x runs strips [x q, (x+1) q)
@@ -620,10 +620,10 @@ k_therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, 
 template <bool DIS, int MODE>
 __global__ void __launch_bounds__(64 * TC_W)
 k_therm_cols(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, ThermGeo g, int arp, ThermSlots sl,
-             int ops)
+             ClockOps ops)
 {
     therm_clear_other(ck, sl);
-    if (ops && blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
+    if (blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
     __shared__ ThermColLds L;
     const int nt = g.nr * g.ns, q = (nt + 7) / 8, t = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
     if ((int)(blockIdx.x / 8) >= q || t >= nt) return;

@@ -992,8 +992,11 @@ extern "C" int gf_itest_mesh(gf_ctx *ctx, int32_t mode_rem, double dx_rem, doubl
     *value = 0.0;
     const long nx = ctx->p.nx;
     // one launch for the smallest angle (:51-129) and the coordinates the other tests read
+    const bool last = nblk(ctx->ne) <= LAST_BLOCKS;
+    RemOut *const out = &ctx->hout->rem, *const none = nullptr;
     hipLaunchKernelGGL(k_rem_angle, dim3(nblk(ctx->ne)), dim3(256), 0, ctx->stream, ctx->dp, ctx->dck, ctx->a,
-                       &ctx->hout->rem);
+                       last ? out : none);
+    if (!last) hipLaunchKernelGGL(k_rem_out, dim3(1), dim3(64), 0, ctx->stream, ctx->dp, ctx->dck, ctx->a, out);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(ctx->stream));
     const RemOut rem = ctx->hout->rem;
@@ -1596,9 +1599,11 @@ static int enq_diff_topo(gf_ctx *ctx)
 
 static int fetch_clock(gf_ctx *ctx, gf_clock *c, bool check)
 {
-    if (check && ctx->area_pending) {
-        LAUNCH(k_area_check, ctx->ne, ctx->dp, ctx->dck, ctx->a, &ctx->hout->ck);
-    } else {
+    const bool last = nblk(ctx->ne) <= LAST_BLOCKS;
+    GfDevClock *none = nullptr;
+    if (check && ctx->area_pending)
+        LAUNCH(k_area_check, ctx->ne, ctx->dp, ctx->dck, ctx->a, last ? &ctx->hout->ck : none);
+    if (!last || !check || !ctx->area_pending) {
         hipLaunchKernelGGL(k_clock_out, dim3(1), dim3(256), 0, ctx->stream, ctx->dck, &ctx->hout->ck);
         int rc = launch_check(ctx, "k_clock_out");
         if (rc) return rc;

@@ -1,7 +1,8 @@
 """gf_flac and itest_mesh hand their results to the host from the call's last launch: a
 loop of gf_flac with the caller's own nloop and time leaves what gf_step leaves, a time
 the caller sets comes back unchanged, and the smallest angle does not depend on earlier
-calls.  Meshes of one workgroup of elements, of exactly two, and of one element more."""
+calls.  Meshes of one workgroup of elements, of exactly two, of one element more, and of 64
+workgroups (up to which that launch hands over itself) and 65."""
 import os
 
 import numpy as np
@@ -14,7 +15,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("nelx,nelz,precision", [
-    (2, 2, abi.PREC_FP64), (32, 16, abi.PREC_FP64), (19, 27, abi.PREC_FP64), (60, 20, abi.PREC_MIXED)])
+    (2, 2, abi.PREC_FP64), (32, 16, abi.PREC_FP64), (19, 27, abi.PREC_FP64), (60, 20, abi.PREC_MIXED),
+    (128, 128, abi.PREC_FP64), (129, 128, abi.PREC_FP64)])
 def test_flac_loop_equals_step(nelx, nelz, precision):
     p = sweep.variant(inp.read_inp(os.path.join(HERE, "golden", "inputs", "box60x20.inp")), nelx, nelz)
     print("case: %dx%d elements, precision %d" % (nelx, nelz, precision), flush=True)

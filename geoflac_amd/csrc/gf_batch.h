@@ -64,9 +64,10 @@ GF_DEV const BatchEntry &bentry(const BatchEntry *tab, int m)
 // workgroup k is dispatched to XCD k % 8: give each XCD one contiguous run of the
 // index range (the first G % 8 XCDs one workgroup more), so that the node rows two
 // neighbouring workgroups share stay in one L2 (a bijection for any grid size G)
-GF_DEV unsigned xcd_block()
+// (skip, a multiple of 8: the first workgroups of the launch do something else)
+GF_DEV unsigned xcd_block(unsigned skip = 0)
 {
-    const unsigned G = gridDim.x, k = blockIdx.x, x = k % 8, q = G / 8, r = G % 8;
+    const unsigned G = gridDim.x - skip, k = blockIdx.x - skip, x = k % 8, q = G / 8, r = G % 8;
     return x * q + min(x, r) + k / 8;
 }
 
@@ -248,13 +249,26 @@ __global__ void __launch_bounds__(256) kb_visc(const BatchEntry *__restrict__ ta
     batch_apply<BK_ELEM>(tab, map, [&](const BatchEntry &b, long e) { visc_body<M>(b.P, b.ck, b.A, e, rot); });
 }
 
-// rot: the batch's last element move left its stress/strain rotation to this kernel
+// rot: the batch's last element move left its stress/strain rotation to this kernel.
+// chk: its first workgroups check the thermal borders of all models (`border` entries),
+// as k_rheol1's do: the check's launch took 9.4 us of a step of 12 FP64 models.
+// FP32 arithmetic: three waves per SIMD (168 VGPRs, with a few spills) where a model alone
+// takes two: 24 models of 100-600 x 40-150 cells keep them all busy, 197 -> 191 us a step;
+// 1000x250 cells alone lost 1.4 of 69 us that way.
 template <bool SHEARH, int M>
-__global__ void __launch_bounds__(256) kb_rheol(const BatchEntry *__restrict__ tab, BatchMap map, int avgsr,
-                                                int rot)
+__global__ void __launch_bounds__(256, M == 1 ? 3 : 2)
+kb_rheol(const BatchEntry *__restrict__ tab, BatchMap map, int avgsr, int rot, int chk, long border, int arp)
 {
+    if (M != 1 && blockIdx.x < (unsigned)chk) {
+        const long g = (long)blockIdx.x * blockDim.x;
+        if (g >= border) return;
+        const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_BORD][g / BATCH_ALIGN]));
+        const long t = g + threadIdx.x - b.pb;
+        if (t < b.cb) therm_check_one(b.P, b.ck, bthermal(b), b.tg, t, 0, arp, bslots(b));
+        return;
+    }
     __shared__ RheolPhases phs;
-    const long g0 = (long)xcd_block() * blockDim.x;
+    const long g0 = (long)xcd_block((unsigned)chk) * blockDim.x;
     const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_ELEM][g0 / BATCH_ALIGN]));
     const long e = g0 + threadIdx.x - b.pe;
     rheol_single<SHEARH, typename Prec<M>::SV, typename Prec<M>::AT>(

@@ -2653,6 +2653,7 @@ static int enq_batch_flac(gf_batch *b)
     b->pend_ops = 0;
     const bool dis = p.ishearh == 1 && p.itherm != 2;
     const int npass = b->m[0]->therm_passes, arp = b->area_pending ? 1 : 0;
+    unsigned chk = 0;  // workgroups of kb_rheol's launch that check the thermal borders
     if (!b->m[0]->therm_proof) {
         BLAUNCH((dis ? kb_therm_pipe<true> : kb_therm_pipe<false>), b->therm_grid, TH_J * TH_I, b->dtab, map, b->tot_t,
                 GF_THERM_STOL, arp, b->fold ? 1 : 0);
@@ -2665,9 +2666,16 @@ static int enq_batch_flac(gf_batch *b)
             BLAUNCH((dis ? kb_therm_strip<true, 2> : kb_therm_strip<false, 2>), grid, 64, b->dtab, map, total, arp);
         else
             BLAUNCH((dis ? kb_therm_strip<true, 0> : kb_therm_strip<false, 0>), grid, 64, b->dtab, map, total, arp);
-        BLAUNCH(kb_therm_check, bgrid(b->tot_b, 256), 256, b->dtab, map, arp);
-        BLAUNCH((dis ? kb_therm_rest<true> : kb_therm_rest<false>), b->therm_grid, 256, b->dtab, map, total, b->tot_b,
-                arp, npass);
+        // (as enq_flac's: the check may go with kb_rheol, the rest then follows it)
+        bool defer = !b->no_mech && !rm && b->nloop % p.ifreq_visc != 0 && p.ishearh != 1;
+        for (const gf_ctx *c : b->m) defer = defer && c->p.istress_therm == 0;
+        if (defer) {
+            chk = (bgrid(b->tot_b, b->bs[0]) + 7) / 8 * 8;
+        } else {
+            BLAUNCH(kb_therm_check, bgrid(b->tot_b, 256), 256, b->dtab, map, arp);
+            BLAUNCH((dis ? kb_therm_rest<true> : kb_therm_rest<false>), b->therm_grid, 256, b->dtab, map, total,
+                    b->tot_b, arp, npass);
+        }
     }
     b->temp0_prev = true;
     if (!b->no_mech) {
@@ -2684,7 +2692,9 @@ static int enq_batch_flac(gf_batch *b)
         }
         const int rot = (b->rot_pending ? RH_ROT : 0) | (b->area_pending ? RH_AREA : 0);
         if (do_visc) BLAUNCH(kb_visc<M>, bgrid(b->tot_e, 256), 256, b->dtab, map, (rot & RH_ROT) ? 1 : 0);
-        BTIMED(0, BLAUNCH((kb_rheol<SH, M>), bgrid(b->tot_e, b->bs[0]), b->bs[0], b->dtab, map, avgsr, rot));
+        BTIMED(0, BLAUNCH((kb_rheol<SH, M>), chk + bgrid(b->tot_e, b->bs[0]), b->bs[0], b->dtab, map, avgsr, rot,
+                          (int)chk, b->tot_b, arp));
+        if (chk) BLAUNCH(kb_therm_rest<false>, b->therm_grid, 256, b->dtab, map, (int)b->tot_t, b->tot_b, arp, npass);
         b->rot_pending = false;
         b->area_pending = false;
         if (avgsr == 1) {

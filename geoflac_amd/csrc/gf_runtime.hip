@@ -1630,13 +1630,15 @@ static int enq_flac(gf_ctx *ctx, int pending = 0, bool last = true)
         if (phases && (rc = enq_change_phase(ctx))) return rc;
         if ((rc = enq_rheol(ctx, true, last))) return rc;
         // fl_node's launch also ends the thermal call where it reads no temperature that a
-        // further pass could still change (the Winkler support reads the bottom row's), on
+        // further pass could still change (the Winkler support reads the bottom row's), and
+        // nothing before it does (the hydrostatic side walls' densities), on
         // meshes whose tiles are all resident at once: a step 33.1 -> 31.4 us at 400x100
-        // cells, 35.7 -> 34.1 at 60x20, 44.0 -> 42.3 at 151x47.  Where they are not, the
+        // cells, 35.7 -> 34.1 at 60x20.  Where they are not, the
         // registers of the further passes cost fl_node waves: 0.6 us more at 901x301, 1 us at
         // 1200x500 with FP32 storage (3 us less at 2000x1000).
         const bool with_node = ctx->therm_rest && !ctx->node_direct && ctx->p.movegrid != 0 && ctx->in_batch == 0 &&
-                               (ctx->p.nyhydro <= 0 || ctx->p.itemp_bc == 1) && node_tiles(ctx) <= 3L * ctx->therm_grid;
+                               (ctx->p.nyhydro <= 0 || ctx->p.itemp_bc == 1) &&
+                               !(ctx->p.nystressbc == 1 && ctx->p.nydrsides == 1) && node_tiles(ctx) <= 3L * ctx->therm_grid;
         if (defer && (rc = enq_therm_rest(ctx, with_node))) return rc;
         if (ctx->p.nystressbc == 1 && (rc = enq_bc_update(ctx))) return rc;
         const bool rm = phases, im = ctx->nloop % ctx->p.ifreq_imasses == 0;

@@ -15,12 +15,17 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 # 64 x 4 nodes a tile, at most 768: 3071 x 63 cells have 768 tiles, 3075 x 63 have 769
 @pytest.mark.gpu
 @pytest.mark.parametrize("nelx,nelz,option,extra", [
-    (200, 40, "", True), (200, 40, "flux", True), (3071, 63, "", False), (3075, 63, "", False), (40, 12, "flux", False)])
+    (200, 40, "", True), (200, 40, "flux", True), (3071, 63, "", False), (3075, 63, "", False), (40, 12, "flux", False),
+    (200, 40, "sides", True)])
 def test_thermal_end_with_the_node_update(nelx, nelz, option, extra):
     from tests import oracle_lib as ol
     p = sweep.variant(inp.read_inp(os.path.join(HERE, "golden", "inputs", "box60x20.inp")), nelx, nelz)
     if option == "flux":
         p["itemp_bc"], p["bot_bc"] = 2, 0.03
+    if option == "sides":  # hydrostatic side walls, whose densities read the step's temperature
+        p["nystressbc"], p["nydrsides"] = 1, 1
+        p["bcs"] = [b for b in p["bcs"] if b["nofside"] in (1, 3)]
+        p["nofbc"] = len(p["bcs"])
     print("case: %dx%d elements, %s" % (nelx, nelz, option or "plain"), flush=True)
     gp, st, m = sweep.make_model(p, abi.PREC_FP64)
     with m:

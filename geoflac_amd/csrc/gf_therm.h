@@ -15,9 +15,9 @@
 // and 150 others (lane shifts among them) a column; the latency of that chain, 1.3 us a
 // column, where a SIMD holds one wave.  The tiles it replaced (64 x 16 nodes in LDS, a
 // workgroup barrier per application, 58% of the nodes evaluated in halos) waited on LDS
-// and barriers; their thermal step took 137 us on 2001x1001 nodes, this one 95, and on
-// square cells (902x302 nodes), where their four halo columns needed a second pass in
-// every step, 125 us against 30.
+// and barriers; their thermal step took 137 us on 2001x1001 nodes, the strips take 68 (and 6
+// for the rest of the call), and on square cells (902x302 nodes), where their four halo
+// columns needed a second pass in every step, 125 us against 27.
 //
 // Strips: rows are cut into strips of 64 lanes that overlap by 2 * TS_HB rows (none at
 // the mesh's top and bottom), columns into strips of `w` output columns that start

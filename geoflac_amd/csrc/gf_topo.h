@@ -18,7 +18,7 @@
 //                 increasing i, so each chunk of elements takes the new markers' numbers
 //                 from a prefix sum.  The elements it changed are stamped for the
 //                 recount that count_phase_ratio does there (k_phase_plan,
-//                 k_phase_replane, k_phase_recount without the plastic-strain share).
+//                 k_phase_update without the plastic-strain share).
 #pragma once
 #include "gf_phase.h"
 

@@ -43,3 +43,63 @@ def test_thermal_end_with_the_node_update(nelx, nelz, option, extra):
     assert stats[0] == 0
     assert not extra or stats[1] > 0
     assert not diff
+
+
+def _variant(nelx, nelz):
+    return sweep.variant(inp.read_inp(os.path.join(HERE, "golden", "inputs", "box60x20.inp")), nelx, nelz)
+
+
+@pytest.mark.gpu
+def test_further_passes_inside_the_node_launch():
+    """An upload forgets the thermal history, so that the step after it, not a multiple of
+    ifreq_visc, needs a further pass, which fl_node's launch then runs."""
+    from tests import oracle_lib as ol
+    print("case: 200x40 elements, upload after 3 steps", flush=True)
+    gp, st, m = sweep.make_model(_variant(200, 40), abi.PREC_FP64)
+    with m:
+        m.download()
+        ref = st.copy()
+        m.step(3)
+        m.download()
+        m.upload()
+        m.therm_stats()
+        m.step(4)
+        stats = m.therm_stats()
+        m.download()
+    assert ol.step(gp, ref, 7, cr=True) == 0
+    diff = [f for f in state.State.FIELDS if not np.array_equal(getattr(st, f), getattr(ref, f))]
+    assert stats[0] == 0 and stats[1] > 0
+    assert not diff
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("meshes", [[(200, 40), (60, 20), (37, 70)], [(200, 40), (230, 75), (240, 80), (60, 20)]])
+def test_further_passes_inside_a_batch(meshes):
+    """The same in a batch, after its element update's launch checked the borders; each
+    model against itself alone."""
+    print("case: batch of %s, upload after 3 steps" % meshes, flush=True)
+    alone = []
+    for nelx, nelz in meshes:
+        gp, st, m = sweep.make_model(_variant(nelx, nelz), abi.PREC_FP64)
+        with m:
+            m.step(17)
+            m.download()
+        alone.append(st)
+    made = [sweep.make_model(_variant(nelx, nelz), abi.PREC_FP64) for nelx, nelz in meshes]
+    models = [x[2] for x in made]
+    b = sweep.Batch(models)
+    b.step(3)
+    b.close()
+    for m in models:
+        m.download()
+        m.upload()
+        m.therm_stats()
+    b = sweep.Batch(models)
+    b.step(14)
+    b.close()
+    extra = sum(m.therm_stats()[1] for m in models)
+    for (gp, st, m), ref in zip(made, alone):
+        m.download()
+        assert not [f for f in state.State.FIELDS if not np.array_equal(getattr(st, f), getattr(ref, f))]
+        m.close()
+    assert extra > 0

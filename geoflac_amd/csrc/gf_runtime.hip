@@ -2758,8 +2758,8 @@ static int batch_pointers(gf_batch *b)
         e.A = c->a;
         e.A.tbord = tbord;
         e.tprev = c->a.xa;
-        e.cord_next = c->cord_alt;
-        if (batch_turns_cord(b)) std::swap(e.A.cord, e.cord_next);
+        e.cord_next = c->a.cord;  // (what bmoved reads: the coordinates in force where none turn)
+        if (batch_turns_cord(b)) e.A.cord = c->cord_alt;
         same = same && memcmp(&e, &b->tab[k], sizeof e) == 0;
         mine = mine && c->therm_batch == b;
         c->therm_batch = b;
@@ -2787,8 +2787,10 @@ static void batch_turn(gf_batch *b, int32_t steps)
         c->a.temp = e.A.temp;
         c->a.temp0 = e.A.temp0;
         c->a.xa = e.tprev;
-        c->a.cord = cord ? e.cord_next : e.A.cord;
-        c->cord_alt = cord ? e.A.cord : e.cord_next;
+        if (cord) {
+            c->a.cord = e.cord_next;
+            c->cord_alt = e.A.cord;
+        }
         e.A.xa = c->a.xa;  // (as batch_pointers finds it; the kernels use the names above)
     }
     b->tab_valid = true;

@@ -105,6 +105,7 @@ __global__ void kb_begin(BatchEntry *tab, BatchMap map, int op, int cord)
     clock_op(b.ck, op);
     b.ck->th_call = (b.ck->th_call + 1) % 3;
     b.ck->th_hist = min(b.ck->th_hist + 1, 3);
+    b.ck->q_next = b.ck->q_done = 0u;  // (kb_therm_rest)
     double *t = b.tprev;
     b.tprev = b.A.temp0;
     b.A.temp0 = b.A.temp;
@@ -158,8 +159,12 @@ __global__ void __launch_bounds__(256) kb_therm_check(const BatchEntry *__restri
     });
 }
 // Returns at once when every model's pass 0 is proven.  Otherwise the further passes of
-// the models that are not, with grid barriers on the first model's counters (one workgroup
-// per CU at most, as k_therm_rest).
+// the models that are not, in phases of gridDim.x units (queue_take on the first model's
+// counters): phase 2 (p - 1) runs the strips of pass p, phase 2 p - 1 checks its borders,
+// and the phase after the last pass that anyone needs settles the results.  Several batches
+// may run at once, on streams of their own: none needs all its workgroups resident, as grid
+// barriers would.  (Nor is it slower: 12 models of 200-360 x 34-60 cells of 25-50 m, some
+// with a further pass in nearly every step, take 203 us a step, with grid barriers 241.)
 template <bool DIS>
 __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restrict__ tab, BatchMap map, int total,
                                                      long border, int arp, int npass)
@@ -176,38 +181,56 @@ __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restric
     if (!open_after(0)) return;
     __shared__ double sPhw[4][4][GF_MAXPH];
     double(*sPh)[GF_MAXPH] = sPhw[threadIdx.x / 64];
-    GfDevClock *bar = tab[0].ck;
-    const long tid = (long)blockIdx.x * 256 + threadIdx.x, nthr = (long)gridDim.x * 256;
-    for (int pass = 1; pass < npass; pass++) {
-        for (int g = (int)(tid / 64); g < total; g += (int)(nthr / 64)) {
-            const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_TILE][g]));
-            if (__hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
-                continue;
-            const GfDevArrays A = bthermal(b);
-            therm_phase_table(b.P, sPh);
-            const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, arp, pass};
-            const int t = g - (int)b.pt;
-            therm_strip<DIS, 1>(b.P, b.ck, A, b.tg, t, it, bslots(b), A.tbord + (long)t * TS_NB(b.tg.w),
-                                b.ck->dt, sPh);
+    GfDevClock *queue = tab[0].ck;
+    const unsigned units = gridDim.x;
+    const long nthr = (long)units * 256;
+    for (;;) {
+        const unsigned unit = queue_take(queue), phase = unit / units;
+        const long tid = (long)(unit % units) * 256 + threadIdx.x;
+        if (phase > 2u * (unsigned)(npass - 1)) return;
+        if (!queue_wait(queue, phase * units)) {  // (not expected; no model's result is known then)
+            for (int m = threadIdx.x; m < map.nm; m += 256)
+                __hip_atomic_fetch_or(&tab[m].ck->bar_timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
         }
-        if (!grid_sync(bar, gridDim.x)) return;  // every strip's iterate is written
-        for (long g = (long)blockIdx.x * 256; g < border; g += nthr) {
-            const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_BORD][g / BATCH_ALIGN]));
-            const long t = g + threadIdx.x - b.pb;
-            if (t < b.cb &&
-                __hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)
-                therm_check_one(b.P, b.ck, bthermal(b), b.tg, t, pass, arp, bslots(b));
+        // passes 1 .. checked are checked; last: the one that ended the call, if one has
+        const int checked = (int)(phase / 2u), pass = checked + 1;
+        int last = -1;
+        for (int k = 1; k <= checked && last < 0; k++)
+            if (!open_after(k)) last = k;
+        if (last < 0 && checked == npass - 1) last = checked;
+        if (last >= 0) {
+            if (phase != 2u * (unsigned)last) return;  // (settled)
+            for (int m = 0; m < map.nm; m++) {
+                if (flag(m, 0) == 0u) continue;
+                int proven = -1;
+                for (int k = npass - 1; k >= 0; k--)
+                    if (flag(m, k) == 0u) proven = k;
+                if (tid == 0) therm_outcome(tab[m].ck, proven);
+                therm_settle(tab[m].P, bthermal(tab[m]), bslots(tab[m]), proven < 0 ? npass - 1 : proven, tid, nthr);
+            }
+        } else if (phase % 2u == 0u) {
+            for (int g = (int)(tid / 64); g < total; g += (int)(nthr / 64)) {
+                const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_TILE][g]));
+                if (__hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
+                    continue;
+                const GfDevArrays A = bthermal(b);
+                therm_phase_table(b.P, sPh);
+                const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, arp, pass};
+                const int t = g - (int)b.pt;
+                therm_strip<DIS, 1>(b.P, b.ck, A, b.tg, t, it, bslots(b), A.tbord + (long)t * TS_NB(b.tg.w),
+                                    b.ck->dt, sPh);
+            }
+        } else {
+            for (long g = tid - threadIdx.x; g < border; g += nthr) {
+                const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_BORD][g / BATCH_ALIGN]));
+                const long t = g + threadIdx.x - b.pb;
+                if (t < b.cb &&
+                    __hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)
+                    therm_check_one(b.P, b.ck, bthermal(b), b.tg, t, pass, arp, bslots(b));
+            }
         }
-        if (!grid_sync(bar, gridDim.x)) return;  // every border is checked
-        if (!open_after(pass)) break;
-    }
-    for (int m = 0; m < map.nm; m++) {
-        if (flag(m, 0) == 0u) continue;
-        int proven = -1;
-        for (int k = npass - 1; k >= 0; k--)
-            if (flag(m, k) == 0u) proven = k;
-        if (tid == 0) therm_outcome(tab[m].ck, proven);
-        therm_settle(tab[m].P, bthermal(tab[m]), bslots(tab[m]), proven < 0 ? npass - 1 : proven, tid, nthr);
+        queue_done(queue);
     }
 }
 

@@ -89,6 +89,7 @@ struct GfDevClock {
     // itest_mesh's smallest triangle angle, as an order-preserving key (rem_angle_key)
     unsigned long long rem_key;
     unsigned int out_cnt, out_pad;  // workgroups of a launch that ends with clock_out and are done
+    unsigned int q_next, q_done;    // units of a launch's phases handed out and done (queue_take)
 };
 
 // ---------------------------------------------------------------- buffer access

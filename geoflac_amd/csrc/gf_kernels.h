@@ -822,6 +822,48 @@ GF_DEV bool grid_sync(GfDevClock *ck, unsigned nblocks)
     return s_ok != 0;
 }
 
+// Phases of work in one launch whose workgroups need not all be resident: each phase is
+// cut into units, which the workgroups take in order, one after the other, until none is
+// left; a unit starts once all those of the phases before it are done (queue_wait).  What a
+// workgroup waits for was taken by workgroups that run already, and those of the earliest
+// open phase wait for nothing, so every wait ends whatever else holds the CUs.  (q_next and
+// q_done start at 0: an earlier launch clears them.  The wait is bounded all the same.)
+GF_DEV unsigned queue_take(GfDevClock *ck)
+{
+    __shared__ unsigned s_unit;
+    __syncthreads();  // (the unit before is read)
+    if (threadIdx.x == 0) s_unit = __hip_atomic_fetch_add(&ck->q_next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    return (unsigned)__builtin_amdgcn_readfirstlane((int)s_unit);
+}
+GF_DEV bool queue_wait(GfDevClock *ck, unsigned before)
+{
+    __shared__ int s_ok;
+    if (threadIdx.x == 0) {
+        int ok = 1, spin = 0;
+        while (__hip_atomic_load(&ck->q_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < before) {
+            if (++spin > GF_BAR_SPIN) {
+                ok = 0;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(2);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        s_ok = ok;
+    }
+    __syncthreads();
+    return s_ok != 0;
+}
+GF_DEV void queue_done(GfDevClock *ck)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __hip_atomic_fetch_add(&ck->q_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 #include "gf_therm.h"
 
 // ------------------------------------------------------------------ material properties

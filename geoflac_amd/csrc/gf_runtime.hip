@@ -2449,6 +2449,7 @@ struct gf_batch {
     int therm_w = 2;      // output columns of a strip
     bool fold = true;     // FP32-arithmetic mode: the tiles apply the boundary conditions
     unsigned therm_grid = 8;  // workgroups of the thermal kernels with one per CU
+    unsigned rest_grid = 8;   // ... of kb_therm_rest: fewer where there are fewer strips than waves
     BatchMap map{};
     int nm = 0;
     long tot_e = 0, tot_n = 0, tot_t = 0, tot_b = 0, tot_m = 0;
@@ -2576,6 +2577,7 @@ extern "C" int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out)
     for (gf_ctx *c : b->m) b->temp0_prev = b->temp0_prev && c->temp0_prev;
     b->noguess = c0->therm_noguess;
     b->therm_grid = c0->therm_grid;
+    b->rest_grid = (unsigned)std::min<long>(b->therm_grid, (pt + 31) / 32 * 8);
     const size_t nmap = me.size() + mn.size() + mt.size() + mb.size() + mm.size() + 1;
     if (hipMalloc((void **)&b->dmap, sizeof(int) * nmap) != hipSuccess) return fail(GF_ERR_HIP, "allocation");
     {
@@ -2675,7 +2677,7 @@ static int enq_batch_flac(gf_batch *b)
             chk = (bgrid(b->tot_b, b->bs[0]) + 7) / 8 * 8;
         } else {
             BLAUNCH(kb_therm_check, bgrid(b->tot_b, 256), 256, b->dtab, map, arp);
-            BLAUNCH((dis ? kb_therm_rest<true> : kb_therm_rest<false>), b->therm_grid, 256, b->dtab, map, total,
+            BLAUNCH((dis ? kb_therm_rest<true> : kb_therm_rest<false>), b->rest_grid, 256, b->dtab, map, total,
                     b->tot_b, arp, npass);
         }
     }
@@ -2696,7 +2698,7 @@ static int enq_batch_flac(gf_batch *b)
         if (do_visc) BLAUNCH(kb_visc<M>, bgrid(b->tot_e, 256), 256, b->dtab, map, (rot & RH_ROT) ? 1 : 0);
         BTIMED(0, BLAUNCH((kb_rheol<SH, M>), chk + bgrid(b->tot_e, b->bs[0]), b->bs[0], b->dtab, map, avgsr, rot,
                           (int)chk, b->tot_b, arp));
-        if (chk) BLAUNCH(kb_therm_rest<false>, b->therm_grid, 256, b->dtab, map, (int)b->tot_t, b->tot_b, arp, npass);
+        if (chk) BLAUNCH(kb_therm_rest<false>, b->rest_grid, 256, b->dtab, map, (int)b->tot_t, b->tot_b, arp, npass);
         b->rot_pending = false;
         b->area_pending = false;
         if (avgsr == 1) {

@@ -28,7 +28,8 @@
 #pragma once
 
 #define TS_HB 6                  // rows of a strip above and below its output rows: one ring row, five halo rows
-#define TS_HI_MAX 8              // most halo columns left of its output columns (after one ring column)
+#define TS_HI_MAX 12             // most halo columns left of its output columns (after one ring column)
+#define TS_HI_FEW 8              // ... where more would not be enough either
 #define TS_OJ (64 - 2 * TS_HB)   // output rows of an inner strip
 #define TS_SWEEP0 2              // applications before the first stillness test
 #define TS_MAXSWEEP 48
@@ -77,17 +78,23 @@ __host__ __device__ inline ThermGeo therm_geo(int nz, int nx, int w)
     return g;
 }
 // Halo columns of a strip: each damps what the ring's start leaves by the coupling of
-// columns c = diff dt / dx^2, and that error is some 1e-5 of a value's change (rows 1 and
-// nz, whose start follows the last two calls).  Enough of them that c^hi <= 1e-11 (at
-// least 2): at c = 1.3e-2 (901x301 cells of 333 m) 4, 5 and 6 columns need a further pass
-// in 45%, 2% and none of the steps; more columns only cost their own time, and what a
-// strip leaves unsettled the border check finds.
+// columns c = diff dt / dx^2.  That error is some 1e-5 of a value's change (rows 1 and nz,
+// whose start follows the last two calls), and grows as c^2 itself, the second difference in
+// time that the extrapolated start leaves out.  Enough of them that c^hi <= 1e-11 and
+// c^(hi + 2) <= 1e-15 (at least 2): at c = 1.3e-2 (901x301 cells of 333 m) 4, 5 and 6 columns
+// need a further pass in 45%, 2% and none of the steps.  The second bound tells from c = 1e-2
+// on: at c = 3e-2 to 6e-2 (200-360 x 34-60 cells of 25-45 m) the first one's 8 or fewer need
+// one in 3-100% of the steps, its 9 to 11 in 0-12%.  Where TS_HI_MAX are not enough (c > 8.5e-2)
+// further passes run in every step anyway, and TS_HI_FEW cost less: 131x70 cells at c = 0.11
+// take 127 us a step with 8, 150 with 12.  What a strip leaves unsettled the border check
+// finds.
 __host__ __device__ inline int therm_halo(double diff_max, double rxbo, int nx, double dt)
 {
     const double dx = rxbo / (double)(nx - 1), c = diff_max * dt / (dx * dx);
-    int hi = 2;
-    for (double v = c * c; v > 1.0e-11 && hi < TS_HI_MAX; v *= c) hi++;
-    return hi;
+    double v = c * c;
+    for (int hi = 2; hi <= TS_HI_MAX; hi++, v *= c)
+        if (v <= 1.0e-11 && v * c * c <= 1.0e-15) return hi;
+    return TS_HI_FEW;
 }
 struct ThermStrip {
     int jb, fo, lo, c0, c1;

@@ -159,12 +159,8 @@ __global__ void __launch_bounds__(256) kb_therm_check(const BatchEntry *__restri
     });
 }
 // Returns at once when every model's pass 0 is proven.  Otherwise the further passes of
-// the models that are not, in phases of gridDim.x units (queue_take on the first model's
-// counters): phase 2 (p - 1) runs the strips of pass p, phase 2 p - 1 checks its borders,
-// and the phase after the last pass that anyone needs settles the results.  Several batches
-// may run at once, on streams of their own: none needs all its workgroups resident, as grid
-// barriers would.  (Nor is it slower: 12 models of 200-360 x 34-60 cells of 25-50 m, some
-// with a further pass in nearly every step, take 203 us a step, with grid barriers 241.)
+// the models that are not, in the phases of k_therm_rest over the strips and borders of all
+// of them (queue_take on the first model's counters).
 template <bool DIS>
 __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restrict__ tab, BatchMap map, int total,
                                                      long border, int arp, int npass)
@@ -190,15 +186,10 @@ __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restric
         if (phase > 2u * (unsigned)(npass - 1)) return;
         if (!queue_wait(queue, phase * units)) {  // (not expected; no model's result is known then)
             for (int m = threadIdx.x; m < map.nm; m += 256)
-                __hip_atomic_fetch_or(&tab[m].ck->bar_timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_or(&tab[m].ck->q_timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return;
         }
-        // passes 1 .. checked are checked; last: the one that ended the call, if one has
-        const int checked = (int)(phase / 2u), pass = checked + 1;
-        int last = -1;
-        for (int k = 1; k <= checked && last < 0; k++)
-            if (!open_after(k)) last = k;
-        if (last < 0 && checked == npass - 1) last = checked;
+        const int checked = (int)(phase / 2u), pass = checked + 1, last = therm_last_pass(checked, npass, open_after);
         if (last >= 0) {
             if (phase != 2u * (unsigned)last) return;  // (settled)
             for (int m = 0; m < map.nm; m++) {

@@ -76,10 +76,9 @@ struct GfDevClock {
     int ph_nz[GF_MAXACT];       // elements with a nonzero ratio, per plane
     int ph_count[GF_MAXPH];     // elements whose iphase is id-1 (the dt_mass minima run over ids present)
     int nmarkers, mk_pad;       // markers in use (resurface appends)
-    // grid barrier of the thermal step's fallback passes: arrivals, generation, a
-    // bounded wait that ran out
-    unsigned int bar_cnt, bar_gen;
-    int bar_timeout, bar_pad;
+    // units of a launch's phases handed out and done (queue_take); a wait that ran out
+    unsigned int q_next, q_done;
+    int q_timeout, q_pad;
     // dt_mass's minimum side measure as the largest product area x side length over
     // the elements (bits of a non-negative double); dlmin is its reciprocal
     unsigned long long dly_bits;
@@ -89,7 +88,6 @@ struct GfDevClock {
     // itest_mesh's smallest triangle angle, as an order-preserving key (rem_angle_key)
     unsigned long long rem_key;
     unsigned int out_cnt, out_pad;  // workgroups of a launch that ends with clock_out and are done
-    unsigned int q_next, q_done;    // units of a launch's phases handed out and done (queue_take)
 };
 
 // ---------------------------------------------------------------- buffer access

@@ -783,51 +783,16 @@ __global__ void __launch_bounds__(256) k_therm_bc(const GfDevParams *__restrict_
     therm_bc_node(P, A, (long)blockIdx.x * 256 + threadIdx.x);
 }
 
-// Grid-wide barrier of a launch whose workgroups are all resident.  Every wave
-// waits for its own memory operations; thread 0 then publishes the workgroup's writes
-// (agent-scope release), counts in, waits for the last workgroup to bump the
-// generation, and acquires.  The wait is bounded: a workgroup that polls GF_BAR_SPIN
-// times raises bar_timeout and returns false, so the launch always ends (the host
-// then reports the call as failed).
-#define GF_BAR_SPIN (1 << 22)
-GF_DEV bool grid_sync(GfDevClock *ck, unsigned nblocks)
-{
-    __shared__ int s_ok;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int ok = 1;
-        const unsigned g0 = __hip_atomic_load(&ck->bar_gen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const unsigned arrived =
-            __hip_atomic_fetch_add(&ck->bar_cnt, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-        if (arrived == nblocks) {
-            __hip_atomic_store(&ck->bar_cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(&ck->bar_gen, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            int spin = 0;
-            while (__hip_atomic_load(&ck->bar_gen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == g0) {
-                if (++spin > GF_BAR_SPIN) {
-                    ok = 0;
-                    __hip_atomic_fetch_or(&ck->bar_timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(2);
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        s_ok = ok;
-    }
-    __syncthreads();
-    return s_ok != 0;
-}
-
 // Phases of work in one launch whose workgroups need not all be resident: each phase is
 // cut into units, which the workgroups take in order, one after the other, until none is
 // left; a unit starts once all those of the phases before it are done (queue_wait).  What a
 // workgroup waits for was taken by workgroups that run already, and those of the earliest
-// open phase wait for nothing, so every wait ends whatever else holds the CUs.  (q_next and
-// q_done start at 0: an earlier launch clears them.  The wait is bounded all the same.)
+// open phase wait for nothing, so every wait ends whatever else holds the CUs.  Every wave
+// waits for its own memory operations before a unit counts as done, whose writes thread 0
+// then publishes (agent-scope release); the waiting side acquires.  (q_next and q_done start
+// at 0: an earlier launch clears them.  The wait is bounded all the same: a workgroup that
+// polls GF_WAIT_SPIN times gives up, and its kernel raises q_timeout.)
+#define GF_WAIT_SPIN (1 << 22)
 GF_DEV unsigned queue_take(GfDevClock *ck)
 {
     __shared__ unsigned s_unit;
@@ -842,7 +807,7 @@ GF_DEV bool queue_wait(GfDevClock *ck, unsigned before)
     if (threadIdx.x == 0) {
         int ok = 1, spin = 0;
         while (__hip_atomic_load(&ck->q_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < before) {
-            if (++spin > GF_BAR_SPIN) {
+            if (++spin > GF_WAIT_SPIN) {
                 ok = 0;
                 break;
             }
@@ -2423,8 +2388,7 @@ __global__ void __launch_bounds__(256) k_node_t(const GfDevParams *__restrict__ 
 }
 // ... with the end of the step's thermal call (k_therm_rest) in its first workgroups, which
 // find pass 0 proven in nearly every step and return: a launch of its own takes 3 us for
-// that answer.  They are the launch's first, so all of them are resident when they need
-// their barriers.  (At 128 VGPRs, four workgroups per CU, a further pass spills.)
+// that answer.  (At 128 VGPRs, four workgroups per CU, a further pass spills.)
 template <int M>
 __global__ void __launch_bounds__(256, 4) k_node_rest(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
                                                       double *cord_out, int ops, ThermRest R)
@@ -2439,7 +2403,7 @@ __global__ void __launch_bounds__(256, 4) k_node_rest(const GfDevParams *__restr
     B.temp = A.temp0;
     B.xa = A.temp;
     B.temp0 = A.xa;
-    therm_rest_body<false>(P, ck, B, R, blockIdx.x);
+    therm_rest_body<false>(P, ck, B, R);
 }
 
 // ------------------------------------------------------------------ fl_move

@@ -97,8 +97,7 @@ struct gf_ctx {
     int therm_passes = TH_MAXPASS;
     bool therm_proof = true;  // false: FP32-arithmetic mode, the single pass is not proven
     // the thermal step's further passes as one launch (k_therm_rest) instead of a launch
-    // per pass and check (GF_THERM=multi, or a device on which a workgroup of it does not
-    // fit on every CU)
+    // per pass and check (GF_THERM=multi)
     bool therm_rest = false;
     int therm_w = 0;     // output columns of a thermal strip
     bool therm_cols = false;  // pass 0 by a workgroup a strip (k_therm_cols)
@@ -332,15 +331,12 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
             goto fail;
         }
         ctx->therm_grid = (unsigned)std::max(8, ncu / 8 * 8);
-        int nb = 0;
         const char *tm = getenv("GF_THERM");
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_therm_rest<true>, 256, 0) != hipSuccess) nb = 0;
-        ctx->therm_rest = nb >= 1 && ncu >= 8 && !(tm && strcmp(tm, "multi") == 0);
+        ctx->therm_rest = !(tm && strcmp(tm, "multi") == 0);
         // a workgroup a strip where every strip then has a CU of its own
         const ThermGeo gc = therm_geo(p->nz, p->nx, TC_W - 1 - TC_HI);
         ctx->therm_cols = gc.nr * gc.ns <= ncu;
         ctx->therm_w = ctx->therm_cols ? gc.w : therm_strip_width({p});
-        (void)hipGetLastError();
     }
     ALLOC(ctx->dp, sizeof(GfDevParams));
     ALLOC(ctx->dck, sizeof(GfDevClock));
@@ -1056,12 +1052,12 @@ static int read_clock(gf_ctx *ctx, gf_clock *c)
     const GfDevClock ck = ctx->hout->ck;
     ctx->dt_seen = ck.dt;
     if (ctx->markers_uploaded && ctx->p.topo_kappa > 0.0) ctx->a.nmarkers = ck.nmarkers;  // (resurface appends)
-    if (ck.bar_timeout != 0) {  // (not expected: every workgroup of the launch is resident)
+    if (ck.q_timeout != 0) {  // (not expected, queue_take)
         GfDevClock z = ck;
-        z.bar_cnt = 0;
-        z.bar_timeout = 0;
+        z.q_timeout = 0;
         HIPCHK(hipMemcpy(ctx->dck, &z, sizeof(z), hipMemcpyHostToDevice));
-        return set_err(ctx, GF_ERR_HIP, "the thermal step's grid barrier timed out: the results of this call are invalid");
+        return set_err(ctx, GF_ERR_HIP,
+                       "a wait between the thermal step's passes timed out: the results of this call are invalid");
     }
     if (c) {
         c->nloop = ctx->nloop; c->nsrate = ctx->nsrate;
@@ -1262,13 +1258,7 @@ static int enq_therm_rest(gf_ctx *ctx, bool with_node)
         const ThermGeo g = ctx->chk.g;
         const ThermSlots sl = ctx->chk.sl;
         if (ctx->therm_rest) {
-            // A plain launch: its grid (one workgroup per CU, at most the CUs) is resident
-            // once the kernels before it on this stream are done, unless other streams hold
-            // CUs, whose kernels then finish first.  The grid barriers of the further passes
-            // wait boundedly, so a launch that is not resident reports an error instead of
-            // waiting for ever.  (A cooperative launch guarantees residency but costs
-            // ~16 us more per launch on MI355X, more than the launches it replaces.)
-            // Fewer where there are fewer strips than waves.
+            // At most one workgroup per CU, fewer where there are fewer strips than waves.
             ctx->rest = ThermRest{(int)std::min<long>(ctx->therm_grid, ((long)g.nr * g.ns + 31) / 32 * 8), arp, npass, g, sl};
             if (!with_node) {
                 auto rest = dis ? k_therm_rest<true> : k_therm_rest<false>;

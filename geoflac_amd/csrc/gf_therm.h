@@ -53,9 +53,11 @@ __host__ __device__ inline ThermSlots therm_slots(int call, int hist, int set = 
     const int c = call % 3;
     return ThermSlots{c, (c + 2) % 3, (c + 1) % 3, hist, set ? GF_MAX_SWEEPS : 0};
 }
-// the flags of the next call (those of the one before this, whose passes are over)
+// the flags of the next call (those of the one before this, whose passes are over), and the
+// counters of this call's further passes
 GF_DEV void therm_clear_other(GfDevClock *ck, const ThermSlots &sl)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) ck->q_next = ck->q_done = 0u;
     if (blockIdx.x == 0 && threadIdx.x < GF_MAX_SWEEPS)
         ck->therm_pass_changed[(sl.flag ^ GF_MAX_SWEEPS) + threadIdx.x] = 0u;
 }
@@ -744,21 +746,32 @@ GF_DEV void therm_settle(const GfDevParams *__restrict__ P, const GfDevArrays &A
     for (long t = tid; t < 2L * (P->nx + P->nz); t += nthr) to[t] = from[t];
 }
 
-// The rest of the call after pass 0 and its check, in one launch of at most one
-// workgroup per CU.  When pass 0 is proven it returns at once.  Otherwise the further
-// passes run here, each over all strips and followed by its border check, with grid
-// barriers between the phases, until one is proven or npass ran.  The flags that decide
-// another pass are read with coherent loads after a barrier, so every workgroup takes
-// the same decision; flag 0 was written by earlier launches.
+// The rest of the call after pass 0 and its check, in one launch.  When pass 0 is proven it
+// returns at once.  Otherwise the further passes run here in phases of R.grid units each
+// (queue_take): phase 2 (p - 1) runs the strips of pass p, phase 2 p - 1 checks its borders,
+// and the phase after the pass that ends the call settles its result.  The flags that decide
+// another pass are read with coherent loads once the phases before are done, so every unit
+// takes the same decision; flag 0 was written by earlier launches.  No workgroup needs the
+// others resident, so that models and batches may run their passes at the same time, on
+// streams of their own; grid barriers after each phase did, and were slower: 12 models of
+// 200-360 x 34-60 cells in a batch, a further pass in nearly every step, 241 us a step to
+// 203.
 struct ThermRest {
     int grid, arp, npass;
     ThermGeo g;
     ThermSlots sl;
 };
-// (workgroup `block` of R.grid of 256 threads)
+// the pass that ends the call, of passes 1 .. checked: the first that is proven, or the last
+// there may be; -1: another follows
+template <typename Open>
+GF_DEV int therm_last_pass(int checked, int npass, const Open &open_after)
+{
+    for (int k = 1; k <= checked; k++)
+        if (!open_after(k)) return k;
+    return checked == npass - 1 ? checked : -1;
+}
 template <bool DIS>
-GF_DEV void therm_rest_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, const ThermRest &R,
-                            unsigned block)
+GF_DEV void therm_rest_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, const ThermRest &R)
 {
     const ThermSlots sl = R.sl;
     if (ck->therm_pass_changed[sl.flag] == 0u) return;
@@ -767,31 +780,42 @@ GF_DEV void therm_rest_body(const GfDevParams *__restrict__ P, GfDevClock *ck, c
     __shared__ double sPhw[4][4][GF_MAXPH];  // (a table a wave)
     double(*sPh)[GF_MAXPH] = sPhw[threadIdx.x / 64];
     therm_phase_table(P, sPh);
+    auto open_after = [&](int pass) {
+        return __hip_atomic_load(&ck->therm_pass_changed[sl.flag + pass], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
+               0u;
+    };
     const int nt = g.nr * g.ns;
     const long nb = (long)nt * TS_NB(g.w);
-    const long tid = (long)block * 256 + threadIdx.x, nthr = (long)R.grid * 256;
-    int proven = -1, pass = 1;
-    for (; pass < npass; pass++) {
-        const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, R.arp, pass};
-        for (int t = (int)(tid / 64); t < nt; t += (int)(nthr / 64))
-            therm_strip<DIS, 1>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(g.w), ck->dt, sPh);
-        if (!grid_sync(ck, R.grid)) return;  // every strip's iterate is written
-        for (long t = tid; t < nb; t += nthr) therm_check_one(P, ck, A, g, t, pass, R.arp, sl);
-        if (!grid_sync(ck, R.grid)) return;  // every border is checked
-        if (__hip_atomic_load(&ck->therm_pass_changed[sl.flag + pass], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-            0u) {
-            proven = pass;
-            break;
+    const unsigned units = (unsigned)R.grid;
+    const long nthr = (long)units * 256;
+    for (;;) {
+        const unsigned unit = queue_take(ck), phase = unit / units;
+        const long tid = (long)(unit % units) * 256 + threadIdx.x;
+        if (phase > 2u * (unsigned)(npass - 1)) return;
+        if (!queue_wait(ck, phase * units)) {  // (not expected)
+            if (threadIdx.x == 0) __hip_atomic_fetch_or(&ck->q_timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
         }
+        const int checked = (int)(phase / 2u), pass = checked + 1, last = therm_last_pass(checked, npass, open_after);
+        if (last >= 0) {
+            if (phase != 2u * (unsigned)last) return;  // (settled)
+            if (tid == 0) therm_outcome(ck, open_after(last) || last == 0 ? -1 : last);
+            therm_settle(P, A, sl, last, tid, nthr);
+        } else if (phase % 2u == 0u) {
+            const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, R.arp, pass};
+            for (int t = (int)(tid / 64); t < nt; t += (int)(nthr / 64))
+                therm_strip<DIS, 1>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(g.w), ck->dt, sPh);
+        } else {
+            for (long t = tid; t < nb; t += nthr) therm_check_one(P, ck, A, g, t, pass, R.arp, sl);
+        }
+        queue_done(ck);
     }
-    if (tid == 0) therm_outcome(ck, proven);
-    therm_settle(P, A, sl, proven < 0 ? npass - 1 : proven, tid, nthr);
 }
 template <bool DIS>
 __global__ void __launch_bounds__(256) k_therm_rest(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
                                                     ThermRest R)
 {
-    therm_rest_body<DIS>(P, ck, A, R, blockIdx.x);
+    therm_rest_body<DIS>(P, ck, A, R);
 }
 
 // the end of a call whose further passes ran as launches of their own

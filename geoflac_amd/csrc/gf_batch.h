@@ -105,6 +105,7 @@ __global__ void kb_begin(BatchEntry *tab, BatchMap map, int op, int cord)
     clock_op(b.ck, op);
     b.ck->th_call = (b.ck->th_call + 1) % 3;
     b.ck->th_hist = min(b.ck->th_hist + 1, 3);
+    b.ck->th_last = 0;
     b.ck->q_next = b.ck->q_done = 0u;  // (kb_therm_rest)
     double *t = b.tprev;
     b.tprev = b.A.temp0;
@@ -165,16 +166,18 @@ template <bool DIS>
 __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restrict__ tab, BatchMap map, int total,
                                                      long border, int arp, int npass)
 {
-    auto flag = [&](int m, int pass) {  // written by other workgroups of this launch too
-        return __hip_atomic_load(&tab[m].ck->therm_pass_changed[pass], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // of a batch, whose calls all use the first set (bslots)
+    auto flag = [&](GfDevClock *ck, int pass) { return &ck->therm_pass_changed[pass % GF_THERM_FLAGS]; };
+    auto is_open = [&](GfDevClock *ck, int pass) {  // (written by other workgroups of this launch too)
+        return __hip_atomic_load(flag(ck, pass), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
     };
     // whether a model's pass is not proven (nor any before it: later flags stay 0 then)
-    auto open_after = [&](int pass) {
+    auto any_open = [&](int pass) {
         int any = 0;
-        for (int m = threadIdx.x; m < map.nm; m += 256) any |= flag(m, pass) != 0u;
+        for (int m = threadIdx.x; m < map.nm; m += 256) any |= is_open(tab[m].ck, pass);
         return __syncthreads_or(any) != 0;
     };
-    if (!open_after(0)) return;
+    if (!any_open(0)) return;
     __shared__ double sPhw[4][4][GF_MAXPH];
     double(*sPh)[GF_MAXPH] = sPhw[threadIdx.x / 64];
     GfDevClock *queue = tab[0].ck;
@@ -189,26 +192,31 @@ __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restric
                 __hip_atomic_fetch_or(&tab[m].ck->q_timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return;
         }
-        const int checked = (int)(phase / 2u), pass = checked + 1, last = therm_last_pass(checked, npass, open_after);
-        if (last >= 0) {
-            if (phase != 2u * (unsigned)last) return;  // (settled)
+        // passes up to `checked` are checked
+        const int checked = (int)(phase / 2u), pass = checked + 1;
+        if (pass == npass || (checked > 0 && !any_open(checked))) {
+            if (phase % 2u != 0u) return;  // (settled)
             for (int m = 0; m < map.nm; m++) {
-                if (flag(m, 0) == 0u) continue;
-                int proven = -1;
-                for (int k = npass - 1; k >= 0; k--)
-                    if (flag(m, k) == 0u) proven = k;
-                if (tid == 0) therm_outcome(tab[m].ck, proven);
-                therm_settle(tab[m].P, bthermal(tab[m]), bslots(tab[m]), proven < 0 ? npass - 1 : proven, tid, nthr);
+                GfDevClock *ck = tab[m].ck;
+                const int last = __hip_atomic_load(&ck->th_last, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const bool open = is_open(ck, checked);
+                if (!open && last == 0) continue;
+                if (tid == 0) therm_outcome(ck, open ? -1 : last);
+                therm_settle(tab[m].P, bthermal(tab[m]), bslots(tab[m]), last, tid, nthr);
             }
         } else if (phase % 2u == 0u) {
+            if (unit % units == 0u)
+                for (int m = threadIdx.x; m < map.nm; m += 256)
+                    __hip_atomic_store(flag(tab[m].ck, pass + 1), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             for (int g = (int)(tid / 64); g < total; g += (int)(nthr / 64)) {
                 const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_TILE][g]));
-                if (__hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
-                    continue;
+                if (!is_open(b.ck, pass - 1)) continue;
                 const GfDevArrays A = bthermal(b);
                 therm_phase_table(b.P, sPh);
                 const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, arp, pass};
                 const int t = g - (int)b.pt;
+                if (t == 0 && threadIdx.x % 64 == 0)
+                    __hip_atomic_store(&b.ck->th_last, pass, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 therm_strip<DIS, 1>(b.P, b.ck, A, b.tg, t, it, bslots(b), A.tbord + (long)t * TS_NB(b.tg.w),
                                     b.ck->dt, sPh);
             }
@@ -216,8 +224,7 @@ __global__ void __launch_bounds__(256) kb_therm_rest(const BatchEntry *__restric
             for (long g = tid - threadIdx.x; g < border; g += nthr) {
                 const BatchEntry &b = bentry(tab, __builtin_amdgcn_readfirstlane(map.chunk[BK_BORD][g / BATCH_ALIGN]));
                 const long t = g + threadIdx.x - b.pb;
-                if (t < b.cb &&
-                    __hip_atomic_load(&b.ck->therm_pass_changed[pass - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)
+                if (t < b.cb && is_open(b.ck, pass - 1))
                     therm_check_one(b.P, b.ck, bthermal(b), b.tg, t, pass, arp, bslots(b));
             }
         }

@@ -54,7 +54,7 @@ struct GfDevParams {
 };
 
 // Time-stepping scalars and reduction cells kept on the device.
-#define GF_MAX_SWEEPS 32
+#define GF_THERM_FLAGS 4  // flags of a thermal call's passes, used in turn (a power of two)
 // phase-ratio planes kept per element: the phases present anywhere, in increasing id
 #define GF_MAXACT 8
 struct GfDevClock {
@@ -65,7 +65,7 @@ struct GfDevClock {
     unsigned long long therm_unconverged, therm_extra_passes, therm_mismatch, therm_mismatch_ulp;
     // flags of a thermal call's passes: bit 0: a border differs from its owner; bit 1: a
     // strip (tile) did not settle.  Two sets, used in turn (ThermSlots)
-    unsigned int therm_pass_changed[2 * GF_MAX_SWEEPS];
+    unsigned int therm_pass_changed[2 * GF_THERM_FLAGS];
     double dt_move;             // dt of the last element move (its stress rotation may still be pending)
     // change_phase (src/change_phase.f90:1-260) on the device
     unsigned int ph_newmask;    // phases (bit id-1) that markers turned into in the current call
@@ -85,6 +85,7 @@ struct GfDevClock {
     // a batch's thermal calls: their number modulo 3, and how many before this one left
     // their boundary values (0..2, counted one ahead)
     int th_call, th_hist;
+    int th_last, th_pad;  // ... and the last pass of the call under way
     // itest_mesh's smallest triangle angle, as an order-preserving key (rem_angle_key)
     unsigned long long rem_key;
     unsigned int out_cnt, out_pad;  // workgroups of a launch that ends with clock_out and are done

@@ -124,7 +124,7 @@ GF_DEV void clock_op(GfDevClock *ck, int op)
 {
     if (op & CK_TIME_ADVANCE) ck->time = ck->time + ck->dt;
     if (op & CK_THERM_BEGIN)
-        for (int k = 0; k < 2 * GF_MAX_SWEEPS; k++) ck->therm_pass_changed[k] = 0u;
+        for (int k = 0; k < 2 * GF_THERM_FLAGS; k++) ck->therm_pass_changed[k] = 0u;
     if (op & CK_DTAVG_ADD) ck->dtavg = ck->dtavg + ck->dt;
     if (op & CK_DTAVG_RESET) ck->dtavg = 0.0;
     if (op & CK_DT_BEGIN) {

@@ -92,13 +92,11 @@ struct gf_ctx {
     // before it forms the areas it needs from the coordinates)
     bool area_pending = false;
     unsigned therm_grid = 8;  // workgroups of the pipelined thermal kernel: the CUs, a multiple of 8
-    // TH_MAXPASS: the thermal result is proven to be the reference's serial one (fallback
-    // passes when needed); 1: FP32-arithmetic mode takes the single tile pass as it is
+    // TH_MAXPASS: the thermal result is proven to be the reference's serial one, by as many
+    // passes as that takes; less: by so many at most.  1: FP32-arithmetic mode takes the
+    // single tile pass as it is
     int therm_passes = TH_MAXPASS;
     bool therm_proof = true;  // false: FP32-arithmetic mode, the single pass is not proven
-    // the thermal step's further passes as one launch (k_therm_rest) instead of a launch
-    // per pass and check (GF_THERM=multi)
-    bool therm_rest = false;
     int therm_w = 0;     // output columns of a thermal strip
     bool therm_cols = false;  // pass 0 by a workgroup a strip (k_therm_cols)
     int therm_call = 0;  // thermal calls, modulo 3: the slot of a.tpre this call writes
@@ -331,8 +329,6 @@ extern "C" int gf_create(const gf_params *p, int32_t precision, gf_ctx **out)
             goto fail;
         }
         ctx->therm_grid = (unsigned)std::max(8, ncu / 8 * 8);
-        const char *tm = getenv("GF_THERM");
-        ctx->therm_rest = !(tm && strcmp(tm, "multi") == 0);
         // a workgroup a strip where every strip then has a CU of its own
         const ThermGeo gc = therm_geo(p->nz, p->nx, TC_W - 1 - TC_HI);
         ctx->therm_cols = gc.nr * gc.ns <= ncu;
@@ -1241,10 +1237,10 @@ static int enq_therm(gf_ctx *ctx, int clock_ops = 0, bool defer = false)
     } else {
         auto kern = ex ? (dis ? k_therm_strip<true, 2> : k_therm_strip<false, 2>)
                        : (dis ? k_therm_strip<true, 0> : k_therm_strip<false, 0>);
-        LAUNCH_DIM("k_therm_strip", kern, grid, 64, ctx->dp, ctx->dck, ctx->a, g, 0, arp, ctx->chk.sl, ops);
+        LAUNCH_DIM("k_therm_strip", kern, grid, 64, ctx->dp, ctx->dck, ctx->a, g, arp, ctx->chk.sl, ops);
     }
     if (defer) return GF_OK;
-    LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, g, 0, arp, ctx->chk.sl, nb);
+    LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, g, arp, ctx->chk.sl, nb);
     return enq_therm_rest(ctx);
 }
 
@@ -1254,26 +1250,14 @@ static int enq_therm_rest(gf_ctx *ctx, bool with_node)
 {
     if (ctx->therm_proof) {
         const bool dis = ctx->p.ishearh == 1 && ctx->p.itherm != 2;
-        const int npass = ctx->therm_passes, arp = ctx->chk.arp;
         const ThermGeo g = ctx->chk.g;
-        const ThermSlots sl = ctx->chk.sl;
-        if (ctx->therm_rest) {
-            // At most one workgroup per CU, fewer where there are fewer strips than waves.
-            ctx->rest = ThermRest{(int)std::min<long>(ctx->therm_grid, ((long)g.nr * g.ns + 31) / 32 * 8), arp, npass, g, sl};
-            if (!with_node) {
-                auto rest = dis ? k_therm_rest<true> : k_therm_rest<false>;
-                LAUNCH_DIM("k_therm_rest", rest, ctx->rest.grid, 256, ctx->dp, ctx->dck, ctx->a, ctx->rest);
-                ctx->rest.grid = 0;
-            }
-        } else {
-            const unsigned grid = 8u * (unsigned)((g.nr * g.ns + 7) / 8);
-            const long nb = (long)g.nr * g.ns * TS_NB(g.w);
-            auto extra = dis ? k_therm_strip<true, 1> : k_therm_strip<false, 1>;
-            for (int pass = 1; pass < npass; pass++) {
-                LAUNCH_DIM("k_therm_strip_extra", extra, grid, 64, ctx->dp, ctx->dck, ctx->a, g, pass, arp, sl, ClockOps{});
-                LAUNCH(k_therm_check, nb, ctx->dp, ctx->dck, ctx->a, g, pass, arp, sl, nb);
-            }
-            LAUNCH_DIM("k_therm_last", k_therm_last, ctx->therm_grid, 256, ctx->dp, ctx->dck, ctx->a, sl, npass);
+        const int npass = ctx->therm_passes < TH_MAXPASS ? ctx->therm_passes : therm_pass_limit(g);
+        // at most one workgroup per CU, fewer where there are fewer strips than waves
+        ctx->rest = ThermRest{(int)std::min<long>(ctx->therm_grid, ((long)g.nr * g.ns + 31) / 32 * 8), ctx->chk.arp, npass, g, ctx->chk.sl};
+        if (!with_node) {
+            auto rest = dis ? k_therm_rest<true> : k_therm_rest<false>;
+            LAUNCH_DIM("k_therm_rest", rest, ctx->rest.grid, 256, ctx->dp, ctx->dck, ctx->a, ctx->rest);
+            ctx->rest.grid = 0;
         }
         ctx->therm_call = (ctx->therm_call + 1) % 3;
         ctx->therm_set ^= 1;
@@ -1626,7 +1610,7 @@ static int enq_flac(gf_ctx *ctx, int pending = 0, bool last = true)
         // cells, 35.7 -> 34.1 at 60x20.  Where they are not, the
         // registers of the further passes cost fl_node waves: 0.6 us more at 901x301, 1 us at
         // 1200x500 with FP32 storage (3 us less at 2000x1000).
-        const bool with_node = ctx->therm_rest && !ctx->node_direct && ctx->p.movegrid != 0 && ctx->in_batch == 0 &&
+        const bool with_node = !ctx->node_direct && ctx->p.movegrid != 0 && ctx->in_batch == 0 &&
                                (ctx->p.nyhydro <= 0 || ctx->p.itemp_bc == 1) &&
                                !(ctx->p.nystressbc == 1 && ctx->p.nydrsides == 1) && node_tiles(ctx) <= 3L * ctx->therm_grid;
         if (defer && (rc = enq_therm_rest(ctx, with_node))) return rc;
@@ -2440,6 +2424,7 @@ struct gf_batch {
     bool fold = true;     // FP32-arithmetic mode: the tiles apply the boundary conditions
     unsigned therm_grid = 8;  // workgroups of the thermal kernels with one per CU
     unsigned rest_grid = 8;   // ... of kb_therm_rest: fewer where there are fewer strips than waves
+    int pass_limit = 1;       // ... and its most passes
     BatchMap map{};
     int nm = 0;
     long tot_e = 0, tot_n = 0, tot_t = 0, tot_b = 0, tot_m = 0;
@@ -2546,6 +2531,7 @@ extern "C" int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out)
         const long nmk = c->markers_uploaded ? c->a.nmarkers : 0;
         tab[k] = BatchEntry{c->dp, c->dck, c->a, nullptr, nullptr, tg, &c->hout->ck, pe, pn, pt, pb, pm, c->ne, c->nn, ntiles, nbord, nmk};
         b->fold = b->fold && q.itemp_bc != 2;
+        b->pass_limit = std::max(b->pass_limit, therm_pass_limit(tg));
         if (nmk > 0) b->markers = true;
         mm.insert(mm.end(), align(nmk) / BATCH_ALIGN, k);
         pm += align(nmk);
@@ -2646,7 +2632,7 @@ static int enq_batch_flac(gf_batch *b)
             b->movegrid && !b->no_mech ? 1 : 0);
     b->pend_ops = 0;
     const bool dis = p.ishearh == 1 && p.itherm != 2;
-    const int npass = b->m[0]->therm_passes, arp = b->area_pending ? 1 : 0;
+    const int npass = b->m[0]->therm_passes < TH_MAXPASS ? b->m[0]->therm_passes : b->pass_limit, arp = b->area_pending ? 1 : 0;
     unsigned chk = 0;  // workgroups of kb_rheol's launch that check the thermal borders
     if (!b->m[0]->therm_proof) {
         BLAUNCH((dis ? kb_therm_pipe<true> : kb_therm_pipe<false>), b->therm_grid, TH_J * TH_I, b->dtab, map, b->tot_t,

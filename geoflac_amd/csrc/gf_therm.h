@@ -46,20 +46,21 @@ struct ThermSlots {
     int cur, prev, prev2, hist;
     int flag;  // first flag of the call's passes; the other set's are cleared by pass 0
     GF_DEVM int of(int pass) const { return pass & 1 ? GF_NPRE - 1 : cur; }
+    GF_DEVM int flag_of(int pass) const { return flag + pass % GF_THERM_FLAGS; }
 };
 // consecutive calls number `call` turn three slots over; an odd pass uses the fourth
 __host__ __device__ inline ThermSlots therm_slots(int call, int hist, int set = 0)
 {
     const int c = call % 3;
-    return ThermSlots{c, (c + 2) % 3, (c + 1) % 3, hist, set ? GF_MAX_SWEEPS : 0};
+    return ThermSlots{c, (c + 2) % 3, (c + 1) % 3, hist, set ? GF_THERM_FLAGS : 0};
 }
 // the flags of the next call (those of the one before this, whose passes are over), and the
 // counters of this call's further passes
 GF_DEV void therm_clear_other(GfDevClock *ck, const ThermSlots &sl)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) ck->q_next = ck->q_done = 0u;
-    if (blockIdx.x == 0 && threadIdx.x < GF_MAX_SWEEPS)
-        ck->therm_pass_changed[(sl.flag ^ GF_MAX_SWEEPS) + threadIdx.x] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x < GF_THERM_FLAGS)
+        ck->therm_pass_changed[(sl.flag ^ GF_THERM_FLAGS) + threadIdx.x] = 0u;
 }
 GF_DEV double *therm_pre(const GfDevParams *P, const GfDevArrays &A, int slot)
 {
@@ -472,7 +473,7 @@ GF_DEV void therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, const
         ydn0 = ydn1;
         tdn0 = tdn1;
     }
-    if (!still && w.lane == 0) atomicOr(&ck->therm_pass_changed[sl.flag + it.pass], 2u);
+    if (!still && w.lane == 0) atomicOr(&ck->therm_pass_changed[sl.flag_of(it.pass)], 2u);
 }
 
 // One strip by one workgroup, a wave a column, for meshes of so few strips that each has a
@@ -589,7 +590,7 @@ GF_DEV void therm_cols(const GfDevParams *__restrict__ P, GfDevClock *ck, const 
         }
     }
     if (in) w.store(i, x, n0.y, phs);
-    if (!still && threadIdx.x == 0) atomicOr(&ck->therm_pass_changed[sl.flag + it.pass], 2u);
+    if (!still && threadIdx.x == 0) atomicOr(&ck->therm_pass_changed[sl.flag_of(it.pass)], 2u);
 }
 
 // by the lanes of one wave, for that wave
@@ -608,21 +609,20 @@ GF_DEV void therm_phase_table(const GfDevParams *__restrict__ P, double (*sPh)[G
     __builtin_amdgcn_wave_barrier();
 }
 
-// pass 0 (mode 0 or 2) or, with launches per phase, a fallback pass: one wave a strip
+// pass 0 (mode 0 or 2), one wave a strip
 template <bool DIS, int MODE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
-k_therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, ThermGeo g, int pass, int arp,
-              ThermSlots sl, ClockOps ops)
+k_therm_strip(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, ThermGeo g, int arp, ThermSlots sl,
+              ClockOps ops)
 {
-    if (pass == 0) therm_clear_other(ck, sl);
+    therm_clear_other(ck, sl);
     if (blockIdx.x == 0 && threadIdx.x == 0) clock_op(ck, ops);  // (fields nothing here reads)
     __shared__ double sPh[4][GF_MAXPH];
-    if (pass > 0 && ck->therm_pass_changed[sl.flag + pass - 1] == 0u) return;  // already proven
     const int nt = g.nr * g.ns, q = (nt + 7) / 8;  // XCD x runs strips [x q, (x+1) q)
     const int t = (int)(blockIdx.x % 8) * q + (int)(blockIdx.x / 8);
     if ((int)(blockIdx.x / 8) >= q || t >= nt) return;
     therm_phase_table(P, sPh);
-    const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, arp, pass};
+    const ThermIter it{A.xb, A.xa, arp, 0};
     therm_strip<DIS, MODE>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(g.w), ck->dt, sPh);
 }
 // pass 0, one workgroup a strip
@@ -640,6 +640,12 @@ k_therm_cols(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A, T
     therm_cols<DIS, MODE>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(g.w), L);
 }
 
+// the same bits; not-a-numbers count as the same (which of them a diverged model holds is no
+// matter, and no reason for further passes)
+GF_DEV bool therm_same(double a, double b)
+{
+    return __double_as_longlong(a) == __double_as_longlong(b) || (a != a && b != b);
+}
 // Compares border value t of the strips with the value its owner wrote.  A node whose
 // values differ is harmless when every output node of this strip that reads it still
 // satisfies x = F(x) with the global values: those (at most three) are evaluated again
@@ -679,8 +685,9 @@ GF_DEV void therm_check_one(const GfDevParams *__restrict__ P, GfDevClock *ck, c
         if (ii == nx) return pre[2 * nx + nz + jj - 1];
         return x[IN(jj, ii)];
     };
-    const long long a = __double_as_longlong(A.tbord[t]), b = __double_as_longlong(X(j, i));
-    if (a == b) return;
+    const double xb = A.tbord[t], xo = X(j, i);
+    if (therm_same(xb, xo)) return;
+    const long long a = __double_as_longlong(xb), b = __double_as_longlong(xo);
     const int dj[3] = {1, 0, -1}, di[3] = {0, 1, 1};  // read as up, left, left-down
     const double dt = ck->dt;
     auto T = [&](int jj, int ii) { return A.temp[IN(jj, ii)]; };  // the old temperature
@@ -695,19 +702,18 @@ GF_DEV void therm_check_one(const GfDevParams *__restrict__ P, GfDevClock *ck, c
         const double xl = mi > 1 ? X(mj, mi - 1) : 0.0;
         const double xd = (mi > 1 && mj < nz) ? X(mj + 1, mi - 1) : 0.0;
         const double f = therm_eval(c, xu, xl, xd, dt);
-        bad |= __double_as_longlong(f) != __double_as_longlong(X(mj, mi));
+        bad |= !therm_same(f, X(mj, mi));
     }
     atomicAdd(&ck->therm_mismatch, 1ull);  // (statistics)
     atomicMax(&ck->therm_mismatch_ulp, (unsigned long long)(a > b ? a - b : b - a));
-    if (bad) atomicOr(&ck->therm_pass_changed[sl.flag + pass], 1u);
+    if (bad) atomicOr(&ck->therm_pass_changed[sl.flag_of(pass)], 1u);
 }
 
 __global__ void __launch_bounds__(256) k_therm_check(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                    ThermGeo g, int pass, int arp, ThermSlots sl, long total)
+                                                    ThermGeo g, int arp, ThermSlots sl, long total)
 {
-    if (pass > 0 && ck->therm_pass_changed[sl.flag + pass - 1] == 0u) return;  // that pass did not run
     const long t = (long)blockIdx.x * 256 + threadIdx.x;
-    if (t < total) therm_check_one(P, ck, A, g, t, pass, arp, sl);
+    if (t < total) therm_check_one(P, ck, A, g, t, 0, arp, sl);
 }
 // The check of pass 0 as the first `grid` workgroups of a launch that neither reads the
 // temperature nor writes what the check reads (grid 0: none; a multiple of 8, so that the
@@ -749,27 +755,24 @@ GF_DEV void therm_settle(const GfDevParams *__restrict__ P, const GfDevArrays &A
 // The rest of the call after pass 0 and its check, in one launch.  When pass 0 is proven it
 // returns at once.  Otherwise the further passes run here in phases of R.grid units each
 // (queue_take): phase 2 (p - 1) runs the strips of pass p, phase 2 p - 1 checks its borders,
-// and the phase after the pass that ends the call settles its result.  The flags that decide
-// another pass are read with coherent loads once the phases before are done, so every unit
-// takes the same decision; flag 0 was written by earlier launches.  No workgroup needs the
-// others resident, so that models and batches may run their passes at the same time, on
-// streams of their own; grid barriers after each phase did, and were slower: 12 models of
-// 200-360 x 34-60 cells in a batch, a further pass in nearly every step, 241 us a step to
-// 203.
+// and the phase after the pass that ends the call settles its result.  The flag that decides
+// another pass is read with coherent loads once the phases before are done, so every unit
+// takes the same decision (strips of pass p clear the one of pass p + 1); flag 0 was written
+// by earlier launches.  No workgroup needs the others resident, so that models and batches
+// may run their passes at the same time, on streams of their own; grid barriers after each
+// phase did, and were slower: 12 models of 200-360 x 34-60 cells in a batch, a further pass
+// in nearly every step, 241 us a step to 203.
+//
+// As many passes as the proof takes (therm_pass_limit), two at most in nearly every call.
+// In a start that is the same in every column, though, some row's sum may lie so near a
+// rounding tie that the last bit of a value hangs on the value to its left all along the
+// row: the serial order's bit then moves on by a strip, or its halo, a pass.
+__host__ __device__ inline int therm_pass_limit(const ThermGeo &g) { return g.nx + 4; }  // (some 3 columns a pass or more)
 struct ThermRest {
     int grid, arp, npass;
     ThermGeo g;
     ThermSlots sl;
 };
-// the pass that ends the call, of passes 1 .. checked: the first that is proven, or the last
-// there may be; -1: another follows
-template <typename Open>
-GF_DEV int therm_last_pass(int checked, int npass, const Open &open_after)
-{
-    for (int k = 1; k <= checked; k++)
-        if (!open_after(k)) return k;
-    return checked == npass - 1 ? checked : -1;
-}
 template <bool DIS>
 GF_DEV void therm_rest_body(const GfDevParams *__restrict__ P, GfDevClock *ck, const GfDevArrays &A, const ThermRest &R)
 {
@@ -780,10 +783,6 @@ GF_DEV void therm_rest_body(const GfDevParams *__restrict__ P, GfDevClock *ck, c
     __shared__ double sPhw[4][4][GF_MAXPH];  // (a table a wave)
     double(*sPh)[GF_MAXPH] = sPhw[threadIdx.x / 64];
     therm_phase_table(P, sPh);
-    auto open_after = [&](int pass) {
-        return __hip_atomic_load(&ck->therm_pass_changed[sl.flag + pass], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
-               0u;
-    };
     const int nt = g.nr * g.ns;
     const long nb = (long)nt * TS_NB(g.w);
     const unsigned units = (unsigned)R.grid;
@@ -796,12 +795,18 @@ GF_DEV void therm_rest_body(const GfDevParams *__restrict__ P, GfDevClock *ck, c
             if (threadIdx.x == 0) __hip_atomic_fetch_or(&ck->q_timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return;
         }
-        const int checked = (int)(phase / 2u), pass = checked + 1, last = therm_last_pass(checked, npass, open_after);
-        if (last >= 0) {
-            if (phase != 2u * (unsigned)last) return;  // (settled)
-            if (tid == 0) therm_outcome(ck, open_after(last) || last == 0 ? -1 : last);
-            therm_settle(P, A, sl, last, tid, nthr);
+        // passes up to `checked` are checked
+        const int checked = (int)(phase / 2u), pass = checked + 1;
+        const bool open = __hip_atomic_load(&ck->therm_pass_changed[sl.flag_of(checked)], __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT) != 0u;
+        if ((checked > 0 && !open) || pass == npass) {
+            if (phase % 2u != 0u) return;  // (settled)
+            if (tid == 0) therm_outcome(ck, checked > 0 && !open ? checked : -1);
+            therm_settle(P, A, sl, checked, tid, nthr);
         } else if (phase % 2u == 0u) {
+            if (tid == 0)
+                __hip_atomic_store(&ck->therm_pass_changed[sl.flag_of(pass + 1)], 0u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
             const ThermIter it{pass % 2 == 1 ? A.xa : A.xb, pass % 2 == 0 ? A.xa : A.xb, R.arp, pass};
             for (int t = (int)(tid / 64); t < nt; t += (int)(nthr / 64))
                 therm_strip<DIS, 1>(P, ck, A, g, t, it, sl, A.tbord + (long)t * TS_NB(g.w), ck->dt, sPh);
@@ -816,18 +821,6 @@ __global__ void __launch_bounds__(256) k_therm_rest(const GfDevParams *__restric
                                                     ThermRest R)
 {
     therm_rest_body<DIS>(P, ck, A, R);
-}
-
-// the end of a call whose further passes ran as launches of their own
-__global__ void __launch_bounds__(256) k_therm_last(const GfDevParams *__restrict__ P, GfDevClock *ck, GfDevArrays A,
-                                                    ThermSlots sl, int npass)
-{
-    int proven = -1;
-    for (int k = npass - 1; k >= 0; k--)
-        if (ck->therm_pass_changed[sl.flag + k] == 0u) proven = k;
-    const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x, nthr = (long)gridDim.x * blockDim.x;
-    if (tid == 0) therm_outcome(ck, proven);
-    therm_settle(P, A, sl, proven < 0 ? npass - 1 : proven, tid, nthr);
 }
 
 // While a batch's table holds the context's array pointers the result is copied to temp

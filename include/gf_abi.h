@@ -242,16 +242,17 @@ int gf_init_visc(gf_ctx *ctx);                   /* src/init_visc.f90:1-18  */
  * counterpart).  stats[0]: thermal calls whose fixed-point iteration was not proven
  * equal to the reference's in-place serial order (the result is bitwise the serial
  * one whenever this stays 0); stats[1]: fixed-point passes beyond the first that the
- * proofs needed; stats[2]: tile border values that differed from their owner's;
+ * proofs needed; stats[2]: border values of strips that differed from their owner's;
  * stats[3]: the largest such difference in units in the last place. */
 int gf_therm_stats(gf_ctx *ctx, int64_t stats[4]);
 
-/* Most fixed-point passes of the thermal step per call (1..4; default 4).  The FP64
- * thermal step reproduces the reference's in-place serial sweep (src/fl_therm.f90:
- * 393-571) by a tiled fixed-point iteration whose result a border check proves equal
- * to the serial one; when no pass within the limit is proven, the step goes on with
- * the last pass and the call returns GF_ERR_THERM_SWEEPS.  No reference counterpart
- * (a limit for tests and callers that prefer an error to a fallback pass). */
+/* Most fixed-point passes of the thermal step per call: 1, 2 or 3, or 4 (the default)
+ * for as many as the proof takes.  The FP64 thermal step reproduces the reference's
+ * in-place serial sweep (src/fl_therm.f90:393-571) by a fixed-point iteration over strips
+ * whose result a border check proves equal to the serial one; when no pass within the
+ * limit is proven, the step goes on with the last pass and the call returns
+ * GF_ERR_THERM_SWEEPS.  No reference counterpart (a limit for tests and callers that
+ * prefer an error to a further pass). */
 int gf_set_therm_passes(gf_ctx *ctx, int32_t npass);
 
 /* Synchronise the context's stream (all queued steps finished). */

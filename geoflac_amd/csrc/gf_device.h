@@ -12,6 +12,7 @@
 
 #include "../../include/gf_abi.h"
 #include "gf_ddmath.h"
+#include "gf_rcp.h"
 
 #define GF_DEV static __device__ __forceinline__
 #define GF_DEVM __device__ __forceinline__  // (members)

@@ -182,7 +182,8 @@ GF_DEV bool last_block(GfDevClock *ck)
 }
 
 // correctly rounded math of the FP64 path, evaluated for a list of arguments
-// (fn: 0 sin, 1 tan, 2 exp, 3 pow with y = args2)
+// (fn: 0 sin, 1 tan, 2 exp, 3 pow with y = args2, 4 the thermal strips' 1 / x, 5 their
+// 1 / (1 / x))
 __global__ void k_math_check(const double *x, const double *y, double *out, long n, int fn)
 {
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -192,6 +193,10 @@ __global__ void k_math_check(const double *x, const double *y, double *out, long
     if (fn == 1) v = cr_tan(x[t]);
     if (fn == 2) v = cr_exp(x[t]);
     if (fn == 3) v = cr_pow(x[t], y[t]);
+    if (fn >= 4) {
+        const double d = x[t], a = rcp_safe(d) ? rcp_core(d) : 1.0 / d;
+        v = fn == 4 ? a : rcp_safe(a) ? rcp_back(a, d) : 1.0 / a;
+    }
     out[t] = v;
 }
 

@@ -2020,7 +2020,7 @@ extern "C" int gf_kernel_time(gf_ctx *ctx, const char *name, double *total_ms, i
 extern "C" int gf_math_check(int32_t fn, const double *x, const double *y, double *out, int64_t n)
 {
     gf_ctx *ctx = nullptr;
-    if (!x || !out || n <= 0 || fn < 0 || fn > 3 || (fn == 3 && !y)) return GF_ERR_ARG;
+    if (!x || !out || n <= 0 || fn < 0 || fn > 5 || (fn == 3 && !y)) return GF_ERR_ARG;
     double *dx = nullptr, *dy = nullptr, *dout = nullptr;
     int rc = GF_OK;
     if (hipMalloc((void **)&dx, 8 * n) != hipSuccess || hipMalloc((void **)&dy, 8 * n) != hipSuccess ||

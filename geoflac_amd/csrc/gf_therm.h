@@ -145,27 +145,6 @@ GF_DEV ThermTri therm_tri(const double d[6], double inv, double dm, double hdf)
     return t;
 }
 
-// 1 / d, correctly rounded for an operand that rcp_safe accepts: two Newton steps from
-// the hardware's estimate and a last step from the exact remainder (the steps of an IEEE
-// division without the scaling that keeps extreme exponents in range)
-GF_DEV double rcp_core(double d)
-{
-    double y = __builtin_amdgcn_rcp(d);
-    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
-    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
-    return __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
-}
-// |d| in [2^-400, 2^400], and a significand that is not all ones (the operands for which
-// the last step need not round correctly: Markstein's exception)
-GF_DEV bool rcp_safe(double d)
-{
-    const unsigned h = (unsigned)__double2hiint(d), e = (h >> 20) & 0x7ffu;
-    return e - (1023u - 400u) <= 800u && ((h | 0xfff00000u) & (unsigned)__double2loint(d)) != 0xffffffffu;
-}
-// 1 / a where a = RN(1 / d), correctly rounded where rcp_safe(a): the remainder 1 - a d is
-// exact and d is within one ulp of 1 / a, so one step from d does
-GF_DEV double rcp_back(double a, double d) { return __builtin_fma(__builtin_fma(-a, d, 1.0), d, d); }
-
 struct ThermIter {
     const double *xin;  // starting iterate of a pass > 0
     double *xout;

@@ -298,7 +298,8 @@ class Model:
 
 
 def math_check(fn, x, y=None):
-    """Device values of the correctly rounded sin (0), tan (1), exp (2), pow (3)."""
+    """Device values of the correctly rounded sin (0), tan (1), exp (2), pow (3), 1 / x (4)
+    and 1 / (1 / x) (5)."""
     import numpy as np
     x = np.ascontiguousarray(x, dtype=np.float64)
     out = np.empty_like(x)

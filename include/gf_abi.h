@@ -269,7 +269,8 @@ int gf_set_timing(gf_ctx *ctx, int32_t on);
 int gf_stream_probe(int64_t bytes, int32_t reps, double *ms_per_launch);
 /* Evaluates on the device, for n host arguments, the correctly rounded functions the
  * FP64 path uses in place of libm (fn: 0 sin, 1 tan, 2 exp, 3 pow(x, y)), so a test
- * can compare them with the host libm the reference calls.  No reference counterpart. */
+ * can compare them with the host libm the reference calls, and the reciprocals of the
+ * thermal step (4: 1 / x, 5: 1 / (1 / x)).  No reference counterpart. */
 int gf_math_check(int32_t fn, const double *x, const double *y, double *out, int64_t n);
 int gf_kernel_time(gf_ctx *ctx, const char *name, double *total_ms, int64_t *launches);
 

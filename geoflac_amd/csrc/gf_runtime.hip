@@ -2041,7 +2041,7 @@ extern "C" int gf_math_check(int32_t fn, const double *x, const double *y, doubl
 }
 
 // ------------------------------------------------------------------ viscosity surrogate
-#define MLP_GRAD_BLOCKS 256  // most workgroups of a gradient launch (one 64-sample tile each or more)
+#define MLP_GRAD_BLOCKS 256  // most workgroups of a gradient launch (a wave takes a tile of MG_TS samples, or more)
 
 extern "C" int gf_surrogate_sample(gf_ctx *ctx, int64_t capacity, int64_t *count)
 {
@@ -2436,7 +2436,7 @@ struct gf_batch {
     hipStream_t stream = nullptr;
     int32_t nloop = 0, nsrate = 0;
     int pend_ops = 0;       // clock updates left to the next launch that makes them
-    int bs[3] = {256, 256, 256};  // threads per workgroup of the rheology and node kernels (the third is unused)
+    int bs[2] = {256, 256};  // threads per workgroup of the rheology and node kernels
     bool use_graph = false;
     // the batch's last element move left its rotation, its areas and dvol to the next
     // kb_rheol (the kernels between form what they read of them)
@@ -2446,7 +2446,7 @@ struct gf_batch {
     // optional per-kernel timing (autotuner)
     bool timing = false;
     hipEvent_t ev[2] = {nullptr, nullptr};
-    double t_ms[3] = {0, 0, 0};
+    double t_ms[2] = {0, 0};
     char msg[256] = {0};
 };
 
@@ -2875,18 +2875,19 @@ extern "C" int gf_batch_step(gf_batch *b, int32_t nsteps)
     return first;
 }
 
-// Picks the workgroup size of the three heaviest kernels from {64, 128, 256} by timing
-// `steps` real steps per candidate (the models advance by 3 * steps).
+// Picks the workgroup sizes of the rheology and node kernels from {64, 128, 256} by timing
+// `steps` real steps per candidate (the models advance by 3 * steps; a border check in the
+// rheology kernel's launch is timed with it).
 extern "C" int gf_batch_autotune(gf_batch *b, int32_t steps, int32_t chosen[3])
 {
     if (!b || steps < 1) return GF_ERR_ARG;
     if (int frc = batch_flush(b)) return frc;
     if (int prc = batch_pointers(b)) return prc;
     const int cand[3] = {64, 128, 256};
-    double best[3] = {1e30, 1e30, 1e30};
-    int pick[3] = {256, 256, 256};
+    double best[2] = {1e30, 1e30};
+    int pick[2] = {256, 256};
     for (int c = 0; c < 3; c++) {
-        for (int q = 0; q < 3; q++) {
+        for (int q = 0; q < 2; q++) {
             b->bs[q] = cand[c];
             b->t_ms[q] = 0.0;
         }
@@ -2895,7 +2896,7 @@ extern "C" int gf_batch_autotune(gf_batch *b, int32_t steps, int32_t chosen[3])
         for (int k = 0; k < steps && rc == GF_OK; k++) rc = enq_batch_step(b);
         b->timing = false;
         if (rc) return rc;
-        for (int q = 0; q < 3; q++)  // (a kernel that did not run in these steps keeps 256)
+        for (int q = 0; q < 2; q++)  // (a kernel that did not run in these steps keeps 256)
             if (b->t_ms[q] > 0.0 && b->t_ms[q] < best[q]) {
                 best[q] = b->t_ms[q];
                 pick[q] = cand[c];
@@ -2912,10 +2913,11 @@ extern "C" int gf_batch_autotune(gf_batch *b, int32_t steps, int32_t chosen[3])
         c->temp0_prev = b->temp0_prev;
         c->therm_clean = false;
     }
-    for (int q = 0; q < 3; q++) {
+    for (int q = 0; q < 2; q++) {
         b->bs[q] = pick[q];
         if (chosen) chosen[q] = pick[q];
     }
+    if (chosen) chosen[2] = 256;
     if (b->gexec) {  // captured with the old sizes
         BCHK(hipGraphExecDestroy(b->gexec));
         b->gexec = nullptr;

@@ -151,8 +151,8 @@ GF_DEV void clock_op(GfDevClock *ck, const ClockOps &o)
 
 // The clock goes to page-locked host memory from the call's last launch, so that the host
 // waits once and copies nothing: a call of gf_flac at 60x20 cells, with a tenth of an
-// itest_mesh, took 87 us with copies of pageable memory both ways and takes 58 (34 of them
-// in the kernels).
+// itest_mesh, took 87 us with copies of pageable memory both ways and takes 44 (some 33 of
+// them in the kernels).
 // (the threads of one workgroup; the values other workgroups of the launch wrote are read
 // past the caches)
 GF_DEV void clock_out(const GfDevClock *ck, GfDevClock *host)

@@ -144,8 +144,9 @@ static int set_err(gf_ctx *c, int code, const char *fmt, ...)
 // Output columns of the thermal strips of one or more meshes that a launch marches over.  A
 // strip of w columns takes some w + 6 column times (halo, ring, start); a column takes a
 // wave alone on its SIMD 1.3 us (latency), n waves 0.6 us more each, 0.9 us each where
-// issue bounds.  The width of least time over the 1024 SIMDs.  Measured, us a step (whole step) at widths 2, 4, 8, 16, 24: 401x101 nodes
-// 38, 41, 47, 59, 70; 902x302 101, 97, 102, 110, 121; 2001x1001 541, 508, 492, 493, 497.
+// issue bounds.  The width of least time over the 1024 SIMDs.  Measured, us a whole step at
+// widths 2, 4, 8, 16, 24: 601x151 nodes 48, 47, 53, 65, 77 (2 is chosen); 902x302 89, 85, 91,
+// 98, 110 (5: 87); 2001x1001 458, 429, 413, 411, 416 (17: 413).
 static int therm_strip_width(const std::vector<const gf_params *> &ps)
 {
     int best = 2;

@@ -328,7 +328,8 @@ int gf_mlp_grad_noalloc(const float *samples, int64_t n, const float *w, float *
  * The models are contexts created, bound and uploaded as usual, with the same
  * precision, switches, ifreq_* frequencies and loop counters; they stay owned by the
  * caller (destroy the batch first).  One launch per kernel of the step covers all of
- * them; each keeps its own parameters, clock and arrays. */
+ * them; each keeps its own parameters, clock and arrays.  Batches of different models may
+ * step at the same time, each from a thread of its own. */
 typedef struct gf_batch gf_batch;
 int gf_batch_create(gf_ctx *const *models, int32_t n, gf_batch **out);
 void gf_batch_destroy(gf_batch *b);
